@@ -94,6 +94,9 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   // Saved-P 16-bit tiles stream straight into two LDS buffers per operand
   // (TileDma): with kPar, two sets in distinct arrays with a compile-time role
   // per loop step (so that the current tile's LDS reads need not wait for the
@@ -101,19 +104,19 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   constexpr bool kDma = L::kSwizzle && (LOADP || D == 64);
   constexpr bool kPar = kDma && (D == 128 || !LOADP);
   constexpr bool kRt = kDma && !kPar;
-  constexpr int kE1 = kPar ? L::kRowElems : 8, kER = kRt ? L::kRowElems : 8;
-  __shared__ __align__(16) T sK0[kRt ? 8 : L::kRowElems];
-  __shared__ __align__(16) T sV0[kRt ? 8 : L::kRowElems];
-  __shared__ __align__(16) T sK1[kE1];
-  __shared__ __align__(16) T sV1[kE1];
-  __shared__ __align__(16) T sKr[kRt ? 2 : 1][kER];
-  __shared__ __align__(16) T sVr[kRt ? 2 : 1][kER];
-  auto set_k = [&](auto par) __attribute__((always_inline)) -> T* {
+  constexpr int kE1 = kPar ? M::kElems : 8, kER = kRt ? M::kElems : 8;
+  __shared__ __align__(16) lds sK0[kRt ? 8 : M::kElems];
+  __shared__ __align__(16) lds sV0[kRt ? 8 : M::kElems];
+  __shared__ __align__(16) lds sK1[kE1];
+  __shared__ __align__(16) lds sV1[kE1];
+  __shared__ __align__(16) lds sKr[kRt ? 2 : 1][kER];
+  __shared__ __align__(16) lds sVr[kRt ? 2 : 1][kER];
+  auto set_k = [&](auto par) __attribute__((always_inline)) -> lds* {
     if constexpr (std::is_same_v<decltype(par), RtBuf>) return sKr[par.cur];
     else if constexpr (decltype(par)::value == 0) return sK0;
     else return sK1;
   };
-  auto set_v = [&](auto par) __attribute__((always_inline)) -> T* {
+  auto set_v = [&](auto par) __attribute__((always_inline)) -> lds* {
     if constexpr (std::is_same_v<decltype(par), RtBuf>) return sVr[par.cur];
     else if constexpr (decltype(par)::value == 0) return sV0;
     else return sV1;
@@ -143,20 +146,23 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   const T* V = at<const T>(a.v, b, h);
   const T* dO = at<const T>(a.dout, b, h);
 
-  frag dof[D / 32], qf[D / 32];
+  frag dor[D / 32];
+  mfrag dof[D / 32], qf[D / 32];
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
-    dof[ks] = load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g);
-    if constexpr (!LOADP) qf[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
+    dor[ks] = load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g);
+    if constexpr (!LOADP) qf[ks] = M::from(load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g));
   }
   const int64_t ridx = (int64_t)bh * T_ + m;
   float Dm;
   if (a.rowsum_in) {
     Dm = row_ok ? a.rowsum_in[ridx] : 0.f;
   } else {
-    Dm = row_dot_do_o<T, D>(dof, at<const T>(a.o, b, h), a.o.st, m, T_);
+    Dm = row_dot_do_o<T, D>(dor, at<const T>(a.o, b, h), a.o.st, m, T_);
     if (a.rowsum_out && ch == 0 && row_ok && g == 0) a.rowsum_out[ridx] = Dm;
   }
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) dof[ks] = M::from(dor[ks]);
   const f32x4 mDm4 = f32x4{-Dm, -Dm, -Dm, -Dm};  // dP's MFMAs start from -D: they give dP - D
   const float lse2 = (!LOADP && row_ok) ? a.lse[ridx] * kLog2e : 0.f;
   const T* Pm = LOADP ? at<const T>(a.p, b, h) + (int64_t)(row_ok ? m : 0) * a.p.st : nullptr;
@@ -239,12 +245,12 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
       __syncthreads();  // everyone's, and everyone is done with the other set
     } else {
       __syncthreads();
-      stage_store_rows<T, D>(stK, sK0);
-      stage_store_rows<T, D>(stV, sV0);
+      stage_store_tile<M>(stK, sK0);
+      stage_store_tile<M>(stV, sV0);
       __syncthreads();
     }
-    const T* cK = set_k(par);
-    const T* cV = set_v(par);
+    const lds* cK = set_k(par);
+    const lds* cV = set_v(par);
     Tile p;
     if constexpr (LOADP) frags_to_tile<T>(p, pn);
     if constexpr (kDma) {
@@ -258,7 +264,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     }
     if constexpr (!LOADP) {
       p.zero();
-      mm_d<T, D>(p, cK, qf);
+      mm_d<M>(p, cK, qf);
       recompute_p_row<T, XM>(p, a, brow, n0, lse2, a.scale_log2);
     }
     if (mk.tile(nb)) {
@@ -271,16 +277,16 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     Tile dp;
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) dp.q[q4] = mDm4;
-    mm_d<T, D>(dp, cV, dof);  // dP - D
-    frag dsf[2];
+    mm_d<M>(dp, cV, dof);  // dP - D
+    mfrag dsf[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       float v[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[j] = p.at(kb, j) * dp.at(kb, j);
-      dsf[kb] = vals_frag<T>(v);
+      dsf[kb] = M::vals(v);
     }
-    mm_s<T, D>(acc, cK, dsf);
+    mm_s<M>(acc, cK, dsf);
   };
   if constexpr (kPar && D == 64) {
     // Pairs of tiles with unconditional prefetch; the last one or two peeled.
@@ -335,6 +341,9 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   typedef Lds<T, kBlk> LP;
   constexpr bool kNeedQ = !DV_ONLY || !LOADP;
   // Staged row statistics of the streamed tile: D (unless DV_ONLY), then lse
@@ -353,17 +362,18 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   // them, the compiler waits for the outstanding direct loads before one of
   // those transposed reads.
   constexpr bool kLateFetch = kDma && LOADP;
-  constexpr int kQE = kNeedQ ? L::kRowElems : 8, kPE = LOADP ? LP::kRowElems : 8, kSE = kNS > 0 ? kNS * kBlk : 4;
-  __shared__ __align__(16) T sdO0[L::kRowElems];
-  __shared__ __align__(16) T sQ0[kQE];
+  constexpr int kQE = kNeedQ ? M::kElems : 8, kPE = LOADP ? LP::kRowElems : 8, kSE = kNS > 0 ? kNS * kBlk : 4;
+  __shared__ __align__(16) lds sdO0[M::kElems];
+  __shared__ __align__(16) lds sQ0[kQE];
   __shared__ __align__(16) T sP0[kPE];
   __shared__ __align__(16) float sS0[kSE];
-  __shared__ __align__(16) T sdO1[kDma ? L::kRowElems : 8];
-  __shared__ __align__(16) T sQ1[kDma ? kQE : 8];
+  __shared__ __align__(16) lds sdO1[kDma ? M::kElems : 8];
+  __shared__ __align__(16) lds sQ1[kDma ? kQE : 8];
   __shared__ __align__(16) T sP1[kDma && !kMix ? kPE : 8];
   __shared__ __align__(16) float sS1[kDma ? kSE : 4];
   struct Bufs {
-    T *dout, *q, *p;
+    lds *dout, *q;
+    T* p;
     float* st;
   };
   auto bufs = [&](auto par) __attribute__((always_inline)) -> Bufs {
@@ -405,16 +415,16 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const float* rs = DV_ONLY ? nullptr : a.rowsum_in + (int64_t)bh * T_;
   const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * T_;
 
-  frag vf[D / 32], kf[D / 32];
+  mfrag vf[D / 32], kf[D / 32];
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
     // negated: dP's MFMAs start from the streamed rows' D and give D - dP;
     // kept as computed (left to itself the compiler redoes the negation per tile)
     if constexpr (!DV_ONLY) {
-      vf[ks] = scale_frag<T>(load_frag_row<T>(V, a.v.st, n, T_, 32 * ks + 8 * g), -1.f);
-      asm volatile("" : "+v"(vf[ks]));
+      vf[ks] = M::from(scale_frag<T>(load_frag_row<T>(V, a.v.st, n, T_, 32 * ks + 8 * g), -1.f));
+      M::keep(vf[ks]);
     }
-    if constexpr (!LOADP) kf[ks] = load_frag_row<T>(K, a.k.st, n, T_, 32 * ks + 8 * g);
+    if constexpr (!LOADP) kf[ks] = M::from(load_frag_row<T>(K, a.k.st, n, T_, 32 * ks + 8 * g));
   }
 
   f32x4 acc_dv[D / 16], acc_dk[D / 16];
@@ -453,23 +463,25 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   }
   const StatDma<kNS> sdma(DV_ONLY ? lse : rs, lse, nullptr, nullptr);
   auto dma_tile = [&](int mb, auto par) __attribute__((always_inline)) {
-    const int m0 = mb * kBlk;
-    const Bufs bf = bufs(par);
-    if (m0 + kBlk <= T_ && cols_full) {
-      dd.load_full(bf.dout, dOn, odO);
-      dd.load_full(bf.q, Qn, oQ);
-      if constexpr (LOADP && !kMix) dpt.load_full(bf.p, Pn, oP);
-    } else {
-      dd.load_ragged(bf.dout, dOn, a.dout.st, T_ - m0, D);
-      dd.load_ragged(bf.q, Qn, a.q.st, T_ - m0, D);
-      if constexpr (LOADP && !kMix) dpt.load_ragged(bf.p, Pn, a.p.st, T_ - m0, T_ - n0);
-      dma_wait();
+    if constexpr (kDma) {
+      const int m0 = mb * kBlk;
+      const Bufs bf = bufs(par);
+      if (m0 + kBlk <= T_ && cols_full) {
+        dd.load_full(bf.dout, dOn, odO);
+        dd.load_full(bf.q, Qn, oQ);
+        if constexpr (LOADP && !kMix) dpt.load_full(bf.p, Pn, oP);
+      } else {
+        dd.load_ragged(bf.dout, dOn, a.dout.st, T_ - m0, D);
+        dd.load_ragged(bf.q, Qn, a.q.st, T_ - m0, D);
+        if constexpr (LOADP && !kMix) dpt.load_ragged(bf.p, Pn, a.p.st, T_ - m0, T_ - n0);
+        dma_wait();
+      }
+      sdma.load(bf.st, m0, T_ - m0);
+      if constexpr (kMix) stage_load<T, kBlk>(stP, Pn, a.p.st, T_ - m0, T_ - n0);
+      dOn += kBlk * a.dout.st;
+      Qn += kBlk * a.q.st;
+      if constexpr (LOADP) Pn += kBlk * a.p.st;
     }
-    sdma.load(bf.st, m0, T_ - m0);
-    if constexpr (kMix) stage_load<T, kBlk>(stP, Pn, a.p.st, T_ - m0, T_ - n0);
-    dOn += kBlk * a.dout.st;
-    Qn += kBlk * a.q.st;
-    if constexpr (LOADP) Pn += kBlk * a.p.st;
   };
   if constexpr (kDma)
     dma_tile(cr.t0, Parity<0>{});
@@ -494,8 +506,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       }
     } else {
       __syncthreads();
-      stage_store_rows<T, D>(stdO, sdO0);
-      if constexpr (kNeedQ) stage_store_rows<T, D>(stQ, sQ0);
+      stage_store_tile<M>(stdO, sdO0);
+      if constexpr (kNeedQ) stage_store_tile<M>(stQ, sQ0);
       if constexpr (LOADP) stage_store_rows<T, kBlk>(stP, sP0);
       if constexpr (kNS > 0) stat_store<kNS>(stv, sS0);
       __syncthreads();
@@ -504,8 +516,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
         if (mb + 1 < cr.t1) load_tile(mb + 1);
     }
     const Bufs cb = bufs(par);
-    const T* cdO = cb.dout;
-    const T* cQ = cb.q;
+    const lds* cdO = cb.dout;
+    const lds* cQ = cb.q;
     const T* cP = cb.p;
     const float* cS = cb.st;
 
@@ -525,7 +537,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       }
     } else {
       p.zero();
-      mm_d<T, D>(p, cQ, kf);
+      mm_d<M>(p, cQ, kf);
       recompute_p_col<T, XM>(p, a, bcol, m0, cS, kSL, a.scale_log2);
     }
     if (mk.tile(mb)) {
@@ -535,10 +547,10 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
         for (int j = 0; j < 8; ++j)
           p.set(kb, j, mk.masked(m0 + stream_index(kb, g, j)) ? 0.f : p.at(kb, j));
     }
-    frag pf[2];
+    mfrag pf[2];
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) pf[kb] = tile_frag<T>(p, kb);
-    mm_s<T, D>(acc_dv, cdO, pf);
+    for (int kb = 0; kb < 2; ++kb) pf[kb] = tile_frag<M>(p, kb);
+    mm_s<M>(acc_dv, cdO, pf);
     if constexpr (!DV_ONLY) {
       Tile dp;
 #pragma unroll
@@ -548,16 +560,16 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
         dp.q[2 * kb] = f32x4{d8[0], d8[1], d8[2], d8[3]};
         dp.q[2 * kb + 1] = f32x4{d8[4], d8[5], d8[6], d8[7]};
       }
-      mm_d<T, D>(dp, cdO, vf);  // D - dP
-      frag dsf[2];
+      mm_d<M>(dp, cdO, vf);  // D - dP
+      mfrag dsf[2];
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb) {
         float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = p.at(kb, j) * dp.at(kb, j);  // -dS
-        dsf[kb] = vals_frag<T>(v);
+        dsf[kb] = M::vals(v);
       }
-      mm_s<T, D>(acc_dk, cQ, dsf);  // -dK / s
+      mm_s<M>(acc_dk, cQ, dsf);  // -dK / s
     }
   };
   if constexpr (kDma) {
@@ -589,8 +601,10 @@ template <typename T, int D, bool XM>
 __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   typedef Elem<T> E;
   typedef typename E::frag frag;
-  typedef Lds<T, D> L;
-  __shared__ __align__(16) T sV[L::kRowElems];
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
+  __shared__ __align__(16) lds sV[M::kElems];
 
   const int T_ = a.T;
   const Slot sl = grid_slot();
@@ -604,9 +618,9 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   const T* dO = at<const T>(a.dout, b, h);
   const T* Pm = at<const T>(a.p, b, h) + (int64_t)(row_ok ? m : 0) * a.p.st;
 
-  frag dof[D / 32];
+  mfrag dof[D / 32];
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) dof[ks] = load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g);
+  for (int ks = 0; ks < D / 32; ++ks) dof[ks] = M::from(load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g));
 
   float sum = 0.f;
   const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
@@ -616,7 +630,7 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   for (int nb = rg.lo; nb < rg.hi; ++nb) {
     const int n0 = nb * kBlk;
     __syncthreads();
-    stage_store_rows<T, D>(stV, sV);
+    stage_store_tile<M>(stV, sV);
     __syncthreads();
     if (nb + 1 < rg.hi) stage_load<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, T_ - n0 - kBlk, D);
     frag pr[2];
@@ -631,7 +645,7 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
           p.set(kb, j, mk.masked(n0 + stream_index(kb, g, j)) ? 0.f : p.at(kb, j));
     }
     dp.zero();
-    mm_d<T, D>(dp, sV, dof);
+    mm_d<M>(dp, sV, dof);
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll

@@ -552,17 +552,7 @@ __device__ __forceinline__ int sigma(int a, int r) {
   return 32 * (a >> 1) + 8 * (r >> 2) + 4 * (a & 1) + (r & 3);
 }
 
-// B fragment for k-block kb built from a score tile (converted to T).
-template <typename T>
-__device__ __forceinline__ typename Elem<T>::frag tile_frag(const Tile& s, int kb) {
-  typename Elem<T>::frag f;
-#pragma unroll
-  for (int j = 0; j < 8; ++j) f[j] = Elem<T>::cvt(s.at(kb, j));
-  return f;
-}
-
-// Same, from a pair of values arrays v[kb][j] (used when the values already
-// sit in a plain array).
+// Eight values converted to T.
 template <typename T>
 __device__ __forceinline__ typename Elem<T>::frag vals_frag(const float* v) {
   typename Elem<T>::frag f;
@@ -610,6 +600,178 @@ struct Lds {
     return r * kRowPitch + (((col / kChunk) ^ swz(r)) * kChunk) + col % kChunk;
   }
 };
+
+// ---------------------------------------------------------------------------
+// fp32 products on the 16-bit matrix cores.  x = h + m + l exactly, each part
+// a bf16 (8 significant bits): h is x truncated, m the rest rounded to
+// nearest, l what is left.  Of the nine products of two split operands the
+// six largest are formed (bf16 products are exact in fp32); the three dropped
+// ones, m*l, l*m and l*l, are below 2^-24 |x y| and of random sign, since m
+// is rounded.  Six v_mfma_f32_16x16x32_bf16 take 96 cycles where the eight
+// v_mfma_f32_16x16x4_f32 of the same product take 256, so the kernels are
+// bound by the VALU work around the products (eleven operations split a pair
+// of values, once per streamed tile and workgroup and once per operand formed
+// in registers), no longer by the products.  An infinite or NaN element gives
+// NaN (inf - inf) where fp32 products could give infinities.
+// Measured against the fp32 products (launch times, us): b8 h6 T1024 d64
+// window 512 O+LSE 63 -> 50, dQ 90 -> 63, dK/dV 120 -> 78, grad-grad row
+// 219 -> 155, column 219 -> 152.  Errors of the seven outputs against 64 bits
+// there: 2.8e-7 .. 8.0e-7 before, 1.3e-7 .. 3.5e-7 now (the sums of mm_tile).
+// ---------------------------------------------------------------------------
+struct SplitFrag {
+  bf16x8 h, m, l;
+};
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+
+// Words holding the bf16 parts of (x0, x1), x0 in the low half.
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& h, uint32_t& m, uint32_t& l) {
+  const uint32_t u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+  h = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+  const float r0 = x0 - __uint_as_float(u0 & 0xffff0000u), r1 = x1 - __uint_as_float(u1 & 0xffff0000u);
+  const bf16x2 mv = __builtin_convertvector(f32x2{r0, r1}, bf16x2);
+  __builtin_memcpy(&m, &mv, 4);
+  const float l0 = r0 - __uint_as_float(m << 16), l1 = r1 - __uint_as_float(m & 0xffff0000u);
+  l = __builtin_amdgcn_perm(__float_as_uint(l1), __float_as_uint(l0), 0x07060302u);  // exact: 8 bits left
+}
+
+__device__ __forceinline__ SplitFrag split8(const float* v) {
+  u32x4 h, m, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    uint32_t a, b, c;
+    split_pair(v[2 * i], v[2 * i + 1], a, b, c);
+    h[i] = a;
+    m[i] = b;
+    l[i] = c;
+  }
+  SplitFrag f;
+  __builtin_memcpy(&f.h, &h, 16);
+  __builtin_memcpy(&f.m, &m, 16);
+  __builtin_memcpy(&f.l, &l, 16);
+  return f;
+}
+
+// Operands of the tile products of element type T_ at head dim D_: the type of
+// an MFMA fragment (eight k-slots of one lane), how a streamed tile lies in
+// LDS, and the product, in kTerms steps.  16-bit types, and fp32 at D = 128:
+// the elements themselves.  kSplit (fp32 at D = 64): three bf16 planes, each in
+// the 16-bit layout.  At D = 128 the grad-grad kernels do not fit (the row
+// kernel's four streamed tiles would take 192 KB of LDS, and split fragments
+// spill 560-1400 bytes per lane), and every kernel of a step must form its
+// scores the same way: with the forward and first backward split alone (5 to
+// 30 % faster) a one-key row's recomputed P misses 1 by the difference, and GK
+// went past 1e-5 there.
+template <typename T_, int D_>
+struct Mm {
+  typedef T_ T;
+  static constexpr int D = D_;
+  static constexpr bool kSplit = std::is_same_v<T, float> && D == 64;
+  typedef std::conditional_t<kSplit, SplitFrag, typename Elem<T>::frag> frag;
+  typedef std::conditional_t<kSplit, __bf16, T> lds;
+  typedef Lds<lds, D> L;
+  static constexpr int kElems = (kSplit ? 3 : 1) * L::kRowElems;  // of a tile in LDS
+  static constexpr bool kBatch = sizeof(lds) == 2;  // fragment reads issued ahead of their MFMAs
+  static constexpr int kTerms = kSplit ? 6 : 1;
+  // Eight elements of row r from column col (mm_d); eight rows from r0 + 8g of
+  // column c0 + c (mm_s).
+  static __device__ __forceinline__ frag row(const lds* x, int r, int col);
+  static __device__ __forceinline__ frag tr(const lds* x, int r0, int c0);
+  // Step t of c + a.b, the smallest parts first.
+  template <int t>
+  static __device__ __forceinline__ f32x4 mma(f32x4 c, const frag& a, const frag& b) {
+    if constexpr (!kSplit) {
+      return Elem<T>::mma(c, a, b);
+    } else {
+      const bf16x8& x = t == 0 ? a.l : (t == 2 || t == 3) ? a.m : a.h;
+      const bf16x8& y = t == 1 ? b.l : (t == 2 || t == 4) ? b.m : b.h;
+      return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
+    }
+  }
+  // Every step (one product by itself).
+  static __device__ __forceinline__ f32x4 mma_all(f32x4 c, const frag& a, const frag& b) {
+    c = mma<0>(c, a, b);
+    if constexpr (kSplit) {
+      c = mma<1>(c, a, b);
+      c = mma<2>(c, a, b);
+      c = mma<3>(c, a, b);
+      c = mma<4>(c, a, b);
+      c = mma<5>(c, a, b);
+    }
+    return c;
+  }
+  // Fragment from eight elements as loaded, or from eight fp32 values.
+  static __device__ __forceinline__ frag from(const typename Elem<T>::frag& f) {
+    if constexpr (kSplit) {
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j] = f[j];
+      return split8(v);
+    } else {
+      return f;
+    }
+  }
+  static __device__ __forceinline__ frag vals(const float* v) {
+    if constexpr (kSplit) {
+      return split8(v);
+    } else {
+      frag f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = Elem<T>::cvt(v[j]);
+      return f;
+    }
+  }
+  // Keeps a fragment in registers as computed.
+  static __device__ __forceinline__ void keep(frag& f) {
+    if constexpr (kSplit)
+      asm volatile("" : "+v"(f.h), "+v"(f.m), "+v"(f.l));
+    else
+      asm volatile("" : "+v"(f));
+  }
+};
+
+// Runs body(std::integral_constant<int, t>) for the steps t of M's product:
+// with the independent accumulators inside, consecutive MFMAs do not wait for
+// one another.
+template <typename M, typename F>
+__device__ __forceinline__ void mma_steps(F&& body) {
+  body(std::integral_constant<int, 0>{});
+  if constexpr (M::kTerms > 1) {
+    body(std::integral_constant<int, 1>{});
+    body(std::integral_constant<int, 2>{});
+    body(std::integral_constant<int, 3>{});
+    body(std::integral_constant<int, 4>{});
+    body(std::integral_constant<int, 5>{});
+  }
+}
+
+// f(a, ks) over the NA subtiles and the k-blocks of mm_d: subtile by subtile,
+// or, where a product takes several steps, k-block by k-block.
+template <typename M, int NA, typename F>
+__device__ __forceinline__ void each_sub_ks(F&& f) {
+  constexpr int KS = M::D / 32;
+  if constexpr (M::kSplit) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) f(a, ks);
+  } else {
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) f(a, ks);
+  }
+}
+
+// B fragment for k-block kb built from a score tile.
+template <typename M>
+__device__ __forceinline__ typename M::frag tile_frag(const Tile& s, int kb) {
+  float v[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = s.at(kb, j);
+  return M::vals(v);
+}
 
 // Staged registers of one 64 x NCOL tile: each thread owns pairs of
 // consecutive rows (2r, 2r+1) at one 16-byte column chunk.
@@ -770,6 +932,41 @@ __device__ __forceinline__ void stage_store_rows(const Stage<T, NCOL>& st, T* ld
   }
 }
 
+// The same into an MFMA tile of M (split types: each 16-byte chunk of four
+// values becomes half a 16-byte chunk of each plane).
+template <typename M>
+__device__ __forceinline__ void stage_store_tile(const Stage<typename M::T, M::D>& st, typename M::lds* lds) {
+  if constexpr (!M::kSplit) {
+    stage_store_rows<typename M::T, M::D>(st, lds);
+  } else {
+    typedef Stage<typename M::T, M::D> S;
+    typedef typename M::L L;
+    const int tid = threadIdx.x;
+    const int col = (tid % S::kChunksPerRow) * S::kChunk;
+#pragma unroll
+    for (int ps = 0; ps < S::kPasses; ++ps) {
+      const int r = 2 * (tid / S::kChunksPerRow + ps * S::kPairsPerPass);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const u32x4& x = i ? st.x1[ps] : st.x0[ps];
+        u32x2 h, m, l;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          uint32_t a, b, c;
+          split_pair(__uint_as_float(x[2 * j]), __uint_as_float(x[2 * j + 1]), a, b, c);
+          h[j] = a;
+          m[j] = b;
+          l[j] = c;
+        }
+        typename M::lds* p = lds + L::off(r + i, col);
+        *reinterpret_cast<u32x2*>(p) = h;
+        *reinterpret_cast<u32x2*>(p + L::kRowElems) = m;
+        *reinterpret_cast<u32x2*>(p + 2 * L::kRowElems) = l;
+      }
+    }
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Column fragment of an LDS tile X (layout Lds<T, NCOL>):
 //   f[j] = X[r0 + 8g + j][c0 + c],  j = 0..7,  lane (c, g);  r0 % 8 == 0, c0 % 16 == 0.
@@ -801,6 +998,24 @@ __device__ __forceinline__ typename Elem<T>::frag load_frag_tr(const T* X, int r
   return f;
 }
 
+template <typename T_, int D_>
+__device__ __forceinline__ typename Mm<T_, D_>::frag Mm<T_, D_>::row(const lds* x, int r, int col) {
+  const lds* p = x + L::off(r, col);
+  if constexpr (kSplit)
+    return SplitFrag{load_frag<lds>(p), load_frag<lds>(p + L::kRowElems), load_frag<lds>(p + 2 * L::kRowElems)};
+  else
+    return load_frag<lds>(p);
+}
+
+template <typename T_, int D_>
+__device__ __forceinline__ typename Mm<T_, D_>::frag Mm<T_, D_>::tr(const lds* x, int r0, int c0) {
+  if constexpr (kSplit)
+    return SplitFrag{load_frag_tr<lds, D>(x, r0, c0), load_frag_tr<lds, D>(x + L::kRowElems, r0, c0),
+                     load_frag_tr<lds, D>(x + 2 * L::kRowElems, r0, c0)};
+  else
+    return load_frag_tr<lds, D>(x, r0, c0);
+}
+
 // ---------------------------------------------------------------------------
 // Tile products over a row-major LDS tile X of the streamed operand (64 x D).
 //
@@ -815,90 +1030,153 @@ __device__ __forceinline__ typename Elem<T>::frag load_frag_tr(const T* X, int r
 // the streamed tile for mm_s, all of D = 64 for mm_d) ahead of the MFMAs that
 // consume them; the scheduling barrier keeps the compiler from sinking each
 // read next to its MFMA.
-template <typename T, int D>
-__device__ __forceinline__ void mm_d(Tile& out, const T* rows, const typename Elem<T>::frag* sta) {
-  typedef Lds<T, D> L;
-  typedef typename Elem<T>::frag frag;
+//
+// Split types: a product over the streamed index is summed for the tile from
+// zero and then added to the running accumulators in fp32 (mm_tile), so those
+// take one rounding per tile, not one per MFMA (b2 h4 T2048 d64 causal, error
+// of GK against 64 bits: 9.3e-7 accumulated in place, 4.1e-7 so; 16 additions
+// a product, no time).
+template <typename M>
+__device__ __forceinline__ void mm_d(Tile& out, const typename M::lds* rows, const typename M::frag* sta) {
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   constexpr int KS = D / 32;
-  constexpr int AB = (sizeof(T) == 2) ? (KS <= 2 ? 4 : 2) : 1;  // subtiles per batch
+  constexpr int AB = M::kSplit ? 2 : M::kBatch ? (KS <= 2 ? 4 : 2) : 1;  // subtiles per batch
 #pragma unroll
   for (int a0 = 0; a0 < 4; a0 += AB) {
     frag x[AB][KS];
 #pragma unroll
     for (int a = 0; a < AB; ++a)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) x[a][ks] = load_frag<T>(rows + L::off(sigma(a0 + a, c), 32 * ks + 8 * g));
-    if constexpr (AB > 1) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int a = 0; a < AB; ++a)
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) out.q[a0 + a] = Elem<T>::mma(out.q[a0 + a], x[a][ks], sta[ks]);
+      for (int ks = 0; ks < KS; ++ks) x[a][ks] = M::row(rows, sigma(a0 + a, c), 32 * ks + 8 * g);
+    if constexpr (M::kBatch) __builtin_amdgcn_sched_barrier(0);
+    mma_steps<M>([&](auto t) __attribute__((always_inline)) {
+      each_sub_ks<M, AB>([&](int a, int ks) __attribute__((always_inline)) {
+        out.q[a0 + a] = M::template mma<decltype(t)::value>(out.q[a0 + a], x[a][ks], sta[ks]);
+      });
+    });
   }
 }
 
-template <typename T, int D>
-__device__ __forceinline__ void mm_s(f32x4* acc, const T* X, const typename Elem<T>::frag* y) {
-  typedef typename Elem<T>::frag frag;
-  constexpr int NB = (sizeof(T) == 2) ? 8 : 1;  // fragments per batch
+// Split types: acc[n][ds] += sum over k-blocks kb0 .. kb1-1 of X . y[n][kb]
+// for N products over one tile, a few column groups at a time.
+template <typename M, int N>
+__device__ __forceinline__ void mm_tile(f32x4* const (&acc)[N], const typename M::lds* X,
+                                        const typename M::frag* const (&y)[N], int kb0, int kb1) {
+  typedef typename M::frag frag;
+  constexpr int DSN = M::D / 16;
+  constexpr int G = N == 1 ? 4 : 2;  // column groups at a time
+#pragma unroll
+  for (int d0 = 0; d0 < DSN; d0 += G) {
+    f32x4 t[N][G];
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+      for (int i = 0; i < G; ++i) t[n][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = kb0; kb < kb1; ++kb) {
+      frag x[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i) x[i] = M::tr(X, 32 * kb, 16 * (d0 + i));
+      mma_steps<M>([&](auto st) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < G; ++i)
+#pragma unroll
+          for (int n = 0; n < N; ++n)
+            t[n][i] = M::template mma<decltype(st)::value>(t[n][i], x[i], y[n][kb - kb0]);
+      });
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+      for (int i = 0; i < G; ++i) acc[n][d0 + i] += t[n][i];
+  }
+}
+
+template <typename M>
+__device__ __forceinline__ void mm_s(f32x4* acc, const typename M::lds* X, const typename M::frag* y) {
+  if constexpr (M::kSplit) {
+    mm_tile<M, 1>({acc}, X, {y}, 0, 2);
+    return;
+  }
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
+  constexpr int NB = M::kBatch ? 8 : 1;  // fragments per batch
   constexpr int DSN = D / 16;
 #pragma unroll
   for (int i0 = 0; i0 < 2 * DSN; i0 += NB) {
     frag x[NB];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) x[i] = load_frag_tr<T, D>(X, 32 * ((i0 + i) / DSN), 16 * ((i0 + i) % DSN));
+    for (int i = 0; i < NB; ++i) x[i] = M::tr(X, 32 * ((i0 + i) / DSN), 16 * ((i0 + i) % DSN));
     if constexpr (NB > 1) __builtin_amdgcn_sched_barrier(0);
+    mma_steps<M>([&](auto t) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int kb = (i0 + i) / DSN, ds = (i0 + i) % DSN;
-      acc[ds] = Elem<T>::mma(acc[ds], x[i], y[kb]);
-    }
+      for (int i = 0; i < NB; ++i) {
+        const int kb = (i0 + i) / DSN, ds = (i0 + i) % DSN;
+        acc[ds] = M::template mma<decltype(t)::value>(acc[ds], x[i], y[kb]);
+      }
+    });
   }
 }
 
 // mm_s for two or three products over the same tile X (acc_n += y_n . X):
 // each fragment of X is read from LDS once and feeds every product.
-template <typename T, int D>
-__device__ __forceinline__ void mm_s2(f32x4* acc0, const typename Elem<T>::frag* y0, f32x4* acc1,
-                                      const typename Elem<T>::frag* y1, const T* X) {
-  typedef typename Elem<T>::frag frag;
-  constexpr int NB = (sizeof(T) == 2) ? 8 : 1;
+template <typename M>
+__device__ __forceinline__ void mm_s2(f32x4* acc0, const typename M::frag* y0, f32x4* acc1,
+                                      const typename M::frag* y1, const typename M::lds* X) {
+  if constexpr (M::kSplit) {
+    mm_tile<M, 2>({acc0, acc1}, X, {y0, y1}, 0, 2);
+    return;
+  }
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
+  constexpr int NB = M::kBatch ? 8 : 1;
   constexpr int DSN = D / 16;
 #pragma unroll
   for (int i0 = 0; i0 < 2 * DSN; i0 += NB) {
     frag x[NB];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) x[i] = load_frag_tr<T, D>(X, 32 * ((i0 + i) / DSN), 16 * ((i0 + i) % DSN));
+    for (int i = 0; i < NB; ++i) x[i] = M::tr(X, 32 * ((i0 + i) / DSN), 16 * ((i0 + i) % DSN));
     if constexpr (NB > 1) __builtin_amdgcn_sched_barrier(0);
+    mma_steps<M>([&](auto t) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int kb = (i0 + i) / DSN, ds = (i0 + i) % DSN;
-      acc0[ds] = Elem<T>::mma(acc0[ds], x[i], y0[kb]);
-      acc1[ds] = Elem<T>::mma(acc1[ds], x[i], y1[kb]);
-    }
+      for (int i = 0; i < NB; ++i) {
+        const int kb = (i0 + i) / DSN, ds = (i0 + i) % DSN;
+        acc0[ds] = M::template mma<decltype(t)::value>(acc0[ds], x[i], y0[kb]);
+        acc1[ds] = M::template mma<decltype(t)::value>(acc1[ds], x[i], y1[kb]);
+      }
+    });
   }
 }
 
-template <typename T, int D>
-__device__ __forceinline__ void mm_s3(f32x4* acc0, const typename Elem<T>::frag* y0, f32x4* acc1,
-                                      const typename Elem<T>::frag* y1, f32x4* acc2,
-                                      const typename Elem<T>::frag* y2, const T* X) {
-  typedef typename Elem<T>::frag frag;
-  constexpr int NB = (sizeof(T) == 2) ? 8 : 1;
+template <typename M>
+__device__ __forceinline__ void mm_s3(f32x4* acc0, const typename M::frag* y0, f32x4* acc1,
+                                      const typename M::frag* y1, f32x4* acc2,
+                                      const typename M::frag* y2, const typename M::lds* X) {
+  if constexpr (M::kSplit) {
+    mm_tile<M, 3>({acc0, acc1, acc2}, X, {y0, y1, y2}, 0, 2);
+    return;
+  }
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
+  constexpr int NB = M::kBatch ? 8 : 1;
   constexpr int DSN = D / 16;
 #pragma unroll
   for (int i0 = 0; i0 < 2 * DSN; i0 += NB) {
     frag x[NB];
 #pragma unroll
-    for (int i = 0; i < NB; ++i) x[i] = load_frag_tr<T, D>(X, 32 * ((i0 + i) / DSN), 16 * ((i0 + i) % DSN));
+    for (int i = 0; i < NB; ++i) x[i] = M::tr(X, 32 * ((i0 + i) / DSN), 16 * ((i0 + i) % DSN));
     if constexpr (NB > 1) __builtin_amdgcn_sched_barrier(0);
+    mma_steps<M>([&](auto t) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int kb = (i0 + i) / DSN, ds = (i0 + i) % DSN;
-      acc0[ds] = Elem<T>::mma(acc0[ds], x[i], y0[kb]);
-      acc1[ds] = Elem<T>::mma(acc1[ds], x[i], y1[kb]);
-      acc2[ds] = Elem<T>::mma(acc2[ds], x[i], y2[kb]);
-    }
+      for (int i = 0; i < NB; ++i) {
+        const int kb = (i0 + i) / DSN, ds = (i0 + i) % DSN;
+        acc0[ds] = M::template mma<decltype(t)::value>(acc0[ds], x[i], y0[kb]);
+        acc1[ds] = M::template mma<decltype(t)::value>(acc1[ds], x[i], y1[kb]);
+        acc2[ds] = M::template mma<decltype(t)::value>(acc2[ds], x[i], y2[kb]);
+      }
+    });
   }
 }
 
@@ -907,96 +1185,109 @@ __device__ __forceinline__ void mm_s3(f32x4* acc0, const typename Elem<T>::frag*
 // a = 2kb, 2kb+1 of mm_d's output, mm_s_half adds k-block kb of mm_s.  Work on
 // one half does not depend on the other, so the second half's products can
 // run while the first half's elementwise work does.
-template <typename T, int D>
-__device__ __forceinline__ void mm_d_half(Tile& out, int kb, const T* rows, const typename Elem<T>::frag* sta) {
-  typedef Lds<T, D> L;
-  typedef typename Elem<T>::frag frag;
+template <typename M>
+__device__ __forceinline__ void mm_d_half(Tile& out, int kb, const typename M::lds* rows, const typename M::frag* sta) {
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   constexpr int KS = D / 32;
   frag x[2][KS];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) x[a][ks] = load_frag<T>(rows + L::off(sigma(2 * kb + a, c), 32 * ks + 8 * g));
-  if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) out.q[2 * kb + a] = Elem<T>::mma(out.q[2 * kb + a], x[a][ks], sta[ks]);
+    for (int ks = 0; ks < KS; ++ks) x[a][ks] = M::row(rows, sigma(2 * kb + a, c), 32 * ks + 8 * g);
+  if constexpr (M::kBatch) __builtin_amdgcn_sched_barrier(0);
+  mma_steps<M>([&](auto t) __attribute__((always_inline)) {
+    each_sub_ks<M, 2>([&](int a, int ks) __attribute__((always_inline)) {
+      out.q[2 * kb + a] = M::template mma<decltype(t)::value>(out.q[2 * kb + a], x[a][ks], sta[ks]);
+    });
+  });
 }
 
 // mm_d_half for two products over the same rows (out0 from sta0, out1 from
 // sta1), reading each row fragment once.
-template <typename T, int D>
-__device__ __forceinline__ void mm_d2_half(Tile& out0, Tile& out1, int kb, const T* rows,
-                                           const typename Elem<T>::frag* sta0, const typename Elem<T>::frag* sta1) {
-  typedef Lds<T, D> L;
-  typedef typename Elem<T>::frag frag;
+template <typename M>
+__device__ __forceinline__ void mm_d2_half(Tile& out0, Tile& out1, int kb, const typename M::lds* rows,
+                                           const typename M::frag* sta0, const typename M::frag* sta1) {
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
   const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   constexpr int KS = D / 32;
   frag x[2][KS];
 #pragma unroll
   for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) x[a][ks] = load_frag<T>(rows + L::off(sigma(2 * kb + a, c), 32 * ks + 8 * g));
-  if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      out0.q[2 * kb + a] = Elem<T>::mma(out0.q[2 * kb + a], x[a][ks], sta0[ks]);
-      out1.q[2 * kb + a] = Elem<T>::mma(out1.q[2 * kb + a], x[a][ks], sta1[ks]);
-    }
+    for (int ks = 0; ks < KS; ++ks) x[a][ks] = M::row(rows, sigma(2 * kb + a, c), 32 * ks + 8 * g);
+  if constexpr (M::kBatch) __builtin_amdgcn_sched_barrier(0);
+  mma_steps<M>([&](auto t) __attribute__((always_inline)) {
+    each_sub_ks<M, 2>([&](int a, int ks) __attribute__((always_inline)) {
+      out0.q[2 * kb + a] = M::template mma<decltype(t)::value>(out0.q[2 * kb + a], x[a][ks], sta0[ks]);
+      out1.q[2 * kb + a] = M::template mma<decltype(t)::value>(out1.q[2 * kb + a], x[a][ks], sta1[ks]);
+    });
+  });
 }
 
-template <typename T, int D>
-__device__ __forceinline__ void mm_s_half(f32x4* acc, int kb, const T* X, typename Elem<T>::frag y) {
-  typedef typename Elem<T>::frag frag;
+template <typename M>
+__device__ __forceinline__ void mm_s_half(f32x4* acc, int kb, const typename M::lds* X, typename M::frag y) {
+  if constexpr (M::kSplit) {
+    mm_tile<M, 1>({acc}, X, {&y}, kb, kb + 1);
+    return;
+  }
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
   constexpr int DSN = D / 16;
   frag x[DSN];
 #pragma unroll
-  for (int ds = 0; ds < DSN; ++ds) x[ds] = load_frag_tr<T, D>(X, 32 * kb, 16 * ds);
-  if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);
+  for (int ds = 0; ds < DSN; ++ds) x[ds] = M::tr(X, 32 * kb, 16 * ds);
+  if constexpr (M::kBatch) __builtin_amdgcn_sched_barrier(0);
+  mma_steps<M>([&](auto t) __attribute__((always_inline)) {
 #pragma unroll
-  for (int ds = 0; ds < DSN; ++ds) acc[ds] = Elem<T>::mma(acc[ds], x[ds], y);
+    for (int ds = 0; ds < DSN; ++ds) acc[ds] = M::template mma<decltype(t)::value>(acc[ds], x[ds], y);
+  });
 }
 
 // mm_s_half for two products over the same half tile (acc_n += y_n . X),
 // reading each fragment of X once.
-template <typename T, int D>
-__device__ __forceinline__ void mm_s2_half(f32x4* acc0, typename Elem<T>::frag y0, f32x4* acc1,
-                                           typename Elem<T>::frag y1, int kb, const T* X) {
-  typedef typename Elem<T>::frag frag;
+template <typename M>
+__device__ __forceinline__ void mm_s2_half(f32x4* acc0, typename M::frag y0, f32x4* acc1,
+                                           typename M::frag y1, int kb, const typename M::lds* X) {
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
   constexpr int DSN = D / 16;
   frag x[DSN];
 #pragma unroll
-  for (int ds = 0; ds < DSN; ++ds) x[ds] = load_frag_tr<T, D>(X, 32 * kb, 16 * ds);
-  if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);
+  for (int ds = 0; ds < DSN; ++ds) x[ds] = M::tr(X, 32 * kb, 16 * ds);
+  if constexpr (M::kBatch) __builtin_amdgcn_sched_barrier(0);
+  mma_steps<M>([&](auto t) __attribute__((always_inline)) {
 #pragma unroll
-  for (int ds = 0; ds < DSN; ++ds) {
-    acc0[ds] = Elem<T>::mma(acc0[ds], x[ds], y0);
-    acc1[ds] = Elem<T>::mma(acc1[ds], x[ds], y1);
-  }
+    for (int ds = 0; ds < DSN; ++ds) {
+      acc0[ds] = M::template mma<decltype(t)::value>(acc0[ds], x[ds], y0);
+      acc1[ds] = M::template mma<decltype(t)::value>(acc1[ds], x[ds], y1);
+    }
+  });
 }
 
 // mm_s_half for three products over the same half tile (acc_n += y_n . X),
 // reading each fragment of X once.
-template <typename T, int D>
-__device__ __forceinline__ void mm_s3_half(f32x4* acc0, typename Elem<T>::frag y0, f32x4* acc1,
-                                           typename Elem<T>::frag y1, f32x4* acc2, typename Elem<T>::frag y2,
-                                           int kb, const T* X) {
-  typedef typename Elem<T>::frag frag;
+template <typename M>
+__device__ __forceinline__ void mm_s3_half(f32x4* acc0, typename M::frag y0, f32x4* acc1,
+                                           typename M::frag y1, f32x4* acc2, typename M::frag y2,
+                                           int kb, const typename M::lds* X) {
+  typedef typename M::frag frag;
+  constexpr int D = M::D;
   constexpr int DSN = D / 16;
   frag x[DSN];
 #pragma unroll
-  for (int ds = 0; ds < DSN; ++ds) x[ds] = load_frag_tr<T, D>(X, 32 * kb, 16 * ds);
-  if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);
+  for (int ds = 0; ds < DSN; ++ds) x[ds] = M::tr(X, 32 * kb, 16 * ds);
+  if constexpr (M::kBatch) __builtin_amdgcn_sched_barrier(0);
+  mma_steps<M>([&](auto t) __attribute__((always_inline)) {
 #pragma unroll
-  for (int ds = 0; ds < DSN; ++ds) {
-    acc0[ds] = Elem<T>::mma(acc0[ds], x[ds], y0);
-    acc1[ds] = Elem<T>::mma(acc1[ds], x[ds], y1);
-    acc2[ds] = Elem<T>::mma(acc2[ds], x[ds], y2);
-  }
+    for (int ds = 0; ds < DSN; ++ds) {
+      acc0[ds] = M::template mma<decltype(t)::value>(acc0[ds], x[ds], y0);
+      acc1[ds] = M::template mma<decltype(t)::value>(acc1[ds], x[ds], y1);
+      acc2[ds] = M::template mma<decltype(t)::value>(acc2[ds], x[ds], y2);
+    }
+  });
 }
 
 // Reductions over the four lane groups (same c), with the gfx950 VALU lane

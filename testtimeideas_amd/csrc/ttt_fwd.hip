@@ -57,11 +57,11 @@ namespace ttt {
 // Scores of key tile nb (rows sK) for query row m, in base-2 units; masked
 // entries are -inf.  brow: this row of the additive bias, or nullptr.
 template <typename T, int D, bool XM>
-__device__ __forceinline__ void fwd_scores(Tile& s, const T* sK, const typename Elem<T>::frag* qf,
-                                           const Params& a, const RowMask<XM>& mk, const T* brow, int nb) {
+__device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds* sK,
+                                           const typename Mm<T, D>::frag* qf, const Params& a, const RowMask<XM>& mk, const T* brow, int nb) {
   const int g = (threadIdx.x & 63) >> 4;
   s.zero();
-  mm_d<T, D>(s, sK, qf);
+  mm_d<Mm<T, D>>(s, sK, qf);
   const int n0 = nb * kBlk;
   const bool need_mask = mk.tile(nb);
 #pragma unroll
@@ -119,16 +119,19 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   // 16-bit tiles stream straight into two LDS buffer sets (TileDma) in
   // distinct arrays with a compile-time role per loop step; fp32 tiles are
   // staged through registers.  At D = 128 the two sets take 64 KB of LDS (two
   // workgroups per CU instead of three) and still measured faster: b4 h16
   // T8192 bf16 causal -9 %, b2 h4 T2048 fp16 -19 %.
   constexpr bool kDma = L::kSwizzle;
-  __shared__ __align__(16) T sK[L::kRowElems];
-  __shared__ __align__(16) T sV[L::kRowElems];
-  __shared__ __align__(16) T sK1[kDma ? L::kRowElems : 8];
-  __shared__ __align__(16) T sV1[kDma ? L::kRowElems : 8];
+  __shared__ __align__(16) lds sK[M::kElems];
+  __shared__ __align__(16) lds sV[M::kElems];
+  __shared__ __align__(16) lds sK1[kDma ? M::kElems : 8];
+  __shared__ __align__(16) lds sV1[kDma ? M::kElems : 8];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
@@ -150,9 +153,9 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
   const T* V = at<const T>(a.v, b, h);
-  frag qf[D / 32];
+  frag qr[D / 32];
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
+  for (int ks = 0; ks < D / 32; ++ks) qr[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
 
   f32x4 acc[D / 16];
 #pragma unroll
@@ -187,14 +190,17 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     if (csl < 0.f) {
       csl = -csl;
 #pragma unroll
-      for (int ks = 0; ks < D / 32; ++ks) qf[ks] = scale_frag<T>(qf[ks], -1.f);
+      for (int ks = 0; ks < D / 32; ++ks) qr[ks] = scale_frag<T>(qr[ks], -1.f);
     }
   }
+  mfrag qf[D / 32];
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
   float sh = -INFINITY;
-  auto body_raw = [&](int nb, const T* cK, const T* cV) __attribute__((always_inline)) {
+  auto body_raw = [&](int nb, const lds* cK, const lds* cV) __attribute__((always_inline)) {
     Tile s;
     s.zero();
-    mm_d<T, D>(s, cK, qf);
+    mm_d<M>(s, cK, qf);
     const bool need_mask = mk.tile(nb);
     if (need_mask) {
       const int n0 = nb * kBlk;
@@ -214,7 +220,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       for (int i = 0; i < D / 16; ++i) acc[i] *= alpha;
       sh = sn;
     }
-    frag pf[2];
+    mfrag pf[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       float pv[8];
@@ -226,11 +232,11 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) l += pv[j];
-      pf[kb] = vals_frag<T>(pv);
+      pf[kb] = M::vals(pv);
     }
-    mm_s<T, D>(acc, cV, pf);
+    mm_s<M>(acc, cV, pf);
   };
-  auto body = [&](int nb, const T* cK, const T* cV) __attribute__((always_inline)) {
+  auto body = [&](int nb, const lds* cK, const lds* cV) __attribute__((always_inline)) {
     if constexpr (!XM) {
       body_raw(nb, cK, cV);
       return;
@@ -242,7 +248,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     const float msh = (XM && mnew == -INFINITY) ? 0.f : mnew;
     const float alpha = fast_exp2(mx - msh);
     float ts = 0.f;
-    frag pf[2];
+    mfrag pf[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       float pv[8];
@@ -251,13 +257,13 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
         pv[j] = fast_exp2(s.at(kb, j) - msh);
         ts += pv[j];
       }
-      pf[kb] = vals_frag<T>(pv);
+      pf[kb] = M::vals(pv);
     }
     l = l * alpha + ts;  // this lane's share of the row sum (all lanes share mnew)
     mx = mnew;
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) acc[i] *= alpha;
-    mm_s<T, D>(acc, cV, pf);
+    mm_s<M>(acc, cV, pf);
   };
   if constexpr (kDma) {
     const TileDma<T, D> dd;
@@ -302,8 +308,8 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     load_kv(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
       __syncthreads();
-      stage_store_rows<T, D>(stK, sK);
-      stage_store_rows<T, D>(stV, sV);
+      stage_store_tile<M>(stK, sK);
+      stage_store_tile<M>(stV, sV);
       __syncthreads();
       if (nb + 1 < cr.t1) load_kv(nb + 1);
       body(nb, sK, sV);
@@ -368,6 +374,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
   constexpr int KS = D / 32;
   __shared__ __align__(16) T sK0[L::kRowElems];
   __shared__ __align__(16) T sK1[L::kRowElems];
@@ -470,7 +477,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
         pv[j] = fast_exp2(x);
       }
       ts[kb] = ((pv[0] + pv[1]) + (pv[2] + pv[3])) + ((pv[4] + pv[5]) + (pv[6] + pv[7]));
-      pf[kb] = vals_frag<T>(pv);
+      pf[kb] = M::vals(pv);
     }
     return ts[0] + ts[1];
   };
@@ -555,7 +562,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     }
     l0 += ts0;
     l1 += ts1;
-    mm_s2<T, D>(acc0, pf0, acc1, pf1, P == 0 ? sV0 : sV1);
+    mm_s2<M>(acc0, pf0, acc1, pf1, P == 0 ? sV0 : sV1);
     s[0] = sn[0];
     s[1] = sn[1];
   };
@@ -607,17 +614,18 @@ struct FwdPWaves {
 template <typename T, int D, bool XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Params a) {
-  typedef Elem<T> E;
-  typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   // R key tiles per round: one pair of barriers and R independent score
   // products per round.
   constexpr int R = 2;
   // 16-bit types: the R tiles of a round stream straight into LDS (TileDma),
   // alternating between two sets in distinct arrays with compile-time roles.
   constexpr bool kDma = L::kSwizzle;
-  __shared__ __align__(16) T sK[R][L::kRowElems];
-  __shared__ __align__(16) T sK1[R][kDma ? L::kRowElems : 8];
+  __shared__ __align__(16) lds sK[R][M::kElems];
+  __shared__ __align__(16) lds sK1[R][kDma ? M::kElems : 8];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
@@ -638,9 +646,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
-  frag qf[D / 32];
+  mfrag qf[D / 32];
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
+  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g));
 
   float mx = -INFINITY, l = 0.f;
   const float csl = a.scale_log2;
@@ -667,7 +675,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   #pragma unroll
           for (int i = 0; i < R; ++i) {
             s[i].zero();
-            mm_d<T, D>(s[i], tile_k(i), qf);
+            mm_d<M>(s[i], tile_k(i), qf);
             const int n0 = (nb + i) * kBlk;
             if ((i > 0 && nb + i >= cr.t1) || mk.tile(nb + i)) {
               const bool past = i > 0 && nb + i >= cr.t1;
@@ -756,7 +764,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       dma_wait();       // this wave's loads of round nb
       __syncthreads();  // everyone's, and everyone is done with the other set
       if (nb + R < cr.t1) fetch_set(nb + R, Parity<1 - P>{});
-      round(nb, [&](int i) -> const T* { return P == 0 ? sK[i] : sK1[i]; });
+      round(nb, [&](int i) -> const lds* { return P == 0 ? sK[i] : sK1[i]; });
     };
     fetch_set(cr.t0, Parity<0>{});
     for (int nb = cr.t0; nb < cr.t1; nb += 2 * R) {
@@ -769,13 +777,13 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
     for (int nb = cr.t0; nb < cr.t1; nb += R) {
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < R; ++i) stage_store_rows<T, D>(stK[i], sK[i]);
+      for (int i = 0; i < R; ++i) stage_store_tile<M>(stK[i], sK[i]);
       __syncthreads();
       if (nb + R < cr.t1) {
 #pragma unroll
         for (int i = 0; i < R; ++i) load_k(nb + R + i, stK[i]);
       }
-      round(nb, [&](int i) -> const T* { return sK[i]; });
+      round(nb, [&](int i) -> const lds* { return sK[i]; });
     }
   }
   if (!XM && raw_units && mx != -INFINITY) mx *= csl;  // back to base-2 units
@@ -844,14 +852,17 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   // 16-bit tiles stream straight into two LDS buffer sets (TileDma) in
   // distinct arrays with a compile-time role per loop step, one tile per
   // barrier round; fp32 tiles are staged through registers.
   constexpr bool kDma = L::kSwizzle;
-  __shared__ __align__(16) T sK[L::kRowElems];
-  __shared__ __align__(16) T sV[L::kRowElems];
-  __shared__ __align__(16) T sK1[kDma ? L::kRowElems : 8];
-  __shared__ __align__(16) T sV1[kDma ? L::kRowElems : 8];
+  __shared__ __align__(16) lds sK[M::kElems];
+  __shared__ __align__(16) lds sV[M::kElems];
+  __shared__ __align__(16) lds sK1[kDma ? M::kElems : 8];
+  __shared__ __align__(16) lds sV1[kDma ? M::kElems : 8];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
@@ -880,9 +891,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   // 16-bit d = 64: full tiles of P stored in whole row segments (store_p_rows;
   // at d = 128 the same stores measured slower steps).
   constexpr bool kRowPair = sizeof(T) == 2 && D == 64;
-  frag qf[D / 32];
+  mfrag qf[D / 32];
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
+  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g));
 
   f32x4 acc[D / 16];
 #pragma unroll
@@ -925,16 +936,16 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
     }
   };
   // Key tile `nt` from LDS tiles cK, cV.
-  auto body = [&](int nt, const T* cK, const T* cV) __attribute__((always_inline)) {
+  auto body = [&](int nt, const lds* cK, const lds* cV) __attribute__((always_inline)) {
       const int n0 = nt * kBlk;
-      frag pf[2];
+      mfrag pf[2];
       if constexpr (!XM && sizeof(T) == 2) {
         // Raw scores; P = exp2(raw * scale*log2e - lse) in one FMA, masked
         // entries selected to 0 afterwards, and one rounding to T gives both
         // the MFMA fragment and the stored P.
         Tile s;
         s.zero();
-        mm_d<T, D>(s, cK, qf);
+        mm_d<M>(s, cK, qf);
         const bool need_mask = mk.tile(nt);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
@@ -945,7 +956,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
 #pragma unroll
             for (int j = 0; j < 8; ++j) pv[j] = mk.masked(n0 + stream_index(kb, g, j)) ? 0.f : pv[j];
           }
-          pf[kb] = vals_frag<T>(pv);
+          pf[kb] = M::vals(pv);
           if (kRowPair && n0 + kBlk <= T_) {
             // stored whole below (or deferred)
           } else if (kDma && a.defer_p && n0 + kBlk <= T_) {
@@ -989,9 +1000,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
           float pv[8];
 #pragma unroll
           for (int j = 0; j < 8; ++j) pv[j] = E::f32(E::cvt(fast_exp2(s.at(kb, j) - lse2)));
-          pf[kb] = vals_frag<T>(pv);
+          pf[kb] = M::vals(pv);
           if (kDma && a.defer_p && n0 + kBlk <= T_) {
-            pend[kb] = pf[kb];
+            if constexpr (kDma) pend[kb] = pf[kb];
             if (kb == 1) {
               if constexpr (kRowPair)
                 pend_n0 = n0;
@@ -1010,7 +1021,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
           }
         }
       }
-      mm_s<T, D>(acc, cV, pf);
+      mm_s<M>(acc, cV, pf);
   };
   if constexpr (kDma) {
     const TileDma<T, D> dd;
@@ -1057,8 +1068,8 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
     load_kv(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
       __syncthreads();
-      stage_store_rows<T, D>(stK, sK);
-      stage_store_rows<T, D>(stV, sV);
+      stage_store_tile<M>(stK, sK);
+      stage_store_tile<M>(stV, sV);
       __syncthreads();
       if (nb + 1 < cr.t1) load_kv(nb + 1);
       body(nb, sK, sV);

@@ -83,12 +83,11 @@ static_assert(TTT_GG_HEAD_DIM == 64 || TTT_GG_HEAD_DIM == 128, "head dim of this
 #define TTT_GG_ROW8 (TTT_GG_HEAD_DIM == 128 && (TTT_GG_TYPES & 1) && (TTT_GG_ROW_GDO & 1))
 
 // Waves per SIMD the four-wave grad-grad kernels are compiled for (registers
-// are limited to 512 / this per lane): two at D = 64 (16-bit types; and fp32
-// in the column kernel, whose few spills cost less than half the waves), one
-// otherwise, where two spill heavily (fp32 fragments take twice the
-// registers, D = 128 twice the accumulators).  Measured on MI355X: b4 h16
-// T8192 d128 bf16 grad-grad 43.8 -> 14.9 ms, fp32 D = 64 row pass
-// 352 -> 268 us.  16-bit types at D = 128 (no window, bias or GdO) take the
+// are limited to 512 / this per lane): two for 16-bit types at D = 64, one
+// otherwise, where two spill heavily (fp32 fragments take two to three times
+// the registers, D = 128 twice the accumulators; the fp32 D = 64 column kernel
+// 560-600 bytes per lane).  Measured on MI355X: b4 h16 T8192 d128 bf16
+// grad-grad 43.8 -> 14.9 ms.  16-bit types at D = 128 (no window, bias or GdO) take the
 // eight-wave kernels k_gg_row8 / k_gg_col8 instead, which fit two waves per
 // SIMD by splitting each streamed tile between two waves (C5 grad-grad
 // 9.66 -> 9.04 ms with P loaded, 10.2 -> 9.3 ms with P recomputed).
@@ -122,18 +121,21 @@ struct Gg8Waves {
   static constexpr int value = 2;
 };
 
-template <typename T, int D, bool COL>
+template <typename T, int D>
 struct GgWaves {
-  static constexpr int value = ((sizeof(T) == 2 || COL) && D == 64) ? 2 : 1;
+  static constexpr int value = (sizeof(T) == 2 && D == 64) ? 2 : 1;
 };
 
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool LOADP, bool GDO, bool XM, bool DQ>
 __global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(Params a) {
+__attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params a) {
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   static_assert(!(DQ && GDO), "the dQ form has no GdO variant");
   // split partials: dS*gK + Z1*K, Z2*K, P*K (+ P*gV + (P o gdS)*V, P*V), the
   // dQ form without Z2*K; row sums E, X and rowsum(Z2) (dQ form: X in fp32)
@@ -146,20 +148,20 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
   constexpr bool kPar = L::kSwizzle && (D == 128 || !GDO);
   constexpr bool kDma = L::kSwizzle && D == 64 && !kPar;
   constexpr int kBuf = kDma ? 2 : 1;
-  constexpr int kE = kPar ? 8 : L::kRowElems;  // the run-time-indexed arrays (unused with kPar)
-  __shared__ __align__(16) T sK[kBuf][kE];
-  __shared__ __align__(16) T sV[kBuf][kE];
-  __shared__ __align__(16) T sgK[kBuf][kE];
-  __shared__ __align__(16) T sgV[kBuf][kE];
-  constexpr int kPE = kPar ? L::kRowElems : 8;
-  __shared__ __align__(16) T pK0[kPE];
-  __shared__ __align__(16) T pV0[kPE];
-  __shared__ __align__(16) T pgK0[kPE];
-  __shared__ __align__(16) T pgV0[kPE];
-  __shared__ __align__(16) T pK1[kPE];
-  __shared__ __align__(16) T pV1[kPE];
-  __shared__ __align__(16) T pgK1[kPE];
-  __shared__ __align__(16) T pgV1[kPE];
+  constexpr int kE = kPar ? 8 : M::kElems;  // the run-time-indexed arrays (unused with kPar)
+  __shared__ __align__(16) lds sK[kBuf][kE];
+  __shared__ __align__(16) lds sV[kBuf][kE];
+  __shared__ __align__(16) lds sgK[kBuf][kE];
+  __shared__ __align__(16) lds sgV[kBuf][kE];
+  constexpr int kPE = kPar ? M::kElems : 8;
+  __shared__ __align__(16) lds pK0[kPE];
+  __shared__ __align__(16) lds pV0[kPE];
+  __shared__ __align__(16) lds pgK0[kPE];
+  __shared__ __align__(16) lds pgV0[kPE];
+  __shared__ __align__(16) lds pK1[kPE];
+  __shared__ __align__(16) lds pV1[kPE];
+  __shared__ __align__(16) lds pgK1[kPE];
+  __shared__ __align__(16) lds pgV1[kPE];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
@@ -188,16 +190,14 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
   const T* gK = at<const T>(a.gk, b, h);
   const T* gV = at<const T>(a.gv, b, h);
 
-  frag qf[D / 32], gqf[D / 32], dof[D / 32];
+  mfrag qf[D / 32], gqf[D / 32], dof[D / 32];
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
-    qf[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
-    gqf[ks] = load_frag_row<T>(gQ, a.gq.st, m, T_, 32 * ks + 8 * g);
-    {
-      qf[ks] = scale_frag<T>(qf[ks], a.scale);
-      gqf[ks] = scale_frag<T>(gqf[ks], a.scale);
-    }
-    dof[ks] = load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g);
+    const frag qr = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
+    const frag gqr = load_frag_row<T>(gQ, a.gq.st, m, T_, 32 * ks + 8 * g);
+    qf[ks] = M::from(scale_frag<T>(qr, a.scale));
+    gqf[ks] = M::from(scale_frag<T>(gqr, a.scale));
+    dof[ks] = M::from(load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g));
   }
   const int64_t ridx = (int64_t)bh * T_ + m;
   const float Dm = row_ok ? a.rowsum_in[ridx] : 0.f;
@@ -220,10 +220,10 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
   // c in all four accumulator slots.
   constexpr bool kMfmaSums = sizeof(T) == 2 && !GDO;  // GdO variants spill with it
   f32x4 xs4 = f32x4{0.f, 0.f, 0.f, 0.f}, ds4 = f32x4{0.f, 0.f, 0.f, 0.f};
-  frag ones;
+  mfrag ones;
   {
     const float one8[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
-    ones = vals_frag<T>(one8);
+    ones = M::vals(one8);
   }
 
   // Tiles are fetched in order t0, t0 + 1, ... through running pointers
@@ -280,13 +280,13 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
   };
   // One streamed tile (key block nb) from LDS tiles cK, cV, cgK, cgV; with
   // LOADP, p already holds its probabilities.
-  auto tile_body = [&](int nb, const T* cK, const T* cV, const T* cgK, const T* cgV, Tile& p)
+  auto tile_body = [&](int nb, const lds* cK, const lds* cV, const lds* cgK, const lds* cgV, Tile& p)
       __attribute__((always_inline)) {
     const int n0 = nb * kBlk;
     Tile dp, gds, gp1;
     if constexpr (!LOADP) {
       p.zero();
-      mm_d<T, D>(p, cK, qf);
+      mm_d<M>(p, cK, qf);
       recompute_p_row<T, XM>(p, a, brow, n0, lse2, kSl2);
     }
     if (mk.tile(nb)) {
@@ -305,12 +305,12 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
     }
     gds.zero();
     gp1.zero();
-    mm_d<T, D>(dp, cV, dof);
-    mm_d<T, D>(gds, cgK, qf);
-    mm_d<T, D>(gds, cK, gqf);
-    mm_d<T, D>(gp1, cgV, dof);
+    mm_d<M>(dp, cV, dof);
+    mm_d<M>(gds, cgK, qf);
+    mm_d<M>(gds, cK, gqf);
+    mm_d<M>(gp1, cgV, dof);
 
-    frag dsf[2], z1f[2], z2f[2], pf[2], z4f[2];
+    mfrag dsf[2], z1f[2], z2f[2], pf[2], z4f[2];
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb) {
       float vds[8], vz1[8], vz2[8], vz4[8];
@@ -333,24 +333,24 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
         vz2[j] = z2;
         vz4[j] = P * gd;
       }
-      dsf[kb] = vals_frag<T>(vds);
-      z1f[kb] = vals_frag<T>(vz1);
-      if constexpr (!DQ) z2f[kb] = vals_frag<T>(vz2);
+      dsf[kb] = M::vals(vds);
+      z1f[kb] = M::vals(vz1);
+      if constexpr (!DQ) z2f[kb] = M::vals(vz2);
       if constexpr (kMfmaSums) {
-        xs4 = E::mma(xs4, ones, z1f[kb]);
-        if constexpr (!DQ) ds4 = E::mma(ds4, ones, z2f[kb]);
+        xs4 = M::mma_all(xs4, ones, z1f[kb]);
+        if constexpr (!DQ) ds4 = M::mma_all(ds4, ones, z2f[kb]);
       }
-      pf[kb] = tile_frag<T>(p, kb);
-      if constexpr (GDO) z4f[kb] = vals_frag<T>(vz4);
+      pf[kb] = tile_frag<M>(p, kb);
+      if constexpr (GDO) z4f[kb] = M::vals(vz4);
     }
-    mm_s<T, D>(a1, cgK, dsf);
+    mm_s<M>(a1, cgK, dsf);
     if constexpr (DQ)
-      mm_s2<T, D>(a2, z1f, a4, pf, cK);
+      mm_s2<M>(a2, z1f, a4, pf, cK);
     else
-      mm_s3<T, D>(a2, z1f, a3, z2f, a4, pf, cK);
+      mm_s3<M>(a2, z1f, a3, z2f, a4, pf, cK);
     if constexpr (GDO) {
-      mm_s<T, D>(b1, cgV, pf);
-      mm_s2<T, D>(b2, z4f, b3, pf, cV);
+      mm_s<M>(b1, cgV, pf);
+      mm_s2<M>(b2, z4f, b3, pf, cV);
     }
   };
   auto p_from_frags = [&](Tile& p) __attribute__((always_inline)) {
@@ -431,10 +431,10 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
         __syncthreads();  // everyone's, and everyone is done with the other buffer
       } else {
         __syncthreads();
-        stage_store_rows<T, D>(s0, sK[0]);
-        stage_store_rows<T, D>(s1, sV[0]);
-        stage_store_rows<T, D>(s2, sgK[0]);
-        stage_store_rows<T, D>(s3, sgV[0]);
+        stage_store_tile<M>(s0, sK[0]);
+        stage_store_tile<M>(s1, sV[0]);
+        stage_store_tile<M>(s2, sgK[0]);
+        stage_store_tile<M>(s3, sgV[0]);
         __syncthreads();
       }
       Tile p;
@@ -509,30 +509,34 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, false>::value))) void k_gg_row(
 // ---------------------------------------------------------------------------
 template <typename T, int D, bool LOADP, bool XM>
 __global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(GgWaves<T, D, true>::value))) void k_gg_col(Params a, Params rowc, int nx) {
+__attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params a, Params rowc, int nx) {
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
   typedef Lds<T, kBlk> LP;
   // 16-bit types at D = 64 stream tiles straight into two LDS buffers
   // (TileDma), set 0 and set 1, in distinct arrays with a compile-time role per
   // loop step; the rest stage them through registers into set 0.
   constexpr bool kDma = L::kSwizzle;
   constexpr int kNS = LOADP ? 3 : 4;  // staged row statistics: D, E, F, then lse (recompute)
-  constexpr int kE1 = kDma ? L::kRowElems : 8;
+  constexpr int kE1 = kDma ? M::kElems : 8;
   constexpr int kP0 = LOADP ? LP::kRowElems : 8, kP1 = (LOADP && kDma) ? LP::kRowElems : 8;
-  __shared__ __align__(16) T sQ0[L::kRowElems];
-  __shared__ __align__(16) T sgQ0[L::kRowElems];
-  __shared__ __align__(16) T sdO0[L::kRowElems];
+  __shared__ __align__(16) lds sQ0[M::kElems];
+  __shared__ __align__(16) lds sgQ0[M::kElems];
+  __shared__ __align__(16) lds sdO0[M::kElems];
   __shared__ __align__(16) T sP0[kP0];
   __shared__ __align__(16) float sS0[kNS * kBlk];
-  __shared__ __align__(16) T sQ1[kE1];
-  __shared__ __align__(16) T sgQ1[kE1];
-  __shared__ __align__(16) T sdO1[kE1];
+  __shared__ __align__(16) lds sQ1[kE1];
+  __shared__ __align__(16) lds sgQ1[kE1];
+  __shared__ __align__(16) lds sdO1[kE1];
   __shared__ __align__(16) T sP1[kP1];
   __shared__ __align__(16) float sS1[kDma ? kNS * kBlk : 4];
   struct Bufs {
-    T *q, *gq, *dout, *p;
+    lds *q, *gq, *dout;
+    T* p;
     float* st;
   };
   auto bufs = [&](auto par) __attribute__((always_inline)) -> Bufs {
@@ -587,15 +591,18 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, true>::value))) void k_gg_col(P
   // Stationary fragments negated (K and gK also scaled by s): the products
   // that start from the staged row statistics come out as D - dP, E - gdS
   // and G - gP1 (G = F + E D), and the scores of the recomputed P as -s q.k.
-  frag kf[D / 32], gkf[D / 32], vf[D / 32], gvf[D / 32];
+  mfrag kf[D / 32], gkf[D / 32], vf[D / 32], gvf[D / 32];
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
-    kf[ks] = scale_frag<T>(load_frag_row<T>(K, a.k.st, n, T_, 32 * ks + 8 * g), -a.scale);
-    gkf[ks] = scale_frag<T>(load_frag_row<T>(gK, a.gk.st, n, T_, 32 * ks + 8 * g), -a.scale);
-    vf[ks] = scale_frag<T>(load_frag_row<T>(V, a.v.st, n, T_, 32 * ks + 8 * g), -1.f);
-    gvf[ks] = scale_frag<T>(load_frag_row<T>(gV, a.gv.st, n, T_, 32 * ks + 8 * g), -1.f);
+    kf[ks] = M::from(scale_frag<T>(load_frag_row<T>(K, a.k.st, n, T_, 32 * ks + 8 * g), -a.scale));
+    gkf[ks] = M::from(scale_frag<T>(load_frag_row<T>(gK, a.gk.st, n, T_, 32 * ks + 8 * g), -a.scale));
+    vf[ks] = M::from(scale_frag<T>(load_frag_row<T>(V, a.v.st, n, T_, 32 * ks + 8 * g), -1.f));
+    gvf[ks] = M::from(scale_frag<T>(load_frag_row<T>(gV, a.gv.st, n, T_, 32 * ks + 8 * g), -1.f));
     // kept as computed (left to itself the compiler redoes a negation per tile)
-    asm volatile("" : "+v"(kf[ks]), "+v"(gkf[ks]), "+v"(vf[ks]), "+v"(gvf[ks]));
+    M::keep(kf[ks]);
+    M::keep(gkf[ks]);
+    M::keep(vf[ks]);
+    M::keep(gvf[ks]);
   }
 
   f32x4 acc_gk[D / 16], acc_gv[D / 16];
@@ -615,7 +622,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, true>::value))) void k_gg_col(P
       }
     } else {
       p.zero();
-      mm_d<T, D>(p, cb.q, kf);  // -s q.k
+      mm_d<M>(p, cb.q, kf);  // -s q.k
       recompute_p_col<T, XM>(p, a, bcol, m0, cb.st, 3, -kSl2);
     }
     if (mk.tile(mb)) {
@@ -647,9 +654,9 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, true>::value))) void k_gg_col(P
         for (int i = 0; i < 4; ++i) g4[i] = f8[4 * h2 + i] + e8[4 * h2 + i] * d8[4 * h2 + i];
         gp1.q[2 * kb + h2] = g4;
       }
-      mm_d2_half<T, D>(dp, gp1, kb, cb.dout, vf, gvf);
-      mm_d_half<T, D>(gds, kb, cb.gq, kf);
-      mm_d_half<T, D>(gds, kb, cb.q, gkf);
+      mm_d2_half<M>(dp, gp1, kb, cb.dout, vf, gvf);
+      mm_d_half<M>(gds, kb, cb.gq, kf);
+      mm_d_half<M>(gds, kb, cb.q, gkf);
       float vds[8], vgs[8], vgdp[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -660,9 +667,9 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, true>::value))) void k_gg_col(P
         vgdp[j] = P * ng;
         vgs[j] = P * (gp1.at(kb, j) - ng * nd);
       }
-      mm_s_half<T, D>(acc_gk, kb, cb.gq, vals_frag<T>(vds));
-      mm_s_half<T, D>(acc_gk, kb, cb.q, vals_frag<T>(vgs));
-      mm_s_half<T, D>(acc_gv, kb, cb.dout, vals_frag<T>(vgdp));
+      mm_s_half<M>(acc_gk, kb, cb.gq, M::vals(vds));
+      mm_s_half<M>(acc_gk, kb, cb.q, M::vals(vgs));
+      mm_s_half<M>(acc_gv, kb, cb.dout, M::vals(vgdp));
     }
   };
 
@@ -733,9 +740,9 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D, true>::value))) void k_gg_col(P
     load_tile(cr.t0);
     for (int mb = cr.t0; mb < cr.t1; ++mb) {
       __syncthreads();
-      stage_store_rows<T, D>(s0, sQ0);
-      stage_store_rows<T, D>(s1, sgQ0);
-      stage_store_rows<T, D>(s2, sdO0);
+      stage_store_tile<M>(s0, sQ0);
+      stage_store_tile<M>(s1, sgQ0);
+      stage_store_tile<M>(s2, sdO0);
       if constexpr (LOADP) stage_store_rows<T, kBlk>(sp, sP0);
       stat_store<kNS>(stv, sS0);
       __syncthreads();
@@ -782,6 +789,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
   typedef Lds<T, kBlk> LP;
   constexpr int kNS = LOADP ? 3 : 4;  // staged row statistics: D, E, F, then lse (recompute)
   constexpr int kP = LOADP ? LP::kRowElems : 8;
@@ -885,7 +893,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
       for (int j = 0; j < 8; ++j) p.set(0, j, E::f32(pf[j]));
     } else {
       p.zero();
-      mm_d_half<T, D>(p, 0, cb.q + hq, kf);
+      mm_d_half<M>(p, 0, cb.q + hq, kf);
       float l2[8];
       stat_read8(l2, st, 3, 0);
 #pragma unroll
@@ -910,9 +918,9 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
       for (int i = 0; i < 4; ++i) g4[i] = f8[4 * h2 + i] + e8[4 * h2 + i] * d8[4 * h2 + i];
       gp1.q[h2] = g4;
     }
-    mm_d2_half<T, D>(dp, gp1, 0, cb.dout + hq, vf, gvf);
-    mm_d_half<T, D>(gds, 0, cb.gq + hq, kf);
-    mm_d_half<T, D>(gds, 0, cb.q + hq, gkf);
+    mm_d2_half<M>(dp, gp1, 0, cb.dout + hq, vf, gvf);
+    mm_d_half<M>(gds, 0, cb.gq + hq, kf);
+    mm_d_half<M>(gds, 0, cb.q + hq, gkf);
     float vds[8], vgs[8], vgdp[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -924,20 +932,20 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
       vgs[j] = P * (gp1.at(0, j) - ng * nd);
     }
     if constexpr (HALF == 0) {
-      xk[128] = vals_frag<T>(vgdp);
-      mm_s_half<T, D>(acc, 0, cb.gq + hq, vals_frag<T>(vds));
-      mm_s_half<T, D>(acc, 0, cb.q + hq, vals_frag<T>(vgs));
+      xk[128] = M::vals(vgdp);
+      mm_s_half<M>(acc, 0, cb.gq + hq, M::vals(vds));
+      mm_s_half<M>(acc, 0, cb.q + hq, M::vals(vgs));
     } else {
-      xk[0] = vals_frag<T>(vds);
-      xk[64] = vals_frag<T>(vgs);
-      mm_s_half<T, D>(acc, 0, cb.dout + hq, vals_frag<T>(vgdp));
+      xk[0] = M::vals(vds);
+      xk[64] = M::vals(vgs);
+      mm_s_half<M>(acc, 0, cb.dout + hq, M::vals(vgdp));
     }
     __syncthreads();  // the partner's operands are in sX
     if constexpr (HALF == 0) {
-      mm_s_half<T, D>(acc, 0, cb.gq + oq, xk[0]);
-      mm_s_half<T, D>(acc, 0, cb.q + oq, xk[64]);
+      mm_s_half<M>(acc, 0, cb.gq + oq, xk[0]);
+      mm_s_half<M>(acc, 0, cb.q + oq, xk[64]);
     } else {
-      mm_s_half<T, D>(acc, 0, cb.dout + oq, xk[128]);
+      mm_s_half<M>(acc, 0, cb.dout + oq, xk[128]);
     }
   };
 
@@ -1040,6 +1048,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
+  typedef Mm<T, D> M;
   __shared__ __align__(16) T pK0[L::kRowElems];
   __shared__ __align__(16) T pV0[L::kRowElems];
   __shared__ __align__(16) T pgK0[L::kRowElems];
@@ -1114,7 +1123,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   frag ones;
   {
     const float one8[8] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
-    ones = vals_frag<T>(one8);
+    ones = M::vals(one8);
   }
 
   // Key tile nb (its 32-key half HALF) from LDS tiles cK, cV, cgK, cgV; with
@@ -1129,7 +1138,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
     Tile dp, gds, gp1;
     if constexpr (!LOADP) {
       p.zero();
-      mm_d_half<T, D>(p, 0, cK + hk, qf);
+      mm_d_half<M>(p, 0, cK + hk, qf);
 #pragma unroll
       for (int j = 0; j < 8; ++j) p.set(0, j, fast_exp2(p.at(0, j) * kSl2 - lse2));
     }
@@ -1154,11 +1163,11 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
       frag dof[D / 32];
 #pragma unroll
       for (int ks = 0; ks < D / 32; ++ks) dof[ks] = sdo[64 * ks + z];
-      mm_d_half<T, D>(dp, 0, cV + hk, dof);
-      mm_d_half<T, D>(gp1, 0, cgV + hk, dof);
+      mm_d_half<M>(dp, 0, cV + hk, dof);
+      mm_d_half<M>(gp1, 0, cgV + hk, dof);
     }
-    mm_d_half<T, D>(gds, 0, cgK + hk, qf);
-    mm_d_half<T, D>(gds, 0, cK + hk, gqf);
+    mm_d_half<M>(gds, 0, cgK + hk, qf);
+    mm_d_half<M>(gds, 0, cK + hk, gqf);
     float vds[8], vz1[8], vz2[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -1175,15 +1184,15 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
         x_acc += vz1[j];
       }
     }
-    const frag z1f = vals_frag<T>(vz1);
+    const frag z1f = M::vals(vz1);
     xs4 = E::mma(xs4, ones, z1f);
-    mm_s_half<T, D>(a12, 0, cgK + hk, vals_frag<T>(vds));
+    mm_s_half<M>(a12, 0, cgK + hk, M::vals(vds));
     if constexpr (DQ) {
-      mm_s2_half<T, D>(a12, z1f, a4, tile_frag<T>(p, 0), 0, cK + hk);
+      mm_s2_half<M>(a12, z1f, a4, tile_frag<M>(p, 0), 0, cK + hk);
     } else {
-      const frag z2f = vals_frag<T>(vz2);
+      const frag z2f = M::vals(vz2);
       ds4 = E::mma(ds4, ones, z2f);
-      mm_s3_half<T, D>(a12, z1f, a3, z2f, a4, tile_frag<T>(p, 0), 0, cK + hk);
+      mm_s3_half<M>(a12, z1f, a3, z2f, a4, tile_frag<M>(p, 0), 0, cK + hk);
     }
   };
 
