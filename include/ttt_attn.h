@@ -139,6 +139,15 @@ typedef struct ttt_problem {
                           shape (triton_attention.py:78-85).      */
 } ttt_problem;
 
+/* Shape of a problem whose operands are not square (the *_shape entry points):
+ * queries and keys of different number.  With keys != seqlen the problem is
+ * neither causal nor windowed; q, o, dout, gq, dq and gq_out, gdout have
+ * seqlen rows, k, v, gk, gv, dk, dv, gk_out and gv_out have `keys` rows, P and
+ * the bias are [B,H,seqlen,keys], row statistics stay [B*H*seqlen]. */
+typedef struct ttt_shape {
+  int64_t keys; /* key and value rows; 0 = seqlen */
+} ttt_shape;
+
 /* Library version (major*10000 + minor*100 + patch). */
 int ttt_version(void);
 
@@ -151,6 +160,10 @@ const char* ttt_last_error(void);
  * reference counterpart: the reference's kernels are not split.
  */
 int64_t ttt_attn_workspace_size(const ttt_problem* pr, int32_t entry, int32_t want_gdout);
+
+/* The same for a *_shape entry point (shape NULL: square). */
+int64_t ttt_attn_workspace_size_shape(const ttt_problem* pr, const ttt_shape* shape, int32_t entry,
+                                      int32_t want_gdout);
 
 /*
  * The split a single-family entry (FWD, FWD_P, BWD_DQ, BWD_DKDV, GG_ROW,
@@ -215,6 +228,12 @@ int ttt_attn_fwd(const ttt_problem* pr, const ttt_view* q, const ttt_view* k,
                  const ttt_view* p, void* workspace,
                  int64_t workspace_bytes, void* stream);
 
+/* ttt_attn_fwd with a ttt_shape (NULL: square), as for GradGradAttentionFn's
+ * rectangular problems (cloud_ttt_e2e/ttt_e2e/attention.py:9-53). */
+int ttt_attn_fwd_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                       const ttt_view* k, const ttt_view* v, const ttt_view* o, float* lse,
+                       const ttt_view* p, void* workspace, int64_t workspace_bytes, void* stream);
+
 /*
  * Zeros into the tiles of P that ttt_attn_fwd leaves unwritten (causal: the
  * tiles past the diagonal and, with a window, before each row block's first
@@ -274,6 +293,13 @@ int ttt_attn_bwd(const ttt_problem* pr, const ttt_view* q, const ttt_view* k,
                  const float* lse, const ttt_view* p, float* rowsum_out,
                  const ttt_view* dq, const ttt_view* dk, const ttt_view* dv,
                  void* workspace, int64_t workspace_bytes, void* stream);
+
+/* ttt_attn_bwd with a ttt_shape (NULL: square). */
+int ttt_attn_bwd_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                       const ttt_view* k, const ttt_view* v, const ttt_view* o,
+                       const ttt_view* dout, const float* lse, const ttt_view* p,
+                       float* rowsum_out, const ttt_view* dq, const ttt_view* dk,
+                       const ttt_view* dv, void* workspace, int64_t workspace_bytes, void* stream);
 
 /*
  * Row statistic from P, with the reference's definition
@@ -340,6 +366,15 @@ int ttt_attn_gg(const ttt_problem* pr, const ttt_view* q, const ttt_view* k,
                 const ttt_view* gv_out, const ttt_view* gdout, float* e_buf,
                 float* f_buf, void* workspace, int64_t workspace_bytes,
                 void* stream);
+
+/* ttt_attn_gg with a ttt_shape (NULL: square). */
+int ttt_attn_gg_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                      const ttt_view* k, const ttt_view* v, const ttt_view* dout, const float* lse,
+                      const ttt_view* p, const float* rowsum, const ttt_view* dq,
+                      const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
+                      const ttt_view* gq_out, const ttt_view* gk_out, const ttt_view* gv_out,
+                      const ttt_view* gdout, float* e_buf, float* f_buf, void* workspace,
+                      int64_t workspace_bytes, void* stream);
 
 /*
  * ttt_attn_gg with no device memory allocation: the same double backward,

@@ -201,16 +201,21 @@ def kernel_timing():
         _timing = prev
 
 
-def _timed(name: str, *args) -> None:
+def _timed_call(name: str, fn, *args):
+    """fn(*args), between two events under `name` while timing is active."""
     if _timing is None:
-        _call(name, *args)
-        return
+        return fn(*args)
     s = torch.cuda.Event(enable_timing=True)
     e = torch.cuda.Event(enable_timing=True)
     s.record()
-    _call(name, *args)
+    out = fn(*args)
     e.record()
     _timing.setdefault(name, []).append((s, e))
+    return out
+
+
+def _timed(name: str, *args) -> None:
+    _timed_call(name, _call, name, *args)
 
 
 def mean_ms(rec: Dict[str, List[Tuple[torch.cuda.Event, torch.cuda.Event]]]) -> Dict[str, float]:
@@ -409,12 +414,16 @@ def _fwd_config(x: torch.Tensor, m, scale: float, run) -> Tuple[int, int]:
     return autotune.choose(key, options, run)
 
 
-def prep_bias(bias: torch.Tensor, b: int, h: int, t: int, dtype: torch.dtype, device) -> torch.Tensor:
-    """An additive score bias broadcastable to [b,h,t,t] as the kernels read
-    it: `dtype` (the input dtype), an expanded [b,h,t,t] view whose broadcast
-    dimensions have stride 0, unit column stride, 16-byte aligned base and
-    strides, and rows readable up to t rounded up to 8 elements.  Copies only when the given
-    tensor does not already satisfy this.  The bias receives no gradient."""
+def prep_bias(bias: torch.Tensor, b: int, h: int, t: int, dtype: torch.dtype, device,
+              tk: Optional[int] = None) -> torch.Tensor:
+    """An additive score bias broadcastable to [b,h,t,tk] (tk: t unless given)
+    as the kernels read it: `dtype` (the input dtype), an expanded [b,h,t,tk]
+    view whose broadcast dimensions have stride 0, unit column stride, 16-byte
+    aligned base and strides, and rows readable up to tk rounded up to 8
+    elements.  Copies only when the given tensor does not already satisfy
+    this.  The bias receives no gradient."""
+    if tk is None:
+        tk = t
     x = bias.detach()
     if x.dtype != dtype:
         x = x.to(dtype)
@@ -425,19 +434,19 @@ def prep_bias(bias: torch.Tensor, b: int, h: int, t: int, dtype: torch.dtype, de
     while x.dim() < 4:
         x = x.unsqueeze(0)
     try:
-        full = x.expand(b, h, t, t)
+        full = x.expand(b, h, t, tk)
     except RuntimeError as e:
         raise ValueError(f"attn_mask of shape {tuple(bias.shape)} does not broadcast to "
-                         f"{(b, h, t, t)}") from e
+                         f"{(b, h, t, tk)}") from e
     eb = x.element_size()
-    tp = (t + ROW_READ - 1) // ROW_READ * ROW_READ
+    tp = (tk + ROW_READ - 1) // ROW_READ * ROW_READ
     if (full.stride(-1) == 1 and full.data_ptr() % 16 == 0
             and all((s * eb) % 16 == 0 for s in full.stride()[:3]) and _rows_readable(full)):
         return full
     keep = tuple(1 if x.size(i) == 1 else n for i, n in enumerate((b, h, t)))
     buf = torch.empty(keep + (tp,), dtype=x.dtype, device=x.device)
-    buf[..., :t].copy_(x.expand(keep + (t,)))
-    return buf[..., :t].expand(b, h, t, t)
+    buf[..., :tk].copy_(x.expand(keep + (tk,)))
+    return buf[..., :tk].expand(b, h, t, tk)
 
 
 _ws_sizes: Dict[tuple, int] = {}
@@ -524,6 +533,10 @@ def fwd(q, k, v, mask, scale: float, want_p: bool):
     if _library_choice():
         return tuple(ext().fwd(q, k, v, m.causal, float(scale), bool(want_p), 0, int(m.window), int(m.window_kind),
                                m.bias, 0))
+    if k.shape[2] != q.shape[2]:
+        # fewer or more keys than queries: one entry call, never tuned
+        return tuple(_timed_call("ttt_attn_fwd", ext().fwd, q, k, v, m.causal, float(scale), bool(want_p),
+                                 _split_chunk, int(m.window), int(m.window_kind), m.bias, _block_rows))
     ent = ENTRY_FWD_P if want_p else ENTRY_FWD
 
     def run(c, rows=0):
@@ -557,7 +570,10 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
     lp = p is not None
     if _library_choice():
         return tuple(ext().bwd_fused(q, k, v, o, do, lse, p, m.causal, float(scale), int(m.window),
-                                     int(m.window_kind), m.bias))
+                                     int(m.window_kind), m.bias, 0))
+    if k.shape[2] != q.shape[2]:
+        return tuple(_timed_call("ttt_attn_bwd", ext().bwd_fused, q, k, v, o, do, lse, p, m.causal, float(scale),
+                                 int(m.window), int(m.window_kind), m.bias, _split_chunk))
 
     def run(cq, ck):
         return ext().bwd(q, k, v, o, do, lse, p, m.causal, float(scale), cq, ck, int(m.window), int(m.window_kind),
@@ -568,7 +584,7 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
     if _timing is None:
         if cq == 0 and ck == 0:
             return tuple(ext().bwd_fused(q, k, v, o, do, lse, p, m.causal, float(scale), int(m.window),
-                                         int(m.window_kind), m.bias))
+                                         int(m.window_kind), m.bias, 0))
         return tuple(run(cq, ck))
     q, k, v, o, do = _ready(q), _ready(k), _ready(v), _ready(o), _ready(do)
     dq = _empty_like_out(q)
@@ -655,7 +671,11 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
                              f"{tuple(dq.shape)} {dq.dtype} {dq.device}")
     if _library_choice():
         return tuple(ext().gg_fused(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale),
-                                    bool(want_gdo), int(m.window), int(m.window_kind), m.bias))
+                                    bool(want_gdo), int(m.window), int(m.window_kind), m.bias, 0))
+    if k.shape[2] != q.shape[2]:
+        return tuple(_timed_call("ttt_attn_gg", ext().gg_fused, q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal,
+                                 float(scale), bool(want_gdo), int(m.window), int(m.window_kind), m.bias,
+                                 _split_chunk))
 
     def run(cr, cc):
         return ext().gg(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale), bool(want_gdo), cr,
@@ -666,7 +686,7 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
     if _timing is None:
         if cr == 0 and cc == 0:
             return tuple(ext().gg_fused(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale),
-                                        bool(want_gdo), int(m.window), int(m.window_kind), m.bias))
+                                        bool(want_gdo), int(m.window), int(m.window_kind), m.bias, 0))
         return tuple(run(cr, cc))
     q, k, v, do, dq, gq, gk, gv = (_ready(t) for t in (q, k, v, do, dq, gq, gk, gv))
     gq_out = _empty_like_out(q)
@@ -753,5 +773,7 @@ def launch_timing(capacity: int = 4096):
 
 def exported_symbols() -> List[str]:
     """Names of the C entry points this binding uses (for ABI checks)."""
-    return list(_SIGS) + ["ttt_last_error", "ttt_version", "ttt_attn_workspace_size", "ttt_attn_split_info",
+    return list(_SIGS) + ["ttt_attn_workspace_size_shape", "ttt_attn_fwd_shape", "ttt_attn_bwd_shape",
+                          "ttt_attn_gg_shape", "ttt_last_error", "ttt_version", "ttt_attn_workspace_size",
+                          "ttt_attn_split_info",
                           "ttt_attn_launch_item", "ttt_kernel_timing", "ttt_kernel_timing_read"]

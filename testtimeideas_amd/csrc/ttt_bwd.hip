@@ -124,13 +124,14 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
   if (it.blk < 0) return;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -184,11 +185,11 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (!LOADP) {
       // Recompute: tile-indexed clamped loads, measured faster for this
       // variant than the running-pointer form below.
-      stage_load<T, D>(stK, K + (int64_t)n1 * a.k.st, a.k.st, T_ - n1, D);
-      stage_load<T, D>(stV, V + (int64_t)n1 * a.v.st, a.v.st, T_ - n1, D);
+      stage_load<T, D>(stK, K + (int64_t)n1 * a.k.st, a.k.st, Tk_ - n1, D);
+      stage_load<T, D>(stV, V + (int64_t)n1 * a.v.st, a.v.st, Tk_ - n1, D);
       return;
     }
-    if (n1 + kBlk <= T_) {
+    if (n1 + kBlk <= Tk_) {
       stage_load_full<T, D>(stK, Kn, soK);
       stage_load_full<T, D>(stV, Vn, soV);
       if constexpr (LOADP) {
@@ -196,9 +197,9 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
         pn[1] = load_frag_g<T>(Pn + 32);
       }
     } else {
-      stage_load<T, D>(stK, Kn, a.k.st, T_ - n1, D);
-      stage_load<T, D>(stV, Vn, a.v.st, T_ - n1, D);
-      if constexpr (LOADP) load_p_frags<T>(pn, Pm, n1, T_);
+      stage_load<T, D>(stK, Kn, a.k.st, Tk_ - n1, D);
+      stage_load<T, D>(stV, Vn, a.v.st, Tk_ - n1, D);
+      if constexpr (LOADP) load_p_frags<T>(pn, Pm, n1, Tk_);
     }
     Kn += kBlk * a.k.st;
     Vn += kBlk * a.v.st;
@@ -213,7 +214,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   }
   auto fetch_dma = [&](int nb, auto par) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
-    if (n1 + kBlk <= T_) {
+    if (n1 + kBlk <= Tk_) {
       dd.load_full(set_k(par), Kn, oK);
       dd.load_full(set_v(par), Vn, oV);
       if constexpr (LOADP) {
@@ -221,9 +222,9 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
         pn[1] = load_frag_g<T>(Pn + 32);
       }
     } else {
-      dd.load_ragged(set_k(par), Kn, a.k.st, T_ - n1, D);
-      dd.load_ragged(set_v(par), Vn, a.v.st, T_ - n1, D);
-      if constexpr (LOADP) load_p_frags<T>(pn, Pm, n1, T_);
+      dd.load_ragged(set_k(par), Kn, a.k.st, Tk_ - n1, D);
+      dd.load_ragged(set_v(par), Vn, a.v.st, Tk_ - n1, D);
+      if constexpr (LOADP) load_p_frags<T>(pn, Pm, n1, Tk_);
       dma_wait();
     }
     Kn += kBlk * a.k.st;
@@ -383,7 +384,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       return Bufs{sdO1, sQ1, kMix ? sP0 : sP1, sS1};
   };
 
-  const int T_ = a.T;
+  const int T_ = a.Tk;  // keys: the stationary rows
+  const int Tq_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const Slot sl = grid_slot();
   // Workgroups past the first nx columns of the grid finish the preceding dQ
@@ -397,7 +399,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   if (it.blk < 0) return;
   const int nb = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
-  const Range rg = col_block_range(nb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = col_block_range(nb, nblk, Tq_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int n0 = nb * kBlk;
@@ -412,8 +414,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const T* V = at<const T>(a.v, b, h);
   const T* dO = at<const T>(a.dout, b, h);
   const T* Pb = LOADP ? at<const T>(a.p, b, h) : nullptr;
-  const float* rs = DV_ONLY ? nullptr : a.rowsum_in + (int64_t)bh * T_;
-  const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * T_;
+  const float* rs = DV_ONLY ? nullptr : a.rowsum_in + (int64_t)bh * Tq_;
+  const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * Tq_;
 
   mfrag vf[D / 32], kf[D / 32];
 #pragma unroll
@@ -443,10 +445,10 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const bool cols_full = n0 + kBlk <= T_;
   auto load_tile = [&](int mb) __attribute__((always_inline)) {
     const int m0 = mb * kBlk;
-    stage_load<T, D>(stdO, dOn, a.dout.st, T_ - m0, D);
-    if constexpr (kNeedQ) stage_load<T, D>(stQ, Qn, a.q.st, T_ - m0, D);
-    if constexpr (LOADP) stage_load<T, kBlk>(stP, Pn, a.p.st, T_ - m0, T_ - n0);
-    if constexpr (kNS > 0) stv = stat_load<kNS>(DV_ONLY ? lse : rs, lse, nullptr, nullptr, m0, T_ - m0);
+    stage_load<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, D);
+    if constexpr (kNeedQ) stage_load<T, D>(stQ, Qn, a.q.st, Tq_ - m0, D);
+    if constexpr (LOADP) stage_load<T, kBlk>(stP, Pn, a.p.st, Tq_ - m0, T_ - n0);
+    if constexpr (kNS > 0) stv = stat_load<kNS>(DV_ONLY ? lse : rs, lse, nullptr, nullptr, m0, Tq_ - m0);
     dOn += kBlk * a.dout.st;
     if constexpr (kNeedQ) Qn += kBlk * a.q.st;
     if constexpr (LOADP) Pn += kBlk * a.p.st;
@@ -466,18 +468,18 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     if constexpr (kDma) {
       const int m0 = mb * kBlk;
       const Bufs bf = bufs(par);
-      if (m0 + kBlk <= T_ && cols_full) {
+      if (m0 + kBlk <= Tq_ && cols_full) {
         dd.load_full(bf.dout, dOn, odO);
         dd.load_full(bf.q, Qn, oQ);
         if constexpr (LOADP && !kMix) dpt.load_full(bf.p, Pn, oP);
       } else {
-        dd.load_ragged(bf.dout, dOn, a.dout.st, T_ - m0, D);
-        dd.load_ragged(bf.q, Qn, a.q.st, T_ - m0, D);
-        if constexpr (LOADP && !kMix) dpt.load_ragged(bf.p, Pn, a.p.st, T_ - m0, T_ - n0);
+        dd.load_ragged(bf.dout, dOn, a.dout.st, Tq_ - m0, D);
+        dd.load_ragged(bf.q, Qn, a.q.st, Tq_ - m0, D);
+        if constexpr (LOADP && !kMix) dpt.load_ragged(bf.p, Pn, a.p.st, Tq_ - m0, T_ - n0);
         dma_wait();
       }
-      sdma.load(bf.st, m0, T_ - m0);
-      if constexpr (kMix) stage_load<T, kBlk>(stP, Pn, a.p.st, T_ - m0, T_ - n0);
+      sdma.load(bf.st, m0, Tq_ - m0);
+      if constexpr (kMix) stage_load<T, kBlk>(stP, Pn, a.p.st, Tq_ - m0, T_ - n0);
       dOn += kBlk * a.dout.st;
       Qn += kBlk * a.q.st;
       if constexpr (LOADP) Pn += kBlk * a.p.st;
@@ -610,6 +612,7 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   const Slot sl = grid_slot();
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const int mb = a.causal ? (nblk - 1 - sl.x) : sl.x;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int m = mb * kBlk + 16 * w + c;
@@ -623,18 +626,18 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   for (int ks = 0; ks < D / 32; ++ks) dof[ks] = M::from(load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g));
 
   float sum = 0.f;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const RowMask<XM> mk(a, mb, m);
   Stage<T, D> stV;
-  stage_load<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, T_ - rg.lo * kBlk, D);
+  stage_load<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, D);
   for (int nb = rg.lo; nb < rg.hi; ++nb) {
     const int n0 = nb * kBlk;
     __syncthreads();
     stage_store_tile<M>(stV, sV);
     __syncthreads();
-    if (nb + 1 < rg.hi) stage_load<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, T_ - n0 - kBlk, D);
+    if (nb + 1 < rg.hi) stage_load<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, Tk_ - n0 - kBlk, D);
     frag pr[2];
-    load_p_frags<T>(pr, Pm, n0, T_);
+    load_p_frags<T>(pr, Pm, n0, Tk_);
     Tile p, dp;
     frags_to_tile<T>(p, pr);
     if (mk.tile(nb)) {
@@ -697,10 +700,9 @@ static void launch_dkdv_x(const Params& a, bool load_p, bool dv_only, dim3 grid,
 template <typename T, int D>
 static hipError_t launch_dkdv_t(int dtype, const Params& a, bool load_p, bool dv_only, hipStream_t st,
                                 const Params* dqc) {
-  const int nblk = (a.T + kBlk - 1) / kBlk;
-  const int nx = nblk * a.nchunk_max;
+  const int nx = (a.Tk + kBlk - 1) / kBlk * a.nchunk_max;
   const bool fold = dqc && dqc->nchunk_max > 1;
-  dim3 grid(nx + (fold ? nblk * CombineSlot<D>::kSub : 0), a.B * a.H);
+  dim3 grid(nx + (fold ? (a.T + kBlk - 1) / kBlk * CombineSlot<D>::kSub : 0), a.B * a.H);
   const Params& c = fold ? *dqc : a;
   if (extended_mask(a))
     launch_dkdv_x<T, D, true>(a, load_p, dv_only, grid, st, c, nx);

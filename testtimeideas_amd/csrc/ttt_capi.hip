@@ -85,8 +85,14 @@ size_t elem_bytes(int dtype) { return dtype == TTT_F32 ? 4 : 2; }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// A problem with its key count: q, o, dout and their gradients have seqlen
+// rows, k, v and theirs `keys`, P and the bias are [B,H,seqlen,keys].
+struct Prob : ttt_problem {
+  int64_t keys;
+};
+
 // Checks a [B,H,T,X] operand and copies it into a kernel View.
-int take_view(const ttt_problem* pr, const ttt_view* v, const char* name, ttt::View* out) {
+int take_view(const Prob* pr, const ttt_view* v, const char* name, ttt::View* out) {
   if (!v || !v->data) return fail(TTT_ERR_INVALID_ARGUMENT, "%s: null pointer", name);
   if (!aligned16(v->data)) return fail(TTT_ERR_INVALID_ARGUMENT, "%s: base pointer not 16-byte aligned", name);
   const size_t eb = elem_bytes(pr->dtype);
@@ -102,8 +108,7 @@ int take_view(const ttt_problem* pr, const ttt_view* v, const char* name, ttt::V
   return TTT_OK;
 }
 
-int check_problem(const ttt_problem* pr) {
-  if (!pr) return fail(TTT_ERR_INVALID_ARGUMENT, "problem: null pointer");
+int check_problem(const Prob* pr) {
   if (pr->dtype != TTT_F16 && pr->dtype != TTT_BF16 && pr->dtype != TTT_F32)
     return fail(TTT_ERR_UNSUPPORTED, "dtype code %d is not f16/bf16/f32", pr->dtype);
   if (pr->head_dim != 64 && pr->head_dim != 128)
@@ -115,6 +120,11 @@ int check_problem(const ttt_problem* pr) {
     return fail(TTT_ERR_INVALID_ARGUMENT, "batch*heads = %lld exceeds 65535", (long long)(pr->batch * pr->heads));
   if (pr->seqlen > (int64_t)1 << 24)
     return fail(TTT_ERR_INVALID_ARGUMENT, "seqlen %lld exceeds 2^24", (long long)pr->seqlen);
+  if (pr->keys < 1 || pr->keys > (int64_t)1 << 24)
+    return fail(TTT_ERR_INVALID_ARGUMENT, "keys %lld: must be 1 .. 2^24", (long long)pr->keys);
+  if (pr->keys != pr->seqlen && (pr->causal != 0 || pr->window != 0))
+    return fail(TTT_ERR_INVALID_ARGUMENT, "%lld keys for %lld queries: neither causal nor windowed",
+                (long long)pr->keys, (long long)pr->seqlen);
   if (pr->causal != 0 && pr->causal != 1) return fail(TTT_ERR_INVALID_ARGUMENT, "causal must be 0 or 1");
   if (pr->split_chunk < 0) return fail(TTT_ERR_INVALID_ARGUMENT, "split_chunk must be >= 0");
   if (pr->window < 0) return fail(TTT_ERR_INVALID_ARGUMENT, "window must be >= 0");
@@ -133,10 +143,18 @@ int check_problem(const ttt_problem* pr) {
   return TTT_OK;
 }
 
-// The window the kernels apply: W >= T sees every earlier key, i.e. none.
-int eff_window(const ttt_problem* pr) { return pr->window > 0 && pr->window < pr->seqlen ? pr->window : 0; }
+// The checked problem of an entry point (shape NULL: square).
+int make_prob(const ttt_problem* pr, const ttt_shape* shape, Prob* out) {
+  if (!pr) return fail(TTT_ERR_INVALID_ARGUMENT, "problem: null pointer");
+  static_cast<ttt_problem&>(*out) = *pr;
+  out->keys = shape && shape->keys != 0 ? shape->keys : pr->seqlen;
+  return check_problem(out);
+}
 
-bool has_xm(const ttt_problem* pr) { return eff_window(pr) > 0 || pr->bias.data != nullptr; }
+// The window the kernels apply: W >= T sees every earlier key, i.e. none.
+int eff_window(const Prob* pr) { return pr->window > 0 && pr->window < pr->seqlen ? pr->window : 0; }
+
+bool has_xm(const Prob* pr) { return eff_window(pr) > 0 || pr->bias.data != nullptr; }
 
 struct Split {
   int nblk, chunk, nchunk_max;
@@ -168,7 +186,7 @@ int device_cus(int* dev_out) {
 
 // Workgroup slots of family `fam`'s kernel (variant load_p) on the current
 // device; cached per (device, family, dtype, head dim, variant).
-int64_t family_slots(const ttt_problem* pr, int fam, bool load_p) {
+int64_t family_slots(const Prob* pr, int fam, bool load_p) {
   static std::atomic<int> per_cu[16][ttt::kNumFams][3][2][2][2];
   int dev = 0;
   const int cus = device_cus(&dev);
@@ -201,18 +219,20 @@ int64_t family_slots(const ttt_problem* pr, int fam, bool load_p) {
   return std::max<int64_t>(1, (int64_t)cus * n * kSlotFill / 100);
 }
 
+int blocks(int64_t rows) { return (int)((rows + ttt::kBlk - 1) / ttt::kBlk); }
+
 bool column_family(int fam) { return fam == ttt::kFamDkdv || fam == ttt::kFamGgCol; }
 
 // Streamed tiles of each block of a slice in launch order: row kernels issue
 // row block nblk-1-i first when causal (block i otherwise), column kernels
 // column block i.  Plain causal gives nblk, nblk-1, ..., 1.
-std::vector<int64_t> block_tiles(const ttt_problem* pr, bool col) {
-  const int T = (int)pr->seqlen, nblk = (T + ttt::kBlk - 1) / ttt::kBlk;
+std::vector<int64_t> block_tiles(const Prob* pr, bool col) {
+  const int T = (int)pr->seqlen, nblk = blocks(col ? pr->keys : pr->seqlen), nkb = blocks(pr->keys);
   const int W = eff_window(pr), kind = pr->window_kind, causal = pr->causal;
   std::vector<int64_t> len(nblk);
   for (int i = 0; i < nblk; ++i) {
     const ttt::Range r = col ? ttt::col_block_range(i, nblk, T, causal, W, kind)
-                             : ttt::row_block_range(causal ? nblk - 1 - i : i, nblk, T, causal, W, kind);
+                             : ttt::row_block_range(causal ? nblk - 1 - i : i, nkb, T, causal, W, kind);
     len[i] = r.hi - r.lo;
   }
   return len;
@@ -270,11 +290,11 @@ double simulate_launch(const std::vector<int64_t>& len, int64_t c, int64_t bh, i
 // split must beat no split by kSplitTiles.  Cached per shape.
 // kind: 0 row blocks, 1 column blocks, 2 row-block pairs (len in their units).
 // cfloor: no chunk below it is considered (0: none).
-int64_t best_chunk(const ttt_problem* pr, const std::vector<int64_t>& len, int kind, int64_t bh, int64_t slots,
+int64_t best_chunk(const Prob* pr, const std::vector<int64_t>& len, int kind, int64_t bh, int64_t slots,
                    int64_t cfloor = 0) {
   static std::mutex mu;
-  static std::map<std::tuple<int64_t, int, int, int, int, int64_t, int64_t, int, int64_t>, int64_t> cache;
-  const auto key = std::make_tuple((int64_t)pr->seqlen, pr->causal, eff_window(pr), pr->window_kind, kind,
+  static std::map<std::tuple<int64_t, int64_t, int, int, int, int, int64_t, int64_t, int, int64_t>, int64_t> cache;
+  const auto key = std::make_tuple((int64_t)pr->seqlen, (int64_t)pr->keys, pr->causal, eff_window(pr), pr->window_kind, kind,
                                    bh, slots, pr->bias.data ? 1 : 0, cfloor);
   // plain causal launches run their chunks longest first (causal_item)
   const bool longest_first = pr->causal && !has_xm(pr);
@@ -314,10 +334,11 @@ int64_t best_chunk(const ttt_problem* pr, const std::vector<int64_t>& len, int k
 // 64-row block: nchunk_max = ceil(nblk / chunk).
 bool pair_family(int fam) { return fam == ttt::kFamFwdPairs; }
 
-Split choose_split_pairs(const ttt_problem* pr) {
+Split choose_split_pairs(const Prob* pr) {
   Split s;
-  s.nblk = (int)((pr->seqlen + ttt::kBlk - 1) / ttt::kBlk);
-  const int64_t nblk = s.nblk, npair = (nblk + 1) / 2;
+  s.nblk = blocks(pr->seqlen);
+  const int64_t nblk = blocks(pr->keys);  // tiles of a walk (= row blocks when causal)
+  const int64_t npair = (s.nblk + 1) / 2;
   const int64_t bh = pr->batch * pr->heads;
   int64_t c;
   if (pr->split_chunk > 0) {
@@ -341,12 +362,12 @@ Split choose_split_pairs(const ttt_problem* pr) {
   return s;
 }
 
-Split choose_split(const ttt_problem* pr, int fam, bool load_p) {
+Split choose_split(const Prob* pr, int fam, bool load_p) {
   if (pair_family(fam)) return choose_split_pairs(pr);
   Split s;
-  s.nblk = (int)((pr->seqlen + ttt::kBlk - 1) / ttt::kBlk);
-  const int64_t bh = pr->batch * pr->heads;
   const bool col = column_family(fam);
+  s.nblk = blocks(col ? pr->keys : pr->seqlen);
+  const int64_t bh = pr->batch * pr->heads;
   const std::vector<int64_t> len = block_tiles(pr, col);
   const int64_t lmax = *std::max_element(len.begin(), len.end());
   int64_t c;
@@ -369,7 +390,7 @@ Split choose_split(const ttt_problem* pr, int fam, bool load_p) {
   return s;
 }
 
-int family_of(const ttt_problem* pr, int entry, bool gdo) {
+int family_of(const Prob* pr, int entry, bool gdo) {
   switch (entry) {
     case TTT_ENTRY_FWD:
       return ttt::fwd_row_pairs(pr->dtype, (int)pr->head_dim, has_xm(pr), pr->block_rows) ? ttt::kFamFwdPairs
@@ -384,7 +405,7 @@ int family_of(const ttt_problem* pr, int entry, bool gdo) {
 }
 
 // Bytes of partial accumulators + partial row scalars for one kernel family.
-int64_t family_bytes(const ttt_problem* pr, const Split& s, int fam) {
+int64_t family_bytes(const Prob* pr, const Split& s, int fam) {
   if (s.nchunk_max <= 1) return 0;
   const int64_t parts = pr->batch * pr->heads * s.nblk * s.nchunk_max;
   return parts * ttt::kBlk * (ttt::kFamNacc[fam] * pr->head_dim + ttt::kFamNsc[fam]) * (int64_t)sizeof(float);
@@ -392,12 +413,12 @@ int64_t family_bytes(const ttt_problem* pr, const Split& s, int fam) {
 
 // Workspace of a family: the larger of its two variants' (with and without
 // P), since a workspace query does not say which one will run.
-int64_t fam_bytes(const ttt_problem* pr, int fam) {
+int64_t fam_bytes(const Prob* pr, int fam) {
   return std::max(family_bytes(pr, choose_split(pr, fam, false), fam),
                   family_bytes(pr, choose_split(pr, fam, true), fam));
 }
 
-int64_t entry_bytes(const ttt_problem* pr, int entry, bool gdo) {
+int64_t entry_bytes(const Prob* pr, int entry, bool gdo) {
   // the fused backward keeps dQ's partials while dK/dV writes its own
   if (entry == TTT_ENTRY_BWD) return fam_bytes(pr, ttt::kFamDq) + fam_bytes(pr, ttt::kFamDkdv);
   // the fused double backward keeps the row pass's partials while the column
@@ -407,12 +428,13 @@ int64_t entry_bytes(const ttt_problem* pr, int entry, bool gdo) {
   return fam < 0 ? -1 : fam_bytes(pr, fam);
 }
 
-ttt::Params base_params(const ttt_problem* pr) {
+ttt::Params base_params(const Prob* pr) {
   ttt::Params a;
   std::memset(&a, 0, sizeof(a));
   a.B = (int)pr->batch;
   a.H = (int)pr->heads;
   a.T = (int)pr->seqlen;
+  a.Tk = (int)pr->keys;
   a.causal = pr->causal;
   a.win = eff_window(pr);
   a.win_kind = pr->window_kind;
@@ -428,7 +450,7 @@ ttt::Params base_params(const ttt_problem* pr) {
 // The split of choose_split, with fewer chunks per block if its partials
 // would need more than `cap` bytes (cap < 0: no limit).  One chunk per block
 // needs none, so some split always fits.
-Split capped_split(const ttt_problem* pr, int fam, bool load_p, int64_t cap) {
+Split capped_split(const Prob* pr, int fam, bool load_p, int64_t cap) {
   Split s = choose_split(pr, fam, load_p);
   if (cap < 0 || family_bytes(pr, s, fam) <= cap) return s;
   const std::vector<int64_t> len = block_tiles(pr, column_family(fam));
@@ -443,7 +465,7 @@ Split capped_split(const ttt_problem* pr, int fam, bool load_p, int64_t cap) {
 
 // Attach the split and the workspace for kernel family `fam`; the split's
 // partials must fit in `cap` bytes (cap < 0: no limit).
-int attach_split(const ttt_problem* pr, int fam, bool load_p, void* ws, int64_t ws_bytes, ttt::Params* a,
+int attach_split(const Prob* pr, int fam, bool load_p, void* ws, int64_t ws_bytes, ttt::Params* a,
                  int64_t cap = -1) {
   const Split s = capped_split(pr, fam, load_p, cap);
   a->chunk = s.chunk;
@@ -601,7 +623,13 @@ int ttt_kernel_timing_read(int32_t kernel, float* mean_ms, int32_t* count) {
 const char* ttt_last_error(void) { return g_err; }
 
 int64_t ttt_attn_workspace_size(const ttt_problem* pr, int32_t entry, int32_t want_gdout) {
-  if (check_problem(pr) != TTT_OK) return -1;
+  return ttt_attn_workspace_size_shape(pr, nullptr, entry, want_gdout);
+}
+
+int64_t ttt_attn_workspace_size_shape(const ttt_problem* problem, const ttt_shape* shape, int32_t entry, int32_t want_gdout) {
+  Prob prob;
+  const Prob* pr = &prob;
+  if (make_prob(problem, shape, &prob) != TTT_OK) return -1;
   if (entry < TTT_ENTRY_FWD || entry > TTT_ENTRY_GG) {
     fail(TTT_ERR_INVALID_ARGUMENT, "unknown entry %d", entry);
     return -1;
@@ -609,9 +637,11 @@ int64_t ttt_attn_workspace_size(const ttt_problem* pr, int32_t entry, int32_t wa
   return entry_bytes(pr, entry, want_gdout != 0);
 }
 
-int ttt_attn_split_info(const ttt_problem* pr, int32_t entry, int32_t load_p, int32_t want_gdout, int32_t* chunk,
+int ttt_attn_split_info(const ttt_problem* problem, int32_t entry, int32_t load_p, int32_t want_gdout, int32_t* chunk,
                         int32_t* nchunk_max, int64_t* slots) {
-  TRY(check_problem(pr));
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   const int fam = family_of(pr, entry, want_gdout != 0);
   if (fam < 0) return fail(TTT_ERR_INVALID_ARGUMENT, "entry %d is not a single kernel family", entry);
   const Split s = choose_split(pr, fam, load_p != 0);
@@ -633,7 +663,15 @@ int ttt_attn_launch_item(int32_t nblk, int32_t chunk, int32_t column, int32_t* b
 int ttt_attn_fwd(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                  const ttt_view* o, float* lse, const ttt_view* p, void* workspace, int64_t workspace_bytes,
                  void* stream) {
-  TRY(check_problem(pr));
+  return ttt_attn_fwd_shape(pr, nullptr, q, k, v, o, lse, p, workspace, workspace_bytes, stream);
+}
+
+int ttt_attn_fwd_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                      const ttt_view* v, const ttt_view* o, float* lse, const ttt_view* p, void* workspace,
+                      int64_t workspace_bytes, void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, shape, &prob));
   ttt::Params a = base_params(pr);
   TRY(take_view(pr, q, "q", &a.q));
   TRY(take_view(pr, k, "k", &a.k));
@@ -653,17 +691,19 @@ int ttt_attn_fwd(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, co
   // rounds of workgroups per slot (b4 h16 T8192 d128: P pass -11 %); with one
   // round they cost about 1 % (b2 h4 T2048 d128).
   if (wp) {
-    const int64_t blocks = pr->batch * pr->heads * ((pr->seqlen + ttt::kBlk - 1) / ttt::kBlk);
-    a.defer_p = blocks >= kDeferRounds * family_slots(pr, ttt::kFamFwdP, true) ? 1 : 0;
-    const int64_t written = pr->batch * pr->heads * pr->seqlen * pr->seqlen * (pr->dtype == TTT_F32 ? 4 : 2) /
+    const int64_t nblocks = pr->batch * pr->heads * blocks(pr->seqlen);
+    a.defer_p = nblocks >= kDeferRounds * family_slots(pr, ttt::kFamFwdP, true) ? 1 : 0;
+    const int64_t written = pr->batch * pr->heads * pr->seqlen * pr->keys * (pr->dtype == TTT_F32 ? 4 : 2) /
                             (pr->causal ? 2 : 1);
     a.p_nt = written > kPStreamBytes ? 1 : 0;
   }
   return launched(ttt::launch_fwd(pr->dtype, (int)pr->head_dim, a, wp, (hipStream_t)stream), "ttt_attn_fwd");
 }
 
-int ttt_attn_fill_masked_p(const ttt_problem* pr, const ttt_view* p, void* stream) {
-  TRY(check_problem(pr));
+int ttt_attn_fill_masked_p(const ttt_problem* problem, const ttt_view* p, void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   ttt::Params a = base_params(pr);
   TRY(take_view(pr, p, "p", &a.p));
   return launched(ttt::launch_fill_masked_p(pr->dtype, a, (hipStream_t)stream), "ttt_attn_fill_masked_p");
@@ -672,10 +712,9 @@ int ttt_attn_fill_masked_p(const ttt_problem* pr, const ttt_view* p, void* strea
 }  // extern "C"
 
 // Parameters of the dQ launch (ttt_attn_bwd_dq), its split and workspace.
-static int prep_dq(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+static int prep_dq(const Prob* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                    const ttt_view* o, const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum_in,
                    float* rowsum_out, const ttt_view* dq, void* workspace, int64_t workspace_bytes, ttt::Params* out) {
-  TRY(check_problem(pr));
   ttt::Params a = base_params(pr);
   TRY(take_view(pr, k, "k", &a.k));
   TRY(take_view(pr, v, "v", &a.v));
@@ -699,11 +738,10 @@ static int prep_dq(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, 
 }
 
 // Parameters of the dK/dV launch (ttt_attn_bwd_dkdv), its split and workspace.
-static int prep_dkdv(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+static int prep_dkdv(const Prob* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                      const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                      const ttt_view* dk, const ttt_view* dv, void* workspace, int64_t workspace_bytes,
                      ttt::Params* out) {
-  TRY(check_problem(pr));
   ttt::Params a = base_params(pr);
   const bool lp = has_p(p);
   const bool dv_only = !(dk && dk->data);
@@ -730,20 +768,26 @@ static int prep_dkdv(const ttt_problem* pr, const ttt_view* q, const ttt_view* k
 
 extern "C" {
 
-int ttt_attn_bwd_dq(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_bwd_dq(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                     const ttt_view* o, const ttt_view* dout, const float* lse, const ttt_view* p,
                     const float* rowsum_in, float* rowsum_out, const ttt_view* dq, void* workspace,
                     int64_t workspace_bytes, void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   ttt::Params a;
   TRY(prep_dq(pr, q, k, v, o, dout, lse, p, rowsum_in, rowsum_out, dq, workspace, workspace_bytes, &a));
   return launched(ttt::launch_bwd_dq(pr->dtype, (int)pr->head_dim, a, has_p(p), (hipStream_t)stream),
                   "ttt_attn_bwd_dq");
 }
 
-int ttt_attn_bwd_dkdv(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_bwd_dkdv(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                       const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                       const ttt_view* dk, const ttt_view* dv, void* workspace, int64_t workspace_bytes,
                       void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   ttt::Params a;
   TRY(prep_dkdv(pr, q, k, v, dout, lse, p, rowsum, dk, dv, workspace, workspace_bytes, &a));
   const bool dv_only = !(dk && dk->data);
@@ -758,9 +802,19 @@ int ttt_attn_bwd(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, co
                  const ttt_view* o, const ttt_view* dout, const float* lse, const ttt_view* p,
                  float* rowsum_out, const ttt_view* dq, const ttt_view* dk, const ttt_view* dv,
                  void* workspace, int64_t workspace_bytes, void* stream) {
+  return ttt_attn_bwd_shape(pr, nullptr, q, k, v, o, dout, lse, p, rowsum_out, dq, dk, dv, workspace,
+                           workspace_bytes, stream);
+}
+
+int ttt_attn_bwd_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                      const ttt_view* v, const ttt_view* o, const ttt_view* dout, const float* lse,
+                      const ttt_view* p, float* rowsum_out, const ttt_view* dq, const ttt_view* dk,
+                      const ttt_view* dv, void* workspace, int64_t workspace_bytes, void* stream) {
   if (!rowsum_out) return fail(TTT_ERR_INVALID_ARGUMENT, "rowsum_out: null pointer");
   if (!dk || !dk->data) return fail(TTT_ERR_INVALID_ARGUMENT, "dk: null pointer");
-  TRY(check_problem(pr));
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, shape, &prob));
   const bool lp = has_p(p);
   const int64_t dq_bytes = family_bytes(pr, choose_split(pr, ttt::kFamDq, lp), ttt::kFamDq);
   const int64_t ws_bytes = workspace ? workspace_bytes : 0;
@@ -775,9 +829,11 @@ int ttt_attn_bwd(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, co
   return launched(ttt::launch_bwd_dkdv(pr->dtype, (int)pr->head_dim, ak, lp, false, st, &aq), "ttt_attn_bwd");
 }
 
-int ttt_attn_bwd_rowsum(const ttt_problem* pr, const ttt_view* p, const ttt_view* dout, const ttt_view* v,
+int ttt_attn_bwd_rowsum(const ttt_problem* problem, const ttt_view* p, const ttt_view* dout, const ttt_view* v,
                         float* rowsum, void* stream) {
-  TRY(check_problem(pr));
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   ttt::Params a = base_params(pr);
   TRY(take_view(pr, p, "p", &a.p));
   TRY(take_view(pr, dout, "dout", &a.dout));
@@ -791,13 +847,12 @@ int ttt_attn_bwd_rowsum(const ttt_problem* pr, const ttt_view* p, const ttt_view
 
 // ttt_attn_gg_row / ttt_attn_gg_col with the split's partials held to `cap`
 // bytes (cap < 0: no limit).
-static int prep_gg_row(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+static int prep_gg_row(const Prob* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                        const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                        const ttt_view* dq, const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
                        const ttt_view* gq_out,
                        const ttt_view* gdout, float* e_out, float* f_out, void* workspace, int64_t workspace_bytes,
                        int64_t cap, ttt::Params* out) {
-  TRY(check_problem(pr));
   ttt::Params a = base_params(pr);
   TRY(take_view(pr, q, "q", &a.q));
   TRY(take_view(pr, k, "k", &a.k));
@@ -826,7 +881,7 @@ static int prep_gg_row(const ttt_problem* pr, const ttt_view* q, const ttt_view*
   return TTT_OK;
 }
 
-static int gg_row_impl(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+static int gg_row_impl(const Prob* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                        const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                        const ttt_view* dq, const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
                        const ttt_view* gq_out, const ttt_view* gdout, float* e_out, float* f_out, void* workspace,
@@ -839,12 +894,11 @@ static int gg_row_impl(const ttt_problem* pr, const ttt_view* q, const ttt_view*
                   "ttt_attn_gg_row");
 }
 
-static int prep_gg_col(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+static int prep_gg_col(const Prob* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                        const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                        const float* e_in, const float* f_in, const ttt_view* gq, const ttt_view* gk,
                        const ttt_view* gv, const ttt_view* gk_out, const ttt_view* gv_out, void* workspace,
                        int64_t workspace_bytes, int64_t cap, ttt::Params* out) {
-  TRY(check_problem(pr));
   ttt::Params a = base_params(pr);
   TRY(take_view(pr, q, "q", &a.q));
   TRY(take_view(pr, k, "k", &a.k));
@@ -869,7 +923,7 @@ static int prep_gg_col(const ttt_problem* pr, const ttt_view* q, const ttt_view*
   return TTT_OK;
 }
 
-static int gg_col_impl(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+static int gg_col_impl(const Prob* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                        const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                        const float* e_in, const float* f_in, const ttt_view* gq, const ttt_view* gk,
                        const ttt_view* gv, const ttt_view* gk_out, const ttt_view* gv_out, void* workspace,
@@ -881,20 +935,26 @@ static int gg_col_impl(const ttt_problem* pr, const ttt_view* q, const ttt_view*
                   "ttt_attn_gg_col");
 }
 
-int ttt_attn_gg_row(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_gg_row(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                     const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                     const ttt_view* dq, const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
                     const ttt_view* gq_out, const ttt_view* gdout, float* e_out, float* f_out, void* workspace,
                     int64_t workspace_bytes, void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   return gg_row_impl(pr, q, k, v, dout, lse, p, rowsum, dq, gq, gk, gv, gq_out, gdout, e_out, f_out, workspace,
                      workspace_bytes, stream, -1);
 }
 
-int ttt_attn_gg_col(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_gg_col(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                     const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                     const float* e_in, const float* f_in, const ttt_view* gq, const ttt_view* gk,
                     const ttt_view* gv, const ttt_view* gk_out, const ttt_view* gv_out, void* workspace,
                     int64_t workspace_bytes, void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   return gg_col_impl(pr, q, k, v, dout, lse, p, rowsum, e_in, f_in, gq, gk, gv, gk_out, gv_out, workspace,
                      workspace_bytes, stream, -1);
 }
@@ -904,11 +964,23 @@ int ttt_attn_gg(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, con
                 const ttt_view* dq, const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
                 const ttt_view* gq_out, const ttt_view* gk_out, const ttt_view* gv_out, const ttt_view* gdout,
                 float* e_buf, float* f_buf, void* workspace, int64_t workspace_bytes, void* stream) {
+  return ttt_attn_gg_shape(pr, nullptr, q, k, v, dout, lse, p, rowsum, dq, gq, gk, gv, gq_out, gk_out,
+                          gv_out, gdout, e_buf, f_buf, workspace, workspace_bytes, stream);
+}
+
+int ttt_attn_gg_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                     const ttt_view* v, const ttt_view* dout, const float* lse, const ttt_view* p,
+                     const float* rowsum, const ttt_view* dq, const ttt_view* gq, const ttt_view* gk,
+                     const ttt_view* gv, const ttt_view* gq_out, const ttt_view* gk_out, const ttt_view* gv_out,
+                     const ttt_view* gdout, float* e_buf, float* f_buf, void* workspace, int64_t workspace_bytes,
+                     void* stream) {
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, shape, &prob));
   // The row pass's partials go in the first part of the workspace and the
   // column pass's after them: the column launch sums the row pass's split
   // blocks (GQ, GdO) in workgroups appended to its grid, after a small launch
   // has formed E and F, which the column pass reads.
-  TRY(check_problem(pr));
   const bool lp = has_p(p);
   const bool gdo = gdout && gdout->data;
   const int fam = gdo ? ttt::kFamGgRowGdo : ttt::kFamGgRow;
@@ -927,12 +999,14 @@ int ttt_attn_gg(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, con
   return launched(ttt::launch_gg_col(pr->dtype, (int)pr->head_dim, ac, lp, st, &ar), "ttt_attn_gg");
 }
 
-int ttt_attn_gg_noalloc(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_gg_noalloc(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                         const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                         const ttt_view* dq, const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
                         const ttt_view* gq_out, const ttt_view* gk_out, const ttt_view* gv_out,
                         const ttt_view* gdout, void* stream) {
-  TRY(check_problem(pr));
+  Prob prob;
+  const Prob* pr = &prob;
+  TRY(make_prob(problem, nullptr, &prob));
   const int64_t nstat = pr->batch * pr->heads * pr->seqlen;
   const int64_t one = (nstat * (int64_t)sizeof(float) + 255) / 256 * 256;  // E, then F, 256-byte aligned
   if (2 * one > kNoAllocStatBytes)

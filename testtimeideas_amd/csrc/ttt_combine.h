@@ -32,9 +32,10 @@ struct CombineSlot {
   }
 };
 
-__device__ __forceinline__ int block_nch(const Params& a, int blk, int nblk, bool col) {
-  const Range r = col ? col_block_range(blk, nblk, a.T, a.causal, a.win, a.win_kind)
-                      : row_block_range(blk, nblk, a.T, a.causal, a.win, a.win_kind);
+__device__ __forceinline__ int block_nch(const Params& a, int blk, bool col) {
+  const int nkb = (a.Tk + kBlk - 1) / kBlk;
+  const Range r = col ? col_block_range(blk, nkb, a.T, a.causal, a.win, a.win_kind)
+                      : row_block_range(blk, nkb, a.T, a.causal, a.win, a.win_kind);
   return (r.hi - r.lo + a.chunk - 1) / a.chunk;
 }
 
@@ -98,15 +99,16 @@ __device__ __forceinline__ void store_slot(const View& o, int b, int h, int row,
 
 // ---------------------------------------------------------------------------
 // Plain sums (O of the save_p forward, dQ, dK/dV, GK/GV) for combine
-// workgroup (bx, by) of a grid of nblk * CombineSlot<D>::kSub by B*H.
+// workgroup (bx, by) of a grid of (the output's blocks) * CombineSlot<D>::kSub
+// by B*H.
 template <typename T, int D>
 __device__ __forceinline__ void combine_sum_block(const Params& a, int which, int bx, int by) {
-  const int T_ = a.T;
+  const bool col = which == kOutDKDV || which == kOutDV || which == kOutGKGV;
+  const int T_ = col ? a.Tk : a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const CombineSlot<D> cs(bx);
   const int bh = by, b = bh / a.H, h = bh % a.H;
-  const bool col = which == kOutDKDV || which == kOutDV || which == kOutGKGV;
-  const int nch = block_nch(a, cs.blk, nblk, col);
+  const int nch = block_nch(a, cs.blk, col);
   if (nch <= 1) return;
   const int row = cs.blk * kBlk + cs.r;
   if (row >= T_) return;
@@ -149,7 +151,7 @@ __device__ __forceinline__ void combine_gg_row_block(const Params& a, int bx, in
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const CombineSlot<D> cs(bx);
   const int bh = by, b = bh / a.H, h = bh % a.H;
-  const int nch = block_nch(a, cs.blk, nblk, false);
+  const int nch = block_nch(a, cs.blk, false);
   if (nch <= 1) return;
   const int r = cs.r;
   const int row = cs.blk * kBlk + r;

@@ -24,7 +24,7 @@ __global__ __launch_bounds__(kThreads) void k_combine_fwd(Params a) {
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const CombineSlot<D> cs(blockIdx.x);
   const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H;
-  const int nch = block_nch(a, cs.blk, nblk, false);
+  const int nch = block_nch(a, cs.blk, false);
   if (nch <= 1) return;
   const int r = cs.r;
   const int row = cs.blk * kBlk + r;
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kThreads) void k_combine_gg_ef(Params a) {
   const int bh = blockIdx.y;
   if (row >= T_) return;
   const int blk = row / kBlk, r = row % kBlk;
-  const int nch = block_nch(a, blk, nblk, false);
+  const int nch = block_nch(a, blk, false);
   if (nch <= 1) return;
   float sc[3];
   sum_scalars<3>(sc, a.ws_sc, part_index(a, bh, nblk, blk, 0), nch, r);
@@ -119,7 +119,8 @@ __global__ __launch_bounds__(kThreads) void k_combine_gg_ef(Params a) {
 // ---------------------------------------------------------------------------
 template <typename T, int D>
 static hipError_t combine_sum_t(const Params& a, int which, hipStream_t st) {
-  dim3 grid((a.T + kBlk - 1) / kBlk * CombineSlot<D>::kSub, a.B * a.H);
+  const bool col = which == kOutDKDV || which == kOutDV || which == kOutGKGV;
+  dim3 grid(((col ? a.Tk : a.T) + kBlk - 1) / kBlk * CombineSlot<D>::kSub, a.B * a.H);
   hipLaunchKernelGGL((k_combine_sum<T, D>), grid, dim3(kThreads), 0, st, a, which);
   return hipGetLastError();
 }

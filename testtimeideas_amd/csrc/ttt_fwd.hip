@@ -69,7 +69,7 @@ __device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds
 #pragma unroll
     for (int j = 0; j < 8; ++j) s.set(kb, j, s.at(kb, j) * a.scale_log2);
   if constexpr (XM)
-    if (brow) add_bias_row<T>(s, brow, n0, a.T);
+    if (brow) add_bias_row<T>(s, brow, n0, a.Tk);
   if (need_mask) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -135,13 +135,14 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
   if (it.blk < 0) return;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -170,12 +171,12 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     const int n1 = nb * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
     const T* vp = V + (int64_t)n1 * a.v.st;
-    if (D == 64 && n1 + kBlk <= T_) {  // full tile: offsets computed once
+    if (D == 64 && n1 + kBlk <= Tk_) {  // full tile: offsets computed once
       stage_load_full<T, D>(stK, kp, soK);
       stage_load_full<T, D>(stV, vp, soV);
     } else {
-      stage_load<T, D>(stK, kp, a.k.st, T_ - n1, D);
-      stage_load<T, D>(stV, vp, a.v.st, T_ - n1, D);
+      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, D);
+      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, D);
     }
   };
   // Key tile nb from LDS tiles cK, cV.
@@ -274,12 +275,12 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       const int n1 = nt * kBlk;
       const T* kp = K + (int64_t)n1 * a.k.st;
       const T* vp = V + (int64_t)n1 * a.v.st;
-      if (n1 + kBlk <= T_) {
+      if (n1 + kBlk <= Tk_) {
         dd.load_full(k, kp, oK);
         dd.load_full(v, vp, oV);
       } else {
-        dd.load_ragged(k, kp, a.k.st, T_ - n1, D);
-        dd.load_ragged(v, vp, a.v.st, T_ - n1, D);
+        dd.load_ragged(k, kp, a.k.st, Tk_ - n1, D);
+        dd.load_ragged(v, vp, a.v.st, Tk_ - n1, D);
         dma_wait();
       }
     };
@@ -383,6 +384,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const int npair = (nblk + 1) >> 1;
   const int C = a.chunk;
   const Slot sl = grid_slot();
@@ -392,7 +394,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   const int pj = a.causal ? npair - 1 - it.blk : it.blk;
   const int ch = it.ch;
   const int mb0 = 2 * pj, mb1 = mb0 + 1;
-  const int hi0 = a.causal ? mb0 + 1 : nblk, hi1 = a.causal ? mb1 + 1 : nblk;
+  const int hi0 = a.causal ? mb0 + 1 : nkb, hi1 = a.causal ? mb1 + 1 : nkb;
   const int t0 = ch * C;
   const bool act0 = t0 < hi0;
   const bool act1 = mb1 < nblk && t0 < hi1;
@@ -437,10 +439,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   auto fetch = [&](const T* base, int64_t ld, const int* off, int t, T* dst) __attribute__((always_inline)) {
     const int n1 = t * kBlk;
     const T* p = base + (int64_t)n1 * ld;
-    if (n1 + kBlk <= T_) {
+    if (n1 + kBlk <= Tk_) {
       dd.load_full(dst, p, off);
     } else {
-      dd.load_ragged(dst, p, ld, T_ - n1, D);
+      dd.load_ragged(dst, p, ld, Tk_ - n1, D);
       dma_wait();
     }
   };
@@ -508,7 +510,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   };
   // Tiles at or past the pair's first diagonal, or ragged, take the masked step.
   auto masked_tile = [&](int t) __attribute__((always_inline)) {
-    return (a.causal && t >= mb0) || (t * kBlk + kBlk > T_);
+    return (a.causal && t >= mb0) || (t * kBlk + kBlk > Tk_);
   };
 
   // Prologue: K and V of tile t0 and K of tile t0 + 1; tile t0's scores and
@@ -566,7 +568,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     s[0] = sn[0];
     s[1] = sn[1];
   };
-  const int tq = min(t1, max(t0, min(a.causal ? mb0 : t1, (T_ % kBlk) ? nblk - 1 : t1)));  // first masked tile
+  const int tq = min(t1, max(t0, min(a.causal ? mb0 : t1, (Tk_ % kBlk) ? nkb - 1 : t1)));  // first masked tile
   int t = t0;
   for (; t + 1 < tq; t += 2) {
     step(Parity<0>{}, std::false_type{}, t);
@@ -629,13 +631,14 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
   if (it.blk < 0) return;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -660,10 +663,10 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   auto load_k = [&](int nb, Stage<T, D>& sk) __attribute__((always_inline)) {
     const int n1 = (nb < cr.t1 ? nb : cr.t1 - 1) * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
-    if (D == 64 && n1 + kBlk <= T_)  // full tile: offsets computed once
+    if (D == 64 && n1 + kBlk <= Tk_)  // full tile: offsets computed once
       stage_load_full<T, D>(sk, kp, soK);
     else
-      stage_load<T, D>(sk, kp, a.k.st, T_ - n1, D);
+      stage_load<T, D>(sk, kp, a.k.st, Tk_ - n1, D);
   };
   // One round: key tiles nb .. nb + R - 1 from the LDS tiles tile_k(i).
   auto round = [&](int nb, auto tile_k) __attribute__((always_inline)) {
@@ -750,10 +753,10 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
         const int n1 = (nb + i < cr.t1 ? nb + i : cr.t1 - 1) * kBlk;
         T* dst = decltype(par)::value == 0 ? sK[i] : sK1[i];
         const T* kp = K + (int64_t)n1 * a.k.st;
-        if (n1 + kBlk <= T_) {
+        if (n1 + kBlk <= Tk_) {
           dd.load_full(dst, kp, oK);
         } else {
-          dd.load_ragged(dst, kp, a.k.st, T_ - n1, D);
+          dd.load_ragged(dst, kp, a.k.st, Tk_ - n1, D);
           dma_wait();
         }
       }
@@ -866,13 +869,14 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
   if (it.blk < 0) return;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -905,12 +909,12 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
     const int n1 = nb * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
     const T* vp = V + (int64_t)n1 * a.v.st;
-    if (D == 64 && n1 + kBlk <= T_) {  // full tile: offsets computed once
+    if (D == 64 && n1 + kBlk <= Tk_) {  // full tile: offsets computed once
       stage_load_full<T, D>(stK, kp, soK);
       stage_load_full<T, D>(stV, vp, soV);
     } else {
-      stage_load<T, D>(stK, kp, a.k.st, T_ - n1, D);
-      stage_load<T, D>(stV, vp, a.v.st, T_ - n1, D);
+      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, D);
+      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, D);
     }
   };
   // With a.defer_p, the P stores of a full tile wait in registers until the
@@ -957,14 +961,14 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
             for (int j = 0; j < 8; ++j) pv[j] = mk.masked(n0 + stream_index(kb, g, j)) ? 0.f : pv[j];
           }
           pf[kb] = M::vals(pv);
-          if (kRowPair && n0 + kBlk <= T_) {
+          if (kRowPair && n0 + kBlk <= Tk_) {
             // stored whole below (or deferred)
-          } else if (kDma && a.defer_p && n0 + kBlk <= T_) {
+          } else if (kDma && a.defer_p && n0 + kBlk <= Tk_) {
             pend[kb] = pf[kb];
             if (kb == 1 && m < T_) pend_ptr = Pm + n0 + stream_index(0, g, 0);
           } else if (m < T_) {
             const int n = n0 + stream_index(kb, g, 0);
-            if (n + 8 <= T_) {
+            if (n + 8 <= Tk_) {
               store_frag_g<T>(Pm + n, pf[kb]);
             } else {
               // Ragged last tile: the stored halves taken from the packed
@@ -974,7 +978,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
               __builtin_memcpy(&raw, &pf[kb], 16);
 #pragma unroll
               for (int j = 0; j < 8; ++j)
-                if (n + j < T_) {
+                if (n + j < Tk_) {
                   const uint16_t h = (uint16_t)(raw[j >> 1] >> (16 * (j & 1)));
                   __builtin_memcpy(Pm + n + j, &h, 2);
                 }
@@ -982,7 +986,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
           }
         }
         if constexpr (kRowPair) {
-          if (n0 + kBlk <= T_) {
+          if (n0 + kBlk <= Tk_) {
             if (kDma && a.defer_p) {
               pend[0] = pf[0];
               pend[1] = pf[1];
@@ -1001,7 +1005,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
 #pragma unroll
           for (int j = 0; j < 8; ++j) pv[j] = E::f32(E::cvt(fast_exp2(s.at(kb, j) - lse2)));
           pf[kb] = M::vals(pv);
-          if (kDma && a.defer_p && n0 + kBlk <= T_) {
+          if (kDma && a.defer_p && n0 + kBlk <= Tk_) {
             if constexpr (kDma) pend[kb] = pf[kb];
             if (kb == 1) {
               if constexpr (kRowPair)
@@ -1011,12 +1015,12 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
             }
           } else if (m < T_) {
             const int n = n0 + stream_index(kb, g, 0);
-            if (n + 8 <= T_) {
+            if (n + 8 <= Tk_) {
               store8<T>(Pm + n, pv);
             } else {
 #pragma unroll
               for (int j = 0; j < 8; ++j)
-                if (n + j < T_) Pm[n + j] = E::cvt(pv[j]);
+                if (n + j < Tk_) Pm[n + j] = E::cvt(pv[j]);
             }
           }
         }
@@ -1032,12 +1036,12 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
       const int n1 = nt * kBlk;
       const T* kp = K + (int64_t)n1 * a.k.st;
       const T* vp = V + (int64_t)n1 * a.v.st;
-      if (n1 + kBlk <= T_) {
+      if (n1 + kBlk <= Tk_) {
         dd.load_full(k, kp, oK);
         dd.load_full(v, vp, oV);
       } else {
-        dd.load_ragged(k, kp, a.k.st, T_ - n1, D);
-        dd.load_ragged(v, vp, a.v.st, T_ - n1, D);
+        dd.load_ragged(k, kp, a.k.st, Tk_ - n1, D);
+        dd.load_ragged(v, vp, a.v.st, Tk_ - n1, D);
         dma_wait();
       }
     };

@@ -165,13 +165,14 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
   if (it.blk < 0) return;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -245,11 +246,11 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   frag pn[2];
   auto load_tile = [&](int nb) {
     const int n0 = nb * kBlk;
-    stage_load<T, D>(s0, Kn, a.k.st, T_ - n0, D);
-    stage_load<T, D>(s1, Vn, a.v.st, T_ - n0, D);
-    stage_load<T, D>(s2, gKn, a.gk.st, T_ - n0, D);
-    stage_load<T, D>(s3, gVn, a.gv.st, T_ - n0, D);
-    if constexpr (LOADP) load_p_frags_run<T>(pn, Pn, Pm, n0, T_);
+    stage_load<T, D>(s0, Kn, a.k.st, Tk_ - n0, D);
+    stage_load<T, D>(s1, Vn, a.v.st, Tk_ - n0, D);
+    stage_load<T, D>(s2, gKn, a.gk.st, Tk_ - n0, D);
+    stage_load<T, D>(s3, gVn, a.gv.st, Tk_ - n0, D);
+    if constexpr (LOADP) load_p_frags_run<T>(pn, Pn, Pm, n0, Tk_);
     advance();
   };
   TileDma<T, D> dd;
@@ -258,7 +259,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   auto dma_tile = [&](int nb, int buf) {
     if constexpr (kDma) {
       const int n0 = nb * kBlk;
-      if (n0 + kBlk <= T_) {  // uniform: one test per tile for all four tiles and P
+      if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
         dd.load_full(sK[buf], Kn, oK);
         dd.load_full(sV[buf], Vn, oV);
         dd.load_full(sgK[buf], gKn, ogK);
@@ -268,11 +269,11 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
           pn[1] = load_frag_g<T>(Pn + 32);
         }
       } else {
-        dd.load_ragged(sK[buf], Kn, a.k.st, T_ - n0, D);
-        dd.load_ragged(sV[buf], Vn, a.v.st, T_ - n0, D);
-        dd.load_ragged(sgK[buf], gKn, a.gk.st, T_ - n0, D);
-        dd.load_ragged(sgV[buf], gVn, a.gv.st, T_ - n0, D);
-        if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, T_);
+        dd.load_ragged(sK[buf], Kn, a.k.st, Tk_ - n0, D);
+        dd.load_ragged(sV[buf], Vn, a.v.st, Tk_ - n0, D);
+        dd.load_ragged(sgK[buf], gKn, a.gk.st, Tk_ - n0, D);
+        dd.load_ragged(sgV[buf], gVn, a.gv.st, Tk_ - n0, D);
+        if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, Tk_);
         dma_wait();
       }
       advance();
@@ -369,7 +370,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     dd.offsets(ogV, a.gv.st);
     auto dma_set = [&](int nb, T* k, T* v, T* gk, T* gv) __attribute__((always_inline)) {
       const int n0 = nb * kBlk;
-      if (n0 + kBlk <= T_) {  // uniform: one test per tile for all four tiles and P
+      if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
         dd.load_full(k, Kn, oK);
         dd.load_full(v, Vn, oV);
         dd.load_full(gk, gKn, ogK);
@@ -379,11 +380,11 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
           pn[1] = load_frag_g<T>(Pn + 32);
         }
       } else {
-        dd.load_ragged(k, Kn, a.k.st, T_ - n0, D);
-        dd.load_ragged(v, Vn, a.v.st, T_ - n0, D);
-        dd.load_ragged(gk, gKn, a.gk.st, T_ - n0, D);
-        dd.load_ragged(gv, gVn, a.gv.st, T_ - n0, D);
-        if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, T_);
+        dd.load_ragged(k, Kn, a.k.st, Tk_ - n0, D);
+        dd.load_ragged(v, Vn, a.v.st, Tk_ - n0, D);
+        dd.load_ragged(gk, gKn, a.gk.st, Tk_ - n0, D);
+        dd.load_ragged(gv, gVn, a.gv.st, Tk_ - n0, D);
+        if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, Tk_);
         dma_wait();
       }
       advance();
@@ -546,7 +547,8 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       return Bufs{sQ1, sgQ1, sdO1, sP1, sS1};
   };
 
-  const int T_ = a.T;
+  const int T_ = a.Tk;  // keys: the stationary rows
+  const int Tq_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const Slot sl = grid_slot();
   // Workgroups past the first nx columns of the grid finish the preceding row
@@ -563,7 +565,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
   if (it.blk < 0) return;
   const int nb = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
-  const Range rg = col_block_range(nb, nblk, T_, a.causal, XM ? a.win : 0, a.win_kind);
+  const Range rg = col_block_range(nb, nblk, Tq_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int n0 = nb * kBlk;
@@ -581,10 +583,10 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
   const T* gK = at<const T>(a.gk, b, h);
   const T* gV = at<const T>(a.gv, b, h);
   const T* Pb = LOADP ? at<const T>(a.p, b, h) : nullptr;
-  const float* rs = a.rowsum_in + (int64_t)bh * T_;
-  const float* ev = a.e + (int64_t)bh * T_;
-  const float* fv = a.f + (int64_t)bh * T_;
-  const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * T_;
+  const float* rs = a.rowsum_in + (int64_t)bh * Tq_;
+  const float* ev = a.e + (int64_t)bh * Tq_;
+  const float* fv = a.f + (int64_t)bh * Tq_;
+  const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * Tq_;
   const float s = a.scale;
   const float kSl2 = kLog2e;  // raw score (in units of s) -> base 2
 
@@ -694,19 +696,19 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     const StatDma<kNS> sdma(rs, ev, fv, lse);
     auto dma_tile = [&](int mb, const Bufs& wb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
-      if (m0 + kBlk <= T_ && cols_full) {  // uniform: one test per tile
+      if (m0 + kBlk <= Tq_ && cols_full) {  // uniform: one test per tile
         dd.load_full(wb.q, Qn, oQ);
         dd.load_full(wb.gq, gQn, ogQ);
         dd.load_full(wb.dout, dOn, odO);
         if constexpr (LOADP) dpt.load_full(wb.p, Pn, oP);
       } else {
-        dd.load_ragged(wb.q, Qn, a.q.st, T_ - m0, D);
-        dd.load_ragged(wb.gq, gQn, a.gq.st, T_ - m0, D);
-        dd.load_ragged(wb.dout, dOn, a.dout.st, T_ - m0, D);
-        if constexpr (LOADP) dpt.load_ragged(wb.p, Pn, a.p.st, T_ - m0, T_ - n0);
+        dd.load_ragged(wb.q, Qn, a.q.st, Tq_ - m0, D);
+        dd.load_ragged(wb.gq, gQn, a.gq.st, Tq_ - m0, D);
+        dd.load_ragged(wb.dout, dOn, a.dout.st, Tq_ - m0, D);
+        if constexpr (LOADP) dpt.load_ragged(wb.p, Pn, a.p.st, Tq_ - m0, T_ - n0);
         dma_wait();
       }
-      sdma.load(wb.st, m0, T_ - m0);
+      sdma.load(wb.st, m0, Tq_ - m0);
       Qn += kBlk * a.q.st;
       gQn += kBlk * a.gq.st;
       dOn += kBlk * a.dout.st;
@@ -731,11 +733,11 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     float stv;
     auto load_tile = [&](int mb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
-      stage_load<T, D>(s0, Q + (int64_t)m0 * a.q.st, a.q.st, T_ - m0, D);
-      stage_load<T, D>(s1, gQ + (int64_t)m0 * a.gq.st, a.gq.st, T_ - m0, D);
-      stage_load<T, D>(s2, dO + (int64_t)m0 * a.dout.st, a.dout.st, T_ - m0, D);
-      if constexpr (LOADP) stage_load<T, kBlk>(sp, Pb + (int64_t)m0 * a.p.st + n0, a.p.st, T_ - m0, T_ - n0);
-      stv = stat_load<kNS>(rs, ev, fv, lse, m0, T_ - m0);
+      stage_load<T, D>(s0, Q + (int64_t)m0 * a.q.st, a.q.st, Tq_ - m0, D);
+      stage_load<T, D>(s1, gQ + (int64_t)m0 * a.gq.st, a.gq.st, Tq_ - m0, D);
+      stage_load<T, D>(s2, dO + (int64_t)m0 * a.dout.st, a.dout.st, Tq_ - m0, D);
+      if constexpr (LOADP) stage_load<T, kBlk>(sp, Pb + (int64_t)m0 * a.p.st + n0, a.p.st, Tq_ - m0, T_ - n0);
+      stv = stat_load<kNS>(rs, ev, fv, lse, m0, Tq_ - m0);
     };
     load_tile(cr.t0);
     for (int mb = cr.t0; mb < cr.t1; ++mb) {
@@ -817,7 +819,8 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
       return Bufs{sQ1, sgQ1, sdO1, sP1, sS1};
   };
 
-  const int T_ = a.T;
+  const int T_ = a.Tk;  // keys: the stationary rows
+  const int Tq_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const Slot sl = grid_slot();
   if (sl.x >= nx) {  // the preceding row launch's split blocks, in the first four waves
@@ -832,7 +835,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   if (it.blk < 0) return;
   const int nb = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
-  const Range rg = col_block_range(nb, nblk, T_, a.causal, 0, a.win_kind);
+  const Range rg = col_block_range(nb, nblk, Tq_, a.causal, 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int n0 = nb * kBlk;
@@ -852,10 +855,10 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   const T* gK = at<const T>(a.gk, b, h);
   const T* gV = at<const T>(a.gv, b, h);
   const T* Pb = LOADP ? at<const T>(a.p, b, h) : nullptr;
-  const float* rs = a.rowsum_in + (int64_t)bh * T_;
-  const float* ev = a.e + (int64_t)bh * T_;
-  const float* fv = a.f + (int64_t)bh * T_;
-  const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * T_;
+  const float* rs = a.rowsum_in + (int64_t)bh * Tq_;
+  const float* ev = a.e + (int64_t)bh * Tq_;
+  const float* fv = a.f + (int64_t)bh * Tq_;
+  const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * Tq_;
   const float s = a.scale;
   const float kSl2 = kLog2e;  // raw score (in units of s) -> base 2
 
@@ -963,19 +966,19 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
     const StatDma<kNS> sdma(rs, ev, fv, lse);
     auto dma_tile = [&](int mb, const Bufs& wb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
-      if (m0 + kBlk <= T_ && cols_full) {  // uniform: one test per tile
+      if (m0 + kBlk <= Tq_ && cols_full) {  // uniform: one test per tile
         dd.load_full0(wb.q, Qn, oQ, a.q.st);
         dd.load_full0(wb.gq, gQn, ogQ, a.gq.st);
         dd.load_full0(wb.dout, dOn, odO, a.dout.st);
         if constexpr (LOADP) dpt.load_full0(wb.p, Pn, oP, a.p.st);
       } else {
-        dd.load_ragged0(wb.q, Qn, a.q.st, T_ - m0, D);
-        dd.load_ragged0(wb.gq, gQn, a.gq.st, T_ - m0, D);
-        dd.load_ragged0(wb.dout, dOn, a.dout.st, T_ - m0, D);
-        if constexpr (LOADP) dpt.load_ragged0(wb.p, Pn, a.p.st, T_ - m0, T_ - n0);
+        dd.load_ragged0(wb.q, Qn, a.q.st, Tq_ - m0, D);
+        dd.load_ragged0(wb.gq, gQn, a.gq.st, Tq_ - m0, D);
+        dd.load_ragged0(wb.dout, dOn, a.dout.st, Tq_ - m0, D);
+        if constexpr (LOADP) dpt.load_ragged0(wb.p, Pn, a.p.st, Tq_ - m0, T_ - n0);
         dma_wait();
       }
-      sdma.load(wb.st, m0, T_ - m0);
+      sdma.load(wb.st, m0, Tq_ - m0);
       Qn += kBlk * a.q.st;
       gQn += kBlk * a.gq.st;
       dOn += kBlk * a.dout.st;
@@ -1063,13 +1066,14 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
+  const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<false>(a, sl.x, nblk);
   if (it.blk < 0) return;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
-  const Range rg = row_block_range(mb, nblk, T_, a.causal, 0, a.win_kind);
+  const Range rg = row_block_range(mb, nkb, T_, a.causal, 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
   if (ch >= cr.nch) return;
   const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
@@ -1207,20 +1211,20 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   frag pn;
   auto dma_set = [&](int nb, T* k, T* v, T* gk, T* gv) __attribute__((always_inline)) {
     const int n0 = nb * kBlk;
-    if (n0 + kBlk <= T_) {  // uniform: one test per tile for all four tiles and P
+    if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
       dd.load_full0(k, Kn, oK, a.k.st);
       dd.load_full0(v, Vn, oV, a.v.st);
       dd.load_full0(gk, gKn, ogK, a.gk.st);
       dd.load_full0(gv, gVn, ogV, a.gv.st);
       if constexpr (LOADP) pn = load_frag_g<T>(Pn);
     } else {
-      dd.load_ragged0(k, Kn, a.k.st, T_ - n0, D);
-      dd.load_ragged0(v, Vn, a.v.st, T_ - n0, D);
-      dd.load_ragged0(gk, gKn, a.gk.st, T_ - n0, D);
-      dd.load_ragged0(gv, gVn, a.gv.st, T_ - n0, D);
+      dd.load_ragged0(k, Kn, a.k.st, Tk_ - n0, D);
+      dd.load_ragged0(v, Vn, a.v.st, Tk_ - n0, D);
+      dd.load_ragged0(gk, gKn, a.gk.st, Tk_ - n0, D);
+      dd.load_ragged0(gv, gVn, a.gv.st, Tk_ - n0, D);
       if constexpr (LOADP) {
         const int n = n0 + 32 * half + stream_index(0, g, 0);
-        pn = load_frag_g<T>(Pm + (n < T_ ? n : 0));
+        pn = load_frag_g<T>(Pm + (n < Tk_ ? n : 0));
       }
       dma_wait();
     }
@@ -1394,10 +1398,9 @@ static hipError_t launch_gg_row_t(int dtype, const Params& a, bool load_p, bool 
 
 template <typename T, int D>
 static hipError_t launch_gg_col_t(int dtype, const Params& a, bool load_p, hipStream_t st, const Params* rowc) {
-  const int nblk = (a.T + kBlk - 1) / kBlk;
-  const int nx = nblk * a.nchunk_max;
+  const int nx = (a.Tk + kBlk - 1) / kBlk * a.nchunk_max;
   const bool fold = rowc && rowc->nchunk_max > 1;
-  dim3 grid(nx + (fold ? nblk * CombineSlot<D>::kSub : 0), a.B * a.H);
+  dim3 grid(nx + (fold ? (a.T + kBlk - 1) / kBlk * CombineSlot<D>::kSub : 0), a.B * a.H);
   const Params& c = fold ? *rowc : a;
   const bool xm = extended_mask(a);
 #if TTT_GG_COL8

@@ -92,25 +92,34 @@ void check(int rc, const char* what) {
   TORCH_CHECK(rc == 0, what, " failed (status ", rc, "): ", ttt_last_error());
 }
 
+// The shape of q [B,H,Tq,D] against k [B,H,Tk,D].
+ttt_shape shape_of(const at::Tensor& q, const at::Tensor& k) {
+  ttt_shape sh;
+  std::memset(&sh, 0, sizeof(sh));
+  sh.keys = k.size(2);
+  return sh;
+}
+
 at::Tensor stats_of(const at::Tensor& x) {
   return at::empty({x.size(0), x.size(1), x.size(2)}, x.options().dtype(at::kFloat));
 }
 
-// [B,H,T,T] P with rows padded to 8 elements (the kernels read rows in runs of 8).
-at::Tensor alloc_p(const at::Tensor& x) {
-  const int64_t t = x.size(2), tp = (t + 7) / 8 * 8;
-  at::Tensor buf = at::empty({x.size(0), x.size(1), t, tp}, x.options());
+// [B,H,Tq,Tk] P with rows padded to 8 elements (the kernels read rows in runs of 8).
+at::Tensor alloc_p(const at::Tensor& x, int64_t t) {
+  const int64_t tp = (t + 7) / 8 * 8;
+  at::Tensor buf = at::empty({x.size(0), x.size(1), x.size(2), tp}, x.options());
   return tp == t ? buf : buf.narrow(3, 0, t);
 }
 
-int64_t workspace_size(const ttt_problem& pr, int32_t entry, bool gdo) {
-  const int64_t n = ttt_attn_workspace_size(&pr, entry, gdo ? 1 : 0);
+int64_t workspace_size(const ttt_problem& pr, int32_t entry, bool gdo, const ttt_shape* shape = nullptr) {
+  const int64_t n = ttt_attn_workspace_size_shape(&pr, shape, entry, gdo ? 1 : 0);
   TORCH_CHECK(n >= 0, "ttt_attn_workspace_size failed: ", ttt_last_error());
   return n;
 }
 
-at::Tensor workspace(const ttt_problem& pr, int32_t entry, bool gdo, const at::Tensor& like, int64_t* bytes) {
-  const int64_t n = workspace_size(pr, entry, gdo);
+at::Tensor workspace(const ttt_problem& pr, const ttt_shape& shape, int32_t entry, bool gdo, const at::Tensor& like,
+                     int64_t* bytes) {
+  const int64_t n = workspace_size(pr, entry, gdo, &shape);
   *bytes = n;
   return n > 0 ? at::empty({n}, like.options().dtype(at::kByte)) : at::Tensor();
 }
@@ -138,12 +147,13 @@ std::vector<at::Tensor> fwd(const at::Tensor& q_, const at::Tensor& k_, const at
   const ttt_problem pr = problem_of(q, causal, scale, split_chunk, window, window_kind, bias, block_rows);
   at::Tensor o = at::empty(q.sizes(), q.options());
   at::Tensor lse = stats_of(q);
-  at::Tensor p = want_p ? alloc_p(q) : at::Tensor();
+  at::Tensor p = want_p ? alloc_p(q, k.size(2)) : at::Tensor();
   int64_t wsb = 0;
-  at::Tensor ws = workspace(pr, want_p ? TTT_ENTRY_FWD_P : TTT_ENTRY_FWD, false, q, &wsb);
+  const ttt_shape sh = shape_of(q, k);
+  at::Tensor ws = workspace(pr, sh, want_p ? TTT_ENTRY_FWD_P : TTT_ENTRY_FWD, false, q, &wsb);
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o);
   const ttt_view vp = want_p ? view_of(p) : none_view();
-  check(ttt_attn_fwd(&pr, &vq, &vk, &vv, &vo, lse.data_ptr<float>(), want_p ? &vp : nullptr, ptr_or_null(ws), wsb,
+  check(ttt_attn_fwd_shape(&pr, &sh, &vq, &vk, &vv, &vo, lse.data_ptr<float>(), want_p ? &vp : nullptr, ptr_or_null(ws), wsb,
                      stream_of(q)),
         "ttt_attn_fwd");
   return {o, lse, p};
@@ -178,25 +188,27 @@ std::vector<at::Tensor> bwd(const at::Tensor& q_, const at::Tensor& k_, const at
   return {dq, dk, dv, rowsum};
 }
 
-// The same through ttt_attn_bwd when both families take the library's split:
-// the dK/dV launch then also finishes dQ's split blocks.
+// The same through ttt_attn_bwd, both families with one split (0: the
+// library's): the dK/dV launch also finishes dQ's split blocks.  Also for
+// fewer or more keys than queries (ttt_shape).
 std::vector<at::Tensor> bwd_fused(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_,
                                   const at::Tensor& o_, const at::Tensor& dout_, const at::Tensor& lse,
                                   const c10::optional<at::Tensor>& p, bool causal, double scale, int64_t window,
-                                  int64_t window_kind, const c10::optional<at::Tensor>& bias) {
+                                  int64_t window_kind, const c10::optional<at::Tensor>& bias, int64_t split) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), o = ready(o_), dout = ready(dout_);
-  const ttt_problem pr = problem_of(q, causal, scale, 0, window, window_kind, bias);
+  const ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
   at::Tensor dq = at::empty(q.sizes(), q.options());
   at::Tensor dk = at::empty(k.sizes(), k.options());
   at::Tensor dv = at::empty(v.sizes(), v.options());
   at::Tensor rowsum = stats_of(q);
   int64_t wsb = 0;
-  at::Tensor ws = workspace(pr, TTT_ENTRY_BWD, false, q, &wsb);
+  const ttt_shape sh = shape_of(q, k);
+  at::Tensor ws = workspace(pr, sh, TTT_ENTRY_BWD, false, q, &wsb);
   const bool lp = p && p->defined();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
   const ttt_view vdq = view_of(dq), vdk = view_of(dk), vdv = view_of(dv);
-  check(ttt_attn_bwd(&pr, &vq, &vk, &vv, &vo, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr,
+  check(ttt_attn_bwd_shape(&pr, &sh, &vq, &vk, &vv, &vo, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr,
                      rowsum.data_ptr<float>(), &vdq, &vdk, &vdv, ptr_or_null(ws), wsb, stream_of(q)),
         "ttt_attn_bwd");
   return {dq, dk, dv, rowsum};
@@ -243,25 +255,27 @@ std::vector<at::Tensor> gg(const at::Tensor& q_, const at::Tensor& k_, const at:
   return {gq_out, gk_out, gv_out, gdo};
 }
 
-// The same through ttt_attn_gg when both passes take the library's split:
-// the column launch then also finishes the row pass's split blocks.
+// The same through ttt_attn_gg, both passes with one split (0: the library's):
+// the column launch also finishes the row pass's split blocks.  Also for
+// fewer or more keys than queries (ttt_shape).
 std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_,
                                  const at::Tensor& dout_, const at::Tensor& lse, const c10::optional<at::Tensor>& p,
                                  const at::Tensor& rowsum, const c10::optional<at::Tensor>& dq_,
                                  const at::Tensor& gq_, const at::Tensor& gk_, const at::Tensor& gv_, bool causal,
                                  double scale, bool want_gdo, int64_t window, int64_t window_kind,
-                                 const c10::optional<at::Tensor>& bias) {
+                                 const c10::optional<at::Tensor>& bias, int64_t split) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), dout = ready(dout_);
   const at::Tensor gq = ready(gq_), gk = ready(gk_), gv = ready(gv_);
   const c10::optional<at::Tensor> dq = ready(dq_);
-  const ttt_problem pr = problem_of(q, causal, scale, 0, window, window_kind, bias);
+  const ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
   at::Tensor gq_out = at::empty(q.sizes(), q.options());
   at::Tensor gk_out = at::empty(k.sizes(), k.options());
   at::Tensor gv_out = at::empty(v.sizes(), v.options());
   at::Tensor gdo = want_gdo ? at::empty(dout.sizes(), dout.options()) : at::Tensor();
   at::Tensor e = stats_of(q), f = stats_of(q);
   int64_t wsb = 0;
-  at::Tensor ws = workspace(pr, TTT_ENTRY_GG, want_gdo, q, &wsb);
+  const ttt_shape sh = shape_of(q, k);
+  at::Tensor ws = workspace(pr, sh, TTT_ENTRY_GG, want_gdo, q, &wsb);
   const bool lp = p && p->defined();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
@@ -270,7 +284,7 @@ std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, con
   const ttt_view ogdo = want_gdo ? view_of(gdo) : none_view();
   const bool ldq = dq && dq->defined();
   const ttt_view vdq = ldq ? view_of(*dq) : none_view();
-  check(ttt_attn_gg(&pr, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rowsum.data_ptr<float>(),
+  check(ttt_attn_gg_shape(&pr, &sh, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rowsum.data_ptr<float>(),
                     ldq ? &vdq : nullptr, &vgq, &vgk, &vgv, &ogq, &ogk, &ogv, want_gdo ? &ogdo : nullptr,
                     e.data_ptr<float>(), f.data_ptr<float>(), ptr_or_null(ws), wsb, stream_of(q)),
         "ttt_attn_gg");

@@ -45,29 +45,40 @@ def _check(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
 
 
 def _kernel_bias(attn_mask: Optional[torch.Tensor], q: torch.Tensor, lq: int, lk: int) -> Optional[torch.Tensor]:
-    """The mask as the kernels' [B,H,T,T] bias, T = max(Lq, Lk): with Lq < Lk
-    the Lk - Lq padded query rows in front get zeros (any finite values do:
-    those rows contribute nothing), with Lq > Lk the padded key columns at
-    the end get -inf."""
-    b, h = q.shape[:2]
-    t = max(lq, lk)
+    """The mask as the kernels' [B,H,Lq,Lk] bias."""
     if attn_mask is None:
-        if lq <= lk:
-            return None
+        return None
+    b, h = q.shape[:2]
+    m = attn_mask.detach()
+    if m.dim() > 4:
+        raise ValueError(f"attn_mask of shape {tuple(attn_mask.shape)} does not broadcast to [B, H, Lq, Lk]")
+    while m.dim() < 4:
+        m = m.unsqueeze(0)
+    if m.size(2) not in (1, lq) or m.size(3) not in (1, lk) or m.size(0) not in (1, b) or m.size(1) not in (1, h):
+        raise ValueError(f"attn_mask of shape {tuple(attn_mask.shape)} does not broadcast to {(b, h, lq, lk)}")
+    return m
+
+
+def _masked_layout(attn_mask: Optional[torch.Tensor], q: torch.Tensor, lq: int, lk: int):
+    """(layout, mask) of a problem of lq queries and lk keys, as it is.  With
+    no queries or no keys at all it is padded square instead, so that every
+    output exists: with Lq < Lk the Lk - Lq query rows in front get zeros (any
+    finite values do: those rows contribute nothing), with Lq > Lk the padded
+    key columns get -inf."""
+    b, h = q.shape[:2]
+    m = _kernel_bias(attn_mask, q, lq, lk)
+    if lq and lk:
+        bias = None if m is None else _lib.prep_bias(m, b, h, lq, q.dtype, q.device, lk)
+        return Layout(q.size(-1)), _lib.Mask(causal=False, bias=bias)
+    if m is None and lq > lk:
         m = torch.zeros((1, 1, 1, lk), dtype=q.dtype, device=q.device)
-    else:
-        m = attn_mask.detach()
-        if m.dim() > 4:
-            raise ValueError(f"attn_mask of shape {tuple(attn_mask.shape)} does not broadcast to [B, H, Lq, Lk]")
-        while m.dim() < 4:
-            m = m.unsqueeze(0)
-        if m.size(2) not in (1, lq) or m.size(3) not in (1, lk) or m.size(0) not in (1, b) or m.size(1) not in (1, h):
-            raise ValueError(f"attn_mask of shape {tuple(attn_mask.shape)} does not broadcast to {(b, h, lq, lk)}")
-    if lq < lk and m.size(2) != 1:
-        m = F.pad(m, (0, 0, lk - lq, 0))
-    if lq > lk:
-        m = F.pad(m.expand(m.size(0), m.size(1), m.size(2), lk), (0, lq - lk), value=float("-inf"))
-    return _lib.prep_bias(m, b, h, t, q.dtype, q.device)
+    if m is not None:
+        if lq < lk and m.size(2) != 1:
+            m = F.pad(m, (0, 0, lk - lq, 0))
+        if lq > lk:
+            m = F.pad(m.expand(m.size(0), m.size(1), m.size(2), lk), (0, lq - lk), value=float("-inf"))
+        m = _lib.prep_bias(m, b, h, max(lq, lk), q.dtype, q.device)
+    return Layout(q.size(-1), qpad=max(0, lk - lq), kpad=max(0, lq - lk)), _lib.Mask(causal=False, bias=m)
 
 
 class GradGradAttentionFn(torch.autograd.Function):
@@ -81,8 +92,7 @@ class GradGradAttentionFn(torch.autograd.Function):
     def forward(ctx, q, k, v, attn_mask, bwd_mode: str = "recompute"):
         _check(q, k, v)
         lq, lk = q.size(-2), k.size(-2)
-        lay = Layout(q.size(-1), qpad=max(0, lk - lq), kpad=max(0, lq - lk))
-        mask = _lib.Mask(causal=False, bias=_kernel_bias(attn_mask, q, lq, lk))
+        lay, mask = _masked_layout(attn_mask, q, lq, lk)
         return attn_forward(ctx, q, k, v, mask, 1.0 / math.sqrt(q.size(-1)), bwd_mode, lay)
 
     @staticmethod
