@@ -139,13 +139,17 @@ typedef struct ttt_problem {
                           shape (triton_attention.py:78-85).      */
 } ttt_problem;
 
-/* Shape of a problem whose operands are not square (the *_shape entry points):
- * queries and keys of different number.  With keys != seqlen the problem is
+/* Shape of a problem beyond seqlen and head_dim (the *_shape entry points):
+ * queries and keys of different number, and rows of fewer columns than the 64
+ * or 128 the kernels compute (head_dim; the columns in between count as zeros
+ * and are neither read nor written).  With keys != seqlen the problem is
  * neither causal nor windowed; q, o, dout, gq, dq and gq_out, gdout have
  * seqlen rows, k, v, gk, gv, dk, dv, gk_out and gv_out have `keys` rows, P and
  * the bias are [B,H,seqlen,keys], row statistics stay [B*H*seqlen]. */
 typedef struct ttt_shape {
   int64_t keys; /* key and value rows; 0 = seqlen */
+  int64_t cols; /* columns of every operand's and output's rows, a multiple
+                   of 8 up to head_dim; 0 = head_dim */
 } ttt_shape;
 
 /* Library version (major*10000 + minor*100 + patch). */

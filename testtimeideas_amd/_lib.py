@@ -2,8 +2,8 @@
 
 This module is the thin layer between torch tensors and the HIP kernels:
 it checks devices, dtypes and shapes, makes operands kernel-compatible
-(unit stride in the last dimension, 16-byte aligned rows, head dim padded to
-64 or 128), allocates outputs with torch's caching allocator, and calls the
+(unit stride in the last dimension, 16-byte aligned rows, a head dim that is
+not a multiple of 8 padded to 64 or 128), allocates outputs with torch's caching allocator, and calls the
 C entry points on torch's current HIP stream.  There is no fallback: if the
 library is missing or an operand is not on a ROCm device, it raises.
 
@@ -246,6 +246,19 @@ def padded_head_dim(d: int) -> int:
     if d <= 128:
         return 128
     raise NotImplementedError(f"head_dim {d} > 128 is not supported (the reference's kernels stop at 128 too)")
+
+
+def native_head_dim(d: int) -> bool:
+    """The fused entry points take rows of d columns as they are (the kernels
+    compute 64 or 128 columns and leave those past d alone)."""
+    return 0 < d <= 128 and d % 8 == 0
+
+
+def _one_call(q: torch.Tensor, k: torch.Tensor) -> bool:
+    """The problem runs through the fused entry points only: key and query
+    counts differ, or the head dim is not one that the per-kernel entries
+    take.  Such problems are not autotuned."""
+    return k.shape[2] != q.shape[2] or q.shape[3] not in (64, 128)
 
 
 def _kernel_ok(t: torch.Tensor) -> bool:
@@ -533,8 +546,7 @@ def fwd(q, k, v, mask, scale: float, want_p: bool):
     if _library_choice():
         return tuple(ext().fwd(q, k, v, m.causal, float(scale), bool(want_p), 0, int(m.window), int(m.window_kind),
                                m.bias, 0))
-    if k.shape[2] != q.shape[2]:
-        # fewer or more keys than queries: one entry call, never tuned
+    if _one_call(q, k):
         return tuple(_timed_call("ttt_attn_fwd", ext().fwd, q, k, v, m.causal, float(scale), bool(want_p),
                                  _split_chunk, int(m.window), int(m.window_kind), m.bias, _block_rows))
     ent = ENTRY_FWD_P if want_p else ENTRY_FWD
@@ -571,7 +583,7 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
     if _library_choice():
         return tuple(ext().bwd_fused(q, k, v, o, do, lse, p, m.causal, float(scale), int(m.window),
                                      int(m.window_kind), m.bias, 0))
-    if k.shape[2] != q.shape[2]:
+    if _one_call(q, k):
         return tuple(_timed_call("ttt_attn_bwd", ext().bwd_fused, q, k, v, o, do, lse, p, m.causal, float(scale),
                                  int(m.window), int(m.window_kind), m.bias, _split_chunk))
 
@@ -672,7 +684,7 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
     if _library_choice():
         return tuple(ext().gg_fused(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale),
                                     bool(want_gdo), int(m.window), int(m.window_kind), m.bias, 0))
-    if k.shape[2] != q.shape[2]:
+    if _one_call(q, k):
         return tuple(_timed_call("ttt_attn_gg", ext().gg_fused, q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal,
                                  float(scale), bool(want_gdo), int(m.window), int(m.window_kind), m.bias,
                                  _split_chunk))

@@ -51,15 +51,14 @@ namespace ttt {
 // layout.
 template <typename T, int D>
 __device__ __forceinline__ float row_dot_do_o(const typename Elem<T>::frag* dof, const T* O, int64_t ld,
-                                              int m, int T_) {
-  const int g = (threadIdx.x & 63) >> 4;
+                                              int m, int T_, int ncols) {
   float acc = 0.f;
+  typename Elem<T>::frag of[D / 32];
+  load_frags_row<T, D>(of, O, ld, m, T_, ncols);
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) {
-    const typename Elem<T>::frag of = load_frag_row<T>(O, ld, m, T_, 32 * ks + 8 * g);
+  for (int ks = 0; ks < D / 32; ++ks)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc += Elem<T>::f32(dof[ks][j]) * Elem<T>::f32(of[j]);
-  }
+    for (int j = 0; j < 8; ++j) acc += Elem<T>::f32(dof[ks][j]) * Elem<T>::f32(of[ks][j]);
   return group_sum(acc);
 }
 
@@ -149,17 +148,19 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
 
   frag dor[D / 32];
   mfrag dof[D / 32], qf[D / 32];
+  load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, a.d);
+  if constexpr (!LOADP) {
+    frag qr[D / 32];
+    load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) {
-    dor[ks] = load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g);
-    if constexpr (!LOADP) qf[ks] = M::from(load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g));
+    for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
   }
   const int64_t ridx = (int64_t)bh * T_ + m;
   float Dm;
   if (a.rowsum_in) {
     Dm = row_ok ? a.rowsum_in[ridx] : 0.f;
   } else {
-    Dm = row_dot_do_o<T, D>(dor, at<const T>(a.o, b, h), a.o.st, m, T_);
+    Dm = row_dot_do_o<T, D>(dor, at<const T>(a.o, b, h), a.o.st, m, T_, a.d);
     if (a.rowsum_out && ch == 0 && row_ok && g == 0) a.rowsum_out[ridx] = Dm;
   }
 #pragma unroll
@@ -176,7 +177,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   // uses offsets computed once, a ragged one clamps (stage_load).
   Stage<T, D> stK, stV;
   frag pn[2];
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st), soV = stage_offsets<T, D>(a.v.st);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d), soV = stage_offsets<T, D>(a.v.st, a.d);
   const T* Kn = K + (int64_t)cr.t0 * kBlk * a.k.st;
   const T* Vn = V + (int64_t)cr.t0 * kBlk * a.v.st;
   const T* Pn = LOADP ? Pm + cr.t0 * kBlk + stream_index(0, g, 0) : nullptr;
@@ -185,8 +186,8 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (!LOADP) {
       // Recompute: tile-indexed clamped loads, measured faster for this
       // variant than the running-pointer form below.
-      stage_load<T, D>(stK, K + (int64_t)n1 * a.k.st, a.k.st, Tk_ - n1, D);
-      stage_load<T, D>(stV, V + (int64_t)n1 * a.v.st, a.v.st, Tk_ - n1, D);
+      stage_load<T, D>(stK, K + (int64_t)n1 * a.k.st, a.k.st, Tk_ - n1, a.d);
+      stage_load<T, D>(stV, V + (int64_t)n1 * a.v.st, a.v.st, Tk_ - n1, a.d);
       return;
     }
     if (n1 + kBlk <= Tk_) {
@@ -197,8 +198,8 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
         pn[1] = load_frag_g<T>(Pn + 32);
       }
     } else {
-      stage_load<T, D>(stK, Kn, a.k.st, Tk_ - n1, D);
-      stage_load<T, D>(stV, Vn, a.v.st, Tk_ - n1, D);
+      stage_load<T, D>(stK, Kn, a.k.st, Tk_ - n1, a.d);
+      stage_load<T, D>(stV, Vn, a.v.st, Tk_ - n1, a.d);
       if constexpr (LOADP) load_p_frags<T>(pn, Pm, n1, Tk_);
     }
     Kn += kBlk * a.k.st;
@@ -206,7 +207,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (LOADP) Pn += kBlk;
   };
   // Direct loads of key tile nb into buffer set `par` (kDma).
-  const TileDma<T, D> dd;
+  const TileDma<T, D> dd(a.d);
   int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
   if constexpr (kDma) {
     dd.offsets(oK, a.k.st);
@@ -320,7 +321,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     for (int nb = cr.t0; nb < cr.t1; ++nb) tile(nb, Parity<2>{}, Parity<0>{});
   }
   if (cr.nch == 1)
-    store_acc_rows<T, D>(at<T>(a.dq, b, h), a.dq.st, m, T_, acc, a.scale);
+    store_acc_rows<T, D>(at<T>(a.dq, b, h), a.dq.st, m, T_, a.d, acc, a.scale);
   else
     store_acc_partial<D>(a.ws_acc + part_index(a, bh, nblk, mb, ch) * kBlk * D, rl, acc);
 }
@@ -418,15 +419,22 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const float* lse = LOADP ? nullptr : a.lse + (int64_t)bh * Tq_;
 
   mfrag vf[D / 32], kf[D / 32];
+  // V negated: dP's MFMAs start from the streamed rows' D and give D - dP;
+  // kept as computed (left to itself the compiler redoes the negation per tile)
+  if constexpr (!DV_ONLY) {
+    frag r[D / 32];
+    load_frags_row<T, D>(r, V, a.v.st, n, T_, a.d);
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) {
-    // negated: dP's MFMAs start from the streamed rows' D and give D - dP;
-    // kept as computed (left to itself the compiler redoes the negation per tile)
-    if constexpr (!DV_ONLY) {
-      vf[ks] = M::from(scale_frag<T>(load_frag_row<T>(V, a.v.st, n, T_, 32 * ks + 8 * g), -1.f));
+    for (int ks = 0; ks < D / 32; ++ks) {
+      vf[ks] = M::from(scale_frag<T>(r[ks], -1.f));
       M::keep(vf[ks]);
     }
-    if constexpr (!LOADP) kf[ks] = M::from(load_frag_row<T>(K, a.k.st, n, T_, 32 * ks + 8 * g));
+  }
+  if constexpr (!LOADP) {
+    frag r[D / 32];
+    load_frags_row<T, D>(r, K, a.k.st, n, T_, a.d);
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) kf[ks] = M::from(r[ks]);
   }
 
   f32x4 acc_dv[D / 16], acc_dk[D / 16];
@@ -445,8 +453,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const bool cols_full = n0 + kBlk <= T_;
   auto load_tile = [&](int mb) __attribute__((always_inline)) {
     const int m0 = mb * kBlk;
-    stage_load<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, D);
-    if constexpr (kNeedQ) stage_load<T, D>(stQ, Qn, a.q.st, Tq_ - m0, D);
+    stage_load<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, a.d);
+    if constexpr (kNeedQ) stage_load<T, D>(stQ, Qn, a.q.st, Tq_ - m0, a.d);
     if constexpr (LOADP) stage_load<T, kBlk>(stP, Pn, a.p.st, Tq_ - m0, T_ - n0);
     if constexpr (kNS > 0) stv = stat_load<kNS>(DV_ONLY ? lse : rs, lse, nullptr, nullptr, m0, Tq_ - m0);
     dOn += kBlk * a.dout.st;
@@ -455,8 +463,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   };
   // Direct loads of query tile mb into buffer set `par` (kDma), in order
   // through the same running pointers.
-  const TileDma<T, D> dd;
-  const TileDma<T, kBlk> dpt;
+  const TileDma<T, D> dd(a.d);
+  const TileDma<T, kBlk> dpt(kBlk);
   int odO[TileDma<T, D>::kPerWave], oQ[TileDma<T, D>::kPerWave], oP[TileDma<T, kBlk>::kPerWave];
   if constexpr (kDma) {
     dd.offsets(odO, a.dout.st);
@@ -583,8 +591,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     for (int mb = cr.t0; mb < cr.t1; ++mb) tile(mb, Parity<2>{}, Parity<0>{});
   }
   if (cr.nch == 1) {
-    store_acc_rows<T, D>(at<T>(a.dv, b, h), a.dv.st, n, T_, acc_dv, 1.f);
-    if constexpr (!DV_ONLY) store_acc_rows<T, D>(at<T>(a.dk, b, h), a.dk.st, n, T_, acc_dk, -a.scale);
+    store_acc_rows<T, D>(at<T>(a.dv, b, h), a.dv.st, n, T_, a.d, acc_dv, 1.f);
+    if constexpr (!DV_ONLY) store_acc_rows<T, D>(at<T>(a.dk, b, h), a.dk.st, n, T_, a.d, acc_dk, -a.scale);
   } else {
     float* base = a.ws_acc + part_index(a, bh, nblk, nb, ch) * 2 * kBlk * D;
     store_acc_partial<D>(base, cl, acc_dv);
@@ -621,21 +629,23 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   const T* dO = at<const T>(a.dout, b, h);
   const T* Pm = at<const T>(a.p, b, h) + (int64_t)(row_ok ? m : 0) * a.p.st;
 
+  frag dor[D / 32];
   mfrag dof[D / 32];
+  load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, a.d);
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) dof[ks] = M::from(load_frag_row<T>(dO, a.dout.st, m, T_, 32 * ks + 8 * g));
+  for (int ks = 0; ks < D / 32; ++ks) dof[ks] = M::from(dor[ks]);
 
   float sum = 0.f;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const RowMask<XM> mk(a, mb, m);
   Stage<T, D> stV;
-  stage_load<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, D);
+  stage_load<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, a.d);
   for (int nb = rg.lo; nb < rg.hi; ++nb) {
     const int n0 = nb * kBlk;
     __syncthreads();
     stage_store_tile<M>(stV, sV);
     __syncthreads();
-    if (nb + 1 < rg.hi) stage_load<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, Tk_ - n0 - kBlk, D);
+    if (nb + 1 < rg.hi) stage_load<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, Tk_ - n0 - kBlk, a.d);
     frag pr[2];
     load_p_frags<T>(pr, Pm, n0, Tk_);
     Tile p, dp;

@@ -85,10 +85,11 @@ size_t elem_bytes(int dtype) { return dtype == TTT_F32 ? 4 : 2; }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// A problem with its key count: q, o, dout and their gradients have seqlen
-// rows, k, v and theirs `keys`, P and the bias are [B,H,seqlen,keys].
+// A problem with its shape: q, o, dout and their gradients have seqlen rows,
+// k, v and theirs `keys`, P and the bias are [B,H,seqlen,keys]; rows have
+// `cols` columns.
 struct Prob : ttt_problem {
-  int64_t keys;
+  int64_t keys, cols;
 };
 
 // Checks a [B,H,T,X] operand and copies it into a kernel View.
@@ -122,6 +123,9 @@ int check_problem(const Prob* pr) {
     return fail(TTT_ERR_INVALID_ARGUMENT, "seqlen %lld exceeds 2^24", (long long)pr->seqlen);
   if (pr->keys < 1 || pr->keys > (int64_t)1 << 24)
     return fail(TTT_ERR_INVALID_ARGUMENT, "keys %lld: must be 1 .. 2^24", (long long)pr->keys);
+  if (pr->cols < 1 || pr->cols > pr->head_dim || pr->cols % 8 != 0)
+    return fail(TTT_ERR_INVALID_ARGUMENT, "cols %lld: must be a multiple of 8 up to head_dim %lld",
+                (long long)pr->cols, (long long)pr->head_dim);
   if (pr->keys != pr->seqlen && (pr->causal != 0 || pr->window != 0))
     return fail(TTT_ERR_INVALID_ARGUMENT, "%lld keys for %lld queries: neither causal nor windowed",
                 (long long)pr->keys, (long long)pr->seqlen);
@@ -148,6 +152,7 @@ int make_prob(const ttt_problem* pr, const ttt_shape* shape, Prob* out) {
   if (!pr) return fail(TTT_ERR_INVALID_ARGUMENT, "problem: null pointer");
   static_cast<ttt_problem&>(*out) = *pr;
   out->keys = shape && shape->keys != 0 ? shape->keys : pr->seqlen;
+  out->cols = shape && shape->cols != 0 ? shape->cols : pr->head_dim;
   return check_problem(out);
 }
 
@@ -435,6 +440,7 @@ ttt::Params base_params(const Prob* pr) {
   a.H = (int)pr->heads;
   a.T = (int)pr->seqlen;
   a.Tk = (int)pr->keys;
+  a.d = (int)pr->cols;
   a.causal = pr->causal;
   a.win = eff_window(pr);
   a.win_kind = pr->window_kind;

@@ -111,7 +111,7 @@ __device__ __forceinline__ void combine_sum_block(const Params& a, int which, in
   const int nch = block_nch(a, cs.blk, col);
   if (nch <= 1) return;
   const int row = cs.blk * kBlk + cs.r;
-  if (row >= T_) return;
+  if (row >= T_ || cs.d0 >= a.d) return;
   const int64_t p0 = part_index(a, bh, nblk, cs.blk, 0);
   if (which == kOutO || which == kOutDQ) {
     f32x4 v;
@@ -155,7 +155,7 @@ __device__ __forceinline__ void combine_gg_row_block(const Params& a, int bx, in
   if (nch <= 1) return;
   const int r = cs.r;
   const int row = cs.blk * kBlk + r;
-  if (row >= T_) return;
+  if (row >= T_ || cs.d0 >= a.d) return;
   const int64_t p0 = part_index(a, bh, nblk, cs.blk, 0);
   if constexpr (!GDO) {
     if (a.dq.p) {

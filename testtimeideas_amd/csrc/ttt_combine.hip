@@ -28,7 +28,7 @@ __global__ __launch_bounds__(kThreads) void k_combine_fwd(Params a) {
   if (nch <= 1) return;
   const int r = cs.r;
   const int row = cs.blk * kBlk + r;
-  if (row >= T_) return;
+  if (row >= T_ || cs.d0 >= a.d) return;
   const int64_t p0 = part_index(a, bh, nblk, cs.blk, 0);
   float mm = -INFINITY;
   if (nch <= kBatch) {

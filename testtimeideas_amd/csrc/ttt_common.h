@@ -69,6 +69,13 @@ struct Params {
   // what they are, where padding the queries to the keys cost the square
   // (b2 h6 d64 fp32, 512 queries of 2048 keys with a mask, step 1315 -> 457 us).
   int Tk;
+  // Columns of every [B,H,T,*] row, a multiple of 8, at most the kernel's head
+  // dim D.  Stationary fragments read as zero past them, so nothing past them
+  // reaches a score; streamed tiles repeat chunk 0 there, and the columns that
+  // gives an output are not stored.  So a head dim of 80 runs the D = 128
+  // kernels on its own rows: padding copies took two launches per operand
+  // (b2 h8 T1000 d80 bf16 causal, forward and backward 100 -> 69 us).
+  int d;
   int causal;
   float scale;       // s
   float scale_log2;  // s * log2(e): scores are kept in base-2 units
@@ -482,13 +489,26 @@ __device__ __forceinline__ typename Elem<T>::frag zero_frag() {
   return r;
 }
 
-// Row `row` of a [T][*] matrix, eight elements from column `col`; zero when
-// row >= nrows.
-template <typename T>
-__device__ __forceinline__ typename Elem<T>::frag load_frag_row(const T* base, int64_t ld, int row,
-                                                                int nrows, int col) {
-  if (row < nrows) return load_frag_g<T>(base + (int64_t)row * ld + col);
-  return zero_frag<T>();
+// The D/32 fragments of row `row` of a [T][ncols] matrix (f[ks]: eight elements
+// from column 32ks + 8g); zero when row >= nrows, and past ncols (a multiple
+// of 8).  Rows of D columns take one uniform test for it.
+template <typename T, int D>
+__device__ __forceinline__ void load_frags_row(typename Elem<T>::frag* f, const T* base, int64_t ld, int row,
+                                               int nrows, int ncols) {
+  const int g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+  for (int ks = 0; ks < D / 32; ++ks) {
+    const int col = 32 * ks + 8 * g;
+    if (row < nrows)
+      f[ks] = load_frag_g<T>(base + (int64_t)row * ld + (col < ncols ? col : 0));
+    else
+      f[ks] = zero_frag<T>();
+  }
+  if (ncols < D) {
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks)
+      if (32 * ks + 8 * g >= ncols) f[ks] = zero_frag<T>();
+  }
 }
 
 // Store eight consecutive elements (16-bit types: one 16-byte store).
@@ -801,7 +821,9 @@ __device__ __forceinline__ u32x4 load16(const void* p) {
   return *(global_u32x4*)p;  // address-space cast (C-style: the only form C++ allows)
 }
 
-// Load a 64 x NCOL tile whose element [0][0] is at g (row stride ld).
+// Load a 64 x NCOL tile whose element [0][0] is at g (row stride ld).  Columns
+// past cols_valid of an operand's rows are never consumed (Params::d); of P's
+// and the statistics' they are masked.
 // Every thread issues the same unconditional loads on every tile: rows at or
 // beyond rows_valid repeat row rows_valid-1 and 16-byte chunks starting at or
 // beyond cols_valid repeat chunk 0, and a chunk that straddles cols_valid is
@@ -834,10 +856,11 @@ struct StageOff {
 };
 
 template <typename T, int NCOL>
-__device__ __forceinline__ StageOff<T, NCOL> stage_offsets(int64_t ld) {
+__device__ __forceinline__ StageOff<T, NCOL> stage_offsets(int64_t ld, int ncols) {
   typedef Stage<T, NCOL> S;
   const int tid = threadIdx.x;
-  const int col = (tid % S::kChunksPerRow) * S::kChunk;
+  const int c0 = (tid % S::kChunksPerRow) * S::kChunk;
+  const int col = c0 < ncols ? c0 : 0;  // as stage_load
   StageOff<T, NCOL> so;
 #pragma unroll
   for (int ps = 0; ps < S::kPasses; ++ps) {
@@ -1318,25 +1341,27 @@ __device__ __forceinline__ float group_max(float x) {
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // Store a transposed accumulator acc^T[d][stationary] (this lane: stationary
-// row `row`, d = 16*ds + 4*g + i) to a row-major [T][D] output, scaled.
+// row `row`, d = 16*ds + 4*g + i) to a row-major [T][ncols] output, scaled.
 template <typename T, int D>
-__device__ __forceinline__ void store_acc_rows(T* base, int64_t ld, int row, int nrows, const f32x4* acc,
+__device__ __forceinline__ void store_acc_rows(T* base, int64_t ld, int row, int nrows, int ncols, const f32x4* acc,
                                                float mul) {
   if (row >= nrows) return;
   const int g = (threadIdx.x & 63) >> 4;
   T* rp = base + (int64_t)row * ld + 4 * g;
 #pragma unroll
-  for (int ds = 0; ds < D / 16; ++ds) store4<T>(rp + 16 * ds, acc[ds] * mul);
+  for (int ds = 0; ds < D / 16; ++ds)
+    if (16 * ds + 4 * g < ncols) store4<T>(rp + 16 * ds, acc[ds] * mul);
 }
 
 // The elements store_acc_rows would write (this lane: row `row`, columns
-// 16*ds + 4g .. +3), read as fp32; zero past nrows.
+// 16*ds + 4g .. +3), read as fp32; zero past nrows and ncols.
 template <typename T, int D>
-__device__ __forceinline__ void load_acc_rows(const T* base, int64_t ld, int row, int nrows, f32x4* out) {
+__device__ __forceinline__ void load_acc_rows(const T* base, int64_t ld, int row, int nrows, int ncols, f32x4* out) {
   const int g = (threadIdx.x & 63) >> 4;
   const T* rp = base + (int64_t)(row < nrows ? row : 0) * ld + 4 * g;
 #pragma unroll
-  for (int ds = 0; ds < D / 16; ++ds) out[ds] = row < nrows ? load4<T>(rp + 16 * ds) : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int ds = 0; ds < D / 16; ++ds)
+    out[ds] = row < nrows && 16 * ds + 4 * g < ncols ? load4<T>(rp + 16 * ds) : f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
 // Offset (floats) of element (row r, column d) in one 64 x D block of fp32
@@ -1419,7 +1444,8 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
   static_assert(kPerWave * NW == kInstr, "tile shape");
   int row[kPerWave], col[kPerWave];  // this lane's logical row and first column per instruction
   int wslice;                         // 1024 * wave index, uniform
-  __device__ __forceinline__ TileDma() {
+  // ncols: columns the rows have; chunks past them repeat chunk 0.
+  __device__ __forceinline__ explicit TileDma(int ncols) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     wslice = 1024 * __builtin_amdgcn_readfirstlane(w);
 #pragma unroll
@@ -1427,7 +1453,8 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
       const int byte = 1024 * (w + NW * q) + 16 * lane;
       const int r = byte / kRowBytes;
       row[q] = r;
-      col[q] = (((byte % kRowBytes) / 16) ^ L::swz(r)) * L::kChunk;
+      const int c = (((byte % kRowBytes) / 16) ^ L::swz(r)) * L::kChunk;
+      col[q] = c < ncols ? c : 0;
     }
   }
   // Byte offsets (row stride ld elements) of this lane's fetches for an

@@ -155,8 +155,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const T* K = at<const T>(a.k, b, h);
   const T* V = at<const T>(a.v, b, h);
   frag qr[D / 32];
-#pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) qr[ks] = load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g);
+  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
 
   f32x4 acc[D / 16];
 #pragma unroll
@@ -166,7 +165,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   // Register stage of the next tile's K and V (loads issued one tile ahead
   // of their use).
   Stage<T, D> stK, stV;
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st), soV = stage_offsets<T, D>(a.v.st);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d), soV = stage_offsets<T, D>(a.v.st, a.d);
   auto load_kv = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
@@ -175,8 +174,8 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       stage_load_full<T, D>(stK, kp, soK);
       stage_load_full<T, D>(stV, vp, soV);
     } else {
-      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, D);
-      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, D);
+      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, a.d);
+      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, a.d);
     }
   };
   // Key tile nb from LDS tiles cK, cV.
@@ -267,7 +266,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     mm_s<M>(acc, cV, pf);
   };
   if constexpr (kDma) {
-    const TileDma<T, D> dd;
+    const TileDma<T, D> dd(a.d);
     int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
     dd.offsets(oK, a.k.st);
     dd.offsets(oV, a.v.st);
@@ -322,7 +321,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const int64_t ridx = (int64_t)bh * T_ + m;
   if (cr.nch == 1) {
     if (m < T_ && g == 0) a.lse[ridx] = (mx + __log2f(l)) * kLn2;
-    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, acc, 1.f / l);
+    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, a.d, acc, 1.f / l);
   } else {
     const int64_t part = part_index(a, bh, nblk, mb, ch);
     store_acc_partial<D>(a.ws_acc + part * kBlk * D, rl, acc);
@@ -410,11 +409,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   const T* K = at<const T>(a.k, b, h);
   const T* V = at<const T>(a.v, b, h);
   frag qf[2][KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    qf[0][ks] = load_frag_row<T>(Q, a.q.st, m0, T_, 32 * ks + 8 * g);
-    qf[1][ks] = load_frag_row<T>(Q, a.q.st, m1, T_, 32 * ks + 8 * g);
-  }
+  load_frags_row<T, D>(qf[0], Q, a.q.st, m0, T_, a.d);
+  load_frags_row<T, D>(qf[1], Q, a.q.st, m1, T_, a.d);
   // Raw scores q.k; c = |s| log2(e) is folded into one FMA per element (q
   // negated for a negative scale).  Masks are applied after that FMA, so a
   // zero scale (c = 0) gives every visible key the same probability.
@@ -432,7 +428,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   for (int i = 0; i < D / 16; ++i) acc0[i] = acc1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float l0 = 0.f, l1 = 0.f, sh0, sh1;
 
-  const TileDma<T, D> dd;
+  const TileDma<T, D> dd(a.d);
   int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
   dd.offsets(oK, a.k.st);
   dd.offsets(oV, a.v.st);
@@ -590,7 +586,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     const float lt = group_sum(lv);
     if ((hi + C - 1) / C == 1) {
       if (m < T_ && g == 0) a.lse[rbase + m] = (shv + __log2f(lt)) * kLn2;
-      store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, ac, 1.f / lt);
+      store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, a.d, ac, 1.f / lt);
     } else {
       const int64_t part = part_index(a, bh, nblk, mb, ch);
       store_acc_partial<D>(a.ws_acc + part * kBlk * D, rl, ac);
@@ -649,9 +645,11 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
+  typename Elem<T>::frag qr[D / 32];
   mfrag qf[D / 32];
+  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g));
+  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
 
   float mx = -INFINITY, l = 0.f;
   const float csl = a.scale_log2;
@@ -659,14 +657,14 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   Stage<T, D> stK[R];
   // Tiles past the chunk load its last tile again (unconditional loads; the
   // round masks them out).
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d);
   auto load_k = [&](int nb, Stage<T, D>& sk) __attribute__((always_inline)) {
     const int n1 = (nb < cr.t1 ? nb : cr.t1 - 1) * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
     if (D == 64 && n1 + kBlk <= Tk_)  // full tile: offsets computed once
       stage_load_full<T, D>(sk, kp, soK);
     else
-      stage_load<T, D>(sk, kp, a.k.st, Tk_ - n1, D);
+      stage_load<T, D>(sk, kp, a.k.st, Tk_ - n1, a.d);
   };
   // One round: key tiles nb .. nb + R - 1 from the LDS tiles tile_k(i).
   auto round = [&](int nb, auto tile_k) __attribute__((always_inline)) {
@@ -743,7 +741,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       mx = mnew;
   };
   if constexpr (kDma) {
-    const TileDma<T, D> dd;
+    const TileDma<T, D> dd(a.d);
     int oK[TileDma<T, D>::kPerWave];
     dd.offsets(oK, a.k.st);
     // Tiles past the chunk load its last tile again (the round masks them).
@@ -895,16 +893,18 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   // 16-bit d = 64: full tiles of P stored in whole row segments (store_p_rows;
   // at d = 128 the same stores measured slower steps).
   constexpr bool kRowPair = sizeof(T) == 2 && D == 64;
+  frag qr[D / 32];
   mfrag qf[D / 32];
+  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(load_frag_row<T>(Q, a.q.st, m, T_, 32 * ks + 8 * g));
+  for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
 
   f32x4 acc[D / 16];
 #pragma unroll
   for (int i = 0; i < D / 16; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   Stage<T, D> stK, stV;
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st), soV = stage_offsets<T, D>(a.v.st);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d), soV = stage_offsets<T, D>(a.v.st, a.d);
   auto load_kv = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
@@ -913,8 +913,8 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
       stage_load_full<T, D>(stK, kp, soK);
       stage_load_full<T, D>(stV, vp, soV);
     } else {
-      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, D);
-      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, D);
+      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, a.d);
+      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, a.d);
     }
   };
   // With a.defer_p, the P stores of a full tile wait in registers until the
@@ -1028,7 +1028,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
       mm_s<M>(acc, cV, pf);
   };
   if constexpr (kDma) {
-    const TileDma<T, D> dd;
+    const TileDma<T, D> dd(a.d);
     int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
     dd.offsets(oK, a.k.st);
     dd.offsets(oV, a.v.st);
@@ -1080,7 +1080,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
     }
   }
   if (cr.nch == 1) {
-    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, acc, 1.f);
+    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, a.d, acc, 1.f);
   } else {
     store_acc_partial<D>(a.ws_acc + part_index(a, bh, nblk, mb, ch) * kBlk * D, rl, acc);
   }

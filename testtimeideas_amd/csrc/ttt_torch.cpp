@@ -7,8 +7,8 @@
 // The ctypes binding (testtimeideas_amd/_lib.py) spends tens of microseconds
 // of Python per call building views, problems and outputs; the autograd path
 // of one grad-grad step makes three such calls.  This module does the same
-// work in C++: it takes tensors with the head dim already padded (by the
-// Python layer), copies any whose strides the C ABI does not take (ready),
+// work in C++: it takes tensors whose head dim is a multiple of 8 up to 128
+// (the Python layer pads others), copies any whose strides the C ABI does not take (ready),
 // allocates outputs, statistics and the workspace with torch's caching
 // allocator on the tensors' device, and calls the C entry points on torch's
 // current HIP stream.  A nonzero status raises
@@ -92,11 +92,16 @@ void check(int rc, const char* what) {
   TORCH_CHECK(rc == 0, what, " failed (status ", rc, "): ", ttt_last_error());
 }
 
-// The shape of q [B,H,Tq,D] against k [B,H,Tk,D].
-ttt_shape shape_of(const at::Tensor& q, const at::Tensor& k) {
+// The shape of q [B,H,Tq,d] against k [B,H,Tk,d], for the entry points that
+// take one; their problem's head_dim is d rounded up to 64 or 128 (the others
+// refuse rows of any other length).
+ttt_shape shape_of(const at::Tensor& q, const at::Tensor& k, ttt_problem* pr) {
+  const int64_t d = q.size(3);
+  pr->head_dim = d <= 64 ? 64 : d <= 128 ? 128 : d;
   ttt_shape sh;
   std::memset(&sh, 0, sizeof(sh));
   sh.keys = k.size(2);
+  sh.cols = d;
   return sh;
 }
 
@@ -144,12 +149,12 @@ std::vector<at::Tensor> fwd(const at::Tensor& q_, const at::Tensor& k_, const at
                             double scale, bool want_p, int64_t split_chunk, int64_t window, int64_t window_kind,
                             const c10::optional<at::Tensor>& bias, int64_t block_rows) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_);
-  const ttt_problem pr = problem_of(q, causal, scale, split_chunk, window, window_kind, bias, block_rows);
+  ttt_problem pr = problem_of(q, causal, scale, split_chunk, window, window_kind, bias, block_rows);
+  const ttt_shape sh = shape_of(q, k, &pr);
   at::Tensor o = at::empty(q.sizes(), q.options());
   at::Tensor lse = stats_of(q);
   at::Tensor p = want_p ? alloc_p(q, k.size(2)) : at::Tensor();
   int64_t wsb = 0;
-  const ttt_shape sh = shape_of(q, k);
   at::Tensor ws = workspace(pr, sh, want_p ? TTT_ENTRY_FWD_P : TTT_ENTRY_FWD, false, q, &wsb);
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o);
   const ttt_view vp = want_p ? view_of(p) : none_view();
@@ -196,13 +201,13 @@ std::vector<at::Tensor> bwd_fused(const at::Tensor& q_, const at::Tensor& k_, co
                                   const c10::optional<at::Tensor>& p, bool causal, double scale, int64_t window,
                                   int64_t window_kind, const c10::optional<at::Tensor>& bias, int64_t split) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), o = ready(o_), dout = ready(dout_);
-  const ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
+  ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
+  const ttt_shape sh = shape_of(q, k, &pr);
   at::Tensor dq = at::empty(q.sizes(), q.options());
   at::Tensor dk = at::empty(k.sizes(), k.options());
   at::Tensor dv = at::empty(v.sizes(), v.options());
   at::Tensor rowsum = stats_of(q);
   int64_t wsb = 0;
-  const ttt_shape sh = shape_of(q, k);
   at::Tensor ws = workspace(pr, sh, TTT_ENTRY_BWD, false, q, &wsb);
   const bool lp = p && p->defined();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o), vdo = view_of(dout);
@@ -267,14 +272,14 @@ std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, con
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), dout = ready(dout_);
   const at::Tensor gq = ready(gq_), gk = ready(gk_), gv = ready(gv_);
   const c10::optional<at::Tensor> dq = ready(dq_);
-  const ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
+  ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
+  const ttt_shape sh = shape_of(q, k, &pr);
   at::Tensor gq_out = at::empty(q.sizes(), q.options());
   at::Tensor gk_out = at::empty(k.sizes(), k.options());
   at::Tensor gv_out = at::empty(v.sizes(), v.options());
   at::Tensor gdo = want_gdo ? at::empty(dout.sizes(), dout.options()) : at::Tensor();
   at::Tensor e = stats_of(q), f = stats_of(q);
   int64_t wsb = 0;
-  const ttt_shape sh = shape_of(q, k);
   at::Tensor ws = workspace(pr, sh, TTT_ENTRY_GG, want_gdo, q, &wsb);
   const bool lp = p && p->defined();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vdo = view_of(dout);

@@ -42,18 +42,19 @@ BWD_MODES = RECOMPUTE_MODES + SAVE_P_MODES + ("custom",)
 
 
 class Layout:
-    """How a problem's operands map onto the kernels' square [B, H, T, Dp]
-    operands: the head dim is zero-padded to Dp (64 or 128); with fewer
-    queries than keys, query-side tensors (q, O, dO and their gradients) get
-    `qpad` zero rows in front; with more queries than keys, key-side tensors
-    (k, v and their gradients) get `kpad` zero rows at the end.  Zero query
+    """How a problem's operands map onto the kernels' [B, H, T, D] operands.
+    Head dims that are multiples of 8 go as they are, others are zero-padded
+    to 64 or 128.  A problem without queries or without keys is made square:
+    query-side tensors (q, O, dO and their gradients) get `qpad` zero rows in
+    front, key-side tensors (k, v and their gradients) `kpad` zero rows at the
+    end.  Zero query
     rows (q = dO = 0, cotangent 0) contribute nothing to any gradient, and
     padded keys are masked by the bias, so the results on the real rows are
     those of the rectangular problem."""
 
     def __init__(self, d: int, qpad: int = 0, kpad: int = 0):
         self.d = d
-        self.dpad = _lib.padded_head_dim(d)
+        self.dpad = d if _lib.native_head_dim(d) else _lib.padded_head_dim(d)
         self.qpad = qpad
         self.kpad = kpad
         # operands go to the kernels as they are (when their strides allow)
