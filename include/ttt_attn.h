@@ -149,7 +149,8 @@ typedef struct ttt_problem {
 typedef struct ttt_shape {
   int64_t keys; /* key and value rows; 0 = seqlen */
   int64_t cols; /* columns of every operand's and output's rows, a multiple
-                   of 8 up to head_dim; 0 = head_dim */
+                   of 8 up to head_dim (fp32 at head_dim 128: 128);
+                   0 = head_dim */
 } ttt_shape;
 
 /* Library version (major*10000 + minor*100 + patch). */

@@ -248,10 +248,11 @@ def padded_head_dim(d: int) -> int:
     raise NotImplementedError(f"head_dim {d} > 128 is not supported (the reference's kernels stop at 128 too)")
 
 
-def native_head_dim(d: int) -> bool:
+def native_head_dim(d: int, dtype: torch.dtype) -> bool:
     """The fused entry points take rows of d columns as they are (the kernels
-    compute 64 or 128 columns and leave those past d alone)."""
-    return 0 < d <= 128 and d % 8 == 0
+    compute 64 or 128 columns and leave those past d alone; in fp32 only the
+    64-column kernels do)."""
+    return d % 8 == 0 and (0 < d <= 64 or d == 128 or (64 < d < 128 and dtype != torch.float32))
 
 
 def _one_call(q: torch.Tensor, k: torch.Tensor) -> bool:

@@ -148,10 +148,10 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
 
   frag dor[D / 32];
   mfrag dof[D / 32], qf[D / 32];
-  load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, a.d);
+  load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, cols_of<T, D>(a));
   if constexpr (!LOADP) {
     frag qr[D / 32];
-    load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
+    load_frags_row<T, D>(qr, Q, a.q.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
   }
@@ -160,7 +160,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   if (a.rowsum_in) {
     Dm = row_ok ? a.rowsum_in[ridx] : 0.f;
   } else {
-    Dm = row_dot_do_o<T, D>(dor, at<const T>(a.o, b, h), a.o.st, m, T_, a.d);
+    Dm = row_dot_do_o<T, D>(dor, at<const T>(a.o, b, h), a.o.st, m, T_, cols_of<T, D>(a));
     if (a.rowsum_out && ch == 0 && row_ok && g == 0) a.rowsum_out[ridx] = Dm;
   }
 #pragma unroll
@@ -175,9 +175,11 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
 
   // Key tiles are fetched in order through running pointers; a full tile
   // uses offsets computed once, a ragged one clamps (stage_load).
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stK, stV;
   frag pn[2];
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d), soV = stage_offsets<T, D>(a.v.st, a.d);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, cols_of<T, D>(a));
+  const StageOff<T, D> soV = stage_offsets<T, D>(a.v.st, cols_of<T, D>(a));
   const T* Kn = K + (int64_t)cr.t0 * kBlk * a.k.st;
   const T* Vn = V + (int64_t)cr.t0 * kBlk * a.v.st;
   const T* Pn = LOADP ? Pm + cr.t0 * kBlk + stream_index(0, g, 0) : nullptr;
@@ -186,8 +188,8 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (!LOADP) {
       // Recompute: tile-indexed clamped loads, measured faster for this
       // variant than the running-pointer form below.
-      stage_load<T, D>(stK, K + (int64_t)n1 * a.k.st, a.k.st, Tk_ - n1, a.d);
-      stage_load<T, D>(stV, V + (int64_t)n1 * a.v.st, a.v.st, Tk_ - n1, a.d);
+      stage_load_at<T, D>(stK, K + (int64_t)n1 * a.k.st, a.k.st, Tk_ - n1, scol);
+      stage_load_at<T, D>(stV, V + (int64_t)n1 * a.v.st, a.v.st, Tk_ - n1, scol);
       return;
     }
     if (n1 + kBlk <= Tk_) {
@@ -198,8 +200,8 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
         pn[1] = load_frag_g<T>(Pn + 32);
       }
     } else {
-      stage_load<T, D>(stK, Kn, a.k.st, Tk_ - n1, a.d);
-      stage_load<T, D>(stV, Vn, a.v.st, Tk_ - n1, a.d);
+      stage_load_at<T, D>(stK, Kn, a.k.st, Tk_ - n1, scol);
+      stage_load_at<T, D>(stV, Vn, a.v.st, Tk_ - n1, scol);
       if constexpr (LOADP) load_p_frags<T>(pn, Pm, n1, Tk_);
     }
     Kn += kBlk * a.k.st;
@@ -207,7 +209,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (LOADP) Pn += kBlk;
   };
   // Direct loads of key tile nb into buffer set `par` (kDma).
-  const TileDma<T, D> dd(a.d);
+  const TileDma<T, D> dd(cols_of<T, D>(a));
   int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
   if constexpr (kDma) {
     dd.offsets(oK, a.k.st);
@@ -321,7 +323,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     for (int nb = cr.t0; nb < cr.t1; ++nb) tile(nb, Parity<2>{}, Parity<0>{});
   }
   if (cr.nch == 1)
-    store_acc_rows<T, D>(at<T>(a.dq, b, h), a.dq.st, m, T_, a.d, acc, a.scale);
+    store_acc_rows<T, D>(at<T>(a.dq, b, h), a.dq.st, m, T_, cols_of<T, D>(a), acc, a.scale);
   else
     store_acc_partial<D>(a.ws_acc + part_index(a, bh, nblk, mb, ch) * kBlk * D, rl, acc);
 }
@@ -423,7 +425,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   // kept as computed (left to itself the compiler redoes the negation per tile)
   if constexpr (!DV_ONLY) {
     frag r[D / 32];
-    load_frags_row<T, D>(r, V, a.v.st, n, T_, a.d);
+    load_frags_row<T, D>(r, V, a.v.st, n, T_, cols_of<T, D>(a));
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) {
       vf[ks] = M::from(scale_frag<T>(r[ks], -1.f));
@@ -432,7 +434,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   }
   if constexpr (!LOADP) {
     frag r[D / 32];
-    load_frags_row<T, D>(r, K, a.k.st, n, T_, a.d);
+    load_frags_row<T, D>(r, K, a.k.st, n, T_, cols_of<T, D>(a));
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) kf[ks] = M::from(r[ks]);
   }
@@ -443,6 +445,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
 
   // Query tiles are fetched in order through running pointers with clamped
   // addressing (stage_load).
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stdO, stQ;
   Stage<T, kBlk> stP;
   float stv = 0.f;
@@ -453,8 +456,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const bool cols_full = n0 + kBlk <= T_;
   auto load_tile = [&](int mb) __attribute__((always_inline)) {
     const int m0 = mb * kBlk;
-    stage_load<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, a.d);
-    if constexpr (kNeedQ) stage_load<T, D>(stQ, Qn, a.q.st, Tq_ - m0, a.d);
+    stage_load_at<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, scol);
+    if constexpr (kNeedQ) stage_load_at<T, D>(stQ, Qn, a.q.st, Tq_ - m0, scol);
     if constexpr (LOADP) stage_load<T, kBlk>(stP, Pn, a.p.st, Tq_ - m0, T_ - n0);
     if constexpr (kNS > 0) stv = stat_load<kNS>(DV_ONLY ? lse : rs, lse, nullptr, nullptr, m0, Tq_ - m0);
     dOn += kBlk * a.dout.st;
@@ -463,7 +466,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   };
   // Direct loads of query tile mb into buffer set `par` (kDma), in order
   // through the same running pointers.
-  const TileDma<T, D> dd(a.d);
+  const TileDma<T, D> dd(cols_of<T, D>(a));
   const TileDma<T, kBlk> dpt(kBlk);
   int odO[TileDma<T, D>::kPerWave], oQ[TileDma<T, D>::kPerWave], oP[TileDma<T, kBlk>::kPerWave];
   if constexpr (kDma) {
@@ -591,8 +594,8 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     for (int mb = cr.t0; mb < cr.t1; ++mb) tile(mb, Parity<2>{}, Parity<0>{});
   }
   if (cr.nch == 1) {
-    store_acc_rows<T, D>(at<T>(a.dv, b, h), a.dv.st, n, T_, a.d, acc_dv, 1.f);
-    if constexpr (!DV_ONLY) store_acc_rows<T, D>(at<T>(a.dk, b, h), a.dk.st, n, T_, a.d, acc_dk, -a.scale);
+    store_acc_rows<T, D>(at<T>(a.dv, b, h), a.dv.st, n, T_, cols_of<T, D>(a), acc_dv, 1.f);
+    if constexpr (!DV_ONLY) store_acc_rows<T, D>(at<T>(a.dk, b, h), a.dk.st, n, T_, cols_of<T, D>(a), acc_dk, -a.scale);
   } else {
     float* base = a.ws_acc + part_index(a, bh, nblk, nb, ch) * 2 * kBlk * D;
     store_acc_partial<D>(base, cl, acc_dv);
@@ -631,21 +634,22 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
 
   frag dor[D / 32];
   mfrag dof[D / 32];
-  load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, a.d);
+  load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) dof[ks] = M::from(dor[ks]);
 
   float sum = 0.f;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const RowMask<XM> mk(a, mb, m);
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stV;
-  stage_load<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, a.d);
+  stage_load_at<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, scol);
   for (int nb = rg.lo; nb < rg.hi; ++nb) {
     const int n0 = nb * kBlk;
     __syncthreads();
     stage_store_tile<M>(stV, sV);
     __syncthreads();
-    if (nb + 1 < rg.hi) stage_load<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, Tk_ - n0 - kBlk, a.d);
+    if (nb + 1 < rg.hi) stage_load_at<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, Tk_ - n0 - kBlk, scol);
     frag pr[2];
     load_p_frags<T>(pr, Pm, n0, Tk_);
     Tile p, dp;

@@ -126,6 +126,8 @@ int check_problem(const Prob* pr) {
   if (pr->cols < 1 || pr->cols > pr->head_dim || pr->cols % 8 != 0)
     return fail(TTT_ERR_INVALID_ARGUMENT, "cols %lld: must be a multiple of 8 up to head_dim %lld",
                 (long long)pr->cols, (long long)pr->head_dim);
+  if (pr->cols != pr->head_dim && pr->head_dim == 128 && pr->dtype == TTT_F32)
+    return fail(TTT_ERR_UNSUPPORTED, "cols %lld of head_dim 128: 16-bit types only", (long long)pr->cols);
   if (pr->keys != pr->seqlen && (pr->causal != 0 || pr->window != 0))
     return fail(TTT_ERR_INVALID_ARGUMENT, "%lld keys for %lld queries: neither causal nor windowed",
                 (long long)pr->keys, (long long)pr->seqlen);
@@ -299,7 +301,8 @@ int64_t best_chunk(const Prob* pr, const std::vector<int64_t>& len, int kind, in
                    int64_t cfloor = 0) {
   static std::mutex mu;
   static std::map<std::tuple<int64_t, int64_t, int, int, int, int, int64_t, int64_t, int, int64_t>, int64_t> cache;
-  const auto key = std::make_tuple((int64_t)pr->seqlen, (int64_t)pr->keys, pr->causal, eff_window(pr), pr->window_kind, kind,
+  const auto key = std::make_tuple((int64_t)pr->seqlen, (int64_t)pr->keys, pr->causal, eff_window(pr),
+                                   pr->window_kind, kind,
                                    bh, slots, pr->bias.data ? 1 : 0, cfloor);
   // plain causal launches run their chunks longest first (causal_item)
   const bool longest_first = pr->causal && !has_xm(pr);
@@ -632,7 +635,8 @@ int64_t ttt_attn_workspace_size(const ttt_problem* pr, int32_t entry, int32_t wa
   return ttt_attn_workspace_size_shape(pr, nullptr, entry, want_gdout);
 }
 
-int64_t ttt_attn_workspace_size_shape(const ttt_problem* problem, const ttt_shape* shape, int32_t entry, int32_t want_gdout) {
+int64_t ttt_attn_workspace_size_shape(const ttt_problem* problem, const ttt_shape* shape, int32_t entry,
+                                      int32_t want_gdout) {
   Prob prob;
   const Prob* pr = &prob;
   if (make_prob(problem, shape, &prob) != TTT_OK) return -1;

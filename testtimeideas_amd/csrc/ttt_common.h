@@ -107,6 +107,16 @@ struct Params {
   int pairs;
 };
 
+// Columns of the rows that a kernel of type T at head dim D is given: fp32 at
+// D = 128 takes whole rows only.  Its kernels fill the 512 registers, and
+// with a run-time column count the compiler moves more of them through AGPRs
+// in the loop (b2 h4 T2048 causal saved-P grad-grad row pass 297 -> 318 us).
+template <typename T, int D>
+__device__ __forceinline__ int cols_of(const Params& a) {
+  if constexpr (sizeof(T) == 4 && D == 128) return D;
+  return a.d;
+}
+
 // Logical grid position (x, slice y) of this workgroup.  The hardware hands
 // workgroups to the 8 XCDs round-robin in linear launch order (x fastest).
 // When the slices divide evenly by 8, slice y runs on XCD y % 8, so the tiles
@@ -497,12 +507,13 @@ __device__ __forceinline__ void load_frags_row(typename Elem<T>::frag* f, const 
                                                int nrows, int ncols) {
   const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
-  for (int ks = 0; ks < D / 32; ++ks) {
-    const int col = 32 * ks + 8 * g;
-    if (row < nrows)
+  for (int ks = 0; ks < D / 32; ++ks) f[ks] = zero_frag<T>();
+  if (row < nrows) {
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) {
+      const int col = 32 * ks + 8 * g;
       f[ks] = load_frag_g<T>(base + (int64_t)row * ld + (col < ncols ? col : 0));
-    else
-      f[ks] = zero_frag<T>();
+    }
   }
   if (ncols < D) {
 #pragma unroll
@@ -832,12 +843,10 @@ __device__ __forceinline__ u32x4 load16(const void* p) {
 // (streamed index >= T) before they reach a product.  Two code paths here
 // would make the compiler wait for the previous tile's loads at their join.
 template <typename T, int NCOL>
-__device__ __forceinline__ void stage_load(Stage<T, NCOL>& st, const T* __restrict__ g, int64_t ld,
-                                           int rows_valid, int cols_valid) {
+__device__ __forceinline__ void stage_load_at(Stage<T, NCOL>& st, const T* __restrict__ g, int64_t ld,
+                                              int rows_valid, int col) {
   typedef Stage<T, NCOL> S;
   const int tid = threadIdx.x;
-  const int c0 = (tid % S::kChunksPerRow) * S::kChunk;
-  const int col = c0 < cols_valid ? c0 : 0;
   const int rmax = rows_valid - 1;
 #pragma unroll
   for (int ps = 0; ps < S::kPasses; ++ps) {
@@ -845,6 +854,22 @@ __device__ __forceinline__ void stage_load(Stage<T, NCOL>& st, const T* __restri
     st.x0[ps] = load16(g + (int64_t)min(r, rmax) * ld + col);
     st.x1[ps] = load16(g + (int64_t)min(r + 1, rmax) * ld + col);
   }
+}
+
+// This thread's first column of stage_load: its chunk's, or 0 from ncols on.
+// Operand tiles take it once per kernel (formed per tile it cost the fp32
+// D = 128 grad-grad row pass 8 %).
+template <typename T, int NCOL>
+__device__ __forceinline__ int stage_col(int ncols) {
+  typedef Stage<T, NCOL> S;
+  const int c0 = (threadIdx.x % S::kChunksPerRow) * S::kChunk;
+  return c0 < ncols ? c0 : 0;
+}
+
+template <typename T, int NCOL>
+__device__ __forceinline__ void stage_load(Stage<T, NCOL>& st, const T* __restrict__ g, int64_t ld,
+                                           int rows_valid, int cols_valid) {
+  stage_load_at<T, NCOL>(st, g, ld, rows_valid, stage_col<T, NCOL>(cols_valid));
 }
 
 // Per-lane byte offsets of stage_load's fetches for a full tile (every row
@@ -859,8 +884,7 @@ template <typename T, int NCOL>
 __device__ __forceinline__ StageOff<T, NCOL> stage_offsets(int64_t ld, int ncols) {
   typedef Stage<T, NCOL> S;
   const int tid = threadIdx.x;
-  const int c0 = (tid % S::kChunksPerRow) * S::kChunk;
-  const int col = c0 < ncols ? c0 : 0;  // as stage_load
+  const int col = stage_col<T, NCOL>(ncols);
   StageOff<T, NCOL> so;
 #pragma unroll
   for (int ps = 0; ps < S::kPasses; ++ps) {

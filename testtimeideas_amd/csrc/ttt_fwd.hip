@@ -58,7 +58,8 @@ namespace ttt {
 // entries are -inf.  brow: this row of the additive bias, or nullptr.
 template <typename T, int D, bool XM>
 __device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds* sK,
-                                           const typename Mm<T, D>::frag* qf, const Params& a, const RowMask<XM>& mk, const T* brow, int nb) {
+                                           const typename Mm<T, D>::frag* qf, const Params& a,
+                                           const RowMask<XM>& mk, const T* brow, int nb) {
   const int g = (threadIdx.x & 63) >> 4;
   s.zero();
   mm_d<Mm<T, D>>(s, sK, qf);
@@ -155,7 +156,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const T* K = at<const T>(a.k, b, h);
   const T* V = at<const T>(a.v, b, h);
   frag qr[D / 32];
-  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
+  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, cols_of<T, D>(a));
 
   f32x4 acc[D / 16];
 #pragma unroll
@@ -164,8 +165,10 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
 
   // Register stage of the next tile's K and V (loads issued one tile ahead
   // of their use).
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stK, stV;
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d), soV = stage_offsets<T, D>(a.v.st, a.d);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, cols_of<T, D>(a));
+  const StageOff<T, D> soV = stage_offsets<T, D>(a.v.st, cols_of<T, D>(a));
   auto load_kv = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
@@ -174,8 +177,8 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       stage_load_full<T, D>(stK, kp, soK);
       stage_load_full<T, D>(stV, vp, soV);
     } else {
-      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, a.d);
-      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, a.d);
+      stage_load_at<T, D>(stK, kp, a.k.st, Tk_ - n1, scol);
+      stage_load_at<T, D>(stV, vp, a.v.st, Tk_ - n1, scol);
     }
   };
   // Key tile nb from LDS tiles cK, cV.
@@ -266,7 +269,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     mm_s<M>(acc, cV, pf);
   };
   if constexpr (kDma) {
-    const TileDma<T, D> dd(a.d);
+    const TileDma<T, D> dd(cols_of<T, D>(a));
     int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
     dd.offsets(oK, a.k.st);
     dd.offsets(oV, a.v.st);
@@ -321,7 +324,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const int64_t ridx = (int64_t)bh * T_ + m;
   if (cr.nch == 1) {
     if (m < T_ && g == 0) a.lse[ridx] = (mx + __log2f(l)) * kLn2;
-    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, a.d, acc, 1.f / l);
+    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, cols_of<T, D>(a), acc, 1.f / l);
   } else {
     const int64_t part = part_index(a, bh, nblk, mb, ch);
     store_acc_partial<D>(a.ws_acc + part * kBlk * D, rl, acc);
@@ -409,8 +412,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   const T* K = at<const T>(a.k, b, h);
   const T* V = at<const T>(a.v, b, h);
   frag qf[2][KS];
-  load_frags_row<T, D>(qf[0], Q, a.q.st, m0, T_, a.d);
-  load_frags_row<T, D>(qf[1], Q, a.q.st, m1, T_, a.d);
+  load_frags_row<T, D>(qf[0], Q, a.q.st, m0, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(qf[1], Q, a.q.st, m1, T_, cols_of<T, D>(a));
   // Raw scores q.k; c = |s| log2(e) is folded into one FMA per element (q
   // negated for a negative scale).  Masks are applied after that FMA, so a
   // zero scale (c = 0) gives every visible key the same probability.
@@ -428,7 +431,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
   for (int i = 0; i < D / 16; ++i) acc0[i] = acc1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float l0 = 0.f, l1 = 0.f, sh0, sh1;
 
-  const TileDma<T, D> dd(a.d);
+  const TileDma<T, D> dd(cols_of<T, D>(a));
   int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
   dd.offsets(oK, a.k.st);
   dd.offsets(oV, a.v.st);
@@ -586,7 +589,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
     const float lt = group_sum(lv);
     if ((hi + C - 1) / C == 1) {
       if (m < T_ && g == 0) a.lse[rbase + m] = (shv + __log2f(lt)) * kLn2;
-      store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, a.d, ac, 1.f / lt);
+      store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, cols_of<T, D>(a), ac, 1.f / lt);
     } else {
       const int64_t part = part_index(a, bh, nblk, mb, ch);
       store_acc_partial<D>(a.ws_acc + part * kBlk * D, rl, ac);
@@ -647,24 +650,25 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   const T* K = at<const T>(a.k, b, h);
   typename Elem<T>::frag qr[D / 32];
   mfrag qf[D / 32];
-  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
+  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
 
   float mx = -INFINITY, l = 0.f;
   const float csl = a.scale_log2;
   const bool raw_units = csl > 0.f;  // uniform; the fused form needs a positive scale
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stK[R];
   // Tiles past the chunk load its last tile again (unconditional loads; the
   // round masks them out).
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, cols_of<T, D>(a));
   auto load_k = [&](int nb, Stage<T, D>& sk) __attribute__((always_inline)) {
     const int n1 = (nb < cr.t1 ? nb : cr.t1 - 1) * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
     if (D == 64 && n1 + kBlk <= Tk_)  // full tile: offsets computed once
       stage_load_full<T, D>(sk, kp, soK);
     else
-      stage_load<T, D>(sk, kp, a.k.st, Tk_ - n1, a.d);
+      stage_load_at<T, D>(sk, kp, a.k.st, Tk_ - n1, scol);
   };
   // One round: key tiles nb .. nb + R - 1 from the LDS tiles tile_k(i).
   auto round = [&](int nb, auto tile_k) __attribute__((always_inline)) {
@@ -741,7 +745,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       mx = mnew;
   };
   if constexpr (kDma) {
-    const TileDma<T, D> dd(a.d);
+    const TileDma<T, D> dd(cols_of<T, D>(a));
     int oK[TileDma<T, D>::kPerWave];
     dd.offsets(oK, a.k.st);
     // Tiles past the chunk load its last tile again (the round masks them).
@@ -895,7 +899,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   constexpr bool kRowPair = sizeof(T) == 2 && D == 64;
   frag qr[D / 32];
   mfrag qf[D / 32];
-  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
+  load_frags_row<T, D>(qr, Q, a.q.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) qf[ks] = M::from(qr[ks]);
 
@@ -903,8 +907,10 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
 #pragma unroll
   for (int i = 0; i < D / 16; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stK, stV;
-  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, a.d), soV = stage_offsets<T, D>(a.v.st, a.d);
+  const StageOff<T, D> soK = stage_offsets<T, D>(a.k.st, cols_of<T, D>(a));
+  const StageOff<T, D> soV = stage_offsets<T, D>(a.v.st, cols_of<T, D>(a));
   auto load_kv = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
     const T* kp = K + (int64_t)n1 * a.k.st;
@@ -913,8 +919,8 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
       stage_load_full<T, D>(stK, kp, soK);
       stage_load_full<T, D>(stV, vp, soV);
     } else {
-      stage_load<T, D>(stK, kp, a.k.st, Tk_ - n1, a.d);
-      stage_load<T, D>(stV, vp, a.v.st, Tk_ - n1, a.d);
+      stage_load_at<T, D>(stK, kp, a.k.st, Tk_ - n1, scol);
+      stage_load_at<T, D>(stV, vp, a.v.st, Tk_ - n1, scol);
     }
   };
   // With a.defer_p, the P stores of a full tile wait in registers until the
@@ -1028,7 +1034,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
       mm_s<M>(acc, cV, pf);
   };
   if constexpr (kDma) {
-    const TileDma<T, D> dd(a.d);
+    const TileDma<T, D> dd(cols_of<T, D>(a));
     int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
     dd.offsets(oK, a.k.st);
     dd.offsets(oV, a.v.st);
@@ -1080,7 +1086,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
     }
   }
   if (cr.nch == 1) {
-    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, a.d, acc, 1.f);
+    store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, cols_of<T, D>(a), acc, 1.f);
   } else {
     store_acc_partial<D>(a.ws_acc + part_index(a, bh, nblk, mb, ch) * kBlk * D, rl, acc);
   }

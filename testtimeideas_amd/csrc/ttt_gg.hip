@@ -194,9 +194,9 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   mfrag qf[D / 32], gqf[D / 32], dof[D / 32];
   {
     frag qr[D / 32], gqr[D / 32], dor[D / 32];
-    load_frags_row<T, D>(qr, Q, a.q.st, m, T_, a.d);
-    load_frags_row<T, D>(gqr, gQ, a.gq.st, m, T_, a.d);
-    load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, a.d);
+    load_frags_row<T, D>(qr, Q, a.q.st, m, T_, cols_of<T, D>(a));
+    load_frags_row<T, D>(gqr, gQ, a.gq.st, m, T_, cols_of<T, D>(a));
+    load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) {
       qf[ks] = M::from(scale_frag<T>(qr[ks], a.scale));
@@ -246,18 +246,19 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     gVn += kBlk * a.gv.st;
     if constexpr (LOADP) Pn += kBlk;
   };
+  const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> s0, s1, s2, s3;  // register staging (not kDma)
   frag pn[2];
   auto load_tile = [&](int nb) {
     const int n0 = nb * kBlk;
-    stage_load<T, D>(s0, Kn, a.k.st, Tk_ - n0, a.d);
-    stage_load<T, D>(s1, Vn, a.v.st, Tk_ - n0, a.d);
-    stage_load<T, D>(s2, gKn, a.gk.st, Tk_ - n0, a.d);
-    stage_load<T, D>(s3, gVn, a.gv.st, Tk_ - n0, a.d);
+    stage_load_at<T, D>(s0, Kn, a.k.st, Tk_ - n0, scol);
+    stage_load_at<T, D>(s1, Vn, a.v.st, Tk_ - n0, scol);
+    stage_load_at<T, D>(s2, gKn, a.gk.st, Tk_ - n0, scol);
+    stage_load_at<T, D>(s3, gVn, a.gv.st, Tk_ - n0, scol);
     if constexpr (LOADP) load_p_frags_run<T>(pn, Pn, Pm, n0, Tk_);
     advance();
   };
-  TileDma<T, D> dd(a.d);
+  TileDma<T, D> dd(cols_of<T, D>(a));
   int oK[TileDma<T, D>::kPerWave], oV[TileDma<T, D>::kPerWave];
   int ogK[TileDma<T, D>::kPerWave], ogV[TileDma<T, D>::kPerWave];
   auto dma_tile = [&](int nb, int buf) {
@@ -463,20 +464,20 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     f32x4 gq[D / 16];
     if constexpr (DQ) {
       f32x4 dq[D / 16];
-      load_acc_rows<T, D>(at<const T>(a.dq, b, h), a.dq.st, m, T_, a.d, dq);
+      load_acc_rows<T, D>(at<const T>(a.dq, b, h), a.dq.st, m, T_, cols_of<T, D>(a), dq);
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) gq[i] = (a1[i] + a2[i] - Gv * a4[i]) * s - Ev * dq[i];
-      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, a.d, gq, 1.f);
+      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, cols_of<T, D>(a), gq, 1.f);
     } else {
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) gq[i] = a1[i] + a2[i] - Ev * a3[i] - Fv * a4[i];
-      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, a.d, gq, s);
+      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, cols_of<T, D>(a), gq, s);
     }
     if constexpr (GDO) {
       f32x4 go[D / 16];
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) go[i] = b1[i] + b2[i] - Ev * b3[i];
-      store_acc_rows<T, D>(at<T>(a.gdout, b, h), a.gdout.st, m, T_, a.d, go, 1.f);
+      store_acc_rows<T, D>(at<T>(a.gdout, b, h), a.gdout.st, m, T_, cols_of<T, D>(a), go, 1.f);
     }
     if (row_ok && g == 0) {
       a.e[ridx] = Ev;
@@ -599,10 +600,10 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
   // and G - gP1 (G = F + E D), and the scores of the recomputed P as -s q.k.
   mfrag kf[D / 32], gkf[D / 32], vf[D / 32], gvf[D / 32];
   frag kr[D / 32], gkr[D / 32], vr[D / 32], gvr[D / 32];
-  load_frags_row<T, D>(kr, K, a.k.st, n, T_, a.d);
-  load_frags_row<T, D>(gkr, gK, a.gk.st, n, T_, a.d);
-  load_frags_row<T, D>(vr, V, a.v.st, n, T_, a.d);
-  load_frags_row<T, D>(gvr, gV, a.gv.st, n, T_, a.d);
+  load_frags_row<T, D>(kr, K, a.k.st, n, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(gkr, gK, a.gk.st, n, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(vr, V, a.v.st, n, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(gvr, gV, a.gv.st, n, T_, cols_of<T, D>(a));
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
     kf[ks] = M::from(scale_frag<T>(kr[ks], -a.scale));
@@ -686,7 +687,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
 
   if constexpr (kDma) {
     // Per-lane fetch offsets of an interior tile, computed once.
-    const TileDma<T, D> dd(a.d);
+    const TileDma<T, D> dd(cols_of<T, D>(a));
     const TileDma<T, kBlk> dpt(kBlk);
     int oQ[TileDma<T, D>::kPerWave], ogQ[TileDma<T, D>::kPerWave], odO[TileDma<T, D>::kPerWave];
     int oP[TileDma<T, kBlk>::kPerWave];
@@ -737,14 +738,15 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       if (mb + 1 < cr.t1) step(Parity<1>{}, mb + 1);
     }
   } else {
+    const int scol = stage_col<T, D>(cols_of<T, D>(a));
     Stage<T, D> s0, s1, s2;
     Stage<T, kBlk> sp;
     float stv;
     auto load_tile = [&](int mb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
-      stage_load<T, D>(s0, Q + (int64_t)m0 * a.q.st, a.q.st, Tq_ - m0, a.d);
-      stage_load<T, D>(s1, gQ + (int64_t)m0 * a.gq.st, a.gq.st, Tq_ - m0, a.d);
-      stage_load<T, D>(s2, dO + (int64_t)m0 * a.dout.st, a.dout.st, Tq_ - m0, a.d);
+      stage_load_at<T, D>(s0, Q + (int64_t)m0 * a.q.st, a.q.st, Tq_ - m0, scol);
+      stage_load_at<T, D>(s1, gQ + (int64_t)m0 * a.gq.st, a.gq.st, Tq_ - m0, scol);
+      stage_load_at<T, D>(s2, dO + (int64_t)m0 * a.dout.st, a.dout.st, Tq_ - m0, scol);
       if constexpr (LOADP) stage_load<T, kBlk>(sp, Pb + (int64_t)m0 * a.p.st + n0, a.p.st, Tq_ - m0, T_ - n0);
       stv = stat_load<kNS>(rs, ev, fv, lse, m0, Tq_ - m0);
     };
@@ -763,8 +765,8 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
   }
   // the accumulators hold -GK/s and -GV
   if (cr.nch == 1) {
-    store_acc_rows<T, D>(at<T>(a.gk_out, b, h), a.gk_out.st, n, T_, a.d, acc_gk, -s);
-    store_acc_rows<T, D>(at<T>(a.gv_out, b, h), a.gv_out.st, n, T_, a.d, acc_gv, -1.f);
+    store_acc_rows<T, D>(at<T>(a.gk_out, b, h), a.gk_out.st, n, T_, cols_of<T, D>(a), acc_gk, -s);
+    store_acc_rows<T, D>(at<T>(a.gv_out, b, h), a.gv_out.st, n, T_, cols_of<T, D>(a), acc_gv, -1.f);
   } else {
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) {
@@ -873,10 +875,10 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
 
   // Stationary fragments negated, as in k_gg_col.
   frag kf[D / 32], gkf[D / 32], vf[D / 32], gvf[D / 32];
-  load_frags_row<T, D>(kf, K, a.k.st, n, T_, a.d);
-  load_frags_row<T, D>(gkf, gK, a.gk.st, n, T_, a.d);
-  load_frags_row<T, D>(vf, V, a.v.st, n, T_, a.d);
-  load_frags_row<T, D>(gvf, gV, a.gv.st, n, T_, a.d);
+  load_frags_row<T, D>(kf, K, a.k.st, n, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(gkf, gK, a.gk.st, n, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(vf, V, a.v.st, n, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(gvf, gV, a.gv.st, n, T_, cols_of<T, D>(a));
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
     kf[ks] = scale_frag<T>(kf[ks], -s);
@@ -966,7 +968,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   };
 
   {
-    const TileDma<T, D, 8> dd(a.d);
+    const TileDma<T, D, 8> dd(cols_of<T, D>(a));
     const int oQ = dd.offset0(a.q.st), ogQ = dd.offset0(a.gq.st), odO = dd.offset0(a.dout.st);
     const TileDma<T, kBlk, 8> dpt(kBlk);
     const int oP = LOADP ? dpt.offset0(a.p.st) : 0;
@@ -1030,9 +1032,9 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   // acc holds -GK/s (half 0) or -GV (half 1)
   if (cr.nch == 1) {
     if (half == 0)
-      store_acc_rows<T, D>(at<T>(a.gk_out, b, h), a.gk_out.st, n, T_, a.d, acc, -s);
+      store_acc_rows<T, D>(at<T>(a.gk_out, b, h), a.gk_out.st, n, T_, cols_of<T, D>(a), acc, -s);
     else
-      store_acc_rows<T, D>(at<T>(a.gv_out, b, h), a.gv_out.st, n, T_, a.d, acc, -1.f);
+      store_acc_rows<T, D>(at<T>(a.gv_out, b, h), a.gv_out.st, n, T_, cols_of<T, D>(a), acc, -1.f);
   } else {
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) acc[i] = -acc[i];
@@ -1106,8 +1108,8 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   const T* gV = at<const T>(a.gv, b, h);
 
   frag qf[D / 32], gqf[D / 32];
-  load_frags_row<T, D>(qf, Q, a.q.st, m, T_, a.d);
-  load_frags_row<T, D>(gqf, gQ, a.gq.st, m, T_, a.d);
+  load_frags_row<T, D>(qf, Q, a.q.st, m, T_, cols_of<T, D>(a));
+  load_frags_row<T, D>(gqf, gQ, a.gq.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
   for (int ks = 0; ks < D / 32; ++ks) {
     qf[ks] = scale_frag<T>(qf[ks], a.scale);
@@ -1117,7 +1119,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   frag* const sdo = sDo + rgp * (D / 32) * 64 + lane;
   if (half == 0) {
     frag dor[D / 32];
-    load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, a.d);
+    load_frags_row<T, D>(dor, dO, a.dout.st, m, T_, cols_of<T, D>(a));
 #pragma unroll
     for (int ks = 0; ks < D / 32; ++ks) sdo[64 * ks] = dor[ks];
   }
@@ -1223,7 +1225,7 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
   const T* gKn = gK + t0r * a.gk.st;
   const T* gVn = gV + t0r * a.gv.st;
   const T* Pn = LOADP ? Pm + t0r + 32 * half + stream_index(0, g, 0) : nullptr;
-  const TileDma<T, D, 8> dd(a.d);
+  const TileDma<T, D, 8> dd(cols_of<T, D>(a));
   const int oK = dd.offset0(a.k.st), oV = dd.offset0(a.v.st), ogK = dd.offset0(a.gk.st), ogV = dd.offset0(a.gv.st);
   frag pn;
   auto dma_set = [&](int nb, T* k, T* v, T* gk, T* gv) __attribute__((always_inline)) {
@@ -1322,14 +1324,14 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
     f32x4 gq[D / 16];
     if constexpr (DQ) {
       f32x4 dq[D / 16];
-      load_acc_rows<T, D>(at<const T>(a.dq, b, h), a.dq.st, m, T_, a.d, dq);
+      load_acc_rows<T, D>(at<const T>(a.dq, b, h), a.dq.st, m, T_, cols_of<T, D>(a), dq);
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) gq[i] = (a12[i] - Gv * a4[i]) * s - Ev * dq[i];
-      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, a.d, gq, 1.f);
+      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, cols_of<T, D>(a), gq, 1.f);
     } else {
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) gq[i] = a12[i] - Ev * a3[i] - Fv * a4[i];
-      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, a.d, gq, s);
+      store_acc_rows<T, D>(at<T>(a.gq_out, b, h), a.gq_out.st, m, T_, cols_of<T, D>(a), gq, s);
     }
     if (row_ok && g == 0) {
       a.e[ridx] = Ev;

@@ -31,7 +31,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .. import _lib
-from ..ttt_kernels.triton_attention import Layout, attn_backward, attn_forward
+from ..ttt_kernels.triton_attention import Layout, attn_backward, attn_forward, plain_layout
 
 
 def _check(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
@@ -69,7 +69,7 @@ def _masked_layout(attn_mask: Optional[torch.Tensor], q: torch.Tensor, lq: int, 
     m = _kernel_bias(attn_mask, q, lq, lk)
     if lq and lk:
         bias = None if m is None else _lib.prep_bias(m, b, h, lq, q.dtype, q.device, lk)
-        return Layout(q.size(-1)), _lib.Mask(causal=False, bias=bias)
+        return plain_layout(q.size(-1), q.dtype), _lib.Mask(causal=False, bias=bias)
     if m is None and lq > lk:
         m = torch.zeros((1, 1, 1, lk), dtype=q.dtype, device=q.device)
     if m is not None:
@@ -78,7 +78,7 @@ def _masked_layout(attn_mask: Optional[torch.Tensor], q: torch.Tensor, lq: int, 
         if lq > lk:
             m = F.pad(m.expand(m.size(0), m.size(1), m.size(2), lk), (0, lq - lk), value=float("-inf"))
         m = _lib.prep_bias(m, b, h, max(lq, lk), q.dtype, q.device)
-    return Layout(q.size(-1), qpad=max(0, lk - lq), kpad=max(0, lq - lk)), _lib.Mask(causal=False, bias=m)
+    return Layout(q.size(-1), q.dtype, qpad=max(0, lk - lq), kpad=max(0, lq - lk)), _lib.Mask(causal=False, bias=m)
 
 
 class GradGradAttentionFn(torch.autograd.Function):
@@ -108,7 +108,7 @@ class _WindowAttentionFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, mask, scale, bwd_mode):
         _lib.check_inputs(q, k, v)
-        return attn_forward(ctx, q, k, v, mask, scale, bwd_mode, Layout(q.size(-1)))
+        return attn_forward(ctx, q, k, v, mask, scale, bwd_mode, plain_layout(q.size(-1), q.dtype))
 
     @staticmethod
     def backward(ctx, grad_out):

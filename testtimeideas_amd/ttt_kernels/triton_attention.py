@@ -43,8 +43,8 @@ BWD_MODES = RECOMPUTE_MODES + SAVE_P_MODES + ("custom",)
 
 class Layout:
     """How a problem's operands map onto the kernels' [B, H, T, D] operands.
-    Head dims that are multiples of 8 go as they are, others are zero-padded
-    to 64 or 128.  A problem without queries or without keys is made square:
+    Head dims that are multiples of 8 go as they are (fp32: up to 64), others
+    are zero-padded to 64 or 128.  A problem without queries or without keys is made square:
     query-side tensors (q, O, dO and their gradients) get `qpad` zero rows in
     front, key-side tensors (k, v and their gradients) `kpad` zero rows at the
     end.  Zero query
@@ -52,9 +52,9 @@ class Layout:
     padded keys are masked by the bias, so the results on the real rows are
     those of the rectangular problem."""
 
-    def __init__(self, d: int, qpad: int = 0, kpad: int = 0):
+    def __init__(self, d: int, dtype: torch.dtype, qpad: int = 0, kpad: int = 0):
         self.d = d
-        self.dpad = d if _lib.native_head_dim(d) else _lib.padded_head_dim(d)
+        self.dpad = d if _lib.native_head_dim(d, dtype) else _lib.padded_head_dim(d)
         self.qpad = qpad
         self.kpad = kpad
         # operands go to the kernels as they are (when their strides allow)
@@ -83,16 +83,16 @@ class Layout:
         return t[..., :t.size(-2) - self.kpad, :self.d]
 
 
-# Layouts without padding rows, one per head dim (immutable), and the two
+# Layouts without padding rows, one per head dim and type (immutable), and the two
 # plain causal masks: shared by every call instead of built per call.
 _PLAIN_LAYOUTS: dict = {}
 _CAUSAL_MASKS = (_lib.Mask(causal=False), _lib.Mask(causal=True))
 
 
-def plain_layout(d: int) -> Layout:
-    lay = _PLAIN_LAYOUTS.get(d)
+def plain_layout(d: int, dtype: torch.dtype) -> Layout:
+    lay = _PLAIN_LAYOUTS.get((d, dtype))
     if lay is None:
-        lay = _PLAIN_LAYOUTS[d] = Layout(d)
+        lay = _PLAIN_LAYOUTS[d, dtype] = Layout(d, dtype)
     return lay
 
 
@@ -217,7 +217,7 @@ class TritonAttentionFn(torch.autograd.Function):
         if scale is None:
             scale = 1.0 / math.sqrt(q.size(-1))
         ctx.causal = causal
-        return attn_forward(ctx, q, k, v, _CAUSAL_MASKS[bool(causal)], scale, bwd_mode, plain_layout(q.size(-1)))
+        return attn_forward(ctx, q, k, v, _CAUSAL_MASKS[bool(causal)], scale, bwd_mode, plain_layout(q.size(-1), q.dtype))
 
     @staticmethod
     def backward(ctx, grad_out: torch.Tensor):
