@@ -532,7 +532,7 @@ def _empty_like_out(x: torch.Tensor) -> torch.Tensor:
 # Tensor-level entry points (inputs already padded and validated).  `mask` is
 # a Mask, or a bool for a plain causal flag.
 # ---------------------------------------------------------------------------
-def _library_choice() -> bool:
+def library_choice() -> bool:
     """Every launch takes the library's own split: nothing forced, no tuning,
     no per-kernel timing (the entry points then call the binding directly)."""
     return not _split_chunk and not _block_rows and _timing is None and not autotune.enabled()
@@ -544,7 +544,7 @@ def fwd(q, k, v, mask, scale: float, want_p: bool):
     if q.numel() == 0:
         return _empty_like_out(q), _stats(q), alloc_p(q) if want_p else None
     m = as_mask(mask)
-    if _library_choice():
+    if library_choice():
         return tuple(ext().fwd(q, k, v, m.causal, float(scale), bool(want_p), 0, int(m.window), int(m.window_kind),
                                m.bias, 0))
     if _one_call(q, k):
@@ -581,7 +581,7 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
         return _empty_like_out(q), _empty_like_out(k), _empty_like_out(v), _stats(q)
     m = as_mask(mask)
     lp = p is not None
-    if _library_choice():
+    if library_choice():
         return tuple(ext().bwd_fused(q, k, v, o, do, lse, p, m.causal, float(scale), int(m.window),
                                      int(m.window_kind), m.bias, 0))
     if _one_call(q, k):
@@ -682,7 +682,7 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
         if dq.shape != q.shape or dq.dtype != q.dtype or dq.device != q.device:
             raise ValueError(f"dq: expected the shape, dtype and device of q {tuple(q.shape)}, got "
                              f"{tuple(dq.shape)} {dq.dtype} {dq.device}")
-    if _library_choice():
+    if library_choice():
         return tuple(ext().gg_fused(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale),
                                     bool(want_gdo), int(m.window), int(m.window_kind), m.bias, 0))
     if _one_call(q, k):

@@ -370,7 +370,7 @@ Split choose_split_pairs(const Prob* pr) {
   return s;
 }
 
-Split choose_split(const Prob* pr, int fam, bool load_p) {
+Split compute_split(const Prob* pr, int fam, bool load_p) {
   if (pair_family(fam)) return choose_split_pairs(pr);
   Split s;
   const bool col = column_family(fam);
@@ -396,6 +396,35 @@ Split choose_split(const Prob* pr, int fam, bool load_p) {
   s.chunk = (int)std::min<int64_t>(c, lmax);
   s.nchunk_max = (int)((lmax + s.chunk - 1) / s.chunk);
   return s;
+}
+
+// compute_split of everything that it depends on, kept per thread for the last
+// problems (an entry call and its workspace query ask for each family's split
+// several times: with the tile counts of every block and the simulation's
+// cache looked up each time, a third of a small call's host time).
+Split choose_split(const Prob* pr, int fam, bool load_p) {
+  struct Entry {
+    int64_t key[11];
+    Split s;
+    bool used;
+  };
+  constexpr int kEntries = 64;
+  static thread_local Entry cache[kEntries] = {};
+  int dev = 0;
+  const int cus = device_cus(&dev);
+  const int64_t key[11] = {pr->dtype | pr->causal << 4 | pr->window_kind << 8 | (pr->bias.data ? 1 : 0) << 12 |
+                               (load_p ? 1 : 0) << 13 | fam << 16,
+                           dev, cus, pr->batch, pr->heads, pr->seqlen, pr->keys, pr->head_dim, pr->split_chunk,
+                           pr->window, pr->block_rows};
+  uint64_t h = 0;
+  for (const int64_t k : key) h = (h ^ (uint64_t)k) * 0x9E3779B97F4A7C15ull;
+  Entry& e = cache[h >> 58];
+  if (!e.used || std::memcmp(e.key, key, sizeof(key)) != 0) {
+    e.s = compute_split(pr, fam, load_p);
+    std::memcpy(e.key, key, sizeof(key));
+    e.used = true;
+  }
+  return e.s;
 }
 
 int family_of(const Prob* pr, int entry, bool gdo) {

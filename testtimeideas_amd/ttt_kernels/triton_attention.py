@@ -108,7 +108,9 @@ def mode_kind(bwd_mode: str) -> str:
 
 class _AttnBwdFn(torch.autograd.Function):
     """First backward as a function of (q, k, v, dO); its backward is the
-    double backward.  The kernel-layout dQ is kept for it: the row pass of the
+    double backward.  For padded operands, and while a split is forced or
+    kernels are timed or tuned; other calls take the same Function in C++
+    (``bwd_graph`` of the binding).  The kernel-layout dQ is kept for it: the row pass of the
     double backward reads dQ = s*(dS*K) instead of forming that product.
 
     `fwd` = (qp, kp, vp, op, lse, p, mask, scale, lay), the saved forward in
@@ -188,7 +190,10 @@ def attn_forward(ctx, q, k, v, mask: "_lib.Mask", scale: float, bwd_mode: str, l
     qp = lay.q(q)
     kp, vp = lay.k(k), lay.k(v)
     op, lse, p = _lib.fwd(qp, kp, vp, mask, scale, want_p=(kind == "save_p"))
-    ctx.save_for_backward(q, k, v, qp, kp, vp, op, lse, p)
+    if lay.plain:
+        ctx.save_for_backward(q, k, v, op, lse, p)
+    else:
+        ctx.save_for_backward(q, k, v, op, lse, p, qp, kp, vp)
     ctx.saved_probs = () if p is None else SavedProbs(p, mask)
     return lay.uq(op)
 
@@ -197,9 +202,16 @@ def attn_backward(ctx, grad_out: torch.Tensor):
     """(dq, dk, dv) of an attention Function.  Under create_graph=True
     (grad mode on in the backward) they come from _AttnBwdFn, whose backward
     is the exact double backward; otherwise straight from the kernels."""
-    q, k, v, qp, kp, vp, op, lse, p = ctx.saved_tensors
     mask, scale, lay = ctx.mask, ctx.scale, ctx.lay
+    if lay.plain:
+        q, k, v, op, lse, p = ctx.saved_tensors
+        qp, kp, vp = q, k, v
+    else:
+        q, k, v, op, lse, p, qp, kp, vp = ctx.saved_tensors
     if torch.is_grad_enabled():
+        if lay.plain and q.is_cuda and q.numel() != 0 and _lib.library_choice():
+            return _lib.ext().bwd_graph(q, k, v, grad_out, op, lse, p, mask.causal, float(scale), int(mask.window),
+                                        int(mask.window_kind), mask.bias)
         # O detached: the saved node holds no edge into the forward's graph
         return _AttnBwdFn.apply(q, k, v, grad_out, (qp, kp, vp, op.detach(), lse, p, mask, scale, lay))
     dq, dk, dv, _ = _lib.bwd(qp, kp, vp, op, lay.q(grad_out), lse, p, mask, scale)
