@@ -15,8 +15,8 @@
 // LOADP = false recomputes P = exp2(s*log2e*QK^T - lse*log2e) per tile.
 // Causal: fully masked tiles are skipped, diagonal tiles masked per element;
 // a key window likewise (RowMask / ColMask).  Recomputed P adds the additive
-// bias when there is one (saved P already holds it).  XM instantiates the
-// window/bias code.
+// bias when there is one (saved P already holds it).  XM is the mask form
+// (kMask*).
 // The next tile's loads are issued before the current tile's math.
 // dP - D comes out of the MFMAs: in k_bwd_dq they start from -D (the
 // stationary row's), in k_bwd_dkdv from the streamed rows' D with the
@@ -87,7 +87,7 @@ struct DqWaves {
 };
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool LOADP, bool XM>
+template <typename T, int D, bool LOADP, int XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(Params a) {
   typedef Elem<T> E;
@@ -137,9 +137,11 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
   const bool row_ok = m < T_;
-  const RowMask<XM> mk(a, mb, m);
-  const T* brow =
-      (XM && !LOADP && a.bias.p) ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
+  const RowMask<XM != kMaskNone> mk(a, mb, m);
+  constexpr bool kBias = XM == kMaskBias;
+  static_assert(!(LOADP && kBias), "a saved P holds the bias");
+  const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
+  frag bn[2], bc[2];  // bias of the next tile and of this one
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -185,6 +187,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   const T* Pn = LOADP ? Pm + cr.t0 * kBlk + stream_index(0, g, 0) : nullptr;
   auto fetch = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
+    if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
     if constexpr (!LOADP) {
       // Recompute: tile-indexed clamped loads, measured faster for this
       // variant than the running-pointer form below.
@@ -217,6 +220,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   }
   auto fetch_dma = [&](int nb, auto par) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
+    if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
     if (n1 + kBlk <= Tk_) {
       dd.load_full(set_k(par), Kn, oK);
       dd.load_full(set_v(par), Vn, oV);
@@ -257,6 +261,10 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     const lds* cV = set_v(par);
     Tile p;
     if constexpr (LOADP) frags_to_tile<T>(p, pn);
+    if constexpr (kBias) {
+      bc[0] = bn[0];
+      bc[1] = bn[1];
+    }
     if constexpr (kDma) {
       if constexpr (decltype(prefetch)::value == 1) fetch_dma(nb + 1, other_buf(par));
       if constexpr (decltype(prefetch)::value == 2)
@@ -269,7 +277,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (!LOADP) {
       p.zero();
       mm_d<M>(p, cK, qf);
-      recompute_p_row<T, XM>(p, a, brow, n0, lse2, a.scale_log2);
+      recompute_p_row<T, kBias>(p, bc, lse2, a.scale_log2);
     }
     if (mk.tile(nb)) {
 #pragma unroll
@@ -338,7 +346,7 @@ struct DkdvWaves {
   static constexpr int value = kDma ? (D == 64 ? 3 : 2) : AccWaves<!LOADP && D == 64>::value;
 };
 
-template <typename T, int D, bool LOADP, bool DV_ONLY, bool XM>
+template <typename T, int D, bool LOADP, bool DV_ONLY, int XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) void k_bwd_dkdv(Params a, Params dqc,
                                                                                               int nx) {
@@ -409,8 +417,11 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int cl = 16 * w + c;
   const int n = n0 + cl;
-  const ColMask<XM> mk(a, nb, n);
-  const T* bcol = (XM && !LOADP && a.bias.p) ? at<const T>(a.bias, b, h) + (n < T_ ? n : 0) : nullptr;
+  const ColMask<XM != kMaskNone> mk(a, nb, n);
+  constexpr bool kBias = XM == kMaskBias;
+  static_assert(!(LOADP && kBias), "a saved P holds the bias");
+  const T* bcol = kBias ? at<const T>(a.bias, b, h) + (n < T_ ? n : 0) : nullptr;
+  BiasCol<T> bn, bc;  // bias of the next tile and of this one
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -456,6 +467,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const bool cols_full = n0 + kBlk <= T_;
   auto load_tile = [&](int mb) __attribute__((always_inline)) {
     const int m0 = mb * kBlk;
+    if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
     stage_load_at<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, scol);
     if constexpr (kNeedQ) stage_load_at<T, D>(stQ, Qn, a.q.st, Tq_ - m0, scol);
     if constexpr (LOADP) stage_load<T, kBlk>(stP, Pn, a.p.st, Tq_ - m0, T_ - n0);
@@ -479,6 +491,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     if constexpr (kDma) {
       const int m0 = mb * kBlk;
       const Bufs bf = bufs(par);
+      if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
       if (m0 + kBlk <= Tq_ && cols_full) {
         dd.load_full(bf.dout, dOn, odO);
         dd.load_full(bf.q, Qn, oQ);
@@ -512,6 +525,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
         stage_store_rows<T, kBlk>(stP, sP0);
         __syncthreads();
       }
+      if constexpr (kBias) bc = bn;
       if constexpr (!kLateFetch) {
         if constexpr (decltype(prefetch)::value == 1) dma_tile(mb + 1, Parity<1 - P>{});
         if constexpr (decltype(prefetch)::value == 2)
@@ -524,6 +538,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       if constexpr (LOADP) stage_store_rows<T, kBlk>(stP, sP0);
       if constexpr (kNS > 0) stat_store<kNS>(stv, sS0);
       __syncthreads();
+      if constexpr (kBias) bc = bn;
       if constexpr (decltype(prefetch)::value == 1) load_tile(mb + 1);
       if constexpr (decltype(prefetch)::value == 2)
         if (mb + 1 < cr.t1) load_tile(mb + 1);
@@ -551,7 +566,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     } else {
       p.zero();
       mm_d<M>(p, cQ, kf);
-      recompute_p_col<T, XM>(p, a, bcol, m0, cS, kSL, a.scale_log2);
+      recompute_p_col<T, kBias>(p, bc, cS, kSL, a.scale_log2);
     }
     if (mk.tile(mb)) {
 #pragma unroll
@@ -610,7 +625,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
 // ---------------------------------------------------------------------------
 // rowsum[m] = sum_n P[m,n] * (dO*V^T)[m,n]; causal skips tiles past the
 // diagonal (they hold zeros in the math path).
-template <typename T, int D, bool XM>
+template <typename T, int D, int XM>
 __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
   typedef Elem<T> E;
   typedef typename E::frag frag;
@@ -640,7 +655,7 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
 
   float sum = 0.f;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
-  const RowMask<XM> mk(a, mb, m);
+  const RowMask<XM != kMaskNone> mk(a, mb, m);
   const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stV;
   stage_load_at<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, scol);
@@ -673,42 +688,43 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool XM>
+template <typename T, int D>
 static void launch_dq_x(const Params& a, bool load_p, dim3 grid, hipStream_t st) {
   const TimedLaunch tl(st, kTagDq);
   if (load_p)
-    hipLaunchKernelGGL((k_bwd_dq<T, D, true, XM>), grid, dim3(kThreads), 0, st, a);
+    DISPATCH_MASK(mask_kind(a, true), false,
+                  hipLaunchKernelGGL((k_bwd_dq<T, D, true, kXM>), grid, dim3(kThreads), 0, st, a));
   else
-    hipLaunchKernelGGL((k_bwd_dq<T, D, false, XM>), grid, dim3(kThreads), 0, st, a);
+    DISPATCH_MASK(mask_kind(a, false), true,
+                  hipLaunchKernelGGL((k_bwd_dq<T, D, false, kXM>), grid, dim3(kThreads), 0, st, a));
 }
 
 template <typename T, int D>
 static hipError_t launch_dq_t(int dtype, const Params& a, bool load_p, hipStream_t st, bool combine) {
   const int nblk = (a.T + kBlk - 1) / kBlk;
   dim3 grid(nblk * a.nchunk_max, a.B * a.H);
-  if (extended_mask(a))
-    launch_dq_x<T, D, true>(a, load_p, grid, st);
-  else
-    launch_dq_x<T, D, false>(a, load_p, grid, st);
+  launch_dq_x<T, D>(a, load_p, grid, st);
   if (combine && a.nchunk_max > 1) return launch_combine_sum(dtype, D, a, kOutDQ, st);
   return hipGetLastError();
 }
 
-template <typename T, int D, bool XM>
+template <typename T, int D>
 static void launch_dkdv_x(const Params& a, bool load_p, bool dv_only, dim3 grid, hipStream_t st, const Params& c,
                           int nx) {
   const TimedLaunch tl(st, kTagDkdv);
-  if (load_p) {
-    if (dv_only)
-      hipLaunchKernelGGL((k_bwd_dkdv<T, D, true, true, XM>), grid, dim3(kThreads), 0, st, a, c, nx);
-    else
-      hipLaunchKernelGGL((k_bwd_dkdv<T, D, true, false, XM>), grid, dim3(kThreads), 0, st, a, c, nx);
-  } else {
-    if (dv_only)
-      hipLaunchKernelGGL((k_bwd_dkdv<T, D, false, true, XM>), grid, dim3(kThreads), 0, st, a, c, nx);
-    else
-      hipLaunchKernelGGL((k_bwd_dkdv<T, D, false, false, XM>), grid, dim3(kThreads), 0, st, a, c, nx);
-  }
+  const int xm = mask_kind(a, load_p);
+  if (load_p && dv_only)
+    DISPATCH_MASK(xm, false,
+                  hipLaunchKernelGGL((k_bwd_dkdv<T, D, true, true, kXM>), grid, dim3(kThreads), 0, st, a, c, nx));
+  else if (load_p)
+    DISPATCH_MASK(xm, false,
+                  hipLaunchKernelGGL((k_bwd_dkdv<T, D, true, false, kXM>), grid, dim3(kThreads), 0, st, a, c, nx));
+  else if (dv_only)
+    DISPATCH_MASK(xm, true,
+                  hipLaunchKernelGGL((k_bwd_dkdv<T, D, false, true, kXM>), grid, dim3(kThreads), 0, st, a, c, nx));
+  else
+    DISPATCH_MASK(xm, true,
+                  hipLaunchKernelGGL((k_bwd_dkdv<T, D, false, false, kXM>), grid, dim3(kThreads), 0, st, a, c, nx));
 }
 
 template <typename T, int D>
@@ -718,10 +734,7 @@ static hipError_t launch_dkdv_t(int dtype, const Params& a, bool load_p, bool dv
   const bool fold = dqc && dqc->nchunk_max > 1;
   dim3 grid(nx + (fold ? (a.T + kBlk - 1) / kBlk * CombineSlot<D>::kSub : 0), a.B * a.H);
   const Params& c = fold ? *dqc : a;
-  if (extended_mask(a))
-    launch_dkdv_x<T, D, true>(a, load_p, dv_only, grid, st, c, nx);
-  else
-    launch_dkdv_x<T, D, false>(a, load_p, dv_only, grid, st, c, nx);
+  launch_dkdv_x<T, D>(a, load_p, dv_only, grid, st, c, nx);
   if (a.nchunk_max > 1) return launch_combine_sum(dtype, D, a, dv_only ? kOutDV : kOutDKDV, st);
   return hipGetLastError();
 }
@@ -729,33 +742,32 @@ static hipError_t launch_dkdv_t(int dtype, const Params& a, bool load_p, bool dv
 template <typename T, int D>
 static hipError_t launch_rowsum_t(const Params& a, hipStream_t st) {
   dim3 grid((a.T + kBlk - 1) / kBlk, a.B * a.H);
-  if (extended_mask(a))
-    hipLaunchKernelGGL((k_bwd_rowsum<T, D, true>), grid, dim3(kThreads), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_bwd_rowsum<T, D, false>), grid, dim3(kThreads), 0, st, a);
+  DISPATCH_MASK(mask_kind(a, true), false,
+                hipLaunchKernelGGL((k_bwd_rowsum<T, D, kXM>), grid, dim3(kThreads), 0, st, a));
   return hipGetLastError();
 }
 
-template <typename T, int D, bool XM>
-static int occupancy_dq_t(bool load_p) {
-  return load_p ? occupancy_of(k_bwd_dq<T, D, true, XM>) : occupancy_of(k_bwd_dq<T, D, false, XM>);
-}
-
-template <typename T, int D, bool XM>
-static int occupancy_dkdv_t(bool load_p) {
-  return load_p ? occupancy_of(k_bwd_dkdv<T, D, true, false, XM>)
-                : occupancy_of(k_bwd_dkdv<T, D, false, false, XM>);
-}
-
-int occupancy_dq(int dtype, int D, bool load_p, bool xm) {
-  if (xm) DISPATCH_DTYPE_D(dtype, D, return occupancy_dq_t<ElemT, kD, true>(load_p));
-  else DISPATCH_DTYPE_D(dtype, D, return occupancy_dq_t<ElemT, kD, false>(load_p));
+template <typename T, int D>
+static int occupancy_dq_t(bool load_p, int xm) {
+  if (load_p) DISPATCH_MASK(xm, false, return occupancy_of(k_bwd_dq<T, D, true, kXM>));
+  else DISPATCH_MASK(xm, true, return occupancy_of(k_bwd_dq<T, D, false, kXM>));
   return 0;
 }
 
-int occupancy_dkdv(int dtype, int D, bool load_p, bool xm) {
-  if (xm) DISPATCH_DTYPE_D(dtype, D, return occupancy_dkdv_t<ElemT, kD, true>(load_p));
-  else DISPATCH_DTYPE_D(dtype, D, return occupancy_dkdv_t<ElemT, kD, false>(load_p));
+template <typename T, int D>
+static int occupancy_dkdv_t(bool load_p, int xm) {
+  if (load_p) DISPATCH_MASK(xm, false, return occupancy_of(k_bwd_dkdv<T, D, true, false, kXM>));
+  else DISPATCH_MASK(xm, true, return occupancy_of(k_bwd_dkdv<T, D, false, false, kXM>));
+  return 0;
+}
+
+int occupancy_dq(int dtype, int D, bool load_p, int xm) {
+  DISPATCH_DTYPE_D(dtype, D, return occupancy_dq_t<ElemT, kD>(load_p, xm));
+  return 0;
+}
+
+int occupancy_dkdv(int dtype, int D, bool load_p, int xm) {
+  DISPATCH_DTYPE_D(dtype, D, return occupancy_dkdv_t<ElemT, kD>(load_p, xm));
   return 0;
 }
 

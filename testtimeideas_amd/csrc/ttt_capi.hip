@@ -194,12 +194,15 @@ int device_cus(int* dev_out) {
 // Workgroup slots of family `fam`'s kernel (variant load_p) on the current
 // device; cached per (device, family, dtype, head dim, variant).
 int64_t family_slots(const Prob* pr, int fam, bool load_p) {
-  static std::atomic<int> per_cu[16][ttt::kNumFams][3][2][2][2];
+  static std::atomic<int> per_cu[16][ttt::kNumFams][3][2][2][3];
   int dev = 0;
   const int cus = device_cus(&dev);
   if (cus == 0) return (int64_t)kFallbackCus * kFallbackPerCu * kSlotFill / 100;
   const int dt = pr->dtype, ds = pr->head_dim == 128 ? 1 : 0, lp = load_p ? 1 : 0;
-  const bool xm = has_xm(pr);
+  // the mask form of the kernel that would run (mask_kind)
+  const bool saved = load_p && fam != ttt::kFamFwdP;
+  const int xm = pr->bias.data ? (saved ? ttt::kMaskWindow : ttt::kMaskBias)
+                 : eff_window(pr) > 0 ? ttt::kMaskWindow : ttt::kMaskNone;
   int n = per_cu[dev][fam][dt][ds][lp][xm].load(std::memory_order_relaxed);
   if (n == 0) {
     const int D = (int)pr->head_dim;

@@ -246,10 +246,19 @@ __host__ __device__ inline Item causal_item(int x, int n, int c) {
   return it;
 }
 
-// The column's chunk: causal_item for plain causal split slices (XM false),
+// Mask code of a kernel instantiation (template parameter XM): none, a key
+// window, or an additive bias (with a window or without).  Kernels that read a
+// saved P, which holds the bias already, have no third form.  Separate, the
+// window kernels carry no bias code, and the bias kernels have registers to
+// load a tile's bias with the tile before: added when it was needed, it cost
+// a memory round trip in every tile (b2 h6 d64 fp32, 512 queries of 2048 keys,
+// grad-grad column pass 177 -> 166 us, dK/dV 83 -> 80).
+enum : int { kMaskNone = 0, kMaskWindow = 1, kMaskBias = 2 };
+
+// The column's chunk: causal_item for plain causal split slices (XM = kMaskNone),
 // else x % nblk, x / nblk (chunk index by chunk index, blocks in launch
 // order; columns past a block's chunks exit on their chunk test).
-template <bool XM>
+template <int XM>
 __device__ __forceinline__ Item launch_item(const Params& a, int x, int nblk) {
   if (!XM && a.causal && a.nchunk_max > 1) return causal_item(x, nblk, a.chunk);
   return Item{x % nblk, x / nblk};
@@ -310,7 +319,7 @@ __host__ __device__ __forceinline__ Range col_block_range(int nb, int nblk, int 
 }
 
 // Per-lane mask of a row-block kernel (stationary query row m).  XM: the
-// problem has a window or a bias (other kernels compile W = 0 in).
+// kernel has a mask form (others compile W = 0 in).
 template <bool XM>
 struct RowMask {
   int m, mb, T, causal, lo, lo_last;
@@ -941,36 +950,40 @@ __device__ __forceinline__ void load_p_frags_run(typename Elem<T>::frag* f, cons
 }
 
 // Additive bias, in base-2 units, onto a streamed tile of a row-block kernel:
-// row pointer brow (this lane's stationary row), columns as load_p_frags
-// (same row-storage contract as P).
+// f, the fragments load_p_frags read of this lane's row of the bias (the same
+// row-storage contract as P's).
 template <typename T>
-__device__ __forceinline__ void add_bias_row(Tile& s, const T* brow, int n0, int T_) {
-  typename Elem<T>::frag f[2];
-  load_p_frags<T>(f, brow, n0, T_);
+__device__ __forceinline__ void add_bias_row(Tile& s, const typename Elem<T>::frag* f) {
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int j = 0; j < 8; ++j) s.set(kb, j, s.at(kb, j) + Elem<T>::f32(f[kb][j]) * kLog2e);
 }
 
-// The same for a column-block kernel: bcol points at this lane's key column
-// of row 0; streamed rows m0 + stream_index(kb, g, j) (rows >= T read row 0).
+// A column-block kernel's bias values of one tile: bcol points at this lane's
+// key column of row 0; streamed rows m0 + stream_index(kb, g, j) (rows >= T
+// read row 0).
 template <typename T>
-__device__ __forceinline__ void add_bias_col(Tile& s, const T* bcol, int64_t st, int m0, int T_) {
-  const int g = (threadIdx.x & 63) >> 4;
-  float v[2][8];
+struct BiasCol {
+  T v[2][8];
+  __device__ __forceinline__ void load(const T* bcol, int64_t st, int m0, int T_) {
+    typedef __attribute__((address_space(1))) const T gT;
+    const int g = (threadIdx.x & 63) >> 4;
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int mm = m0 + stream_index(kb, g, j);
-      v[kb][j] = Elem<T>::f32(bcol[(int64_t)(mm < T_ ? mm : 0) * st]);
-    }
+      for (int j = 0; j < 8; ++j) {
+        const int mm = m0 + stream_index(kb, g, j);
+        v[kb][j] = *(gT*)(bcol + (int64_t)(mm < T_ ? mm : 0) * st);
+      }
+  }
+  __device__ __forceinline__ void add(Tile& s) const {
 #pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) s.set(kb, j, s.at(kb, j) + v[kb][j] * kLog2e);
-}
+      for (int j = 0; j < 8; ++j) s.set(kb, j, s.at(kb, j) + Elem<T>::f32(v[kb][j]) * kLog2e);
+  }
+};
 
 // Write staged registers to an LDS tile (layout of Lds<T, NCOL>).
 template <typename T, int NCOL>
@@ -1626,25 +1639,22 @@ __device__ __forceinline__ RtBuf other_buf(RtBuf b) { return RtBuf{b.cur ^ 1}; }
 
 // ---------------------------------------------------------------------------
 // P = exp2(s*log2e*x [+ bias*log2e] - lse2) from raw scores x of a row-block
-// tile (brow: this lane's bias row, or nullptr).
+// tile (BIAS: bf, the tile's bias fragments).
 // sl2 converts raw scores to base-2 units: s*log2(e), or log2(e) when the
 // stationary fragments were scaled by s beforehand.
-template <typename T, bool XM>
-__device__ __forceinline__ void recompute_p_row(Tile& p, const Params& a, const T* brow, int n0, float lse2,
-                                                float sl2) {
-  if constexpr (XM) {
-    if (brow) {
+template <typename T, bool BIAS>
+__device__ __forceinline__ void recompute_p_row(Tile& p, const typename Elem<T>::frag* bf, float lse2, float sl2) {
+  if constexpr (BIAS) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
-      add_bias_row<T>(p, brow, n0, a.Tk);
+      for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
+    add_bias_row<T>(p, bf);
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) - lse2));
-      return;
-    }
+      for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) - lse2));
+    return;
   }
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
@@ -1652,34 +1662,24 @@ __device__ __forceinline__ void recompute_p_row(Tile& p, const Params& a, const 
     for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) * sl2 - lse2));
 }
 
-// The same for a column-block tile: l2 holds lse2 of the streamed rows of
-// k-block kb; bcol is this lane's bias column (or nullptr).
-template <typename T, bool XM>
-__device__ __forceinline__ void recompute_p_col(Tile& p, const Params& a, const T* bcol, int m0, const float* sS,
-                                                int slot, float sl2) {
-  if constexpr (XM) {
-    if (bcol) {
+// The same for a column-block tile: statistic `slot` of sS holds the streamed
+// rows' lse; bv is the tile's bias.
+template <typename T, bool BIAS>
+__device__ __forceinline__ void recompute_p_col(Tile& p, const BiasCol<T>& bv, const float* sS, int slot, float sl2) {
+  if constexpr (BIAS) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
-      add_bias_col<T>(p, bcol, a.bias.st, m0, a.T);
-#pragma unroll
-      for (int kb = 0; kb < 2; ++kb) {
-        float l2[8];
-        stat_read8(l2, sS, slot, kb);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) - l2[j] * kLog2e));
-      }
-      return;
-    }
+      for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
+    bv.add(p);
   }
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb) {
     float l2[8];
     stat_read8(l2, sS, slot, kb);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) * sl2 - l2[j] * kLog2e));
+    for (int j = 0; j < 8; ++j)
+      p.set(kb, j, fast_exp2(BIAS ? p.at(kb, j) - l2[j] * kLog2e : p.at(kb, j) * sl2 - l2[j] * kLog2e));
   }
 }
 

@@ -18,7 +18,8 @@
 // per element (key > query).  A key window also skips the tiles before the
 // block's first visible key and masks the tiles it cuts.  An additive bias is
 // added to the base-2 scores of every tile.  The window and bias code is a
-// separate instantiation (XM), so plain problems run the kernels without it.
+// separate instantiations (XM, the mask form), so plain problems run the
+// kernels without it.
 // Row blocks are issued heaviest first, and the chunks of a split plain causal
 // launch longest first (launch_item).  Blocks split into several chunks are
 // finished by the combine kernels of ttt_combine.hip.
@@ -55,11 +56,12 @@
 namespace ttt {
 
 // Scores of key tile nb (rows sK) for query row m, in base-2 units; masked
-// entries are -inf.  brow: this row of the additive bias, or nullptr.
-template <typename T, int D, bool XM>
+// entries are -inf.  bf: the tile's bias fragments (kMaskBias).
+template <typename T, int D, int XM>
 __device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds* sK,
                                            const typename Mm<T, D>::frag* qf, const Params& a,
-                                           const RowMask<XM>& mk, const T* brow, int nb) {
+                                           const RowMask<XM != kMaskNone>& mk, const typename Elem<T>::frag* bf,
+                                           int nb) {
   const int g = (threadIdx.x & 63) >> 4;
   s.zero();
   mm_d<Mm<T, D>>(s, sK, qf);
@@ -69,8 +71,7 @@ __device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
     for (int j = 0; j < 8; ++j) s.set(kb, j, s.at(kb, j) * a.scale_log2);
-  if constexpr (XM)
-    if (brow) add_bias_row<T>(s, brow, n0, a.Tk);
+  if constexpr (XM == kMaskBias) add_bias_row<T>(s, bf);
   if (need_mask) {
 #pragma unroll
     for (int kb = 0; kb < 2; ++kb)
@@ -114,7 +115,7 @@ __device__ __forceinline__ float tile_max(const Tile& s) {
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool XM>
+template <typename T, int D, int XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Params a) {
   typedef Elem<T> E;
@@ -149,8 +150,10 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;  // row within the block
   const int m = mb * kBlk + rl;
-  const RowMask<XM> mk(a, mb, m);
-  const T* brow = (XM && a.bias.p) ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
+  const RowMask<XM != kMaskNone> mk(a, mb, m);
+  constexpr bool kBias = XM == kMaskBias;
+  const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
+  frag bn[2], bc[2];  // bias of the next tile and of this one
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -171,6 +174,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const StageOff<T, D> soV = stage_offsets<T, D>(a.v.st, cols_of<T, D>(a));
   auto load_kv = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
+    if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
     const T* kp = K + (int64_t)n1 * a.k.st;
     const T* vp = V + (int64_t)n1 * a.v.st;
     if (D == 64 && n1 + kBlk <= Tk_) {  // full tile: offsets computed once
@@ -182,14 +186,14 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     }
   };
   // Key tile nb from LDS tiles cK, cV.
-  // Without a window or bias the scores stay raw (q.k): c = |s|*log2(e) is
+  // Without a bias the scores stay raw (q.k): c = |s|*log2(e) is
   // folded into one FMA per element (q negated for a negative scale), and the
   // running shift sh (base 2) moves only when a row's max exceeds it by more
   // than kSlack, so most tiles skip rescaling O and l (then P <= 2^kSlack,
   // well inside T's range).  Other problems take the scaled form below.
   constexpr float kSlack = 8.f;
   float csl = a.scale_log2;
-  if constexpr (!XM) {
+  if constexpr (!kBias) {
     if (csl < 0.f) {
       csl = -csl;
 #pragma unroll
@@ -213,11 +217,12 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
         for (int j = 0; j < 8; ++j)
           s.set(kb, j, mk.masked(n0 + stream_index(kb, g, j)) ? -INFINITY : s.at(kb, j));
     }
-    // Every row sees a key of every tile of its walk here, so tm is finite.
+    // Without a window every row sees a key of every tile of its walk, so tm is
+    // finite; with one it is -inf where a row has seen no key yet.
     const float tm = tile_max(s) * csl;
     if (__builtin_amdgcn_ballot_w64(tm > sh + kSlack) != 0) {  // uniform
       const float sn = fmaxf(sh, tm);
-      const float alpha = fast_exp2(sh - sn);
+      const float alpha = XM == kMaskWindow && sn == -INFINITY ? 1.f : fast_exp2(sh - sn);
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) acc[i] *= alpha;
@@ -240,15 +245,15 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     mm_s<M>(acc, cV, pf);
   };
   auto body = [&](int nb, const lds* cK, const lds* cV) __attribute__((always_inline)) {
-    if constexpr (!XM) {
+    if constexpr (!kBias) {
       body_raw(nb, cK, cV);
       return;
     }
     Tile s;
-    fwd_scores<T, D, XM>(s, cK, qf, a, mk, brow, nb);
+    fwd_scores<T, D, XM>(s, cK, qf, a, mk, bc, nb);
     const float mnew = fmaxf(mx, tile_max(s));
     // A window can mask a row's every key of a tile so far: shift by 0 then.
-    const float msh = (XM && mnew == -INFINITY) ? 0.f : mnew;
+    const float msh = (mnew == -INFINITY) ? 0.f : mnew;
     const float alpha = fast_exp2(mx - msh);
     float ts = 0.f;
     mfrag pf[2];
@@ -275,6 +280,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     dd.offsets(oV, a.v.st);
     auto fetch = [&](int nt, T* k, T* v) __attribute__((always_inline)) {
       const int n1 = nt * kBlk;
+      if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
       const T* kp = K + (int64_t)n1 * a.k.st;
       const T* vp = V + (int64_t)n1 * a.v.st;
       if (n1 + kBlk <= Tk_) {
@@ -291,6 +297,10 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       constexpr int P = decltype(par)::value;
       dma_wait();       // this wave's loads of tile nt
       __syncthreads();  // everyone's, and everyone is done with the other set
+      if constexpr (kBias) {
+        bc[0] = bn[0];
+        bc[1] = bn[1];
+      }
       if (nt + 1 < cr.t1) {
         if constexpr (P == 0)
           fetch(nt + 1, sK1, sV1);
@@ -314,13 +324,17 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       stage_store_tile<M>(stK, sK);
       stage_store_tile<M>(stV, sV);
       __syncthreads();
+      if constexpr (kBias) {
+        bc[0] = bn[0];
+        bc[1] = bn[1];
+      }
       if (nb + 1 < cr.t1) load_kv(nb + 1);
       body(nb, sK, sV);
     }
   }
 
   l = group_sum(l);
-  if constexpr (!XM) mx = sh;
+  if constexpr (!kBias) mx = sh;
   const int64_t ridx = (int64_t)bh * T_ + m;
   if (cr.nch == 1) {
     if (m < T_ && g == 0) a.lse[ridx] = (mx + __log2f(l)) * kLn2;
@@ -612,7 +626,7 @@ struct FwdPWaves {
   static constexpr int value = sizeof(T) == 2 ? (D == 64 ? 3 : 2) : AccWaves<false>::value;
 };
 
-template <typename T, int D, bool XM>
+template <typename T, int D, int XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Params a) {
   typedef Lds<T, D> L;
@@ -643,8 +657,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
-  const RowMask<XM> mk(a, mb, m);
-  const T* brow = (XM && a.bias.p) ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
+  const RowMask<XM != kMaskNone> mk(a, mb, m);
+  constexpr bool kBias = XM == kMaskBias;
+  const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -673,7 +688,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   // One round: key tiles nb .. nb + R - 1 from the LDS tiles tile_k(i).
   auto round = [&](int nb, auto tile_k) __attribute__((always_inline)) {
       Tile s[R];
-      if constexpr (!XM) {
+      if constexpr (!kBias) {
         if (raw_units) {
           // Max and sum in raw-score units: exp2(raw * csl - max * csl) with the
           // scale csl = scale*log2e > 0 folded into one FMA per element.
@@ -714,7 +729,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       }
   #pragma unroll
       for (int i = 0; i < R; ++i) {
-        fwd_scores<T, D, XM>(s[i], tile_k(i), qf, a, mk, brow, nb + i);
+        typename Elem<T>::frag bf[2];
+        if constexpr (kBias) load_p_frags<T>(bf, brow, (nb + i) * kBlk, Tk_);
+        fwd_scores<T, D, XM>(s[i], tile_k(i), qf, a, mk, bf, nb + i);
         if (i > 0 && nb + i >= cr.t1) {
   #pragma unroll
           for (int kb = 0; kb < 2; ++kb)
@@ -791,12 +808,12 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       round(nb, [&](int i) -> const lds* { return sK[i]; });
     }
   }
-  if (!XM && raw_units && mx != -INFINITY) mx *= csl;  // back to base-2 units
+  if (!kBias && raw_units && mx != -INFINITY) mx *= csl;  // back to base-2 units
   {
     // Finite without a window (every row sees a key of its first tile); with
     // one a chunk can miss all of a row's keys, and then max -inf, sum 0.
     const float mrow = group_max(mx);
-    l = group_sum(l * fast_exp2(mx - ((XM && mrow == -INFINITY) ? 0.f : mrow)));
+    l = group_sum(l * fast_exp2(mx - ((XM != kMaskNone && mrow == -INFINITY) ? 0.f : mrow)));
     mx = mrow;
   }
   if (g != 0) return;
@@ -851,7 +868,7 @@ __device__ __forceinline__ float p_pass_lse2(const Params& a, int bh, int nblk, 
   return lse2;
 }
 
-template <typename T, int D, bool XM>
+template <typename T, int D, int XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params a) {
   typedef Elem<T> E;
@@ -884,8 +901,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
-  const RowMask<XM> mk(a, mb, m);
-  const T* brow = (XM && a.bias.p) ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
+  const RowMask<XM != kMaskNone> mk(a, mb, m);
+  constexpr bool kBias = XM == kMaskBias;
+  const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
 
   const float lse2 = p_pass_lse2(a, bh, nblk, mb, rl, cr.nch, ch == 0 && g == 0);
 
@@ -949,7 +967,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   auto body = [&](int nt, const lds* cK, const lds* cV) __attribute__((always_inline)) {
       const int n0 = nt * kBlk;
       mfrag pf[2];
-      if constexpr (!XM && sizeof(T) == 2) {
+      if constexpr (!kBias && sizeof(T) == 2) {
         // Raw scores; P = exp2(raw * scale*log2e - lse) in one FMA, masked
         // entries selected to 0 afterwards, and one rounding to T gives both
         // the MFMA fragment and the stored P.
@@ -1004,7 +1022,9 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
         }
       } else {
         Tile s;
-        fwd_scores<T, D, XM>(s, cK, qf, a, mk, brow, nt);
+        frag bf[2];
+        if constexpr (kBias) load_p_frags<T>(bf, brow, n0, Tk_);
+        fwd_scores<T, D, XM>(s, cK, qf, a, mk, bf, nt);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
           float pv[8];
@@ -1131,17 +1151,18 @@ hipError_t launch_fill_masked_p(int dtype, const Params& a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool XM>
+template <typename T, int D>
 static void launch_fwd_x(const Params& a, bool write_p, dim3 grid, hipStream_t st) {
+  const int xm = mask_kind(a, false);
   if (write_p) {
     {
       const TimedLaunch tl(st, kTagFwdStats);
-      hipLaunchKernelGGL((k_fwd_stats<T, D, XM>), grid, dim3(kThreads), 0, st, a);
+      DISPATCH_MASK(xm, true, hipLaunchKernelGGL((k_fwd_stats<T, D, kXM>), grid, dim3(kThreads), 0, st, a));
     }
     const TimedLaunch tl(st, kTagFwdP);
-    hipLaunchKernelGGL((k_fwd_p<T, D, XM>), grid, dim3(kThreads), 0, st, a);
+    DISPATCH_MASK(xm, true, hipLaunchKernelGGL((k_fwd_p<T, D, kXM>), grid, dim3(kThreads), 0, st, a));
   } else {
-    if constexpr (!XM && sizeof(T) == 2) {
+    if constexpr (sizeof(T) == 2) {
       if (a.pairs) {
         const int npair = ((a.T + kBlk - 1) / kBlk + 1) >> 1;
         const int c2 = a.chunk >> 1;
@@ -1152,7 +1173,7 @@ static void launch_fwd_x(const Params& a, bool write_p, dim3 grid, hipStream_t s
       }
     }
     const TimedLaunch tl(st, kTagFwdOnline);
-    hipLaunchKernelGGL((k_fwd_online<T, D, XM>), grid, dim3(kThreads), 0, st, a);
+    DISPATCH_MASK(xm, true, hipLaunchKernelGGL((k_fwd_online<T, D, kXM>), grid, dim3(kThreads), 0, st, a));
   }
 }
 
@@ -1163,26 +1184,24 @@ static hipError_t launch_fwd_t(int dtype, const Params& a, bool write_p, hipStre
   // row pairs: 16-bit types without a window or bias; a split causal walk
   // takes chunks of an even number of tiles
   if (!write_p && a.pairs &&
-      (!fwd_pairs_allowed(dtype, extended_mask(a)) || (a.causal && a.nchunk_max > 1 && (a.chunk & 1))))
+      (!fwd_pairs_allowed(dtype, mask_kind(a, false) != kMaskNone) || (a.causal && a.nchunk_max > 1 && (a.chunk & 1))))
     return hipErrorInvalidValue;
-  if (extended_mask(a))
-    launch_fwd_x<T, D, true>(a, write_p, grid, st);
-  else
-    launch_fwd_x<T, D, false>(a, write_p, grid, st);
+  launch_fwd_x<T, D>(a, write_p, grid, st);
   if (a.nchunk_max > 1)
     return write_p ? launch_combine_sum(dtype, D, a, kOutO, st) : launch_combine_fwd(dtype, D, a, st);
   return hipGetLastError();
 }
 
-template <typename T, int D, bool XM>
-static int occupancy_fwd_t(bool write_p) {
-  if (!write_p) return occupancy_of(k_fwd_online<T, D, XM>);
-  return std::min(occupancy_of(k_fwd_stats<T, D, XM>), occupancy_of(k_fwd_p<T, D, XM>));
+template <typename T, int D>
+static int occupancy_fwd_t(bool write_p, int xm) {
+  if (!write_p) DISPATCH_MASK(xm, true, return occupancy_of(k_fwd_online<T, D, kXM>));
+  DISPATCH_MASK(xm, true,
+                return std::min(occupancy_of(k_fwd_stats<T, D, kXM>), occupancy_of(k_fwd_p<T, D, kXM>)));
+  return 0;
 }
 
-int occupancy_fwd(int dtype, int D, bool write_p, bool xm) {
-  if (xm) DISPATCH_DTYPE_D(dtype, D, return occupancy_fwd_t<ElemT, kD, true>(write_p));
-  else DISPATCH_DTYPE_D(dtype, D, return occupancy_fwd_t<ElemT, kD, false>(write_p));
+int occupancy_fwd(int dtype, int D, bool write_p, int xm) {
+  DISPATCH_DTYPE_D(dtype, D, return occupancy_fwd_t<ElemT, kD>(write_p, xm));
   return 0;
 }
 

@@ -111,6 +111,13 @@ static_assert(TTT_GG_HEAD_DIM == 64 || TTT_GG_HEAD_DIM == 128, "head dim of this
 
 namespace ttt {
 
+// Types whose plain problems the eight-wave kernels run: the four-wave ones
+// exist for their windows and biases (and GdO).
+template <typename T>
+constexpr bool kRow4Plain = !(TTT_GG_ROW8 && sizeof(T) == 2);
+template <typename T>
+constexpr bool kCol4Plain = !(TTT_GG_COL8 && sizeof(T) == 2);
+
 constexpr int kThreads8 = 2 * kThreads;  // the eight-wave kernels
 
 // Waves per SIMD of the eight-wave kernels (built at D = 128 only: at D = 64
@@ -127,7 +134,7 @@ struct GgWaves {
 };
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool LOADP, bool GDO, bool XM, bool DQ>
+template <typename T, int D, bool LOADP, bool GDO, int XM, bool DQ>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params a) {
   typedef Elem<T> E;
@@ -179,9 +186,17 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
   const bool row_ok = m < T_;
-  const RowMask<XM> mk(a, mb, m);
-  const T* brow =
-      (XM && !LOADP && a.bias.p) ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
+  const RowMask<XM != kMaskNone> mk(a, mb, m);
+  constexpr bool kBias = XM == kMaskBias;
+  static_assert(!(LOADP && kBias), "a saved P holds the bias");
+  const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
+  frag bn[2], bc[2];  // bias of the next tile and of this one
+  auto take_bias = [&]() __attribute__((always_inline)) {
+    if constexpr (kBias) {
+      bc[0] = bn[0];
+      bc[1] = bn[1];
+    }
+  };
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -251,6 +266,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   frag pn[2];
   auto load_tile = [&](int nb) {
     const int n0 = nb * kBlk;
+    if constexpr (kBias) load_p_frags<T>(bn, brow, n0, Tk_);
     stage_load_at<T, D>(s0, Kn, a.k.st, Tk_ - n0, scol);
     stage_load_at<T, D>(s1, Vn, a.v.st, Tk_ - n0, scol);
     stage_load_at<T, D>(s2, gKn, a.gk.st, Tk_ - n0, scol);
@@ -264,6 +280,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   auto dma_tile = [&](int nb, int buf) {
     if constexpr (kDma) {
       const int n0 = nb * kBlk;
+      if constexpr (kBias) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
         dd.load_full(sK[buf], Kn, oK);
         dd.load_full(sV[buf], Vn, oV);
@@ -293,7 +310,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     if constexpr (!LOADP) {
       p.zero();
       mm_d<M>(p, cK, qf);
-      recompute_p_row<T, XM>(p, a, brow, n0, lse2, kSl2);
+      recompute_p_row<T, kBias>(p, bc, lse2, kSl2);
     }
     if (mk.tile(nb)) {
 #pragma unroll
@@ -375,6 +392,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     dd.offsets(ogV, a.gv.st);
     auto dma_set = [&](int nb, T* k, T* v, T* gk, T* gv) __attribute__((always_inline)) {
       const int n0 = nb * kBlk;
+      if constexpr (kBias) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
         dd.load_full(k, Kn, oK);
         dd.load_full(v, Vn, oV);
@@ -401,6 +419,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       __syncthreads();  // everyone's, and everyone is done with the other set
       Tile p;
       p_from_frags(p);
+      take_bias();
       // Keep the conversion ahead of the next tile's loads: sunk below them,
       // it would wait for those loads (vmcnt) before the tile's work.
       __builtin_amdgcn_sched_barrier(0);
@@ -445,6 +464,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       }
       Tile p;
       p_from_frags(p);
+      take_bias();
       if (nb + 1 < cr.t1) {
         if constexpr (kDma)
           dma_tile(nb + 1, cur ^ 1);
@@ -513,7 +533,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool LOADP, bool XM>
+template <typename T, int D, bool LOADP, int XM>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params a, Params rowc, int nx) {
   typedef Elem<T> E;
@@ -577,8 +597,11 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int cl = 16 * w + c;
   const int n = n0 + cl;
-  const ColMask<XM> mk(a, nb, n);
-  const T* bcol = (XM && !LOADP && a.bias.p) ? at<const T>(a.bias, b, h) + (n < T_ ? n : 0) : nullptr;
+  const ColMask<XM != kMaskNone> mk(a, nb, n);
+  constexpr bool kBias = XM == kMaskBias;
+  static_assert(!(LOADP && kBias), "a saved P holds the bias");
+  const T* bcol = kBias ? at<const T>(a.bias, b, h) + (n < T_ ? n : 0) : nullptr;
+  BiasCol<T> bn, bc;  // bias of the next tile and of this one
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -635,7 +658,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     } else {
       p.zero();
       mm_d<M>(p, cb.q, kf);  // -s q.k
-      recompute_p_col<T, XM>(p, a, bcol, m0, cb.st, 3, -kSl2);
+      recompute_p_col<T, kBias>(p, bc, cb.st, 3, -kSl2);
     }
     if (mk.tile(mb)) {
 #pragma unroll
@@ -706,6 +729,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     const StatDma<kNS> sdma(rs, ev, fv, lse);
     auto dma_tile = [&](int mb, const Bufs& wb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
+      if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
       if (m0 + kBlk <= Tq_ && cols_full) {  // uniform: one test per tile
         dd.load_full(wb.q, Qn, oQ);
         dd.load_full(wb.gq, gQn, ogQ);
@@ -729,6 +753,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       constexpr int P = decltype(par)::value;
       dma_wait();       // this wave's loads of tile mb
       __syncthreads();  // everyone's, and everyone is done with the other set
+      if constexpr (kBias) bc = bn;
       if (mb + 1 < cr.t1) dma_tile(mb + 1, bufs(Parity<1 - P>{}));
       compute(mb, bufs(Parity<P>{}));
     };
@@ -744,6 +769,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     float stv;
     auto load_tile = [&](int mb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
+      if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
       stage_load_at<T, D>(s0, Q + (int64_t)m0 * a.q.st, a.q.st, Tq_ - m0, scol);
       stage_load_at<T, D>(s1, gQ + (int64_t)m0 * a.gq.st, a.gq.st, Tq_ - m0, scol);
       stage_load_at<T, D>(s2, dO + (int64_t)m0 * a.dout.st, a.dout.st, Tq_ - m0, scol);
@@ -759,6 +785,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       if constexpr (LOADP) stage_store_rows<T, kBlk>(sp, sP0);
       stat_store<kNS>(stv, sS0);
       __syncthreads();
+      if constexpr (kBias) bc = bn;
       if (mb + 1 < cr.t1) load_tile(mb + 1);
       compute(mb, bufs(Parity<0>{}));
     }
@@ -1354,24 +1381,27 @@ __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(Gg8Wa
 #endif
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool XM>
+template <typename T, int D>
 // False when the variant asked for is not in this object (ttt_launch.h
 // routes each variant to the object that has it).  Without GdO, a given dQ
 // (a.dq.p) selects the dQ form.
 static bool launch_gg_row_x(const Params& a, bool load_p, bool gdo, dim3 grid, hipStream_t st) {
   const TimedLaunch tl(st, kTagGgRow);
+  const int xm = mask_kind(a, load_p);
   if (gdo) {
     if constexpr ((TTT_GG_ROW_GDO & 2) != 0) {
       if (load_p)
-        hipLaunchKernelGGL((k_gg_row<T, D, true, true, XM, false>), grid, dim3(kThreads), 0, st, a);
+        DISPATCH_MASK(xm, false,
+                      hipLaunchKernelGGL((k_gg_row<T, D, true, true, kXM, false>), grid, dim3(kThreads), 0, st, a));
       else
-        hipLaunchKernelGGL((k_gg_row<T, D, false, true, XM, false>), grid, dim3(kThreads), 0, st, a);
+        DISPATCH_MASK(xm, true,
+                      hipLaunchKernelGGL((k_gg_row<T, D, false, true, kXM, false>), grid, dim3(kThreads), 0, st, a));
       return true;
     }
   } else {
     const bool dq = a.dq.p != nullptr;
 #if TTT_GG_ROW8
-    if constexpr (sizeof(T) == 2 && !XM) {
+    if (sizeof(T) == 2 && xm == kMaskNone) {
       if (dq) {
         if (load_p)
           hipLaunchKernelGGL((k_gg_row8<T, D, true, true>), grid, dim3(kThreads8), 0, st, a);
@@ -1389,14 +1419,18 @@ static bool launch_gg_row_x(const Params& a, bool load_p, bool gdo, dim3 grid, h
     if constexpr ((TTT_GG_ROW_GDO & 1) != 0) {
       if (dq) {
         if (load_p)
-          hipLaunchKernelGGL((k_gg_row<T, D, true, false, XM, true>), grid, dim3(kThreads), 0, st, a);
+          DISPATCH_MASK_OF(xm, kRow4Plain<T>, false,
+                      hipLaunchKernelGGL((k_gg_row<T, D, true, false, kXM, true>), grid, dim3(kThreads), 0, st, a));
         else
-          hipLaunchKernelGGL((k_gg_row<T, D, false, false, XM, true>), grid, dim3(kThreads), 0, st, a);
+          DISPATCH_MASK_OF(xm, kRow4Plain<T>, true,
+                      hipLaunchKernelGGL((k_gg_row<T, D, false, false, kXM, true>), grid, dim3(kThreads), 0, st, a));
       } else {
         if (load_p)
-          hipLaunchKernelGGL((k_gg_row<T, D, true, false, XM, false>), grid, dim3(kThreads), 0, st, a);
+          DISPATCH_MASK_OF(xm, kRow4Plain<T>, false,
+                      hipLaunchKernelGGL((k_gg_row<T, D, true, false, kXM, false>), grid, dim3(kThreads), 0, st, a));
         else
-          hipLaunchKernelGGL((k_gg_row<T, D, false, false, XM, false>), grid, dim3(kThreads), 0, st, a);
+          DISPATCH_MASK_OF(xm, kRow4Plain<T>, true,
+                      hipLaunchKernelGGL((k_gg_row<T, D, false, false, kXM, false>), grid, dim3(kThreads), 0, st, a));
       }
       return true;
     }
@@ -1408,8 +1442,7 @@ template <typename T, int D>
 static hipError_t launch_gg_row_t(int dtype, const Params& a, bool load_p, bool gdo, hipStream_t st, bool combine) {
   const int nblk = (a.T + kBlk - 1) / kBlk;
   dim3 grid(nblk * a.nchunk_max, a.B * a.H);
-  const bool ok = extended_mask(a) ? launch_gg_row_x<T, D, true>(a, load_p, gdo, grid, st)
-                                    : launch_gg_row_x<T, D, false>(a, load_p, gdo, grid, st);
+  const bool ok = launch_gg_row_x<T, D>(a, load_p, gdo, grid, st);
   if (!ok) return hipErrorInvalidDeviceFunction;
   if (a.nchunk_max > 1) return combine ? launch_combine_gg_row(dtype, D, a, gdo, st) : launch_combine_gg_ef(a, st);
   return hipGetLastError();
@@ -1421,10 +1454,10 @@ static hipError_t launch_gg_col_t(int dtype, const Params& a, bool load_p, hipSt
   const bool fold = rowc && rowc->nchunk_max > 1;
   dim3 grid(nx + (fold ? (a.T + kBlk - 1) / kBlk * CombineSlot<D>::kSub : 0), a.B * a.H);
   const Params& c = fold ? *rowc : a;
-  const bool xm = extended_mask(a);
+  const int xm = mask_kind(a, load_p);
 #if TTT_GG_COL8
   if constexpr (sizeof(T) == 2) {
-    if (!xm) {
+    if (xm == kMaskNone) {
       {
         const TimedLaunch tl(st, kTagGgCol);
         if (load_p)
@@ -1439,17 +1472,12 @@ static hipError_t launch_gg_col_t(int dtype, const Params& a, bool load_p, hipSt
 #endif
   {
     const TimedLaunch tl(st, kTagGgCol);
-    if (load_p) {
-      if (xm)
-        hipLaunchKernelGGL((k_gg_col<T, D, true, true>), grid, dim3(kThreads), 0, st, a, c, nx);
-      else
-        hipLaunchKernelGGL((k_gg_col<T, D, true, false>), grid, dim3(kThreads), 0, st, a, c, nx);
-    } else {
-      if (xm)
-        hipLaunchKernelGGL((k_gg_col<T, D, false, true>), grid, dim3(kThreads), 0, st, a, c, nx);
-      else
-        hipLaunchKernelGGL((k_gg_col<T, D, false, false>), grid, dim3(kThreads), 0, st, a, c, nx);
-    }
+    if (load_p)
+      DISPATCH_MASK_OF(xm, kCol4Plain<T>, false,
+                    hipLaunchKernelGGL((k_gg_col<T, D, true, kXM>), grid, dim3(kThreads), 0, st, a, c, nx));
+    else
+      DISPATCH_MASK_OF(xm, kCol4Plain<T>, true,
+                    hipLaunchKernelGGL((k_gg_col<T, D, false, kXM>), grid, dim3(kThreads), 0, st, a, c, nx));
   }
   if (a.nchunk_max > 1) return launch_combine_sum(dtype, D, a, kOutGKGV, st);
   return hipGetLastError();
@@ -1459,32 +1487,38 @@ static hipError_t launch_gg_col_t(int dtype, const Params& a, bool load_p, hipSt
 // without dQ, so that a workspace sized before the call fits either form; the
 // dQ form runs at least as many (the same waves-per-SIMD target and LDS,
 // fewer registers).
-template <typename T, int D, bool XM>
-static int occupancy_gg_row_t(bool load_p, bool gdo) {
+template <typename T, int D>
+static int occupancy_gg_row_t(bool load_p, bool gdo, int xm) {
   if (gdo) {
-    if constexpr ((TTT_GG_ROW_GDO & 2) != 0)
-      return load_p ? occupancy_of(k_gg_row<T, D, true, true, XM, false>)
-                    : occupancy_of(k_gg_row<T, D, false, true, XM, false>);
+    if constexpr ((TTT_GG_ROW_GDO & 2) != 0) {
+      if (load_p) DISPATCH_MASK(xm, false, return occupancy_of(k_gg_row<T, D, true, true, kXM, false>));
+      else DISPATCH_MASK(xm, true, return occupancy_of(k_gg_row<T, D, false, true, kXM, false>));
+    }
   } else {
 #if TTT_GG_ROW8
-    if constexpr (sizeof(T) == 2 && !XM)
+    if (sizeof(T) == 2 && xm == kMaskNone)
       return load_p ? occupancy_of(k_gg_row8<T, D, true, false>, kThreads8)
                     : occupancy_of(k_gg_row8<T, D, false, false>, kThreads8);
 #endif
-    if constexpr ((TTT_GG_ROW_GDO & 1) != 0)
-      return load_p ? occupancy_of(k_gg_row<T, D, true, false, XM, false>)
-                    : occupancy_of(k_gg_row<T, D, false, false, XM, false>);
+    if constexpr ((TTT_GG_ROW_GDO & 1) != 0) {
+      if (load_p)
+        DISPATCH_MASK_OF(xm, kRow4Plain<T>, false, return occupancy_of(k_gg_row<T, D, true, false, kXM, false>));
+      else
+        DISPATCH_MASK_OF(xm, kRow4Plain<T>, true, return occupancy_of(k_gg_row<T, D, false, false, kXM, false>));
+    }
   }
   return 0;
 }
 
-template <typename T, int D, bool XM>
-static int occupancy_gg_col_t(bool load_p) {
+template <typename T, int D>
+static int occupancy_gg_col_t(bool load_p, int xm) {
 #if TTT_GG_COL8
-  if constexpr (sizeof(T) == 2 && !XM)
+  if (sizeof(T) == 2 && xm == kMaskNone)
     return load_p ? occupancy_of(k_gg_col8<T, D, true>, kThreads8) : occupancy_of(k_gg_col8<T, D, false>, kThreads8);
 #endif
-  return load_p ? occupancy_of(k_gg_col<T, D, true, XM>) : occupancy_of(k_gg_col<T, D, false, XM>);
+  if (load_p) DISPATCH_MASK_OF(xm, kCol4Plain<T>, false, return occupancy_of(k_gg_col<T, D, true, kXM>));
+  else DISPATCH_MASK_OF(xm, kCol4Plain<T>, true, return occupancy_of(k_gg_col<T, D, false, kXM>));
+  return 0;
 }
 
 // Entry points of this object's head dim and element types (D is
@@ -1509,9 +1543,8 @@ static int occupancy_gg_col_t(bool load_p) {
     }                                                                \
   } while (0)
 
-int TTT_GG_NAME(occupancy_gg_row)(int dtype, bool load_p, bool gdo, bool xm) {
-  if (xm) TTT_GG_DISPATCH(dtype, return occupancy_gg_row_t<ElemT, kD, true>(load_p, gdo));
-  else TTT_GG_DISPATCH(dtype, return occupancy_gg_row_t<ElemT, kD, false>(load_p, gdo));
+int TTT_GG_NAME(occupancy_gg_row)(int dtype, bool load_p, bool gdo, int xm) {
+  TTT_GG_DISPATCH(dtype, return occupancy_gg_row_t<ElemT, kD>(load_p, gdo, xm));
   return 0;
 }
 
@@ -1522,9 +1555,8 @@ hipError_t TTT_GG_NAME(launch_gg_row)(int dtype, const Params& a, bool load_p, b
 }
 
 #if TTT_GG_COL
-int TTT_GG_NAME(occupancy_gg_col)(int dtype, bool load_p, bool xm) {
-  if (xm) TTT_GG_DISPATCH(dtype, return occupancy_gg_col_t<ElemT, kD, true>(load_p));
-  else TTT_GG_DISPATCH(dtype, return occupancy_gg_col_t<ElemT, kD, false>(load_p));
+int TTT_GG_NAME(occupancy_gg_col)(int dtype, bool load_p, int xm) {
+  TTT_GG_DISPATCH(dtype, return occupancy_gg_col_t<ElemT, kD>(load_p, xm));
   return 0;
 }
 

@@ -68,9 +68,27 @@ struct TimedLaunch {
   ~TimedLaunch() { timing_mark(st, tag, true); }
 };
 
-// The problem has a key window or an additive bias: launches run the kernels'
-// XM instantiation.
-inline bool extended_mask(const Params& a) { return a.win > 0 || a.bias.p != nullptr; }
+// The mask form of a launch (kMask*): kernels that read a saved P take the
+// window form for a bias.
+inline int mask_kind(const Params& a, bool load_p) {
+  return a.bias.p ? (load_p ? kMaskWindow : kMaskBias) : a.win > 0 ? kMaskWindow : kMaskNone;
+}
+// Runs `stmt` with kXM bound to the mask form: kMaskNone and kMaskBias only
+// where NONE and BIAS say that such a kernel exists.
+#define DISPATCH_MASK_OF(kind, NONE, BIAS, ...)                              \
+  do {                                                                        \
+    if ((NONE) && (kind) == ::ttt::kMaskNone) {                               \
+      constexpr int kXM = (NONE) ? ::ttt::kMaskNone : ::ttt::kMaskWindow;     \
+      __VA_ARGS__;                                                            \
+    } else if ((BIAS) && (kind) == ::ttt::kMaskBias) {                        \
+      constexpr int kXM = (BIAS) ? ::ttt::kMaskBias : ::ttt::kMaskWindow;     \
+      __VA_ARGS__;                                                            \
+    } else {                                                                  \
+      constexpr int kXM = ::ttt::kMaskWindow;                                 \
+      __VA_ARGS__;                                                            \
+    }                                                                         \
+  } while (0)
+#define DISPATCH_MASK(kind, BIAS, ...) DISPATCH_MASK_OF(kind, true, BIAS, __VA_ARGS__)
 
 // The O + LSE forward can run k_fwd_lse, whose workgroups take pairs of row
 // blocks (128 rows; split causal walks in chunks of an even number of
@@ -85,25 +103,25 @@ inline bool fwd_row_pairs(int dtype, int D, bool xm, int block_rows) {
 }
 
 // Occupancy of the kernels a launch of each family runs (the smaller one when
-// it runs two); xm selects the window/bias instantiation.
-int occupancy_fwd(int dtype, int D, bool write_p, bool xm);
+// it runs two); xm: the mask form (mask_kind).
+int occupancy_fwd(int dtype, int D, bool write_p, int xm);
 int occupancy_fwd_pairs(int dtype, int D);
-int occupancy_dq(int dtype, int D, bool load_p, bool xm);
-int occupancy_dkdv(int dtype, int D, bool load_p, bool xm);
+int occupancy_dq(int dtype, int D, bool load_p, int xm);
+int occupancy_dkdv(int dtype, int D, bool load_p, int xm);
 // Grad-grad entry points: ttt_gg.hip is built into one object per head dim
 // (and, at D = 128, per 16-bit / 16-bit with GdO / fp32), suffixed 64, 128h,
 // 128hg and 128f.
 #define TTT_GG_CAT2(a, b) a##b
 #define TTT_GG_CAT(a, b) TTT_GG_CAT2(a, b)
 #define TTT_GG_NAME(name) TTT_GG_CAT(name, TTT_GG_SUFFIX)
-int occupancy_gg_row64(int dtype, bool load_p, bool gdo, bool xm);
-int occupancy_gg_row128h(int dtype, bool load_p, bool gdo, bool xm);
-int occupancy_gg_row128hg(int dtype, bool load_p, bool gdo, bool xm);
-int occupancy_gg_row128f(int dtype, bool load_p, bool gdo, bool xm);
-int occupancy_gg_col64(int dtype, bool load_p, bool xm);
-int occupancy_gg_col128h(int dtype, bool load_p, bool xm);
-int occupancy_gg_col128f(int dtype, bool load_p, bool xm);
-inline int occupancy_gg_row(int dtype, int D, bool load_p, bool gdo, bool xm) {
+int occupancy_gg_row64(int dtype, bool load_p, bool gdo, int xm);
+int occupancy_gg_row128h(int dtype, bool load_p, bool gdo, int xm);
+int occupancy_gg_row128hg(int dtype, bool load_p, bool gdo, int xm);
+int occupancy_gg_row128f(int dtype, bool load_p, bool gdo, int xm);
+int occupancy_gg_col64(int dtype, bool load_p, int xm);
+int occupancy_gg_col128h(int dtype, bool load_p, int xm);
+int occupancy_gg_col128f(int dtype, bool load_p, int xm);
+inline int occupancy_gg_row(int dtype, int D, bool load_p, bool gdo, int xm) {
   if (D == 64) return occupancy_gg_row64(dtype, load_p, gdo, xm);
   if (D == 128)
     return dtype == kF32 ? occupancy_gg_row128f(dtype, load_p, gdo, xm)
@@ -111,7 +129,7 @@ inline int occupancy_gg_row(int dtype, int D, bool load_p, bool gdo, bool xm) {
                          : occupancy_gg_row128h(dtype, load_p, gdo, xm);
   return 0;
 }
-inline int occupancy_gg_col(int dtype, int D, bool load_p, bool xm) {
+inline int occupancy_gg_col(int dtype, int D, bool load_p, int xm) {
   if (D == 64) return occupancy_gg_col64(dtype, load_p, xm);
   if (D == 128) return dtype == kF32 ? occupancy_gg_col128f(dtype, load_p, xm) : occupancy_gg_col128h(dtype, load_p, xm);
   return 0;
