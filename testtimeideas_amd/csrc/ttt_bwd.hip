@@ -141,6 +141,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   constexpr bool kBias = XM == kMaskBias;
   static_assert(!(LOADP && kBias), "a saved P holds the bias");
   const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
+  constexpr bool kAhead = kBias && kBiasAhead<T, D>;
   frag bn[2], bc[2];  // bias of the next tile and of this one
 
   const T* Q = at<const T>(a.q, b, h);
@@ -187,7 +188,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   const T* Pn = LOADP ? Pm + cr.t0 * kBlk + stream_index(0, g, 0) : nullptr;
   auto fetch = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
-    if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
+    if constexpr (kAhead) load_p_frags<T>(bn, brow, n1, Tk_);
     if constexpr (!LOADP) {
       // Recompute: tile-indexed clamped loads, measured faster for this
       // variant than the running-pointer form below.
@@ -220,7 +221,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   }
   auto fetch_dma = [&](int nb, auto par) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
-    if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
+    if constexpr (kAhead) load_p_frags<T>(bn, brow, n1, Tk_);
     if (n1 + kBlk <= Tk_) {
       dd.load_full(set_k(par), Kn, oK);
       dd.load_full(set_v(par), Vn, oV);
@@ -261,9 +262,12 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     const lds* cV = set_v(par);
     Tile p;
     if constexpr (LOADP) frags_to_tile<T>(p, pn);
-    if constexpr (kBias) {
+    if constexpr (kAhead) {
       bc[0] = bn[0];
       bc[1] = bn[1];
+    } else if constexpr (kBias) {
+      load_p_frags<T>(bc, brow, n0, Tk_);
+      if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);  // see kBiasAhead
     }
     if constexpr (kDma) {
       if constexpr (decltype(prefetch)::value == 1) fetch_dma(nb + 1, other_buf(par));
@@ -421,7 +425,16 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   constexpr bool kBias = XM == kMaskBias;
   static_assert(!(LOADP && kBias), "a saved P holds the bias");
   const T* bcol = kBias ? at<const T>(a.bias, b, h) + (n < T_ ? n : 0) : nullptr;
+  constexpr bool kAhead = kBias && kBiasAhead<T, D>;
   BiasCol<T> bn, bc;  // bias of the next tile and of this one
+  auto take_bias = [&](int mb) __attribute__((always_inline)) {
+    if constexpr (kAhead) {
+      bc = bn;
+    } else if constexpr (kBias) {
+      bc.load(bcol, a.bias.st, mb * kBlk, Tq_);
+      if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);  // see kBiasAhead
+    }
+  };
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -467,7 +480,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   const bool cols_full = n0 + kBlk <= T_;
   auto load_tile = [&](int mb) __attribute__((always_inline)) {
     const int m0 = mb * kBlk;
-    if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
+    if constexpr (kAhead) bn.load(bcol, a.bias.st, m0, Tq_);
     stage_load_at<T, D>(stdO, dOn, a.dout.st, Tq_ - m0, scol);
     if constexpr (kNeedQ) stage_load_at<T, D>(stQ, Qn, a.q.st, Tq_ - m0, scol);
     if constexpr (LOADP) stage_load<T, kBlk>(stP, Pn, a.p.st, Tq_ - m0, T_ - n0);
@@ -491,7 +504,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     if constexpr (kDma) {
       const int m0 = mb * kBlk;
       const Bufs bf = bufs(par);
-      if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
+      if constexpr (kAhead) bn.load(bcol, a.bias.st, m0, Tq_);
       if (m0 + kBlk <= Tq_ && cols_full) {
         dd.load_full(bf.dout, dOn, odO);
         dd.load_full(bf.q, Qn, oQ);
@@ -525,7 +538,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
         stage_store_rows<T, kBlk>(stP, sP0);
         __syncthreads();
       }
-      if constexpr (kBias) bc = bn;
+      take_bias(mb);
       if constexpr (!kLateFetch) {
         if constexpr (decltype(prefetch)::value == 1) dma_tile(mb + 1, Parity<1 - P>{});
         if constexpr (decltype(prefetch)::value == 2)
@@ -538,7 +551,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       if constexpr (LOADP) stage_store_rows<T, kBlk>(stP, sP0);
       if constexpr (kNS > 0) stat_store<kNS>(stv, sS0);
       __syncthreads();
-      if constexpr (kBias) bc = bn;
+      take_bias(mb);
       if constexpr (decltype(prefetch)::value == 1) load_tile(mb + 1);
       if constexpr (decltype(prefetch)::value == 2)
         if (mb + 1 < cr.t1) load_tile(mb + 1);

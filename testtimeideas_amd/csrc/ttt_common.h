@@ -255,6 +255,22 @@ __host__ __device__ inline Item causal_item(int x, int n, int c) {
 // grad-grad column pass 177 -> 166 us, dK/dV 83 -> 80).
 enum : int { kMaskNone = 0, kMaskWindow = 1, kMaskBias = 2 };
 
+// Whether a bias kernel loads a tile's bias one tile ahead (with the next
+// tile's operands) or at the head of its own step, before the next tile's
+// loads are issued (in 16-bit kernels behind a scheduling barrier: sunk below
+// the direct loads, it would wait for them too).  Ahead, it is two fragments
+// (column kernels: 32 values) across a whole step, and the line is registers:
+// 16-bit D = 64 row kernels spill at their waves-per-SIMD cap (gg-row 14,
+// dQ 8) and dK/dV drops from three waves to two; fp32 D = 128 dQ drops from
+// two to one.  Both sides measured, ahead -> own step (us): b8 h6 T1024 d64
+// bf16 dQ 37.5 -> 32.7, gg-row 80.7 -> 71.8, dK/dV 53.1 -> 44.5, the step
+// 275 -> 253; b1 h4 T4096 354 -> 333; b2 h4 T1500 d128 fp32 dQ 181 -> 165,
+// the step 1597 -> 1545.  (One loss, from the fill of 512 workgroups: b2 h8
+// T2048 bf16 dK/dV 66 -> 81.)  fp32 D = 64 and 16-bit D = 128 have the
+// registers: 512 queries of 2048 keys fp32 own step -> ahead 459 -> 433.
+template <typename T, int D>
+constexpr bool kBiasAhead = (sizeof(T) == 4) == (D == 64);
+
 // The column's chunk: causal_item for plain causal split slices (XM = kMaskNone),
 // else x % nblk, x / nblk (chunk index by chunk index, blocks in launch
 // order; columns past a block's chunks exit on their chunk test).

@@ -153,7 +153,17 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const RowMask<XM != kMaskNone> mk(a, mb, m);
   constexpr bool kBias = XM == kMaskBias;
   const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(m < T_ ? m : 0) * a.bias.st : nullptr;
+  constexpr bool kAhead = kBias && kBiasAhead<T, D>;
   frag bn[2], bc[2];  // bias of the next tile and of this one
+  auto take_bias = [&](int nt) __attribute__((always_inline)) {
+    if constexpr (kAhead) {
+      bc[0] = bn[0];
+      bc[1] = bn[1];
+    } else if constexpr (kBias) {
+      load_p_frags<T>(bc, brow, nt * kBlk, Tk_);
+      if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);  // see kBiasAhead
+    }
+  };
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -174,7 +184,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   const StageOff<T, D> soV = stage_offsets<T, D>(a.v.st, cols_of<T, D>(a));
   auto load_kv = [&](int nb) __attribute__((always_inline)) {
     const int n1 = nb * kBlk;
-    if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
+    if constexpr (kAhead) load_p_frags<T>(bn, brow, n1, Tk_);
     const T* kp = K + (int64_t)n1 * a.k.st;
     const T* vp = V + (int64_t)n1 * a.v.st;
     if (D == 64 && n1 + kBlk <= Tk_) {  // full tile: offsets computed once
@@ -280,7 +290,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     dd.offsets(oV, a.v.st);
     auto fetch = [&](int nt, T* k, T* v) __attribute__((always_inline)) {
       const int n1 = nt * kBlk;
-      if constexpr (kBias) load_p_frags<T>(bn, brow, n1, Tk_);
+      if constexpr (kAhead) load_p_frags<T>(bn, brow, n1, Tk_);
       const T* kp = K + (int64_t)n1 * a.k.st;
       const T* vp = V + (int64_t)n1 * a.v.st;
       if (n1 + kBlk <= Tk_) {
@@ -297,10 +307,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       constexpr int P = decltype(par)::value;
       dma_wait();       // this wave's loads of tile nt
       __syncthreads();  // everyone's, and everyone is done with the other set
-      if constexpr (kBias) {
-        bc[0] = bn[0];
-        bc[1] = bn[1];
-      }
+      take_bias(nt);
       if (nt + 1 < cr.t1) {
         if constexpr (P == 0)
           fetch(nt + 1, sK1, sV1);
@@ -324,10 +331,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       stage_store_tile<M>(stK, sK);
       stage_store_tile<M>(stV, sV);
       __syncthreads();
-      if constexpr (kBias) {
-        bc[0] = bn[0];
-        bc[1] = bn[1];
-      }
+      take_bias(nb);
       if (nb + 1 < cr.t1) load_kv(nb + 1);
       body(nb, sK, sV);
     }

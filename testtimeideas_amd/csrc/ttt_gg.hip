@@ -190,11 +190,15 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   constexpr bool kBias = XM == kMaskBias;
   static_assert(!(LOADP && kBias), "a saved P holds the bias");
   const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
+  constexpr bool kAhead = kBias && kBiasAhead<T, D>;
   frag bn[2], bc[2];  // bias of the next tile and of this one
-  auto take_bias = [&]() __attribute__((always_inline)) {
-    if constexpr (kBias) {
+  auto take_bias = [&](int nb) __attribute__((always_inline)) {
+    if constexpr (kAhead) {
       bc[0] = bn[0];
       bc[1] = bn[1];
+    } else if constexpr (kBias) {
+      load_p_frags<T>(bc, brow, nb * kBlk, Tk_);
+      if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);  // see kBiasAhead
     }
   };
 
@@ -266,7 +270,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   frag pn[2];
   auto load_tile = [&](int nb) {
     const int n0 = nb * kBlk;
-    if constexpr (kBias) load_p_frags<T>(bn, brow, n0, Tk_);
+    if constexpr (kAhead) load_p_frags<T>(bn, brow, n0, Tk_);
     stage_load_at<T, D>(s0, Kn, a.k.st, Tk_ - n0, scol);
     stage_load_at<T, D>(s1, Vn, a.v.st, Tk_ - n0, scol);
     stage_load_at<T, D>(s2, gKn, a.gk.st, Tk_ - n0, scol);
@@ -280,7 +284,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
   auto dma_tile = [&](int nb, int buf) {
     if constexpr (kDma) {
       const int n0 = nb * kBlk;
-      if constexpr (kBias) load_p_frags<T>(bn, brow, n0, Tk_);
+      if constexpr (kAhead) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
         dd.load_full(sK[buf], Kn, oK);
         dd.load_full(sV[buf], Vn, oV);
@@ -392,7 +396,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     dd.offsets(ogV, a.gv.st);
     auto dma_set = [&](int nb, T* k, T* v, T* gk, T* gv) __attribute__((always_inline)) {
       const int n0 = nb * kBlk;
-      if constexpr (kBias) load_p_frags<T>(bn, brow, n0, Tk_);
+      if constexpr (kAhead) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
         dd.load_full(k, Kn, oK);
         dd.load_full(v, Vn, oV);
@@ -419,7 +423,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       __syncthreads();  // everyone's, and everyone is done with the other set
       Tile p;
       p_from_frags(p);
-      take_bias();
+      take_bias(nb);
       // Keep the conversion ahead of the next tile's loads: sunk below them,
       // it would wait for those loads (vmcnt) before the tile's work.
       __builtin_amdgcn_sched_barrier(0);
@@ -464,7 +468,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       }
       Tile p;
       p_from_frags(p);
-      take_bias();
+      take_bias(nb);
       if (nb + 1 < cr.t1) {
         if constexpr (kDma)
           dma_tile(nb + 1, cur ^ 1);
@@ -601,7 +605,16 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
   constexpr bool kBias = XM == kMaskBias;
   static_assert(!(LOADP && kBias), "a saved P holds the bias");
   const T* bcol = kBias ? at<const T>(a.bias, b, h) + (n < T_ ? n : 0) : nullptr;
+  constexpr bool kAhead = kBias && kBiasAhead<T, D>;
   BiasCol<T> bn, bc;  // bias of the next tile and of this one
+  auto take_bias = [&](int mb) __attribute__((always_inline)) {
+    if constexpr (kAhead) {
+      bc = bn;
+    } else if constexpr (kBias) {
+      bc.load(bcol, a.bias.st, mb * kBlk, Tq_);
+      if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);  // see kBiasAhead
+    }
+  };
 
   const T* Q = at<const T>(a.q, b, h);
   const T* K = at<const T>(a.k, b, h);
@@ -729,7 +742,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     const StatDma<kNS> sdma(rs, ev, fv, lse);
     auto dma_tile = [&](int mb, const Bufs& wb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
-      if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
+      if constexpr (kAhead) bn.load(bcol, a.bias.st, m0, Tq_);
       if (m0 + kBlk <= Tq_ && cols_full) {  // uniform: one test per tile
         dd.load_full(wb.q, Qn, oQ);
         dd.load_full(wb.gq, gQn, ogQ);
@@ -753,7 +766,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       constexpr int P = decltype(par)::value;
       dma_wait();       // this wave's loads of tile mb
       __syncthreads();  // everyone's, and everyone is done with the other set
-      if constexpr (kBias) bc = bn;
+      take_bias(mb);
       if (mb + 1 < cr.t1) dma_tile(mb + 1, bufs(Parity<1 - P>{}));
       compute(mb, bufs(Parity<P>{}));
     };
@@ -769,7 +782,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     float stv;
     auto load_tile = [&](int mb) __attribute__((always_inline)) {
       const int m0 = mb * kBlk;
-      if constexpr (kBias) bn.load(bcol, a.bias.st, m0, Tq_);
+      if constexpr (kAhead) bn.load(bcol, a.bias.st, m0, Tq_);
       stage_load_at<T, D>(s0, Q + (int64_t)m0 * a.q.st, a.q.st, Tq_ - m0, scol);
       stage_load_at<T, D>(s1, gQ + (int64_t)m0 * a.gq.st, a.gq.st, Tq_ - m0, scol);
       stage_load_at<T, D>(s2, dO + (int64_t)m0 * a.dout.st, a.dout.st, Tq_ - m0, scol);
@@ -785,7 +798,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       if constexpr (LOADP) stage_store_rows<T, kBlk>(sp, sP0);
       stat_store<kNS>(stv, sS0);
       __syncthreads();
-      if constexpr (kBias) bc = bn;
+      take_bias(mb);
       if (mb + 1 < cr.t1) load_tile(mb + 1);
       compute(mb, bufs(Parity<0>{}));
     }
