@@ -249,10 +249,9 @@ __host__ __device__ inline Item causal_item(int x, int n, int c) {
 // Mask code of a kernel instantiation (template parameter XM): none, a key
 // window, or an additive bias (with a window or without).  Kernels that read a
 // saved P, which holds the bias already, have no third form.  Separate, the
-// window kernels carry no bias code, and the bias kernels have registers to
-// load a tile's bias with the tile before: added when it was needed, it cost
-// a memory round trip in every tile (b2 h6 d64 fp32, 512 queries of 2048 keys,
-// grad-grad column pass 177 -> 166 us, dK/dV 83 -> 80).
+// window kernels carry no bias code (b8 h6 T8192 d64 bf16 window 512: dK/dV
+// 116 -> 112 us, grad-grad column pass 218 -> 211), and the bias kernels no
+// longer load a tile's bias behind the next tile's operands (kBiasAhead).
 enum : int { kMaskNone = 0, kMaskWindow = 1, kMaskBias = 2 };
 
 // Whether a bias kernel loads a tile's bias one tile ahead (with the next
@@ -267,7 +266,8 @@ enum : int { kMaskNone = 0, kMaskWindow = 1, kMaskBias = 2 };
 // 275 -> 253; b1 h4 T4096 354 -> 333; b2 h4 T1500 d128 fp32 dQ 181 -> 165,
 // the step 1597 -> 1545.  (One loss, from the fill of 512 workgroups: b2 h8
 // T2048 bf16 dK/dV 66 -> 81.)  fp32 D = 64 and 16-bit D = 128 have the
-// registers: 512 queries of 2048 keys fp32 own step -> ahead 459 -> 433.
+// registers: b2 h6 d64 fp32, 512 queries of 2048 keys, loaded where it is
+// added -> ahead: grad-grad column pass 177 -> 166, dK/dV 83 -> 80.
 template <typename T, int D>
 constexpr bool kBiasAhead = (sizeof(T) == 4) == (D == 64);
 
