@@ -281,7 +281,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     if constexpr (!LOADP) {
       p.zero();
       mm_d<M>(p, cK, qf);
-      recompute_p_row<T, kBias>(p, bc, lse2, a.scale_log2);
+      recompute_p_row<T, XM>(p, bc, lse2, a.scale_log2);
     }
     if (mk.tile(nb)) {
 #pragma unroll
@@ -579,7 +579,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
     } else {
       p.zero();
       mm_d<M>(p, cQ, kf);
-      recompute_p_col<T, kBias>(p, bc, cS, kSL, a.scale_log2);
+      recompute_p_col<T, XM>(p, bc, cS, kSL, a.scale_log2);
     }
     if (mk.tile(mb)) {
 #pragma unroll

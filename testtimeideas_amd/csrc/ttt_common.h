@@ -1654,39 +1654,39 @@ __device__ __forceinline__ Parity<1 - P> other_buf(Parity<P>) { return {}; }
 __device__ __forceinline__ RtBuf other_buf(RtBuf b) { return RtBuf{b.cur ^ 1}; }
 
 // ---------------------------------------------------------------------------
-// P = exp2(s*log2e*x [+ bias*log2e] - lse2) from raw scores x of a row-block
-// tile (BIAS: bf, the tile's bias fragments).
-// sl2 converts raw scores to base-2 units: s*log2(e), or log2(e) when the
-// stationary fragments were scaled by s beforehand.
-template <typename T, bool BIAS>
+// Scores x to base-2 units, rounded there: sl2 = s*log2(e), or log2(e) when
+// the stationary fragments were scaled by s beforehand.  Left to contraction,
+// some kernels would fold the product into a later shift and others not, and a
+// window's forward and that of the same mask as a bias would differ.
+__device__ __forceinline__ void scale_scores(Tile& p, float sl2) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
+}
+
+// P = exp2(sl2*x [+ bias*log2e] - lse2) from raw scores x of a row-block tile
+// (bf: the tile's bias fragments, in the bias form XM).
+template <typename T, int XM>
 __device__ __forceinline__ void recompute_p_row(Tile& p, const typename Elem<T>::frag* bf, float lse2, float sl2) {
-  if constexpr (BIAS) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
+  if constexpr (XM == kMaskBias) {
+    scale_scores(p, sl2);
     add_bias_row<T>(p, bf);
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) - lse2));
-    return;
   }
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) * sl2 - lse2));
+    for (int j = 0; j < 8; ++j)
+      p.set(kb, j, fast_exp2(XM == kMaskBias ? p.at(kb, j) - lse2 : p.at(kb, j) * sl2 - lse2));
 }
 
 // The same for a column-block tile: statistic `slot` of sS holds the streamed
 // rows' lse; bv is the tile's bias.
-template <typename T, bool BIAS>
+template <typename T, int XM>
 __device__ __forceinline__ void recompute_p_col(Tile& p, const BiasCol<T>& bv, const float* sS, int slot, float sl2) {
-  if constexpr (BIAS) {
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) p.set(kb, j, p.at(kb, j) * sl2);
+  if constexpr (XM == kMaskBias) {
+    scale_scores(p, sl2);
     bv.add(p);
   }
 #pragma unroll
@@ -1695,7 +1695,7 @@ __device__ __forceinline__ void recompute_p_col(Tile& p, const BiasCol<T>& bv, c
     stat_read8(l2, sS, slot, kb);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      p.set(kb, j, fast_exp2(BIAS ? p.at(kb, j) - l2[j] * kLog2e : p.at(kb, j) * sl2 - l2[j] * kLog2e));
+      p.set(kb, j, fast_exp2(XM == kMaskBias ? p.at(kb, j) - l2[j] * kLog2e : p.at(kb, j) * sl2 - l2[j] * kLog2e));
   }
 }
 

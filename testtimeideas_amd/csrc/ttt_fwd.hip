@@ -17,9 +17,9 @@
 // Causal: key tiles past the diagonal are skipped; the diagonal tile is masked
 // per element (key > query).  A key window also skips the tiles before the
 // block's first visible key and masks the tiles it cuts.  An additive bias is
-// added to the base-2 scores of every tile.  The window and bias code is a
-// separate instantiations (XM, the mask form), so plain problems run the
-// kernels without it.
+// added to the base-2 scores of every tile.  Windows and biases are
+// instantiations of their own (XM, the mask form), so plain problems run the
+// kernels without them.
 // Row blocks are issued heaviest first, and the chunks of a split plain causal
 // launch longest first (launch_item).  Blocks split into several chunks are
 // finished by the combine kernels of ttt_combine.hip.
@@ -67,10 +67,7 @@ __device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds
   mm_d<Mm<T, D>>(s, sK, qf);
   const int n0 = nb * kBlk;
   const bool need_mask = mk.tile(nb);
-#pragma unroll
-  for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s.set(kb, j, s.at(kb, j) * a.scale_log2);
+  scale_scores(s, a.scale_log2);
   if constexpr (XM == kMaskBias) add_bias_row<T>(s, bf);
   if (need_mask) {
 #pragma unroll
@@ -196,14 +193,18 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     }
   };
   // Key tile nb from LDS tiles cK, cV.
-  // Without a bias the scores stay raw (q.k): c = |s|*log2(e) is
+  // Without a window or bias the scores stay raw (q.k): c = |s|*log2(e) is
   // folded into one FMA per element (q negated for a negative scale), and the
   // running shift sh (base 2) moves only when a row's max exceeds it by more
   // than kSlack, so most tiles skip rescaling O and l (then P <= 2^kSlack,
-  // well inside T's range).  Other problems take the scaled form below.
+  // well inside T's range).  Other problems take the scaled form below: in a
+  // window's walk of a few tiles the raw form measured no faster (b8 h6 T8192
+  // d64 bf16 window 512, the step 660 us scaled, 664 us raw), and P <= 2^kSlack
+  // rounds in other places than P <= 1.
+  constexpr bool kRaw = XM == kMaskNone;
   constexpr float kSlack = 8.f;
   float csl = a.scale_log2;
-  if constexpr (!kBias) {
+  if constexpr (kRaw) {
     if (csl < 0.f) {
       csl = -csl;
 #pragma unroll
@@ -227,12 +228,11 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
         for (int j = 0; j < 8; ++j)
           s.set(kb, j, mk.masked(n0 + stream_index(kb, g, j)) ? -INFINITY : s.at(kb, j));
     }
-    // Without a window every row sees a key of every tile of its walk, so tm is
-    // finite; with one it is -inf where a row has seen no key yet.
+    // Every row sees a key of every tile of its walk here, so tm is finite.
     const float tm = tile_max(s) * csl;
     if (__builtin_amdgcn_ballot_w64(tm > sh + kSlack) != 0) {  // uniform
       const float sn = fmaxf(sh, tm);
-      const float alpha = XM == kMaskWindow && sn == -INFINITY ? 1.f : fast_exp2(sh - sn);
+      const float alpha = fast_exp2(sh - sn);
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) acc[i] *= alpha;
@@ -255,7 +255,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
     mm_s<M>(acc, cV, pf);
   };
   auto body = [&](int nb, const lds* cK, const lds* cV) __attribute__((always_inline)) {
-    if constexpr (!kBias) {
+    if constexpr (kRaw) {
       body_raw(nb, cK, cV);
       return;
     }
@@ -338,7 +338,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   }
 
   l = group_sum(l);
-  if constexpr (!kBias) mx = sh;
+  if constexpr (kRaw) mx = sh;
   const int64_t ridx = (int64_t)bh * T_ + m;
   if (cr.nch == 1) {
     if (m < T_ && g == 0) a.lse[ridx] = (mx + __log2f(l)) * kLn2;
@@ -675,6 +675,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
 
   float mx = -INFINITY, l = 0.f;
   const float csl = a.scale_log2;
+  constexpr bool kRaw = XM == kMaskNone;  // as in k_fwd_online
   const bool raw_units = csl > 0.f;  // uniform; the fused form needs a positive scale
   const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stK[R];
@@ -692,7 +693,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
   // One round: key tiles nb .. nb + R - 1 from the LDS tiles tile_k(i).
   auto round = [&](int nb, auto tile_k) __attribute__((always_inline)) {
       Tile s[R];
-      if constexpr (!kBias) {
+      if constexpr (kRaw) {
         if (raw_units) {
           // Max and sum in raw-score units: exp2(raw * csl - max * csl) with the
           // scale csl = scale*log2e > 0 folded into one FMA per element.
@@ -812,7 +813,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       round(nb, [&](int i) -> const lds* { return sK[i]; });
     }
   }
-  if (!kBias && raw_units && mx != -INFINITY) mx *= csl;  // back to base-2 units
+  if (kRaw && raw_units && mx != -INFINITY) mx *= csl;  // back to base-2 units
   {
     // Finite without a window (every row sees a key of its first tile); with
     // one a chunk can miss all of a row's keys, and then max -inf, sum 0.
@@ -971,7 +972,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
   auto body = [&](int nt, const lds* cK, const lds* cV) __attribute__((always_inline)) {
       const int n0 = nt * kBlk;
       mfrag pf[2];
-      if constexpr (!kBias && sizeof(T) == 2) {
+      if constexpr (XM == kMaskNone && sizeof(T) == 2) {
         // Raw scores; P = exp2(raw * scale*log2e - lse) in one FMA, masked
         // entries selected to 0 afterwards, and one rounding to T gives both
         // the MFMA fragment and the stored P.

@@ -314,7 +314,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     if constexpr (!LOADP) {
       p.zero();
       mm_d<M>(p, cK, qf);
-      recompute_p_row<T, kBias>(p, bc, lse2, kSl2);
+      recompute_p_row<T, XM>(p, bc, lse2, kSl2);
     }
     if (mk.tile(nb)) {
 #pragma unroll
@@ -671,7 +671,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     } else {
       p.zero();
       mm_d<M>(p, cb.q, kf);  // -s q.k
-      recompute_p_col<T, kBias>(p, bc, cb.st, 3, -kSl2);
+      recompute_p_col<T, XM>(p, bc, cb.st, 3, -kSl2);
     }
     if (mk.tile(mb)) {
 #pragma unroll
