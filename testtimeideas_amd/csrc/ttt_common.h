@@ -668,19 +668,24 @@ struct Lds {
 // ---------------------------------------------------------------------------
 // fp32 products on the 16-bit matrix cores.  x = h + m + l exactly, each part
 // a bf16 (8 significant bits): h is x truncated, m the rest rounded to
-// nearest, l what is left.  Of the nine products of two split operands the
-// six largest are formed (bf16 products are exact in fp32); the three dropped
-// ones, m*l, l*m and l*l, are below 2^-24 |x y| and of random sign, since m
-// is rounded.  Six v_mfma_f32_16x16x32_bf16 take 96 cycles where the eight
-// v_mfma_f32_16x16x4_f32 of the same product take 256, so the kernels are
-// bound by the VALU work around the products (eleven operations split a pair
-// of values, once per streamed tile and workgroup and once per operand formed
-// in registers), no longer by the products.  An infinite or NaN element gives
-// NaN (inf - inf) where fp32 products could give infinities.
-// Measured against the fp32 products (launch times, us): b8 h6 T1024 d64
-// window 512 O+LSE 63 -> 50, dQ 90 -> 63, dK/dV 120 -> 78, grad-grad row
-// 219 -> 155, column 219 -> 152.  Errors of the seven outputs against 64 bits
-// there: 2.8e-7 .. 8.0e-7 before, 1.3e-7 .. 3.5e-7 now (the sums of mm_tile).
+// nearest, l what is left (|m| < 2^-7 |x|, |l| <= 2^-16 |x|).  Of the nine
+// products of two split operands eight are formed (bf16 products are exact in
+// fp32), the smallest first; l*l, below 2^-31 |x y|, is dropped.  So a single
+// product has one rounding, as in fp32 (simulated, relative r.m.s. 2.5e-8,
+// largest 6.0e-8 both; without m*l and l*m 3.4e-8 and 2.4e-7: those two reach
+// 2^-22 |x y|), and sums of several have fewer.  Parts below 2^-126 are
+// flushed by the matrix cores: an element below 2^-112 loses bits, at most
+// 2^-126 of the other operand.
+// Eight v_mfma_f32_16x16x32_bf16 take 128 cycles where the eight
+// v_mfma_f32_16x16x4_f32 of the same product take 256; eleven VALU operations
+// split a pair of values, once per streamed tile and workgroup and once per
+// operand formed in registers.  An infinite or NaN element gives NaN
+// (inf - inf) where fp32 products could give infinities.
+// Measured (launch times, us): fp32 products -> eight bf16 products (six), b8
+// h6 T1024 d64 window 512: O+LSE 59 -> 50 (46), dQ 85 -> 64 (56), dK/dV
+// 113 -> 78 (70), grad-grad row with GdO 287 -> 216 (192), column 211 -> 153
+// (137).  Errors of the seven outputs against 64 bits there: 2.8e-7 .. 8.0e-7
+// before, 1.3e-7 .. 3.5e-7 now (the sums of mm_tile).
 // ---------------------------------------------------------------------------
 struct SplitFrag {
   bf16x8 h, m, l;
@@ -737,33 +742,22 @@ struct Mm {
   typedef Lds<lds, D> L;
   static constexpr int kElems = (kSplit ? 3 : 1) * L::kRowElems;  // of a tile in LDS
   static constexpr bool kBatch = sizeof(lds) == 2;  // fragment reads issued ahead of their MFMAs
-  static constexpr int kTerms = kSplit ? 6 : 1;
+  static constexpr int kTerms = kSplit ? 8 : 1;
   // Eight elements of row r from column col (mm_d); eight rows from r0 + 8g of
   // column c0 + c (mm_s).
   static __device__ __forceinline__ frag row(const lds* x, int r, int col);
   static __device__ __forceinline__ frag tr(const lds* x, int r0, int c0);
-  // Step t of c + a.b, the smallest parts first.
+  // Step t of c + a.b, the smallest parts first: l.m, m.l, l.h, h.l, m.m, m.h,
+  // h.m, h.h.
   template <int t>
   static __device__ __forceinline__ f32x4 mma(f32x4 c, const frag& a, const frag& b) {
     if constexpr (!kSplit) {
       return Elem<T>::mma(c, a, b);
     } else {
-      const bf16x8& x = t == 0 ? a.l : (t == 2 || t == 3) ? a.m : a.h;
-      const bf16x8& y = t == 1 ? b.l : (t == 2 || t == 4) ? b.m : b.h;
+      const bf16x8& x = (t == 0 || t == 2) ? a.l : (t == 1 || t == 4 || t == 5) ? a.m : a.h;
+      const bf16x8& y = (t == 1 || t == 3) ? b.l : (t == 0 || t == 4 || t == 6) ? b.m : b.h;
       return __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, c, 0, 0, 0);
     }
-  }
-  // Every step (one product by itself).
-  static __device__ __forceinline__ f32x4 mma_all(f32x4 c, const frag& a, const frag& b) {
-    c = mma<0>(c, a, b);
-    if constexpr (kSplit) {
-      c = mma<1>(c, a, b);
-      c = mma<2>(c, a, b);
-      c = mma<3>(c, a, b);
-      c = mma<4>(c, a, b);
-      c = mma<5>(c, a, b);
-    }
-    return c;
   }
   // Fragment from eight elements as loaded, or from eight fp32 values.
   static __device__ __forceinline__ frag from(const typename Elem<T>::frag& f) {
@@ -807,6 +801,8 @@ __device__ __forceinline__ void mma_steps(F&& body) {
     body(std::integral_constant<int, 3>{});
     body(std::integral_constant<int, 4>{});
     body(std::integral_constant<int, 5>{});
+    body(std::integral_constant<int, 6>{});
+    body(std::integral_constant<int, 7>{});
   }
 }
 

@@ -364,8 +364,8 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       z1f[kb] = M::vals(vz1);
       if constexpr (!DQ) z2f[kb] = M::vals(vz2);
       if constexpr (kMfmaSums) {
-        xs4 = M::mma_all(xs4, ones, z1f[kb]);
-        if constexpr (!DQ) ds4 = M::mma_all(ds4, ones, z2f[kb]);
+        xs4 = E::mma(xs4, ones, z1f[kb]);
+        if constexpr (!DQ) ds4 = E::mma(ds4, ones, z2f[kb]);
       }
       pf[kb] = tile_frag<M>(p, kb);
       if constexpr (GDO) z4f[kb] = M::vals(vz4);
