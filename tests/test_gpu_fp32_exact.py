@@ -1,9 +1,12 @@
 """fp32 at head dims up to 64, whose products are formed from bf16 parts: one
-term keeps fp32's relative precision."""
+term keeps fp32's relative precision, and infinities and NaN give what fp32
+products give (the head dim 128 kernels, which form them, on the same operands
+with zero columns behind them)."""
 import pytest
 import torch
 
 from testtimeideas_amd import _lib
+from testtimeideas_amd.ttt_kernels.triton_attention import triton_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -32,3 +35,37 @@ def test_one_term_products():
     assert abs(float(rel.mean())) <= 2.0 ** -24
     # product, scaling, logarithm's sum, scaling back: four roundings and the constants
     assert float(rel.abs().max()) <= 4 * 2.0 ** -24 + 2e-8
+
+
+def _step(xs, causal, mode, scale):
+    q, k, v, do = (x.clone().requires_grad_() for x in xs[:4])
+    o = triton_attention(q, k, v, causal=causal, scale=scale, bwd_mode=mode)
+    first = torch.autograd.grad(o, (q, k, v), do, create_graph=True)
+    return [x.detach() for x in (o, *first, *torch.autograd.grad(first, (q, k, v, do), xs[4:]))]
+
+
+def _same(name, a, b, tol):
+    assert torch.equal(torch.isnan(a), torch.isnan(b)), name
+    assert torch.equal(torch.isinf(a), torch.isinf(b)), name
+    inf = torch.isinf(a)
+    assert torch.equal(a[inf], b[inf]), name
+    fin = torch.isfinite(a)
+    x, y = a[fin].double(), b[fin].double()
+    if x.numel():
+        assert float((x - y).norm()) <= tol * max(float(y.norm()), 1.0), name
+
+
+@pytest.mark.parametrize("which", range(7), ids=["q", "k", "v", "do", "rq", "rk", "rv"])
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("d,causal,mode", [(64, True, "recompute"), (64, False, "save_p")])
+def test_non_finite_operands(which, value, d, causal, mode):
+    t = 150
+    g = torch.Generator().manual_seed(which)
+    xs = [torch.randn((1, 2, t, d), generator=g).cuda() for _ in range(7)]
+    xs[which][0, 1, 70, 3] = value
+    wide = [torch.nn.functional.pad(x, (0, 128 - d)) for x in xs]
+    got = _step(xs, causal, mode, 0.125)
+    want = _step(wide, causal, mode, 0.125)
+    for name, a, b in zip(("o", "dq", "dk", "dv", "gq", "gk", "gv", "gdo"), got, want):
+        _same(name, a[:, 0], b[:, 0, :, :d], 5e-6)  # the untouched slice
+        _same(name, a, b[..., :d], 5e-6)

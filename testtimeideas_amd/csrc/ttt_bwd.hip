@@ -71,7 +71,9 @@ __device__ __forceinline__ void frags_to_tile(Tile& p, const typename Elem<T>::f
 }
 
 // Waves per EU the dQ kernel is compiled for: VGPR accumulators (AccWaves)
-// for the D = 64 recompute variants, and for their 16-bit types a cap of 128
+// for the D = 64 recompute variants and for split products (whose second walk,
+// with AGPR accumulators, takes the kernel past 256 registers), and for the
+// recompute variants' 16-bit types a cap of 128
 // registers, which keeps four waves per SIMD (the window/bias variant sits
 // right at that boundary; at 132 registers it drops to three, measured
 // b8 h6 T8192 d64 bf16 local window 512: dQ 101 -> 113 us).
@@ -82,41 +84,46 @@ struct DqWaves {
   // step): without a register cap the compiler keeps the accumulators in
   // AGPRs and copies them every step.
   static constexpr bool kPar = LOADP && sizeof(T) == 2 && D == 128;
-  static constexpr int value =
-      kVacc ? (sizeof(T) == 2 ? 4 : AccWaves<true>::value) : kPar ? (D == 64 ? 3 : 2) : AccWaves<false>::value;
+  static constexpr int value = kVacc ? (sizeof(T) == 2 ? 4 : AccWaves<true>::value)
+                               : kPar ? (D == 64 ? 3 : 2) : AccWaves<Mm<T, D>::kSplit>::value;
 };
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool LOADP, int XM>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(Params a) {
-  typedef Elem<T> E;
-  typedef typename E::frag frag;
-  typedef Lds<T, D> L;
+// How the dQ kernel holds its tiles, and their sizes in LDS.
+template <typename T, int D, bool LOADP>
+struct DqTiles {
   typedef Mm<T, D> M;
-  typedef typename M::frag mfrag;
-  typedef typename M::lds lds;
   // Saved-P 16-bit tiles stream straight into two LDS buffers per operand
   // (TileDma): with kPar, two sets in distinct arrays with a compile-time role
   // per loop step (so that the current tile's LDS reads need not wait for the
   // next tile's loads), else two buffers of one array picked at run time.
-  constexpr bool kDma = L::kSwizzle && (LOADP || D == 64);
-  constexpr bool kPar = kDma && (D == 128 || !LOADP);
-  constexpr bool kRt = kDma && !kPar;
-  constexpr int kE1 = kPar ? M::kElems : 8, kER = kRt ? M::kElems : 8;
-  __shared__ __align__(16) lds sK0[kRt ? 8 : M::kElems];
-  __shared__ __align__(16) lds sV0[kRt ? 8 : M::kElems];
-  __shared__ __align__(16) lds sK1[kE1];
-  __shared__ __align__(16) lds sV1[kE1];
-  __shared__ __align__(16) lds sKr[kRt ? 2 : 1][kER];
-  __shared__ __align__(16) lds sVr[kRt ? 2 : 1][kER];
+  static constexpr bool kDma = Lds<T, D>::kSwizzle && (LOADP || D == 64);
+  static constexpr bool kPar = kDma && (D == 128 || !LOADP);
+  static constexpr bool kRt = kDma && !kPar;
+  static constexpr int kE0 = kRt ? 8 : M::kElems, kE1 = kPar ? M::kElems : 8, kER = kRt ? M::kElems : 8;
+};
+
+// Row block and chunk of this workgroup, over the LDS tiles of DqTiles.  True:
+// has_nan.
+template <typename M, bool LOADP, int XM>
+__device__ __forceinline__ bool bwd_dq(Params a, typename M::lds* sK0, typename M::lds* sV0,
+                                       typename M::lds* sK1, typename M::lds* sV1, typename M::lds* sKr,
+                                       typename M::lds* sVr) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
+  typedef Elem<T> E;
+  typedef typename E::frag frag;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
+  typedef DqTiles<T, D, LOADP> Tiles;
+  constexpr bool kDma = Tiles::kDma, kPar = Tiles::kPar, kRt = Tiles::kRt;
   auto set_k = [&](auto par) __attribute__((always_inline)) -> lds* {
-    if constexpr (std::is_same_v<decltype(par), RtBuf>) return sKr[par.cur];
+    if constexpr (std::is_same_v<decltype(par), RtBuf>) return sKr + par.cur * M::kElems;
     else if constexpr (decltype(par)::value == 0) return sK0;
     else return sK1;
   };
   auto set_v = [&](auto par) __attribute__((always_inline)) -> lds* {
-    if constexpr (std::is_same_v<decltype(par), RtBuf>) return sVr[par.cur];
+    if constexpr (std::is_same_v<decltype(par), RtBuf>) return sVr + par.cur * M::kElems;
     else if constexpr (decltype(par)::value == 0) return sV0;
     else return sV1;
   };
@@ -126,13 +133,13 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
@@ -243,7 +250,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
     fetch_dma(cr.t0, Parity<0>{});
   else if constexpr (kRt)
     fetch_dma(cr.t0, RtBuf{0});
-  else
+  else if constexpr (M::kPrefetch)
     fetch(cr.t0);
   // Tile nb from buffer set `par`; `prefetch`: 1 fetch tile nb + 1, 2 fetch it
   // if it exists, 0 none.
@@ -253,6 +260,7 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
       dma_wait();       // this wave's loads of tile nb
       __syncthreads();  // everyone's, and everyone is done with the other set
     } else {
+      if constexpr (!M::kPrefetch) fetch(nb);
       __syncthreads();
       stage_store_tile<M>(stK, sK0);
       stage_store_tile<M>(stV, sV0);
@@ -274,8 +282,8 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
       if constexpr (decltype(prefetch)::value == 2)
         if (nb + 1 < cr.t1) fetch_dma(nb + 1, other_buf(par));
     } else {
-      if constexpr (decltype(prefetch)::value == 1) fetch(nb + 1);
-      if constexpr (decltype(prefetch)::value == 2)
+      if constexpr (M::kPrefetch && decltype(prefetch)::value == 1) fetch(nb + 1);
+      if constexpr (M::kPrefetch && decltype(prefetch)::value == 2)
         if (nb + 1 < cr.t1) fetch(nb + 1);
     }
     if constexpr (!LOADP) {
@@ -334,89 +342,104 @@ __attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(
   } else {
     for (int nb = cr.t0; nb < cr.t1; ++nb) tile(nb, Parity<2>{}, Parity<0>{});
   }
+  if (has_nan<M>(0.f, acc)) return true;
   if (cr.nch == 1)
     store_acc_rows<T, D>(at<T>(a.dq, b, h), a.dq.st, m, T_, cols_of<T, D>(a), acc, a.scale);
   else
     store_acc_partial<D>(a.ws_acc + part_index(a, bh, nblk, mb, ch) * kBlk * D, rl, acc);
+  return false;
+}
+
+template <typename T, int D, bool LOADP, int XM>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(DqWaves<T, D, LOADP>::value))) void k_bwd_dq(Params a) {
+  typedef typename Mm<T, D>::lds lds;
+  typedef DqTiles<T, D, LOADP> Tiles;
+  __shared__ __align__(16) lds sK0[Tiles::kE0];
+  __shared__ __align__(16) lds sV0[Tiles::kE0];
+  __shared__ __align__(16) lds sK1[Tiles::kE1];
+  __shared__ __align__(16) lds sV1[Tiles::kE1];
+  __shared__ __align__(16) lds sKr[(Tiles::kRt ? 2 : 1) * Tiles::kER];
+  __shared__ __align__(16) lds sVr[(Tiles::kRt ? 2 : 1) * Tiles::kER];
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return bwd_dq<P, LOADP, XM>(a, tile_as<P>(sK0), tile_as<P>(sV0), tile_as<P>(sK1), tile_as<P>(sV1),
+                                tile_as<P>(sKr), tile_as<P>(sVr));
+  });
 }
 
 // ---------------------------------------------------------------------------
-// Waves per SIMD the dK/dV kernel is compiled for: recompute at D = 64 caps
-// registers for VGPR accumulators; the saved-P 16-bit kernels (direct loads)
+// Waves per SIMD the dK/dV kernel is compiled for: recompute at D = 64 and
+// split products (as DqWaves) cap registers for VGPR accumulators; the saved-P 16-bit kernels (direct loads)
 // for three waves at D = 64 and two at D = 128.
 template <typename T, int D, bool LOADP, bool DV_ONLY>
 struct DkdvWaves {
   static constexpr bool kDma = LOADP && !DV_ONLY && sizeof(T) == 2;
-  static constexpr int value = kDma ? (D == 64 ? 3 : 2) : AccWaves<!LOADP && D == 64>::value;
+  static constexpr int value = kDma ? (D == 64 ? 3 : 2) : AccWaves<(!LOADP && D == 64) || Mm<T, D>::kSplit>::value;
 };
 
-template <typename T, int D, bool LOADP, bool DV_ONLY, int XM>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) void k_bwd_dkdv(Params a, Params dqc,
-                                                                                              int nx) {
-  typedef Elem<T> E;
-  typedef typename E::frag frag;
-  typedef Lds<T, D> L;
+// How the dK/dV kernel holds its tiles, and their sizes in LDS.
+template <typename T, int D, bool LOADP, bool DV_ONLY>
+struct DkdvTiles {
   typedef Mm<T, D> M;
-  typedef typename M::frag mfrag;
-  typedef typename M::lds lds;
   typedef Lds<T, kBlk> LP;
-  constexpr bool kNeedQ = !DV_ONLY || !LOADP;
+  static constexpr bool kNeedQ = !DV_ONLY || !LOADP;
   // Staged row statistics of the streamed tile: D (unless DV_ONLY), then lse
   // (recompute only).
-  constexpr int kNS = (DV_ONLY ? 0 : 1) + (LOADP ? 0 : 1);
-  constexpr int kSD = 0, kSL = DV_ONLY ? 0 : 1;
+  static constexpr int kNS = (DV_ONLY ? 0 : 1) + (LOADP ? 0 : 1);
   // Saved-P 16-bit D = 64 tiles (dO, Q, P and the rowsum slice) stream
   // straight into two LDS buffer sets (TileDma) in distinct arrays with a
   // compile-time role per loop step, so that the current tile's LDS reads
   // need not wait for the next tile's loads.
   // At D = 128 (kMix) P stays staged through registers into one buffer: two
   // sets of all three tiles would need 80 KB of LDS, one workgroup per CU.
-  constexpr bool kDma = !DV_ONLY && L::kSwizzle && (LOADP || D == 64);
-  constexpr bool kMix = kDma && D == 128;
+  static constexpr bool kDma = !DV_ONLY && Lds<T, D>::kSwizzle && (LOADP || D == 64);
+  static constexpr bool kMix = kDma && D == 128;
+  static constexpr int kQE = kNeedQ ? M::kElems : 8, kPE = LOADP ? LP::kRowElems : 8, kSE = kNS > 0 ? kNS * kBlk : 4;
+};
+
+template <typename M>
+struct DkdvBufs {
+  typename M::lds *dout, *q;
+  typename M::T* p;
+  float* st;
+};
+
+// Column block and chunk of this workgroup, over the buffer sets b0 and, for
+// direct loads, b1.  True: has_nan.
+template <typename M, bool LOADP, bool DV_ONLY, int XM>
+__device__ __forceinline__ bool bwd_dkdv(Params a, Slot sl, DkdvBufs<M> b0, DkdvBufs<M> b1) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
+  typedef Elem<T> E;
+  typedef typename E::frag frag;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
+  typedef DkdvTiles<T, D, LOADP, DV_ONLY> Tiles;
+  typedef DkdvBufs<M> Bufs;
+  constexpr bool kNeedQ = Tiles::kNeedQ, kDma = Tiles::kDma, kMix = Tiles::kMix;
+  constexpr int kNS = Tiles::kNS, kSD = 0, kSL = DV_ONLY ? 0 : 1;
   // The next tile's loads are issued after this tile's P reads: issued before
   // them, the compiler waits for the outstanding direct loads before one of
   // those transposed reads.
   constexpr bool kLateFetch = kDma && LOADP;
-  constexpr int kQE = kNeedQ ? M::kElems : 8, kPE = LOADP ? LP::kRowElems : 8, kSE = kNS > 0 ? kNS * kBlk : 4;
-  __shared__ __align__(16) lds sdO0[M::kElems];
-  __shared__ __align__(16) lds sQ0[kQE];
-  __shared__ __align__(16) T sP0[kPE];
-  __shared__ __align__(16) float sS0[kSE];
-  __shared__ __align__(16) lds sdO1[kDma ? M::kElems : 8];
-  __shared__ __align__(16) lds sQ1[kDma ? kQE : 8];
-  __shared__ __align__(16) T sP1[kDma && !kMix ? kPE : 8];
-  __shared__ __align__(16) float sS1[kDma ? kSE : 4];
-  struct Bufs {
-    lds *dout, *q;
-    T* p;
-    float* st;
-  };
   auto bufs = [&](auto par) __attribute__((always_inline)) -> Bufs {
     if constexpr (decltype(par)::value == 0)
-      return Bufs{sdO0, sQ0, sP0, sS0};
+      return b0;
     else
-      return Bufs{sdO1, sQ1, kMix ? sP0 : sP1, sS1};
+      return b1;
   };
 
   const int T_ = a.Tk;  // keys: the stationary rows
   const int Tq_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
-  const Slot sl = grid_slot();
-  // Workgroups past the first nx columns of the grid finish the preceding dQ
-  // launch's split blocks (its partials are complete in stream order), in the
-  // tail of this launch rather than in a launch of their own.
-  if (sl.x >= nx) {
-    combine_sum_block<T, D>(dqc, kOutDQ, sl.x - nx, sl.y);
-    return;
-  }
   const Item it = launch_item<XM>(a, sl.x, nblk);  // causal: column 0 has the most tiles
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int nb = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const Range rg = col_block_range(nb, nblk, Tq_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int n0 = nb * kBlk;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int cl = 16 * w + c;
@@ -524,7 +547,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   };
   if constexpr (kDma)
     dma_tile(cr.t0, Parity<0>{});
-  else
+  else if constexpr (M::kPrefetch)
     load_tile(cr.t0);
   // Tile mb from buffer set `par`; `prefetch`: 1 fetch tile mb + 1, 2 fetch it
   // if it exists, 0 none.
@@ -535,7 +558,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       dma_wait();       // this wave's loads of tile mb
       __syncthreads();  // everyone's; everyone is also done with the other set
       if constexpr (kMix) {
-        stage_store_rows<T, kBlk>(stP, sP0);
+        stage_store_rows<T, kBlk>(stP, b0.p);
         __syncthreads();
       }
       take_bias(mb);
@@ -545,15 +568,16 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
           if (mb + 1 < cr.t1) dma_tile(mb + 1, Parity<1 - P>{});
       }
     } else {
+      if constexpr (!M::kPrefetch) load_tile(mb);
       __syncthreads();
-      stage_store_tile<M>(stdO, sdO0);
-      if constexpr (kNeedQ) stage_store_tile<M>(stQ, sQ0);
-      if constexpr (LOADP) stage_store_rows<T, kBlk>(stP, sP0);
-      if constexpr (kNS > 0) stat_store<kNS>(stv, sS0);
+      stage_store_tile<M>(stdO, b0.dout);
+      if constexpr (kNeedQ) stage_store_tile<M>(stQ, b0.q);
+      if constexpr (LOADP) stage_store_rows<T, kBlk>(stP, b0.p);
+      if constexpr (kNS > 0) stat_store<kNS>(stv, b0.st);
       __syncthreads();
       take_bias(mb);
-      if constexpr (decltype(prefetch)::value == 1) load_tile(mb + 1);
-      if constexpr (decltype(prefetch)::value == 2)
+      if constexpr (M::kPrefetch && decltype(prefetch)::value == 1) load_tile(mb + 1);
+      if constexpr (M::kPrefetch && decltype(prefetch)::value == 2)
         if (mb + 1 < cr.t1) load_tile(mb + 1);
     }
     const Bufs cb = bufs(par);
@@ -621,6 +645,7 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
   } else {
     for (int mb = cr.t0; mb < cr.t1; ++mb) tile(mb, Parity<2>{}, Parity<0>{});
   }
+  if (has_nan<M>(0.f, acc_dv, acc_dk)) return true;
   if (cr.nch == 1) {
     store_acc_rows<T, D>(at<T>(a.dv, b, h), a.dv.st, n, T_, cols_of<T, D>(a), acc_dv, 1.f);
     if constexpr (!DV_ONLY) store_acc_rows<T, D>(at<T>(a.dk, b, h), a.dk.st, n, T_, cols_of<T, D>(a), acc_dk, -a.scale);
@@ -633,19 +658,50 @@ __attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) voi
       store_acc_partial<D>(base + kBlk * D, cl, acc_dk);
     }
   }
+  return false;
+}
+
+template <typename T, int D, bool LOADP, bool DV_ONLY, int XM>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(DkdvWaves<T, D, LOADP, DV_ONLY>::value))) void k_bwd_dkdv(Params a, Params dqc,
+                                                                                              int nx) {
+  typedef Mm<T, D> M;
+  typedef typename M::lds lds;
+  typedef DkdvTiles<T, D, LOADP, DV_ONLY> Tiles;
+  constexpr bool kDma = Tiles::kDma, kMix = Tiles::kMix;
+  __shared__ __align__(16) lds sdO0[M::kElems];
+  __shared__ __align__(16) lds sQ0[Tiles::kQE];
+  __shared__ __align__(16) T sP0[Tiles::kPE];
+  __shared__ __align__(16) float sS0[Tiles::kSE];
+  __shared__ __align__(16) lds sdO1[kDma ? M::kElems : 8];
+  __shared__ __align__(16) lds sQ1[kDma ? Tiles::kQE : 8];
+  __shared__ __align__(16) T sP1[kDma && !kMix ? Tiles::kPE : 8];
+  __shared__ __align__(16) float sS1[kDma ? Tiles::kSE : 4];
+  // Workgroups past the first nx columns of the grid finish the preceding dQ
+  // launch's split blocks (its partials are complete in stream order), in the
+  // tail of this launch rather than in a launch of their own.
+  const Slot sl = grid_slot();
+  if (sl.x >= nx) {
+    combine_sum_block<T, D>(dqc, kOutDQ, sl.x - nx, sl.y);
+    return;
+  }
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return bwd_dkdv<P, LOADP, DV_ONLY, XM>(a, sl, DkdvBufs<P>{tile_as<P>(sdO0), tile_as<P>(sQ0), sP0, sS0},
+                                           DkdvBufs<P>{tile_as<P>(sdO1), tile_as<P>(sQ1), kMix ? sP0 : sP1, sS1});
+  });
 }
 
 // ---------------------------------------------------------------------------
 // rowsum[m] = sum_n P[m,n] * (dO*V^T)[m,n]; causal skips tiles past the
 // diagonal (they hold zeros in the math path).
-template <typename T, int D, int XM>
-__global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
+template <typename M, int XM>
+__device__ __forceinline__ bool bwd_rowsum(Params a, typename M::lds* sV) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
   typedef Elem<T> E;
   typedef typename E::frag frag;
-  typedef Mm<T, D> M;
   typedef typename M::frag mfrag;
-  typedef typename M::lds lds;
-  __shared__ __align__(16) lds sV[M::kElems];
 
   const int T_ = a.T;
   const Slot sl = grid_slot();
@@ -697,7 +753,19 @@ __global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
       for (int j = 0; j < 8; ++j) sum += p.at(kb, j) * dp.at(kb, j);
   }
   sum = group_sum(sum);
+  if (has_nan<M>(sum)) return true;
   if (row_ok && g == 0) a.rowsum_out[(int64_t)bh * T_ + m] = sum;
+  return false;
+}
+
+template <typename T, int D, int XM>
+__global__ __launch_bounds__(kThreads) void k_bwd_rowsum(Params a) {
+  typedef Mm<T, D> M;
+  __shared__ __align__(16) typename M::lds sV[M::kElems];
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return bwd_rowsum<P, XM>(a, tile_as<P>(sV));
+  });
 }
 
 // ---------------------------------------------------------------------------

@@ -679,8 +679,10 @@ struct Lds {
 // Eight v_mfma_f32_16x16x32_bf16 take 128 cycles where the eight
 // v_mfma_f32_16x16x4_f32 of the same product take 256; eleven VALU operations
 // split a pair of values, once per streamed tile and workgroup and once per
-// operand formed in registers.  An infinite or NaN element gives NaN
-// (inf - inf) where fp32 products could give infinities.
+// operand formed in registers.  An infinite element's parts are NaN
+// (inf - inf), as are the sums of products past the largest float, so a
+// workgroup whose results hold a NaN forms them again from fp32 products
+// (repeat_unsplit).
 // Measured (launch times, us): fp32 products -> eight bf16 products (six), b8
 // h6 T1024 d64 window 512: O+LSE 59 -> 50 (46), dQ 85 -> 64 (56), dK/dV
 // 113 -> 78 (70), grad-grad row with GdO 287 -> 216 (192), column 211 -> 153
@@ -725,24 +727,28 @@ __device__ __forceinline__ SplitFrag split8(const float* v) {
 // Operands of the tile products of element type T_ at head dim D_: the type of
 // an MFMA fragment (eight k-slots of one lane), how a streamed tile lies in
 // LDS, and the product, in kTerms steps.  16-bit types, and fp32 at D = 128:
-// the elements themselves.  kSplit (fp32 at D = 64): three bf16 planes, each in
-// the 16-bit layout.  At D = 128 the grad-grad kernels do not fit (the row
+// the elements themselves.  SPLIT (fp32 at D = 64; without it only where a
+// result came out NaN, see repeat_unsplit): three bf16 planes, each in the
+// 16-bit layout.  At D = 128 the grad-grad kernels do not fit (the row
 // kernel's four streamed tiles would take 192 KB of LDS, and split fragments
 // spill 560-1400 bytes per lane), and every kernel of a step must form its
 // scores the same way: with the forward and first backward split alone (5 to
 // 30 % faster) a one-key row's recomputed P misses 1 by the difference, and GK
 // went past 1e-5 there.
-template <typename T_, int D_>
+template <typename T_, int D_, bool SPLIT = std::is_same_v<T_, float> && D_ == 64>
 struct Mm {
   typedef T_ T;
   static constexpr int D = D_;
-  static constexpr bool kSplit = std::is_same_v<T, float> && D == 64;
+  static constexpr bool kSplit = SPLIT;
   typedef std::conditional_t<kSplit, SplitFrag, typename Elem<T>::frag> frag;
   typedef std::conditional_t<kSplit, __bf16, T> lds;
   typedef Lds<lds, D> L;
   static constexpr int kElems = (kSplit ? 3 : 1) * L::kRowElems;  // of a tile in LDS
   static constexpr bool kBatch = sizeof(lds) == 2;  // fragment reads issued ahead of their MFMAs
   static constexpr int kTerms = kSplit ? 8 : 1;
+  // The second walk loads each tile when it comes to it: nothing is prefetched,
+  // and the kernel needs no more registers than its first walk.
+  static constexpr bool kPrefetch = kSplit || !(std::is_same_v<T, float> && D == 64);
   // Eight elements of row r from column col (mm_d); eight rows from r0 + 8g of
   // column c0 + c (mm_s).
   static __device__ __forceinline__ frag row(const lds* x, int r, int col);
@@ -788,6 +794,49 @@ struct Mm {
       asm volatile("" : "+v"(f));
   }
 };
+
+// A kernel's work, walk(M), which returns whether a result came out NaN
+// (has_nan): where split products did that, an infinity or an overflow among
+// the operands may have no NaN in fp32, so the workgroup walks its tiles again
+// with fp32 products, over the same LDS.  The test and the larger kernels cost
+// 1 to 2 % (b8 h6 T1024 window 512 in a layer 1598 -> 1611 us, b2 h6 512
+// queries of 2048 keys with a mask 484 -> 494 us); a row that sees no key at
+// all, whose gradients are NaN, walks twice.
+template <typename T, int D, typename F>
+__device__ __forceinline__ void repeat_unsplit(F&& walk) {
+  typedef Mm<T, D> M;
+  const bool again = walk(M{});
+  if constexpr (M::kSplit) {
+    if (__builtin_expect(again, 0)) walk(Mm<T, D, false>{});
+  }
+}
+
+// An LDS tile of the kernel's main products as one of M's.
+template <typename M, typename E>
+__device__ __forceinline__ typename M::lds* tile_as(E* x) {
+  static_assert(std::is_same_v<E, typename M::lds> ||
+                M::kElems * sizeof(typename M::lds) <= Mm<typename M::T, M::D>::kElems * sizeof(E));
+  return reinterpret_cast<typename M::lds*>(x);
+}
+
+// Whether any lane of the workgroup holds a NaN in the sums of acc (16-bit
+// types and fp32 products: false, without looking).  Sums that are NaN for
+// another reason (infinities of both signs) only cost a second walk.
+template <int N>
+__device__ __forceinline__ float sum_of(const f32x4 (&acc)[N]) {
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) s += (acc[i][0] + acc[i][1]) + (acc[i][2] + acc[i][3]);
+  return s;
+}
+template <typename M, int... N>
+__device__ __forceinline__ bool has_nan(float x, const f32x4 (&... acc)[N]) {
+  if constexpr (M::kSplit) {
+    x = (x + ... + sum_of(acc));
+    return __syncthreads_or(x != x);
+  }
+  return false;
+}
 
 // Runs body(std::integral_constant<int, t>) for the steps t of M's product:
 // with the independent accumulators inside, consecutive MFMAs do not wait for
@@ -1078,8 +1127,8 @@ __device__ __forceinline__ typename Elem<T>::frag load_frag_tr(const T* X, int r
   return f;
 }
 
-template <typename T_, int D_>
-__device__ __forceinline__ typename Mm<T_, D_>::frag Mm<T_, D_>::row(const lds* x, int r, int col) {
+template <typename T_, int D_, bool SPLIT>
+__device__ __forceinline__ typename Mm<T_, D_, SPLIT>::frag Mm<T_, D_, SPLIT>::row(const lds* x, int r, int col) {
   const lds* p = x + L::off(r, col);
   if constexpr (kSplit)
     return SplitFrag{load_frag<lds>(p), load_frag<lds>(p + L::kRowElems), load_frag<lds>(p + 2 * L::kRowElems)};
@@ -1087,8 +1136,8 @@ __device__ __forceinline__ typename Mm<T_, D_>::frag Mm<T_, D_>::row(const lds* 
     return load_frag<lds>(p);
 }
 
-template <typename T_, int D_>
-__device__ __forceinline__ typename Mm<T_, D_>::frag Mm<T_, D_>::tr(const lds* x, int r0, int c0) {
+template <typename T_, int D_, bool SPLIT>
+__device__ __forceinline__ typename Mm<T_, D_, SPLIT>::frag Mm<T_, D_, SPLIT>::tr(const lds* x, int r0, int c0) {
   if constexpr (kSplit)
     return SplitFrag{load_frag_tr<lds, D>(x, r0, c0), load_frag_tr<lds, D>(x + L::kRowElems, r0, c0),
                      load_frag_tr<lds, D>(x + 2 * L::kRowElems, r0, c0)};

@@ -57,14 +57,14 @@ namespace ttt {
 
 // Scores of key tile nb (rows sK) for query row m, in base-2 units; masked
 // entries are -inf.  bf: the tile's bias fragments (kMaskBias).
-template <typename T, int D, int XM>
-__device__ __forceinline__ void fwd_scores(Tile& s, const typename Mm<T, D>::lds* sK,
-                                           const typename Mm<T, D>::frag* qf, const Params& a,
-                                           const RowMask<XM != kMaskNone>& mk, const typename Elem<T>::frag* bf,
-                                           int nb) {
+template <typename M, int XM>
+__device__ __forceinline__ void fwd_scores(Tile& s, const typename M::lds* sK, const typename M::frag* qf,
+                                           const Params& a, const RowMask<XM != kMaskNone>& mk,
+                                           const typename Elem<typename M::T>::frag* bf, int nb) {
+  typedef typename M::T T;
   const int g = (threadIdx.x & 63) >> 4;
   s.zero();
-  mm_d<Mm<T, D>>(s, sK, qf);
+  mm_d<M>(s, sK, qf);
   const int n0 = nb * kBlk;
   const bool need_mask = mk.tile(nb);
   scale_scores(s, a.scale_log2);
@@ -112,13 +112,16 @@ __device__ __forceinline__ float tile_max(const Tile& s) {
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, int XM>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Params a) {
+// Row block and chunk of this workgroup, over the LDS tiles sK, sV and, for
+// direct loads, the second set sK1, sV1.  True: has_nan.
+template <typename M, int XM>
+__device__ __forceinline__ bool fwd_online(Params a, typename M::lds* sK, typename M::lds* sV,
+                                           typename M::lds* sK1, typename M::lds* sV1) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
-  typedef Mm<T, D> M;
   typedef typename M::frag mfrag;
   typedef typename M::lds lds;
   // 16-bit tiles stream straight into two LDS buffer sets (TileDma) in
@@ -127,23 +130,19 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
   // workgroups per CU instead of three) and still measured faster: b4 h16
   // T8192 bf16 causal -9 %, b2 h4 T2048 fp16 -19 %.
   constexpr bool kDma = L::kSwizzle;
-  __shared__ __align__(16) lds sK[M::kElems];
-  __shared__ __align__(16) lds sV[M::kElems];
-  __shared__ __align__(16) lds sK1[kDma ? M::kElems : 8];
-  __shared__ __align__(16) lds sV1[kDma ? M::kElems : 8];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;  // row within the block
   const int m = mb * kBlk + rl;
@@ -260,7 +259,7 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       return;
     }
     Tile s;
-    fwd_scores<T, D, XM>(s, cK, qf, a, mk, bc, nb);
+    fwd_scores<M, XM>(s, cK, qf, a, mk, bc, nb);
     const float mnew = fmaxf(mx, tile_max(s));
     // A window can mask a row's every key of a tile so far: shift by 0 then.
     const float msh = (mnew == -INFINITY) ? 0.f : mnew;
@@ -325,20 +324,23 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       if (nb + 1 < cr.t1) step(Parity<1>{}, nb + 1);
     }
   } else {
-    load_kv(cr.t0);
+    if constexpr (M::kPrefetch) load_kv(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
+      if constexpr (!M::kPrefetch) load_kv(nb);
       __syncthreads();
       stage_store_tile<M>(stK, sK);
       stage_store_tile<M>(stV, sV);
       __syncthreads();
       take_bias(nb);
-      if (nb + 1 < cr.t1) load_kv(nb + 1);
+      if constexpr (M::kPrefetch)
+        if (nb + 1 < cr.t1) load_kv(nb + 1);
       body(nb, sK, sV);
     }
   }
 
   l = group_sum(l);
   if constexpr (kRaw) mx = sh;
+  if (has_nan<M>(l, acc)) return true;
   const int64_t ridx = (int64_t)bh * T_ + m;
   if (cr.nch == 1) {
     if (m < T_ && g == 0) a.lse[ridx] = (mx + __log2f(l)) * kLn2;
@@ -351,6 +353,22 @@ __attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Pa
       a.ws_sc[part * 2 * kBlk + kBlk + rl] = l;
     }
   }
+  return false;
+}
+
+template <typename T, int D, int XM>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(AccWaves<true>::value))) void k_fwd_online(Params a) {
+  typedef Mm<T, D> M;
+  constexpr int kE1 = Lds<T, D>::kSwizzle ? M::kElems : 8;
+  __shared__ __align__(16) typename M::lds sK[M::kElems];
+  __shared__ __align__(16) typename M::lds sV[M::kElems];
+  __shared__ __align__(16) typename M::lds sK1[kE1];
+  __shared__ __align__(16) typename M::lds sV1[kE1];
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return fwd_online<P, XM>(a, tile_as<P>(sK), tile_as<P>(sV), tile_as<P>(sK1), tile_as<P>(sV1));
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -624,40 +642,42 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(D == 6
 // ---------------------------------------------------------------------------
 // Waves per SIMD the statistics and P passes are compiled for: their 16-bit
 // D = 64 two-set forms (two steps per loop iteration) without a register cap
-// keep their MFMA results in AGPRs and copy them every step.
+// keep their MFMA results in AGPRs and copy them every step; split products
+// would go past 256 registers (as in DqWaves).
 template <typename T, int D>
 struct FwdPWaves {
-  static constexpr int value = sizeof(T) == 2 ? (D == 64 ? 3 : 2) : AccWaves<false>::value;
+  static constexpr int value = sizeof(T) == 2 ? (D == 64 ? 3 : 2) : AccWaves<Mm<T, D>::kSplit>::value;
 };
 
-template <typename T, int D, int XM>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Params a) {
+// R key tiles per round: one pair of barriers and R independent score
+// products per round.
+constexpr int kStatTiles = 2;
+
+// Over R tiles from sK and, for direct loads, the second set from sK1.  True:
+// has_nan.
+template <typename M, int XM>
+__device__ __forceinline__ bool fwd_stats(Params a, typename M::lds* sK, typename M::lds* sK1) {
+  typedef typename M::T T;
+  constexpr int D = M::D, R = kStatTiles;
   typedef Lds<T, D> L;
-  typedef Mm<T, D> M;
   typedef typename M::frag mfrag;
   typedef typename M::lds lds;
-  // R key tiles per round: one pair of barriers and R independent score
-  // products per round.
-  constexpr int R = 2;
   // 16-bit types: the R tiles of a round stream straight into LDS (TileDma),
   // alternating between two sets in distinct arrays with compile-time roles.
   constexpr bool kDma = L::kSwizzle;
-  __shared__ __align__(16) lds sK[R][M::kElems];
-  __shared__ __align__(16) lds sK1[R][kDma ? M::kElems : 8];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
@@ -736,7 +756,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       for (int i = 0; i < R; ++i) {
         typename Elem<T>::frag bf[2];
         if constexpr (kBias) load_p_frags<T>(bf, brow, (nb + i) * kBlk, Tk_);
-        fwd_scores<T, D, XM>(s[i], tile_k(i), qf, a, mk, bf, nb + i);
+        fwd_scores<M, XM>(s[i], tile_k(i), qf, a, mk, bf, nb + i);
         if (i > 0 && nb + i >= cr.t1) {
   #pragma unroll
           for (int kb = 0; kb < 2; ++kb)
@@ -775,7 +795,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         const int n1 = (nb + i < cr.t1 ? nb + i : cr.t1 - 1) * kBlk;
-        T* dst = decltype(par)::value == 0 ? sK[i] : sK1[i];
+        T* dst = (decltype(par)::value == 0 ? sK : sK1) + i * M::kElems;
         const T* kp = K + (int64_t)n1 * a.k.st;
         if (n1 + kBlk <= Tk_) {
           dd.load_full(dst, kp, oK);
@@ -791,7 +811,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       dma_wait();       // this wave's loads of round nb
       __syncthreads();  // everyone's, and everyone is done with the other set
       if (nb + R < cr.t1) fetch_set(nb + R, Parity<1 - P>{});
-      round(nb, [&](int i) -> const lds* { return P == 0 ? sK[i] : sK1[i]; });
+      round(nb, [&](int i) -> const lds* { return (P == 0 ? sK : sK1) + i * M::kElems; });
     };
     fetch_set(cr.t0, Parity<0>{});
     for (int nb = cr.t0; nb < cr.t1; nb += 2 * R) {
@@ -799,18 +819,20 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
       if (nb + R < cr.t1) step(Parity<1>{}, nb + R);
     }
   } else {
+    auto load_round = [&](int nb) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < R; ++i) load_k(cr.t0 + i, stK[i]);
+      for (int i = 0; i < R; ++i) load_k(nb + i, stK[i]);
+    };
+    if constexpr (M::kPrefetch) load_round(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; nb += R) {
+      if constexpr (!M::kPrefetch) load_round(nb);
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < R; ++i) stage_store_tile<M>(stK[i], sK[i]);
+      for (int i = 0; i < R; ++i) stage_store_tile<M>(stK[i], sK + i * M::kElems);
       __syncthreads();
-      if (nb + R < cr.t1) {
-#pragma unroll
-        for (int i = 0; i < R; ++i) load_k(nb + R + i, stK[i]);
-      }
-      round(nb, [&](int i) -> const lds* { return sK[i]; });
+      if constexpr (M::kPrefetch)
+        if (nb + R < cr.t1) load_round(nb + R);
+      round(nb, [&](int i) -> const lds* { return sK + i * M::kElems; });
     }
   }
   if (kRaw && raw_units && mx != -INFINITY) mx *= csl;  // back to base-2 units
@@ -821,7 +843,8 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
     l = group_sum(l * fast_exp2(mx - ((XM != kMaskNone && mrow == -INFINITY) ? 0.f : mrow)));
     mx = mrow;
   }
-  if (g != 0) return;
+  if (has_nan<M>(l)) return true;
+  if (g != 0) return false;
   if (cr.nch == 1) {
     if (m < T_) a.lse[(int64_t)bh * T_ + m] = (mx + __log2f(l)) * kLn2;
   } else {
@@ -829,6 +852,19 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Pa
     a.ws_sc[part * 2 * kBlk + rl] = mx;
     a.ws_sc[part * 2 * kBlk + kBlk + rl] = l;
   }
+  return false;
+}
+
+template <typename T, int D, int XM>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_stats(Params a) {
+  typedef Mm<T, D> M;
+  __shared__ __align__(16) typename M::lds sK[kStatTiles * M::kElems];
+  __shared__ __align__(16) typename M::lds sK1[Lds<T, D>::kSwizzle ? kStatTiles * M::kElems : 8];
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return fwd_stats<P, XM>(a, tile_as<P>(sK), tile_as<P>(sK1));
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -873,36 +909,34 @@ __device__ __forceinline__ float p_pass_lse2(const Params& a, int bh, int nblk, 
   return lse2;
 }
 
-template <typename T, int D, int XM>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params a) {
+// LDS tiles and result as fwd_online's.
+template <typename M, int XM>
+__device__ __forceinline__ bool fwd_p(Params a, typename M::lds* sK, typename M::lds* sV,
+                                      typename M::lds* sK1, typename M::lds* sV1) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
   typedef Elem<T> E;
   typedef typename E::frag frag;
   typedef Lds<T, D> L;
-  typedef Mm<T, D> M;
   typedef typename M::frag mfrag;
   typedef typename M::lds lds;
   // 16-bit tiles stream straight into two LDS buffer sets (TileDma) in
   // distinct arrays with a compile-time role per loop step, one tile per
   // barrier round; fp32 tiles are staged through registers.
   constexpr bool kDma = L::kSwizzle;
-  __shared__ __align__(16) lds sK[M::kElems];
-  __shared__ __align__(16) lds sV[M::kElems];
-  __shared__ __align__(16) lds sK1[kDma ? M::kElems : 8];
-  __shared__ __align__(16) lds sV1[kDma ? M::kElems : 8];
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
@@ -1029,7 +1063,7 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
         Tile s;
         frag bf[2];
         if constexpr (kBias) load_p_frags<T>(bf, brow, n0, Tk_);
-        fwd_scores<T, D, XM>(s, cK, qf, a, mk, bf, nt);
+        fwd_scores<M, XM>(s, cK, qf, a, mk, bf, nt);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
           float pv[8];
@@ -1100,21 +1134,40 @@ __attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params
     }
     flush();
   } else {
-    load_kv(cr.t0);
+    if constexpr (M::kPrefetch) load_kv(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
+      if constexpr (!M::kPrefetch) load_kv(nb);
       __syncthreads();
       stage_store_tile<M>(stK, sK);
       stage_store_tile<M>(stV, sV);
       __syncthreads();
-      if (nb + 1 < cr.t1) load_kv(nb + 1);
+      if constexpr (M::kPrefetch)
+        if (nb + 1 < cr.t1) load_kv(nb + 1);
       body(nb, sK, sV);
     }
   }
+  if (has_nan<M>(0.f, acc)) return true;
   if (cr.nch == 1) {
     store_acc_rows<T, D>(at<T>(a.o, b, h), a.o.st, m, T_, cols_of<T, D>(a), acc, 1.f);
   } else {
     store_acc_partial<D>(a.ws_acc + part_index(a, bh, nblk, mb, ch) * kBlk * D, rl, acc);
   }
+  return false;
+}
+
+template <typename T, int D, int XM>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(FwdPWaves<T, D>::value))) void k_fwd_p(Params a) {
+  typedef Mm<T, D> M;
+  constexpr int kE1 = Lds<T, D>::kSwizzle ? M::kElems : 8;
+  __shared__ __align__(16) typename M::lds sK[M::kElems];
+  __shared__ __align__(16) typename M::lds sV[M::kElems];
+  __shared__ __align__(16) typename M::lds sK1[kE1];
+  __shared__ __align__(16) typename M::lds sV1[kE1];
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return fwd_p<P, XM>(a, tile_as<P>(sK), tile_as<P>(sV), tile_as<P>(sK1), tile_as<P>(sV1));
+  });
 }
 
 // ---------------------------------------------------------------------------

@@ -134,54 +134,57 @@ struct GgWaves {
 };
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool LOADP, bool GDO, int XM, bool DQ>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params a) {
-  typedef Elem<T> E;
-  typedef typename E::frag frag;
-  typedef Lds<T, D> L;
+// How the row kernel holds its tiles, and their sizes in LDS.
+template <typename T, int D, bool GDO>
+struct GgRowTiles {
   typedef Mm<T, D> M;
-  typedef typename M::frag mfrag;
-  typedef typename M::lds lds;
-  static_assert(!(DQ && GDO), "the dQ form has no GdO variant");
-  // split partials: dS*gK + Z1*K, Z2*K, P*K (+ P*gV + (P o gdS)*V, P*V), the
-  // dQ form without Z2*K; row sums E, X and rowsum(Z2) (dQ form: X in fp32)
-  constexpr int NACC = DQ ? 2 : GDO ? 5 : 3;
   // 16-bit types stream tiles straight into LDS (TileDma), into two buffer
   // sets in distinct arrays with a compile-time role per loop step (kPar), so
   // that the current tile's LDS reads need not wait for the next tile's loads;
   // the D = 64 GdO variants into two buffers of one array per operand, picked
   // at run time.  The rest stage tiles through registers into one buffer.
-  constexpr bool kPar = L::kSwizzle && (D == 128 || !GDO);
-  constexpr bool kDma = L::kSwizzle && D == 64 && !kPar;
-  constexpr int kBuf = kDma ? 2 : 1;
-  constexpr int kE = kPar ? 8 : M::kElems;  // the run-time-indexed arrays (unused with kPar)
-  __shared__ __align__(16) lds sK[kBuf][kE];
-  __shared__ __align__(16) lds sV[kBuf][kE];
-  __shared__ __align__(16) lds sgK[kBuf][kE];
-  __shared__ __align__(16) lds sgV[kBuf][kE];
-  constexpr int kPE = kPar ? M::kElems : 8;
-  __shared__ __align__(16) lds pK0[kPE];
-  __shared__ __align__(16) lds pV0[kPE];
-  __shared__ __align__(16) lds pgK0[kPE];
-  __shared__ __align__(16) lds pgV0[kPE];
-  __shared__ __align__(16) lds pK1[kPE];
-  __shared__ __align__(16) lds pV1[kPE];
-  __shared__ __align__(16) lds pgK1[kPE];
-  __shared__ __align__(16) lds pgV1[kPE];
+  static constexpr bool kPar = Lds<T, D>::kSwizzle && (D == 128 || !GDO);
+  static constexpr bool kDma = Lds<T, D>::kSwizzle && D == 64 && !kPar;
+  static constexpr int kBuf = kDma ? 2 : 1;
+  static constexpr int kE = kPar ? 8 : M::kElems;   // of a run-time-indexed buffer (unused with kPar)
+  static constexpr int kPE = kPar ? M::kElems : 8;  // of a tile of the two sets
+};
+
+template <typename L>
+struct GgRowSet {
+  L *k, *v, *gk, *gv;
+};
+
+// Row block and chunk of this workgroup, over the run-time-indexed buffers sr
+// and the sets p0 and p1 of GgRowTiles.  True: has_nan.
+template <typename M, bool LOADP, bool GDO, int XM, bool DQ>
+__device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
+                                       GgRowSet<typename M::lds> p0, GgRowSet<typename M::lds> p1) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
+  typedef Elem<T> E;
+  typedef typename E::frag frag;
+  typedef typename M::frag mfrag;
+  typedef typename M::lds lds;
+  typedef GgRowTiles<T, D, GDO> Tiles;
+  constexpr bool kPar = Tiles::kPar, kDma = Tiles::kDma;
+  static_assert(!(DQ && GDO), "the dQ form has no GdO variant");
+  // split partials: dS*gK + Z1*K, Z2*K, P*K (+ P*gV + (P o gdS)*V, P*V), the
+  // dQ form without Z2*K; row sums E, X and rowsum(Z2) (dQ form: X in fp32)
+  constexpr int NACC = DQ ? 2 : GDO ? 5 : 3;
 
   const int T_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
   const int Tk_ = a.Tk, nkb = (Tk_ + kBlk - 1) / kBlk;  // keys
   const Slot sl = grid_slot();
   const Item it = launch_item<XM>(a, sl.x, nblk);
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int bi = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const int mb = a.causal ? (nblk - 1 - bi) : bi;
   const Range rg = row_block_range(mb, nkb, T_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int rl = 16 * w + c;
   const int m = mb * kBlk + rl;
@@ -286,19 +289,19 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       const int n0 = nb * kBlk;
       if constexpr (kAhead) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
-        dd.load_full(sK[buf], Kn, oK);
-        dd.load_full(sV[buf], Vn, oV);
-        dd.load_full(sgK[buf], gKn, ogK);
-        dd.load_full(sgV[buf], gVn, ogV);
+        dd.load_full(sr.k + buf * M::kElems, Kn, oK);
+        dd.load_full(sr.v + buf * M::kElems, Vn, oV);
+        dd.load_full(sr.gk + buf * M::kElems, gKn, ogK);
+        dd.load_full(sr.gv + buf * M::kElems, gVn, ogV);
         if constexpr (LOADP) {
           pn[0] = load_frag_g<T>(Pn);
           pn[1] = load_frag_g<T>(Pn + 32);
         }
       } else {
-        dd.load_ragged(sK[buf], Kn, a.k.st, Tk_ - n0, D);
-        dd.load_ragged(sV[buf], Vn, a.v.st, Tk_ - n0, D);
-        dd.load_ragged(sgK[buf], gKn, a.gk.st, Tk_ - n0, D);
-        dd.load_ragged(sgV[buf], gVn, a.gv.st, Tk_ - n0, D);
+        dd.load_ragged(sr.k + buf * M::kElems, Kn, a.k.st, Tk_ - n0, D);
+        dd.load_ragged(sr.v + buf * M::kElems, Vn, a.v.st, Tk_ - n0, D);
+        dd.load_ragged(sr.gk + buf * M::kElems, gKn, a.gk.st, Tk_ - n0, D);
+        dd.load_ragged(sr.gv + buf * M::kElems, gVn, a.gv.st, Tk_ - n0, D);
         if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, Tk_);
         dma_wait();
       }
@@ -394,23 +397,23 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
     dd.offsets(oV, a.v.st);
     dd.offsets(ogK, a.gk.st);
     dd.offsets(ogV, a.gv.st);
-    auto dma_set = [&](int nb, T* k, T* v, T* gk, T* gv) __attribute__((always_inline)) {
+    auto dma_set = [&](int nb, const GgRowSet<T>& to) __attribute__((always_inline)) {
       const int n0 = nb * kBlk;
       if constexpr (kAhead) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
-        dd.load_full(k, Kn, oK);
-        dd.load_full(v, Vn, oV);
-        dd.load_full(gk, gKn, ogK);
-        dd.load_full(gv, gVn, ogV);
+        dd.load_full(to.k, Kn, oK);
+        dd.load_full(to.v, Vn, oV);
+        dd.load_full(to.gk, gKn, ogK);
+        dd.load_full(to.gv, gVn, ogV);
         if constexpr (LOADP) {
           pn[0] = load_frag_g<T>(Pn);
           pn[1] = load_frag_g<T>(Pn + 32);
         }
       } else {
-        dd.load_ragged(k, Kn, a.k.st, Tk_ - n0, D);
-        dd.load_ragged(v, Vn, a.v.st, Tk_ - n0, D);
-        dd.load_ragged(gk, gKn, a.gk.st, Tk_ - n0, D);
-        dd.load_ragged(gv, gVn, a.gv.st, Tk_ - n0, D);
+        dd.load_ragged(to.k, Kn, a.k.st, Tk_ - n0, D);
+        dd.load_ragged(to.v, Vn, a.v.st, Tk_ - n0, D);
+        dd.load_ragged(to.gk, gKn, a.gk.st, Tk_ - n0, D);
+        dd.load_ragged(to.gv, gVn, a.gv.st, Tk_ - n0, D);
         if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, Tk_);
         dma_wait();
       }
@@ -429,16 +432,16 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       __builtin_amdgcn_sched_barrier(0);
       if (nb + 1 < cr.t1) {
         if constexpr (P == 0)
-          dma_set(nb + 1, pK1, pV1, pgK1, pgV1);
+          dma_set(nb + 1, p1);
         else
-          dma_set(nb + 1, pK0, pV0, pgK0, pgV0);
+          dma_set(nb + 1, p0);
       }
       if constexpr (P == 0)
-        tile_body(nb, pK0, pV0, pgK0, pgV0, p);
+        tile_body(nb, p0.k, p0.v, p0.gk, p0.gv, p);
       else
-        tile_body(nb, pK1, pV1, pgK1, pgV1, p);
+        tile_body(nb, p1.k, p1.v, p1.gk, p1.gv, p);
     };
-    dma_set(cr.t0, pK0, pV0, pgK0, pgV0);
+    dma_set(cr.t0, p0);
     for (int nb = cr.t0; nb < cr.t1; nb += 2) {
       step(Parity<0>{}, nb);
       if (nb + 1 < cr.t1) step(Parity<1>{}, nb + 1);
@@ -451,7 +454,7 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       dd.offsets(ogV, a.gv.st);
       dma_tile(cr.t0, 0);
     } else {
-      load_tile(cr.t0);
+      if constexpr (M::kPrefetch) load_tile(cr.t0);
     }
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
       const int cur = kDma ? ((nb - cr.t0) & 1) : 0;
@@ -459,11 +462,12 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
         dma_wait();  // this wave's loads of tile nb (LDS tiles and P fragments)
         __syncthreads();  // everyone's, and everyone is done with the other buffer
       } else {
+        if constexpr (!M::kPrefetch) load_tile(nb);
         __syncthreads();
-        stage_store_tile<M>(s0, sK[0]);
-        stage_store_tile<M>(s1, sV[0]);
-        stage_store_tile<M>(s2, sgK[0]);
-        stage_store_tile<M>(s3, sgV[0]);
+        stage_store_tile<M>(s0, sr.k);
+        stage_store_tile<M>(s1, sr.v);
+        stage_store_tile<M>(s2, sr.gk);
+        stage_store_tile<M>(s3, sr.gv);
         __syncthreads();
       }
       Tile p;
@@ -472,11 +476,16 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       if (nb + 1 < cr.t1) {
         if constexpr (kDma)
           dma_tile(nb + 1, cur ^ 1);
-        else
+        else if constexpr (M::kPrefetch)
           load_tile(nb + 1);
       }
-      tile_body(nb, sK[cur], sV[cur], sgK[cur], sgV[cur], p);
+      tile_body(nb, sr.k + cur * M::kElems, sr.v + cur * M::kElems, sr.gk + cur * M::kElems, sr.gv + cur * M::kElems, p);
     }
+  }
+  if constexpr (GDO) {
+    if (has_nan<M>(e_acc + x_acc + d_acc, a1, a2, a3, a4, b1, b2, b3)) return true;
+  } else {
+    if (has_nan<M>(e_acc + x_acc + d_acc, a1, a2, a4)) return true;
   }
   const float Ev = group_sum(e_acc);
   const float Xv = kMfmaSums ? xs4[0] : group_sum(x_acc);
@@ -534,69 +543,77 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params 
       sc[2 * kBlk + rl] = Dv;
     }
   }
+  return false;
+}
+
+template <typename T, int D, bool LOADP, bool GDO, int XM, bool DQ>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_row(Params a) {
+  typedef typename Mm<T, D>::lds lds;
+  typedef GgRowTiles<T, D, GDO> Tiles;
+  constexpr int kE = Tiles::kBuf * Tiles::kE, kPE = Tiles::kPE;
+  __shared__ __align__(16) lds sK[kE];
+  __shared__ __align__(16) lds sV[kE];
+  __shared__ __align__(16) lds sgK[kE];
+  __shared__ __align__(16) lds sgV[kE];
+  __shared__ __align__(16) lds pK0[kPE];
+  __shared__ __align__(16) lds pV0[kPE];
+  __shared__ __align__(16) lds pgK0[kPE];
+  __shared__ __align__(16) lds pgV0[kPE];
+  __shared__ __align__(16) lds pK1[kPE];
+  __shared__ __align__(16) lds pV1[kPE];
+  __shared__ __align__(16) lds pgK1[kPE];
+  __shared__ __align__(16) lds pgV1[kPE];
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    typedef GgRowSet<typename P::lds> Set;
+    return gg_row<P, LOADP, GDO, XM, DQ>(
+        a, Set{tile_as<P>(sK), tile_as<P>(sV), tile_as<P>(sgK), tile_as<P>(sgV)},
+        Set{tile_as<P>(pK0), tile_as<P>(pV0), tile_as<P>(pgK0), tile_as<P>(pgV0)},
+        Set{tile_as<P>(pK1), tile_as<P>(pV1), tile_as<P>(pgK1), tile_as<P>(pgV1)});
+  });
 }
 
 // ---------------------------------------------------------------------------
-template <typename T, int D, bool LOADP, int XM>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params a, Params rowc, int nx) {
+template <typename M>
+struct GgColBufs {
+  typename M::lds *q, *gq, *dout;
+  typename M::T* p;
+  float* st;
+};
+
+// Column block and chunk of this workgroup, over the buffer sets b0 and b1.
+// True: has_nan.  16-bit types at D = 64 stream tiles straight into the two
+// sets (TileDma), which lie in distinct arrays with a compile-time role per
+// loop step; the rest stage them through registers into set 0.
+template <typename M, bool LOADP, int XM>
+__device__ __forceinline__ bool gg_col(Params a, Slot sl, GgColBufs<M> b0,
+                                       GgColBufs<M> b1) {
+  typedef typename M::T T;
+  constexpr int D = M::D;
   typedef Elem<T> E;
   typedef typename E::frag frag;
-  typedef Lds<T, D> L;
-  typedef Mm<T, D> M;
   typedef typename M::frag mfrag;
-  typedef typename M::lds lds;
-  typedef Lds<T, kBlk> LP;
-  // 16-bit types at D = 64 stream tiles straight into two LDS buffers
-  // (TileDma), set 0 and set 1, in distinct arrays with a compile-time role per
-  // loop step; the rest stage them through registers into set 0.
-  constexpr bool kDma = L::kSwizzle;
+  typedef GgColBufs<M> Bufs;
+  constexpr bool kDma = Lds<T, D>::kSwizzle;
   constexpr int kNS = LOADP ? 3 : 4;  // staged row statistics: D, E, F, then lse (recompute)
-  constexpr int kE1 = kDma ? M::kElems : 8;
-  constexpr int kP0 = LOADP ? LP::kRowElems : 8, kP1 = (LOADP && kDma) ? LP::kRowElems : 8;
-  __shared__ __align__(16) lds sQ0[M::kElems];
-  __shared__ __align__(16) lds sgQ0[M::kElems];
-  __shared__ __align__(16) lds sdO0[M::kElems];
-  __shared__ __align__(16) T sP0[kP0];
-  __shared__ __align__(16) float sS0[kNS * kBlk];
-  __shared__ __align__(16) lds sQ1[kE1];
-  __shared__ __align__(16) lds sgQ1[kE1];
-  __shared__ __align__(16) lds sdO1[kE1];
-  __shared__ __align__(16) T sP1[kP1];
-  __shared__ __align__(16) float sS1[kDma ? kNS * kBlk : 4];
-  struct Bufs {
-    lds *q, *gq, *dout;
-    T* p;
-    float* st;
-  };
   auto bufs = [&](auto par) __attribute__((always_inline)) -> Bufs {
     if constexpr (decltype(par)::value == 0)
-      return Bufs{sQ0, sgQ0, sdO0, sP0, sS0};
+      return b0;
     else
-      return Bufs{sQ1, sgQ1, sdO1, sP1, sS1};
+      return b1;
   };
 
   const int T_ = a.Tk;  // keys: the stationary rows
   const int Tq_ = a.T;
   const int nblk = (T_ + kBlk - 1) / kBlk;
-  const Slot sl = grid_slot();
-  // Workgroups past the first nx columns of the grid finish the preceding row
-  // launch's split blocks (GQ, GdO; E and F are already written), in the tail
-  // of this launch rather than in a launch of their own.
-  if (sl.x >= nx) {
-    if (rowc.gdout.p)
-      combine_gg_row_block<T, D, true>(rowc, sl.x - nx, sl.y, false);
-    else
-      combine_gg_row_block<T, D, false>(rowc, sl.x - nx, sl.y, false);
-    return;
-  }
   const Item it = launch_item<XM>(a, sl.x, nblk);
-  if (it.blk < 0) return;
+  if (it.blk < 0) return false;
   const int nb = it.blk, ch = it.ch;
   const int bh = sl.y, b = bh / a.H, h = bh % a.H;
   const Range rg = col_block_range(nb, nblk, Tq_, a.causal, XM ? a.win : 0, a.win_kind);
   const Chunk cr = chunk_of(rg.lo, rg.hi, ch, a.chunk);
-  if (ch >= cr.nch) return;
+  if (ch >= cr.nch) return false;
   const int n0 = nb * kBlk;
   const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, c = lane & 15, g = lane >> 4;
   const int cl = 16 * w + c;
@@ -789,20 +806,23 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
       if constexpr (LOADP) stage_load<T, kBlk>(sp, Pb + (int64_t)m0 * a.p.st + n0, a.p.st, Tq_ - m0, T_ - n0);
       stv = stat_load<kNS>(rs, ev, fv, lse, m0, Tq_ - m0);
     };
-    load_tile(cr.t0);
+    if constexpr (M::kPrefetch) load_tile(cr.t0);
     for (int mb = cr.t0; mb < cr.t1; ++mb) {
+      if constexpr (!M::kPrefetch) load_tile(mb);
       __syncthreads();
-      stage_store_tile<M>(s0, sQ0);
-      stage_store_tile<M>(s1, sgQ0);
-      stage_store_tile<M>(s2, sdO0);
-      if constexpr (LOADP) stage_store_rows<T, kBlk>(sp, sP0);
-      stat_store<kNS>(stv, sS0);
+      stage_store_tile<M>(s0, b0.q);
+      stage_store_tile<M>(s1, b0.gq);
+      stage_store_tile<M>(s2, b0.dout);
+      if constexpr (LOADP) stage_store_rows<T, kBlk>(sp, b0.p);
+      stat_store<kNS>(stv, b0.st);
       __syncthreads();
       take_bias(mb);
-      if (mb + 1 < cr.t1) load_tile(mb + 1);
+      if constexpr (M::kPrefetch)
+        if (mb + 1 < cr.t1) load_tile(mb + 1);
       compute(mb, bufs(Parity<0>{}));
     }
   }
+  if (has_nan<M>(0.f, acc_gk, acc_gv)) return true;
   // the accumulators hold -GK/s and -GV
   if (cr.nch == 1) {
     store_acc_rows<T, D>(at<T>(a.gk_out, b, h), a.gk_out.st, n, T_, cols_of<T, D>(a), acc_gk, -s);
@@ -817,6 +837,46 @@ __attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params 
     store_acc_partial<D>(base, cl, acc_gk);
     store_acc_partial<D>(base + kBlk * D, cl, acc_gv);
   }
+  return false;
+}
+
+template <typename T, int D, bool LOADP, int XM>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(GgWaves<T, D>::value))) void k_gg_col(Params a, Params rowc, int nx) {
+  typedef Mm<T, D> M;
+  typedef typename M::lds lds;
+  typedef Lds<T, kBlk> LP;
+  constexpr bool kDma = Lds<T, D>::kSwizzle;
+  constexpr int kNS = LOADP ? 3 : 4;
+  constexpr int kE1 = kDma ? M::kElems : 8;
+  constexpr int kP0 = LOADP ? LP::kRowElems : 8, kP1 = (LOADP && kDma) ? LP::kRowElems : 8;
+  __shared__ __align__(16) lds sQ0[M::kElems];
+  __shared__ __align__(16) lds sgQ0[M::kElems];
+  __shared__ __align__(16) lds sdO0[M::kElems];
+  __shared__ __align__(16) T sP0[kP0];
+  __shared__ __align__(16) float sS0[kNS * kBlk];
+  __shared__ __align__(16) lds sQ1[kE1];
+  __shared__ __align__(16) lds sgQ1[kE1];
+  __shared__ __align__(16) lds sdO1[kE1];
+  __shared__ __align__(16) T sP1[kP1];
+  __shared__ __align__(16) float sS1[kDma ? kNS * kBlk : 4];
+  const Slot sl = grid_slot();
+  // Workgroups past the first nx columns of the grid finish the preceding row
+  // launch's split blocks (GQ, GdO; E and F are already written), in the tail
+  // of this launch rather than in a launch of their own.
+  if (sl.x >= nx) {
+    if (rowc.gdout.p)
+      combine_gg_row_block<T, D, true>(rowc, sl.x - nx, sl.y, false);
+    else
+      combine_gg_row_block<T, D, false>(rowc, sl.x - nx, sl.y, false);
+    return;
+  }
+  repeat_unsplit<T, D>([&](auto m) __attribute__((always_inline)) {
+    typedef decltype(m) P;
+    return gg_col<P, LOADP, XM>(
+        a, sl, GgColBufs<P>{tile_as<P>(sQ0), tile_as<P>(sgQ0), tile_as<P>(sdO0), sP0, sS0},
+        GgColBufs<P>{tile_as<P>(sQ1), tile_as<P>(sgQ1), tile_as<P>(sdO1), sP1, sS1});
+  });
 }
 
 #if TTT_GG_COL8
