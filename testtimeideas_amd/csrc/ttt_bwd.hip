@@ -252,6 +252,10 @@ __device__ __forceinline__ bool bwd_dq(Params a, typename M::lds* sK0, typename 
     fetch_dma(cr.t0, RtBuf{0});
   else if constexpr (M::kPrefetch)
     fetch(cr.t0);
+  if constexpr (!kDma) {
+    zero_columns<M>(sK0, cols_of<T, D>(a));
+    zero_columns<M>(sV0, cols_of<T, D>(a));
+  }
   // Tile nb from buffer set `par`; `prefetch`: 1 fetch tile nb + 1, 2 fetch it
   // if it exists, 0 none.
   auto tile = [&](int nb, auto prefetch, auto par) __attribute__((always_inline)) {
@@ -262,8 +266,8 @@ __device__ __forceinline__ bool bwd_dq(Params a, typename M::lds* sK0, typename 
     } else {
       if constexpr (!M::kPrefetch) fetch(nb);
       __syncthreads();
-      stage_store_tile<M>(stK, sK0);
-      stage_store_tile<M>(stV, sV0);
+      stage_store_tile<M>(stK, sK0, cols_of<T, D>(a));
+      stage_store_tile<M>(stV, sV0, cols_of<T, D>(a));
       __syncthreads();
     }
     const lds* cK = set_k(par);
@@ -549,6 +553,10 @@ __device__ __forceinline__ bool bwd_dkdv(Params a, Slot sl, DkdvBufs<M> b0, Dkdv
     dma_tile(cr.t0, Parity<0>{});
   else if constexpr (M::kPrefetch)
     load_tile(cr.t0);
+  if constexpr (!kDma) {
+    zero_columns<M>(b0.dout, cols_of<T, D>(a));
+    if constexpr (kNeedQ) zero_columns<M>(b0.q, cols_of<T, D>(a));
+  }
   // Tile mb from buffer set `par`; `prefetch`: 1 fetch tile mb + 1, 2 fetch it
   // if it exists, 0 none.
   auto tile = [&](int mb, auto prefetch, auto par) __attribute__((always_inline)) {
@@ -570,8 +578,8 @@ __device__ __forceinline__ bool bwd_dkdv(Params a, Slot sl, DkdvBufs<M> b0, Dkdv
     } else {
       if constexpr (!M::kPrefetch) load_tile(mb);
       __syncthreads();
-      stage_store_tile<M>(stdO, b0.dout);
-      if constexpr (kNeedQ) stage_store_tile<M>(stQ, b0.q);
+      stage_store_tile<M>(stdO, b0.dout, cols_of<T, D>(a));
+      if constexpr (kNeedQ) stage_store_tile<M>(stQ, b0.q, cols_of<T, D>(a));
       if constexpr (LOADP) stage_store_rows<T, kBlk>(stP, b0.p);
       if constexpr (kNS > 0) stat_store<kNS>(stv, b0.st);
       __syncthreads();
@@ -728,10 +736,11 @@ __device__ __forceinline__ bool bwd_rowsum(Params a, typename M::lds* sV) {
   const int scol = stage_col<T, D>(cols_of<T, D>(a));
   Stage<T, D> stV;
   stage_load_at<T, D>(stV, V + (int64_t)rg.lo * kBlk * a.v.st, a.v.st, Tk_ - rg.lo * kBlk, scol);
+  zero_columns<M>(sV, cols_of<T, D>(a));
   for (int nb = rg.lo; nb < rg.hi; ++nb) {
     const int n0 = nb * kBlk;
     __syncthreads();
-    stage_store_tile<M>(stV, sV);
+    stage_store_tile<M>(stV, sV, cols_of<T, D>(a));
     __syncthreads();
     if (nb + 1 < rg.hi) stage_load_at<T, D>(stV, V + (int64_t)(n0 + kBlk) * a.v.st, a.v.st, Tk_ - n0 - kBlk, scol);
     frag pr[2];

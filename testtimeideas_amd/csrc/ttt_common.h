@@ -71,10 +71,11 @@ struct Params {
   int Tk;
   // Columns of every [B,H,T,*] row, a multiple of 8, at most the kernel's head
   // dim D.  Stationary fragments read as zero past them, so nothing past them
-  // reaches a score; streamed tiles repeat chunk 0 there, and the columns that
-  // gives an output are not stored.  So a head dim of 80 runs the D = 128
-  // kernels on its own rows: padding copies took two launches per operand
-  // (b2 h8 T1000 d80 bf16 causal, forward and backward 100 -> 69 us).
+  // reaches a score; streamed tiles hold zeros there too (an infinity would
+  // make a NaN of the zero it meets; split products: stage_store_tile), and an
+  // output's are not stored.  So a head dim of 80 runs the D = 128 kernels on
+  // its own rows: padding copies took two launches per operand (b2 h8 T1000
+  // d80 bf16 causal, forward and backward 100 -> 69 us).
   int d;
   int causal;
   float scale;       // s
@@ -903,8 +904,8 @@ __device__ __forceinline__ u32x4 load16(const void* p) {
 }
 
 // Load a 64 x NCOL tile whose element [0][0] is at g (row stride ld).  Columns
-// past cols_valid of an operand's rows are never consumed (Params::d); of P's
-// and the statistics' they are masked.
+// past cols_valid of an operand's rows (Params::d) stay in registers
+// (stage_store_tile); P's are masked.
 // Every thread issues the same unconditional loads on every tile: rows at or
 // beyond rows_valid repeat row rows_valid-1 and 16-byte chunks starting at or
 // beyond cols_valid repeat chunk 0, and a chunk that straddles cols_valid is
@@ -1061,17 +1062,23 @@ __device__ __forceinline__ void stage_store_rows(const Stage<T, NCOL>& st, T* ld
   }
 }
 
-// The same into an MFMA tile of M (split types: each 16-byte chunk of four
-// values becomes half a 16-byte chunk of each plane).
+// The same for an operand's rows of ncols columns into an MFMA tile of M (split
+// types: each 16-byte chunk of four values becomes half a 16-byte chunk of
+// each plane).  Chunks past ncols are not stored: they hold the zeros of
+// zero_columns, written once per walk (zeros selected on every store took a
+// b2 h8 T1000 d80 bf16 forward and backward from 69 to 74 us).  Split types
+// store what was loaded, chunk 0: finite, it meets zeros, and an infinity there
+// makes a NaN, for which the walk is repeated (repeat_unsplit).
 template <typename M>
-__device__ __forceinline__ void stage_store_tile(const Stage<typename M::T, M::D>& st, typename M::lds* lds) {
+__device__ __forceinline__ void stage_store_tile(const Stage<typename M::T, M::D>& st, typename M::lds* lds,
+                                                 int ncols) {
+  typedef Stage<typename M::T, M::D> S;
+  typedef typename M::L L;
+  const int tid = threadIdx.x;
+  const int col = (tid % S::kChunksPerRow) * S::kChunk;
   if constexpr (!M::kSplit) {
-    stage_store_rows<typename M::T, M::D>(st, lds);
+    if (col < ncols) stage_store_rows<typename M::T, M::D>(st, lds);
   } else {
-    typedef Stage<typename M::T, M::D> S;
-    typedef typename M::L L;
-    const int tid = threadIdx.x;
-    const int col = (tid % S::kChunksPerRow) * S::kChunk;
 #pragma unroll
     for (int ps = 0; ps < S::kPasses; ++ps) {
       const int r = 2 * (tid / S::kChunksPerRow + ps * S::kPairsPerPass);
@@ -1094,6 +1101,18 @@ __device__ __forceinline__ void stage_store_tile(const Stage<typename M::T, M::D
       }
     }
   }
+}
+
+// Zeros in an MFMA tile's columns from ncols on (a multiple of 8), which
+// stage_store_tile leaves alone; before the first barrier of a walk.
+template <typename M>
+__device__ __forceinline__ void zero_columns(typename M::lds* lds, int ncols) {
+  if (M::kSplit || ncols >= M::D) return;  // uniform
+  typedef typename M::L L;
+  constexpr int kEl = 16 / (int)sizeof(typename M::lds);
+  const int r = threadIdx.x % kBlk;
+  for (int col = ncols + (int)(threadIdx.x / kBlk) * kEl; col < M::D; col += kThreads / kBlk * kEl)
+    *reinterpret_cast<u32x4*>(lds + L::off(r, col)) = u32x4{0u, 0u, 0u, 0u};
 }
 
 // ---------------------------------------------------------------------------
@@ -1525,13 +1544,18 @@ __device__ __forceinline__ void stat_read8(float* v, const float* lds, int st, i
 // The loads bypass registers and
 // complete on vmcnt; readers wait for them (dma_wait) and meet at a barrier.
 // As with stage_load, rows at or beyond rows_valid and chunks at or beyond
-// cols_valid read from row 0 / chunk 0 (finite data that consumers mask).
+// cols_valid read from row 0 / chunk 0 (data that consumers mask); chunks past
+// the rows' own columns (Params::d) are filled with zeros.
 // ---------------------------------------------------------------------------
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 // Word 3 of a raw buffer resource on gfx9-family parts (gfx950): 32-bit
 // data format, no swizzle, no index stride.
 constexpr int kBufWord3 = 0x00020000;
+// The range of such a resource (bytes), and the offset of a fetch past it: the
+// buffer returns zeros there and reads no memory.  Tile offsets lie below.
+constexpr uint32_t kBufRange = 0xFFFFFFF0u;
+constexpr int kBufPast = (int)kBufRange;
 
 template <typename T, int NCOL, int NW = 4>
 struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>::kSwizzle
@@ -1542,7 +1566,7 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
   static_assert(kPerWave * NW == kInstr, "tile shape");
   int row[kPerWave], col[kPerWave];  // this lane's logical row and first column per instruction
   int wslice;                         // 1024 * wave index, uniform
-  // ncols: columns the rows have; chunks past them repeat chunk 0.
+  // ncols: columns the rows have; chunks past them (col -1) are zeros.
   __device__ __forceinline__ explicit TileDma(int ncols) {
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     wslice = 1024 * __builtin_amdgcn_readfirstlane(w);
@@ -1552,14 +1576,17 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
       const int r = byte / kRowBytes;
       row[q] = r;
       const int c = (((byte % kRowBytes) / 16) ^ L::swz(r)) * L::kChunk;
-      col[q] = c < ncols ? c : 0;
+      col[q] = c < ncols ? c : -1;
     }
   }
-  // Byte offsets (row stride ld elements) of this lane's fetches for an
-  // interior tile.
+  // Byte offset of the fetch at row r and column c (row stride ld elements).
+  static __device__ __forceinline__ int offset_of(int r, int c, int64_t ld) {
+    return c < 0 ? kBufPast : (int)(((int64_t)r * ld + c) * (int64_t)sizeof(T));
+  }
+  // Byte offsets of this lane's fetches for an interior tile.
   __device__ __forceinline__ void offsets(int* off, int64_t ld) const {
 #pragma unroll
-    for (int q = 0; q < kPerWave; ++q) off[q] = (int)(((int64_t)row[q] * ld + col[q]) * (int64_t)sizeof(T));
+    for (int q = 0; q < kPerWave; ++q) off[q] = offset_of(row[q], col[q], ld);
   }
   // Issue the loads of the tile at g into lds.  `off` from offsets(); ragged
   // tiles (uniform) recompute them with row/column clamping.
@@ -1576,16 +1603,11 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
   // extension next to each load; hoisted out of a loop, it leaves a 64-bit
   // per-lane address (two registers per load, a 64-bit add per issue, and a
   // fresh register whose reuse soon after the load makes the compiler wait
-  // for the load to complete).  The resource does no range checking.
+  // for the load to complete).  The resource's range check only makes the
+  // zeros past the rows' columns.
   __device__ __forceinline__ void load_full(T* lds, const T* g, const int* off) const {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const __amdgpu_buffer_rsrc_t r =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(g), (short)0, (int)0xFFFFFFFF, kBufWord3);
 #pragma unroll
-    for (int q = 0; q < kPerWave; ++q)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          r, (lds_void_t*)(reinterpret_cast<char*>(lds) + wslice + 1024 * NW * q), 16, off[q], 0, 0, 0);
-#endif
+    for (int q = 0; q < kPerWave; ++q) issue(lds, g, off[q], 0, q);
   }
   // A ragged tile's clamped offsets live in temporaries: callers wait for
   // these loads (dma_wait) before leaving the ragged branch, since with loads
@@ -1596,7 +1618,7 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
     for (int q = 0; q < kPerWave; ++q) {
       const int r = row[q] < rows_valid ? row[q] : 0;
       const int c = col[q] < cols_valid ? col[q] : 0;
-      issue(lds, g, (int)(((int64_t)r * ld + c) * (int64_t)sizeof(T)), q);
+      issue(lds, g, offset_of(r, c, ld), 0, q);
     }
   }
   // The compact form (the eight-wave kernels): instruction q of a lane reads
@@ -1606,18 +1628,12 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
   static constexpr int kRowStep = 1024 * NW / kRowBytes;
   __device__ __forceinline__ int offset0(int64_t ld) const {
     static_assert(kRowStep % 16 == 0, "rows of one lane's instructions share the permutation");
-    return (int)(((int64_t)row[0] * ld + col[0]) * (int64_t)sizeof(T));
+    return offset_of(row[0], col[0], ld);
   }
   __device__ __forceinline__ void load_full0(T* lds, const T* g, int off0, int64_t ld) const {
-#if defined(__HIP_DEVICE_COMPILE__)
-    const __amdgpu_buffer_rsrc_t r =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(g), (short)0, (int)0xFFFFFFFF, kBufWord3);
     const int step = (int)(kRowStep * ld * (int64_t)sizeof(T));
 #pragma unroll
-    for (int q = 0; q < kPerWave; ++q)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          r, (lds_void_t*)(reinterpret_cast<char*>(lds) + wslice + 1024 * NW * q), 16, off0, q * step, 0, 0);
-#endif
+    for (int q = 0; q < kPerWave; ++q) issue(lds, g, off0, q * step, q);
   }
   __device__ __forceinline__ void load_ragged0(T* lds, const T* g, int64_t ld, int rows_valid, int cols_valid) const {
 #pragma unroll
@@ -1625,15 +1641,17 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
       const int rq = row[0] + kRowStep * q;
       const int r = rq < rows_valid ? rq : 0;
       const int c = col[0] < cols_valid ? col[0] : 0;
-      issue(lds, g, (int)(((int64_t)r * ld + c) * (int64_t)sizeof(T)), q);
+      issue(lds, g, offset_of(r, c, ld), 0, q);
     }
   }
-  // One 16-byte-per-lane load into the 1 KB slice (wave + NW q) of lds, in the
-  // saddr + voffset form: uniform base g, unsigned 32-bit byte offset.
-  __device__ __forceinline__ void issue(T* lds, const T* g, int byte_off, int q) const {
-#if defined(__HIP_DEVICE_COMPILE__)  // the builtin exists only for the gfx950 target
-    __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(g) + (uint32_t)byte_off,
-                                     (lds_void_t*)(reinterpret_cast<char*>(lds) + wslice + 1024 * NW * q), 16, 0, 0);
+  // One 16-byte-per-lane load into the 1 KB slice (wave + NW q) of lds: uniform
+  // base g and step, unsigned 32-bit byte offset per lane.
+  __device__ __forceinline__ void issue(T* lds, const T* g, int byte_off, int step, int q) const {
+#if defined(__HIP_DEVICE_COMPILE__)  // the builtins exist only for the gfx950 target
+    const __amdgpu_buffer_rsrc_t r =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(g), (short)0, (int)kBufRange, kBufWord3);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        r, (lds_void_t*)(reinterpret_cast<char*>(lds) + wslice + 1024 * NW * q), 16, byte_off, step, 0, 0);
 #endif
   }
 };

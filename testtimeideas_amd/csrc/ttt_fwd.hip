@@ -324,12 +324,14 @@ __device__ __forceinline__ bool fwd_online(Params a, typename M::lds* sK, typena
       if (nb + 1 < cr.t1) step(Parity<1>{}, nb + 1);
     }
   } else {
+    zero_columns<M>(sK, cols_of<T, D>(a));
+    zero_columns<M>(sV, cols_of<T, D>(a));
     if constexpr (M::kPrefetch) load_kv(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
       if constexpr (!M::kPrefetch) load_kv(nb);
       __syncthreads();
-      stage_store_tile<M>(stK, sK);
-      stage_store_tile<M>(stV, sV);
+      stage_store_tile<M>(stK, sK, cols_of<T, D>(a));
+      stage_store_tile<M>(stV, sV, cols_of<T, D>(a));
       __syncthreads();
       take_bias(nb);
       if constexpr (M::kPrefetch)
@@ -823,12 +825,14 @@ __device__ __forceinline__ bool fwd_stats(Params a, typename M::lds* sK, typenam
 #pragma unroll
       for (int i = 0; i < R; ++i) load_k(nb + i, stK[i]);
     };
+#pragma unroll
+    for (int i = 0; i < R; ++i) zero_columns<M>(sK + i * M::kElems, cols_of<T, D>(a));
     if constexpr (M::kPrefetch) load_round(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; nb += R) {
       if constexpr (!M::kPrefetch) load_round(nb);
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < R; ++i) stage_store_tile<M>(stK[i], sK + i * M::kElems);
+      for (int i = 0; i < R; ++i) stage_store_tile<M>(stK[i], sK + i * M::kElems, cols_of<T, D>(a));
       __syncthreads();
       if constexpr (M::kPrefetch)
         if (nb + R < cr.t1) load_round(nb + R);
@@ -1134,12 +1138,14 @@ __device__ __forceinline__ bool fwd_p(Params a, typename M::lds* sK, typename M:
     }
     flush();
   } else {
+    zero_columns<M>(sK, cols_of<T, D>(a));
+    zero_columns<M>(sV, cols_of<T, D>(a));
     if constexpr (M::kPrefetch) load_kv(cr.t0);
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
       if constexpr (!M::kPrefetch) load_kv(nb);
       __syncthreads();
-      stage_store_tile<M>(stK, sK);
-      stage_store_tile<M>(stV, sV);
+      stage_store_tile<M>(stK, sK, cols_of<T, D>(a));
+      stage_store_tile<M>(stV, sV, cols_of<T, D>(a));
       __syncthreads();
       if constexpr (M::kPrefetch)
         if (nb + 1 < cr.t1) load_kv(nb + 1);

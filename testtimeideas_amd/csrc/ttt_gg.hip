@@ -454,6 +454,10 @@ __device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
       dd.offsets(ogV, a.gv.st);
       dma_tile(cr.t0, 0);
     } else {
+      zero_columns<M>(sr.k, cols_of<T, D>(a));
+      zero_columns<M>(sr.v, cols_of<T, D>(a));
+      zero_columns<M>(sr.gk, cols_of<T, D>(a));
+      zero_columns<M>(sr.gv, cols_of<T, D>(a));
       if constexpr (M::kPrefetch) load_tile(cr.t0);
     }
     for (int nb = cr.t0; nb < cr.t1; ++nb) {
@@ -464,10 +468,10 @@ __device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
       } else {
         if constexpr (!M::kPrefetch) load_tile(nb);
         __syncthreads();
-        stage_store_tile<M>(s0, sr.k);
-        stage_store_tile<M>(s1, sr.v);
-        stage_store_tile<M>(s2, sr.gk);
-        stage_store_tile<M>(s3, sr.gv);
+        stage_store_tile<M>(s0, sr.k, cols_of<T, D>(a));
+        stage_store_tile<M>(s1, sr.v, cols_of<T, D>(a));
+        stage_store_tile<M>(s2, sr.gk, cols_of<T, D>(a));
+        stage_store_tile<M>(s3, sr.gv, cols_of<T, D>(a));
         __syncthreads();
       }
       Tile p;
@@ -806,13 +810,16 @@ __device__ __forceinline__ bool gg_col(Params a, Slot sl, GgColBufs<M> b0,
       if constexpr (LOADP) stage_load<T, kBlk>(sp, Pb + (int64_t)m0 * a.p.st + n0, a.p.st, Tq_ - m0, T_ - n0);
       stv = stat_load<kNS>(rs, ev, fv, lse, m0, Tq_ - m0);
     };
+    zero_columns<M>(b0.q, cols_of<T, D>(a));
+    zero_columns<M>(b0.gq, cols_of<T, D>(a));
+    zero_columns<M>(b0.dout, cols_of<T, D>(a));
     if constexpr (M::kPrefetch) load_tile(cr.t0);
     for (int mb = cr.t0; mb < cr.t1; ++mb) {
       if constexpr (!M::kPrefetch) load_tile(mb);
       __syncthreads();
-      stage_store_tile<M>(s0, b0.q);
-      stage_store_tile<M>(s1, b0.gq);
-      stage_store_tile<M>(s2, b0.dout);
+      stage_store_tile<M>(s0, b0.q, cols_of<T, D>(a));
+      stage_store_tile<M>(s1, b0.gq, cols_of<T, D>(a));
+      stage_store_tile<M>(s2, b0.dout, cols_of<T, D>(a));
       if constexpr (LOADP) stage_store_rows<T, kBlk>(sp, b0.p);
       stat_store<kNS>(stv, b0.st);
       __syncthreads();
