@@ -179,6 +179,11 @@ int64_t ttt_attn_workspace_size_shape(const ttt_problem* pr, const ttt_shape* sh
 int ttt_attn_split_info(const ttt_problem* pr, int32_t entry, int32_t load_p, int32_t want_gdout,
                         int32_t* chunk, int32_t* nchunk_max, int64_t* slots);
 
+/* The same for a *_shape entry point (shape NULL: square). */
+int ttt_attn_split_info_shape(const ttt_problem* pr, const ttt_shape* shape, int32_t entry,
+                              int32_t load_p, int32_t want_gdout, int32_t* chunk,
+                              int32_t* nchunk_max, int64_t* slots);
+
 /*
  * The chunk that grid column `column` (0 <= column < nblk * ceil(nblk /
  * chunk)) of a split plain-causal slice runs: block (in launch order: block i
@@ -267,6 +272,13 @@ int ttt_attn_bwd_dq(const ttt_problem* pr, const ttt_view* q,
                     const ttt_view* dq, void* workspace, int64_t workspace_bytes,
                     void* stream);
 
+/* ttt_attn_bwd_dq with a ttt_shape (NULL: square). */
+int ttt_attn_bwd_dq_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                          const ttt_view* k, const ttt_view* v, const ttt_view* o,
+                          const ttt_view* dout, const float* lse, const ttt_view* p,
+                          const float* rowsum_in, float* rowsum_out, const ttt_view* dq,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+
 /*
  * dK and dV (column-block kernel), from P (p != NULL) or recomputed from lse.
  * dk may be NULL: then only dV = P^T*dO is computed and rowsum is not read.
@@ -282,6 +294,13 @@ int ttt_attn_bwd_dkdv(const ttt_problem* pr, const ttt_view* q,
                       const ttt_view* p, const float* rowsum,
                       const ttt_view* dk, const ttt_view* dv, void* workspace,
                       int64_t workspace_bytes, void* stream);
+
+/* ttt_attn_bwd_dkdv with a ttt_shape (NULL: square). */
+int ttt_attn_bwd_dkdv_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                            const ttt_view* k, const ttt_view* v, const ttt_view* dout,
+                            const float* lse, const ttt_view* p, const float* rowsum,
+                            const ttt_view* dk, const ttt_view* dv, void* workspace,
+                            int64_t workspace_bytes, void* stream);
 
 /*
  * Full first backward in one call: the work of ttt_attn_bwd_dq (computing D
@@ -336,6 +355,15 @@ int ttt_attn_gg_row(const ttt_problem* pr, const ttt_view* q,
                     const ttt_view* gdout, float* e_out, float* f_out,
                     void* workspace, int64_t workspace_bytes, void* stream);
 
+/* ttt_attn_gg_row with a ttt_shape (NULL: square). */
+int ttt_attn_gg_row_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                          const ttt_view* k, const ttt_view* v, const ttt_view* dout,
+                          const float* lse, const ttt_view* p, const float* rowsum,
+                          const ttt_view* dq, const ttt_view* gq, const ttt_view* gk,
+                          const ttt_view* gv, const ttt_view* gq_out, const ttt_view* gdout,
+                          float* e_out, float* f_out, void* workspace, int64_t workspace_bytes,
+                          void* stream);
+
 /*
  * Double backward, column-block pass: GK and GV, reading E and F from
  * ttt_attn_gg_row.
@@ -350,6 +378,15 @@ int ttt_attn_gg_col(const ttt_problem* pr, const ttt_view* q,
                     const ttt_view* gv, const ttt_view* gk_out,
                     const ttt_view* gv_out, void* workspace,
                     int64_t workspace_bytes, void* stream);
+
+/* ttt_attn_gg_col with a ttt_shape (NULL: square). */
+int ttt_attn_gg_col_shape(const ttt_problem* pr, const ttt_shape* shape, const ttt_view* q,
+                          const ttt_view* k, const ttt_view* v, const ttt_view* dout,
+                          const float* lse, const ttt_view* p, const float* rowsum,
+                          const float* e_in, const float* f_in, const ttt_view* gq,
+                          const ttt_view* gk, const ttt_view* gv, const ttt_view* gk_out,
+                          const ttt_view* gv_out, void* workspace, int64_t workspace_bytes,
+                          void* stream);
 
 /*
  * Full double backward in one call: the work of ttt_attn_gg_row (with dq as

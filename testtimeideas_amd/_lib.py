@@ -64,6 +64,10 @@ class _Problem(ctypes.Structure):
     ]
 
 
+class _Shape(ctypes.Structure):
+    _fields_ = [("keys", ctypes.c_int64), ("cols", ctypes.c_int64)]
+
+
 # ttt_window_kind (include/ttt_attn.h)
 WINDOW_SLIDING, WINDOW_LOCAL = 0, 1
 
@@ -111,6 +115,11 @@ _SIGS = {
                             _VP] + _ST,
 }
 
+# The entry points that also take a ttt_shape, after the problem
+_SHAPED = ("ttt_attn_fwd", "ttt_attn_bwd_dq", "ttt_attn_bwd_dkdv", "ttt_attn_bwd", "ttt_attn_gg_row",
+           "ttt_attn_gg_col", "ttt_attn_gg")
+_SIGS.update({name + "_shape": [_P(_Problem), _P(_Shape)] + _SIGS[name][1:] for name in _SHAPED})
+
 # ttt_entry codes (include/ttt_attn.h)
 ENTRY_FWD, ENTRY_FWD_P, ENTRY_BWD_DQ, ENTRY_BWD_DKDV, ENTRY_BWD, ENTRY_GG_ROW, ENTRY_GG_COL, ENTRY_GG = range(8)
 
@@ -137,9 +146,13 @@ def load() -> ctypes.CDLL:
     lib.ttt_version.restype = ctypes.c_int
     lib.ttt_attn_workspace_size.argtypes = [_P(_Problem), ctypes.c_int32, ctypes.c_int32]
     lib.ttt_attn_workspace_size.restype = ctypes.c_int64
-    lib.ttt_attn_split_info.argtypes = [_P(_Problem), ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
-                                        _P(ctypes.c_int32), _P(ctypes.c_int32), _P(ctypes.c_int64)]
+    lib.ttt_attn_workspace_size_shape.argtypes = [_P(_Problem), _P(_Shape), ctypes.c_int32, ctypes.c_int32]
+    lib.ttt_attn_workspace_size_shape.restype = ctypes.c_int64
+    info = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _P(ctypes.c_int32), _P(ctypes.c_int32), _P(ctypes.c_int64)]
+    lib.ttt_attn_split_info.argtypes = [_P(_Problem)] + info
     lib.ttt_attn_split_info.restype = ctypes.c_int
+    lib.ttt_attn_split_info_shape.argtypes = [_P(_Problem), _P(_Shape)] + info
+    lib.ttt_attn_split_info_shape.restype = ctypes.c_int
     lib.ttt_attn_launch_item.argtypes = [ctypes.c_int32, ctypes.c_int32, ctypes.c_int32, _P(ctypes.c_int32),
                                          _P(ctypes.c_int32)]
     lib.ttt_attn_launch_item.restype = ctypes.c_int
@@ -218,6 +231,11 @@ def _timed(name: str, *args) -> None:
     _timed_call(name, _call, name, *args)
 
 
+def _timed_shape(name: str, *args) -> None:
+    """The *_shape form of entry point `name`, timed as `name`."""
+    _timed_call(name, _call, name + "_shape", *args)
+
+
 def mean_ms(rec: Dict[str, List[Tuple[torch.cuda.Event, torch.cuda.Event]]]) -> Dict[str, float]:
     return {k: sum(a.elapsed_time(b) for a, b in v) / len(v) for k, v in rec.items() if v}
 
@@ -249,17 +267,10 @@ def padded_head_dim(d: int) -> int:
 
 
 def native_head_dim(d: int, dtype: torch.dtype) -> bool:
-    """The fused entry points take rows of d columns as they are (the kernels
-    compute 64 or 128 columns and leave those past d alone; in fp32 only the
-    64-column kernels do)."""
+    """The kernels take rows of d columns as they are (they compute 64 or 128
+    columns and leave those past d alone; in fp32 only the 64-column kernels
+    do)."""
     return d % 8 == 0 and (0 < d <= 64 or d == 128 or (64 < d < 128 and dtype != torch.float32))
-
-
-def _one_call(q: torch.Tensor, k: torch.Tensor) -> bool:
-    """The problem runs through the fused entry points only: key and query
-    counts differ, or the head dim is not one that the per-kernel entries
-    take.  Such problems are not autotuned."""
-    return k.shape[2] != q.shape[2] or q.shape[3] not in (64, 128)
 
 
 def _kernel_ok(t: torch.Tensor) -> bool:
@@ -378,25 +389,34 @@ def _problem(x: torch.Tensor, mask, scale: float, split: Optional[int] = None, r
                     _split_chunk if split is None else int(split), int(m.window), int(m.window_kind), bv, int(rows))
 
 
-def _split_for(entry: int, x: torch.Tensor, m, scale: float, load_p: bool, gdo: bool, run) -> int:
+def _shaped(q: torch.Tensor, k: torch.Tensor, mask, scale: float, split: int, rows: int = 0) -> Tuple[_Problem, _Shape]:
+    """The problem of q [B,H,Tq,d] and k [B,H,Tk,d] for the *_shape entry
+    points: the head dim the kernels compute, and d and Tk in the shape."""
+    pr = _problem(q, mask, scale, split, rows)
+    d = q.shape[3]
+    pr.head_dim = 64 if d <= 64 else 128 if d <= 128 else d
+    return pr, _Shape(k.shape[2], d)
+
+
+def _split_for(entry: int, x: torch.Tensor, k: torch.Tensor, m, scale: float, load_p: bool, gdo: bool, run) -> int:
     """The split to launch kernel family `entry` with: a split forced by
     ``split_chunk``, else the autotuned one (``autotune``; `run(c)` launches
     the call with split c), else 0, the library's choice."""
     if _split_chunk or not autotune.enabled():
         return _split_chunk
-    key = (entry, x.dtype, m.causal, tuple(x.shape), int(m.window), int(m.window_kind), m.bias is not None,
-           bool(load_p), bool(gdo))
+    key = (entry, x.dtype, m.causal, tuple(x.shape), k.shape[2], int(m.window), int(m.window_kind),
+           m.bias is not None, bool(load_p), bool(gdo))
 
     def pick():
-        pr = _problem(x, m, scale, 0)
-        c0 = split_info(pr, entry, load_p, gdo)[0]
+        pr, sh = _shaped(x, k, m, scale, 0)
+        c0 = split_info(pr, entry, load_p, gdo, sh)[0]
         pr.split_chunk = 1 << 30  # clipped to the longest walk
-        return c0, split_info(pr, entry, load_p, gdo)[0]
+        return c0, split_info(pr, entry, load_p, gdo, sh)[0]
 
     return autotune.chunk(key, pick, run)
 
 
-def _fwd_config(x: torch.Tensor, m, scale: float, run) -> Tuple[int, int]:
+def _fwd_config(x: torch.Tensor, k: torch.Tensor, m, scale: float, run) -> Tuple[int, int]:
     """(block_rows, split) of the O + LSE forward: (0, split_chunk) when a
     split is forced, (0, 0) -- the library's choice -- with tuning off, else
     the fastest of the library's choice and, for each block height the
@@ -405,25 +425,26 @@ def _fwd_config(x: torch.Tensor, m, scale: float, run) -> Tuple[int, int]:
     split))`; (0, 0) again when the library's choice wins."""
     if _block_rows or _split_chunk or not autotune.enabled():
         return _block_rows, _split_chunk
-    key = ("fwd_rows", x.dtype, m.causal, tuple(x.shape), int(m.window), int(m.window_kind), m.bias is not None)
+    key = ("fwd_rows", x.dtype, m.causal, tuple(x.shape), k.shape[2], int(m.window), int(m.window_kind),
+           m.bias is not None)
     t = x.shape[2]
     pairs_ok = x.dtype != torch.float32 and m.bias is None and not (0 < int(m.window) < t)
 
     def options():
         opts = []
         for rows in ((64, 128) if pairs_ok else (64,)):
-            pr = _problem(x, m, scale, 0, rows)
-            c0 = split_info(pr, ENTRY_FWD, False)[0]
+            pr, sh = _shaped(x, k, m, scale, 0, rows)
+            c0 = split_info(pr, ENTRY_FWD, False, shape=sh)[0]
             pr.split_chunk = 1 << 30  # clipped to the longest walk
-            lmax = split_info(pr, ENTRY_FWD, False)[0]
+            lmax = split_info(pr, ENTRY_FWD, False, shape=sh)[0]
             for c in autotune.candidates(c0, lmax):
                 pr.split_chunk = c
-                ce = split_info(pr, ENTRY_FWD, False)[0]  # as launched (causal row pairs: even)
+                ce = split_info(pr, ENTRY_FWD, False, shape=sh)[0]  # as launched (causal row pairs: even)
                 if (rows, ce) not in opts:
                     opts.append((rows, ce))
-        pr = _problem(x, m, scale, 0, 0)
+        pr, sh = _shaped(x, k, m, scale, 0, 0)
         lib_rows = 128 if pairs_ok and x.shape[3] <= 64 else 64
-        return (lib_rows, split_info(pr, ENTRY_FWD, False)[0]), opts
+        return (lib_rows, split_info(pr, ENTRY_FWD, False, shape=sh)[0]), opts
 
     return autotune.choose(key, options, run)
 
@@ -466,21 +487,26 @@ def prep_bias(bias: torch.Tensor, b: int, h: int, t: int, dtype: torch.dtype, de
 _ws_sizes: Dict[tuple, int] = {}
 
 
-def workspace_bytes(pr: _Problem, entry: int, gdo: bool = False) -> int:
-    key = (pr.dtype, pr.causal, pr.batch, pr.heads, pr.seqlen, pr.head_dim, pr.split_chunk, pr.window,
-           pr.window_kind, pr.bias.data is not None, entry, gdo)
+def workspace_bytes(pr: _Problem, entry: int, gdo: bool = False, shape: Optional[_Shape] = None) -> int:
+    keys = shape.keys if shape is not None else pr.seqlen
+    key = (pr.dtype, pr.causal, pr.batch, pr.heads, pr.seqlen, keys, pr.head_dim, pr.split_chunk, pr.window,
+           pr.window_kind, pr.block_rows, pr.bias.data is not None, entry, gdo)
     n = _ws_sizes.get(key)
     if n is None:
-        n = int(load().ttt_attn_workspace_size(ctypes.byref(pr), entry, 1 if gdo else 0))
+        n = int(load().ttt_attn_workspace_size_shape(ctypes.byref(pr), _ref(shape), entry, 1 if gdo else 0))
         if n < 0:
             raise RuntimeError(f"ttt_attn_workspace_size: {load().ttt_last_error().decode(errors='replace')}")
         _ws_sizes[key] = n
     return n
 
 
-def _workspace(pr: _Problem, entry: int, device, gdo: bool = False):
+def _ref(shape: Optional[_Shape]):
+    return None if shape is None else ctypes.byref(shape)
+
+
+def _workspace(pr: _Problem, entry: int, device, gdo: bool = False, shape: Optional[_Shape] = None):
     """(pointer, bytes, tensor) of a fresh workspace from torch's caching allocator."""
-    n = workspace_bytes(pr, entry, gdo)
+    n = workspace_bytes(pr, entry, gdo, shape)
     if n == 0:
         return None, 0, None
     buf = torch.empty(n, dtype=torch.uint8, device=device)
@@ -501,13 +527,15 @@ def _rows_readable(x: torch.Tensor) -> bool:
     return last * x.element_size() <= x.untyped_storage().nbytes()
 
 
-def alloc_p(like: torch.Tensor) -> torch.Tensor:
-    """[B,H,T,T] P buffer whose rows start on 16-byte boundaries and hold T
-    rounded up to 8 elements."""
+def alloc_p(like: torch.Tensor, tk: Optional[int] = None) -> torch.Tensor:
+    """[B,H,T,tk] P buffer (tk: T unless given) whose rows start on 16-byte
+    boundaries and hold tk rounded up to 8 elements."""
     b, h, t, _ = like.shape
-    tp = (t + ROW_READ - 1) // ROW_READ * ROW_READ
+    if tk is None:
+        tk = t
+    tp = (tk + ROW_READ - 1) // ROW_READ * ROW_READ
     buf = torch.empty((b, h, t, tp), dtype=like.dtype, device=like.device)
-    return buf if tp == t else buf[..., :t]
+    return buf if tp == tk else buf[..., :tk]
 
 
 def _stats(like: torch.Tensor) -> torch.Tensor:
@@ -547,9 +575,6 @@ def fwd(q, k, v, mask, scale: float, want_p: bool):
     if library_choice():
         return tuple(ext().fwd(q, k, v, m.causal, float(scale), bool(want_p), 0, int(m.window), int(m.window_kind),
                                m.bias, 0))
-    if _one_call(q, k):
-        return tuple(_timed_call("ttt_attn_fwd", ext().fwd, q, k, v, m.causal, float(scale), bool(want_p),
-                                 _split_chunk, int(m.window), int(m.window_kind), m.bias, _block_rows))
     ent = ENTRY_FWD_P if want_p else ENTRY_FWD
 
     def run(c, rows=0):
@@ -557,18 +582,18 @@ def fwd(q, k, v, mask, scale: float, want_p: bool):
                          rows)
 
     if want_p:
-        rows, c = 0, _split_for(ent, q, m, scale, want_p, False, run)
+        rows, c = 0, _split_for(ent, q, k, m, scale, want_p, False, run)
     else:
-        rows, c = _fwd_config(q, m, scale, lambda rc: run(rc[1], rc[0]))
+        rows, c = _fwd_config(q, k, m, scale, lambda rc: run(rc[1], rc[0]))
     if _timing is None:
         return tuple(run(c, rows))
     q, k, v = _ready(q), _ready(k), _ready(v)
     o = _empty_like_out(q)
     lse = _stats(q)
-    p = alloc_p(q) if want_p else None
-    pr = _problem(q, mask, scale, c, rows)
-    wp, wn, _wbuf = _workspace(pr, ENTRY_FWD_P if want_p else ENTRY_FWD, q.device)
-    _timed("ttt_attn_fwd", ctypes.byref(pr), _view(q), _view(k), _view(v), _view(o), lse.data_ptr(),
+    p = alloc_p(q, k.shape[2]) if want_p else None
+    pr, sh = _shaped(q, k, mask, scale, c, rows)
+    wp, wn, _wbuf = _workspace(pr, ENTRY_FWD_P if want_p else ENTRY_FWD, q.device, shape=sh)
+    _timed_shape("ttt_attn_fwd", ctypes.byref(pr), ctypes.byref(sh), _view(q), _view(k), _view(v), _view(o), lse.data_ptr(),
            _view(p), wp, wn, _stream())
     return o, lse, p
 
@@ -584,16 +609,13 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
     if library_choice():
         return tuple(ext().bwd_fused(q, k, v, o, do, lse, p, m.causal, float(scale), int(m.window),
                                      int(m.window_kind), m.bias, 0))
-    if _one_call(q, k):
-        return tuple(_timed_call("ttt_attn_bwd", ext().bwd_fused, q, k, v, o, do, lse, p, m.causal, float(scale),
-                                 int(m.window), int(m.window_kind), m.bias, _split_chunk))
 
     def run(cq, ck):
         return ext().bwd(q, k, v, o, do, lse, p, m.causal, float(scale), cq, ck, int(m.window), int(m.window_kind),
                          m.bias)
 
-    cq = _split_for(ENTRY_BWD_DQ, q, m, scale, lp, False, lambda c: run(c, 0))
-    ck = _split_for(ENTRY_BWD_DKDV, q, m, scale, lp, False, lambda c: run(cq, c))
+    cq = _split_for(ENTRY_BWD_DQ, q, k, m, scale, lp, False, lambda c: run(c, 0))
+    ck = _split_for(ENTRY_BWD_DKDV, q, k, m, scale, lp, False, lambda c: run(cq, c))
     if _timing is None:
         if cq == 0 and ck == 0:
             return tuple(ext().bwd_fused(q, k, v, o, do, lse, p, m.causal, float(scale), int(m.window),
@@ -606,14 +628,14 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
     rowsum = _stats(q)
     st = _stream()
     lse_p = _fptr(lse)
-    pq = _problem(q, mask, scale, cq)
-    pk = _problem(q, mask, scale, ck)
-    wp, wn, _wbuf = _workspace(pq, ENTRY_BWD_DQ, q.device)
-    _timed("ttt_attn_bwd_dq", ctypes.byref(pq), _view(q), _view(k), _view(v), _view(o), _view(do), lse_p, _view(p),
-           None, rowsum.data_ptr(), _view(dq), wp, wn, st)
-    wp, wn, _wbuf2 = _workspace(pk, ENTRY_BWD_DKDV, q.device)
-    _timed("ttt_attn_bwd_dkdv", ctypes.byref(pk), _view(q), _view(k), _view(v), _view(do), lse_p, _view(p),
-           rowsum.data_ptr(), _view(dk), _view(dv), wp, wn, st)
+    pq, sh = _shaped(q, k, mask, scale, cq)
+    pk, _ = _shaped(q, k, mask, scale, ck)
+    wp, wn, _wbuf = _workspace(pq, ENTRY_BWD_DQ, q.device, shape=sh)
+    _timed_shape("ttt_attn_bwd_dq", ctypes.byref(pq), ctypes.byref(sh), _view(q), _view(k), _view(v), _view(o),
+                 _view(do), lse_p, _view(p), None, rowsum.data_ptr(), _view(dq), wp, wn, st)
+    wp, wn, _wbuf2 = _workspace(pk, ENTRY_BWD_DKDV, q.device, shape=sh)
+    _timed_shape("ttt_attn_bwd_dkdv", ctypes.byref(pk), ctypes.byref(sh), _view(q), _view(k), _view(v), _view(do),
+                 lse_p, _view(p), rowsum.data_ptr(), _view(dk), _view(dv), wp, wn, st)
     return dq, dk, dv, rowsum
 
 
@@ -685,17 +707,13 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
     if library_choice():
         return tuple(ext().gg_fused(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale),
                                     bool(want_gdo), int(m.window), int(m.window_kind), m.bias, 0))
-    if _one_call(q, k):
-        return tuple(_timed_call("ttt_attn_gg", ext().gg_fused, q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal,
-                                 float(scale), bool(want_gdo), int(m.window), int(m.window_kind), m.bias,
-                                 _split_chunk))
 
     def run(cr, cc):
         return ext().gg(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale), bool(want_gdo), cr,
                         cc, int(m.window), int(m.window_kind), m.bias)
 
-    cr = _split_for(ENTRY_GG_ROW, q, m, scale, lp, want_gdo, lambda c: run(c, 0))
-    cc = _split_for(ENTRY_GG_COL, q, m, scale, lp, False, lambda c: run(cr, c))
+    cr = _split_for(ENTRY_GG_ROW, q, k, m, scale, lp, want_gdo, lambda c: run(c, 0))
+    cc = _split_for(ENTRY_GG_COL, q, k, m, scale, lp, False, lambda c: run(cr, c))
     if _timing is None:
         if cr == 0 and cc == 0:
             return tuple(ext().gg_fused(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, m.causal, float(scale),
@@ -710,16 +728,16 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
     f = _stats(q)
     st = _stream()
     lse_p = _fptr(lse)
-    prr = _problem(q, mask, scale, cr)
-    prc = _problem(q, mask, scale, cc)
-    wp, wn, _wbuf = _workspace(prr, ENTRY_GG_ROW, q.device, want_gdo)
-    _timed("ttt_attn_gg_row", ctypes.byref(prr), _view(q), _view(k), _view(v), _view(do), lse_p, _view(p),
-           rowsum.data_ptr(), _view(dq), _view(gq), _view(gk), _view(gv), _view(gq_out), _view(gdo),
-           e.data_ptr(), f.data_ptr(), wp, wn, st)
-    wp, wn, _wbuf2 = _workspace(prc, ENTRY_GG_COL, q.device)
-    _timed("ttt_attn_gg_col", ctypes.byref(prc), _view(q), _view(k), _view(v), _view(do), lse_p, _view(p),
-           rowsum.data_ptr(), e.data_ptr(), f.data_ptr(), _view(gq), _view(gk), _view(gv), _view(gk_out),
-           _view(gv_out), wp, wn, st)
+    prr, sh = _shaped(q, k, mask, scale, cr)
+    prc, _ = _shaped(q, k, mask, scale, cc)
+    wp, wn, _wbuf = _workspace(prr, ENTRY_GG_ROW, q.device, want_gdo, sh)
+    _timed_shape("ttt_attn_gg_row", ctypes.byref(prr), ctypes.byref(sh), _view(q), _view(k), _view(v), _view(do),
+                 lse_p, _view(p), rowsum.data_ptr(), _view(dq), _view(gq), _view(gk), _view(gv), _view(gq_out),
+                 _view(gdo), e.data_ptr(), f.data_ptr(), wp, wn, st)
+    wp, wn, _wbuf2 = _workspace(prc, ENTRY_GG_COL, q.device, shape=sh)
+    _timed_shape("ttt_attn_gg_col", ctypes.byref(prc), ctypes.byref(sh), _view(q), _view(k), _view(v), _view(do),
+                 lse_p, _view(p), rowsum.data_ptr(), e.data_ptr(), f.data_ptr(), _view(gq), _view(gk), _view(gv),
+                 _view(gk_out), _view(gv_out), wp, wn, st)
     return gq_out, gk_out, gv_out, gdo
 
 
@@ -740,12 +758,13 @@ def gg_noalloc(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want
     return gq_out, gk_out, gv_out, gdo
 
 
-def split_info(pr: _Problem, entry: int, load_p: bool, gdo: bool = False) -> Tuple[int, int, int]:
+def split_info(pr: _Problem, entry: int, load_p: bool, gdo: bool = False,
+               shape: Optional[_Shape] = None) -> Tuple[int, int, int]:
     """(tiles per workgroup, chunks of the longest block, workgroup slots) the
     library would use for `entry` on the current device."""
     c, n, sl = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int64()
-    _call("ttt_attn_split_info", ctypes.byref(pr), entry, 1 if load_p else 0, 1 if gdo else 0, ctypes.byref(c),
-          ctypes.byref(n), ctypes.byref(sl))
+    _call("ttt_attn_split_info_shape", ctypes.byref(pr), _ref(shape), entry, 1 if load_p else 0, 1 if gdo else 0,
+          ctypes.byref(c), ctypes.byref(n), ctypes.byref(sl))
     return c.value, n.value, sl.value
 
 
@@ -786,7 +805,6 @@ def launch_timing(capacity: int = 4096):
 
 def exported_symbols() -> List[str]:
     """Names of the C entry points this binding uses (for ABI checks)."""
-    return list(_SIGS) + ["ttt_attn_workspace_size_shape", "ttt_attn_fwd_shape", "ttt_attn_bwd_shape",
-                          "ttt_attn_gg_shape", "ttt_last_error", "ttt_version", "ttt_attn_workspace_size",
-                          "ttt_attn_split_info",
-                          "ttt_attn_launch_item", "ttt_kernel_timing", "ttt_kernel_timing_read"]
+    return list(_SIGS) + ["ttt_last_error", "ttt_version", "ttt_attn_workspace_size", "ttt_attn_workspace_size_shape",
+                          "ttt_attn_split_info", "ttt_attn_split_info_shape", "ttt_attn_launch_item",
+                          "ttt_kernel_timing", "ttt_kernel_timing_read"]

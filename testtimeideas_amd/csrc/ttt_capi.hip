@@ -679,11 +679,16 @@ int64_t ttt_attn_workspace_size_shape(const ttt_problem* problem, const ttt_shap
   return entry_bytes(pr, entry, want_gdout != 0);
 }
 
-int ttt_attn_split_info(const ttt_problem* problem, int32_t entry, int32_t load_p, int32_t want_gdout, int32_t* chunk,
+int ttt_attn_split_info(const ttt_problem* pr, int32_t entry, int32_t load_p, int32_t want_gdout, int32_t* chunk,
                         int32_t* nchunk_max, int64_t* slots) {
+  return ttt_attn_split_info_shape(pr, nullptr, entry, load_p, want_gdout, chunk, nchunk_max, slots);
+}
+
+int ttt_attn_split_info_shape(const ttt_problem* problem, const ttt_shape* shape, int32_t entry, int32_t load_p,
+                              int32_t want_gdout, int32_t* chunk, int32_t* nchunk_max, int64_t* slots) {
   Prob prob;
   const Prob* pr = &prob;
-  TRY(make_prob(problem, nullptr, &prob));
+  TRY(make_prob(problem, shape, &prob));
   const int fam = family_of(pr, entry, want_gdout != 0);
   if (fam < 0) return fail(TTT_ERR_INVALID_ARGUMENT, "entry %d is not a single kernel family", entry);
   const Split s = choose_split(pr, fam, load_p != 0);
@@ -810,26 +815,42 @@ static int prep_dkdv(const Prob* pr, const ttt_view* q, const ttt_view* k, const
 
 extern "C" {
 
-int ttt_attn_bwd_dq(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_bwd_dq(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                     const ttt_view* o, const ttt_view* dout, const float* lse, const ttt_view* p,
                     const float* rowsum_in, float* rowsum_out, const ttt_view* dq, void* workspace,
                     int64_t workspace_bytes, void* stream) {
+  return ttt_attn_bwd_dq_shape(pr, nullptr, q, k, v, o, dout, lse, p, rowsum_in, rowsum_out, dq, workspace,
+                               workspace_bytes, stream);
+}
+
+int ttt_attn_bwd_dq_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                          const ttt_view* v, const ttt_view* o, const ttt_view* dout, const float* lse,
+                          const ttt_view* p, const float* rowsum_in, float* rowsum_out, const ttt_view* dq,
+                          void* workspace, int64_t workspace_bytes, void* stream) {
   Prob prob;
   const Prob* pr = &prob;
-  TRY(make_prob(problem, nullptr, &prob));
+  TRY(make_prob(problem, shape, &prob));
   ttt::Params a;
   TRY(prep_dq(pr, q, k, v, o, dout, lse, p, rowsum_in, rowsum_out, dq, workspace, workspace_bytes, &a));
   return launched(ttt::launch_bwd_dq(pr->dtype, (int)pr->head_dim, a, has_p(p), (hipStream_t)stream),
                   "ttt_attn_bwd_dq");
 }
 
-int ttt_attn_bwd_dkdv(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_bwd_dkdv(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                       const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                       const ttt_view* dk, const ttt_view* dv, void* workspace, int64_t workspace_bytes,
                       void* stream) {
+  return ttt_attn_bwd_dkdv_shape(pr, nullptr, q, k, v, dout, lse, p, rowsum, dk, dv, workspace, workspace_bytes,
+                                 stream);
+}
+
+int ttt_attn_bwd_dkdv_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                            const ttt_view* v, const ttt_view* dout, const float* lse, const ttt_view* p,
+                            const float* rowsum, const ttt_view* dk, const ttt_view* dv, void* workspace,
+                            int64_t workspace_bytes, void* stream) {
   Prob prob;
   const Prob* pr = &prob;
-  TRY(make_prob(problem, nullptr, &prob));
+  TRY(make_prob(problem, shape, &prob));
   ttt::Params a;
   TRY(prep_dkdv(pr, q, k, v, dout, lse, p, rowsum, dk, dv, workspace, workspace_bytes, &a));
   const bool dv_only = !(dk && dk->data);
@@ -977,26 +998,44 @@ static int gg_col_impl(const Prob* pr, const ttt_view* q, const ttt_view* k, con
                   "ttt_attn_gg_col");
 }
 
-int ttt_attn_gg_row(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_gg_row(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                     const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                     const ttt_view* dq, const ttt_view* gq, const ttt_view* gk, const ttt_view* gv,
                     const ttt_view* gq_out, const ttt_view* gdout, float* e_out, float* f_out, void* workspace,
                     int64_t workspace_bytes, void* stream) {
+  return ttt_attn_gg_row_shape(pr, nullptr, q, k, v, dout, lse, p, rowsum, dq, gq, gk, gv, gq_out, gdout, e_out,
+                               f_out, workspace, workspace_bytes, stream);
+}
+
+int ttt_attn_gg_row_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                          const ttt_view* v, const ttt_view* dout, const float* lse, const ttt_view* p,
+                          const float* rowsum, const ttt_view* dq, const ttt_view* gq, const ttt_view* gk,
+                          const ttt_view* gv, const ttt_view* gq_out, const ttt_view* gdout, float* e_out,
+                          float* f_out, void* workspace, int64_t workspace_bytes, void* stream) {
   Prob prob;
   const Prob* pr = &prob;
-  TRY(make_prob(problem, nullptr, &prob));
+  TRY(make_prob(problem, shape, &prob));
   return gg_row_impl(pr, q, k, v, dout, lse, p, rowsum, dq, gq, gk, gv, gq_out, gdout, e_out, f_out, workspace,
                      workspace_bytes, stream, -1);
 }
 
-int ttt_attn_gg_col(const ttt_problem* problem, const ttt_view* q, const ttt_view* k, const ttt_view* v,
+int ttt_attn_gg_col(const ttt_problem* pr, const ttt_view* q, const ttt_view* k, const ttt_view* v,
                     const ttt_view* dout, const float* lse, const ttt_view* p, const float* rowsum,
                     const float* e_in, const float* f_in, const ttt_view* gq, const ttt_view* gk,
                     const ttt_view* gv, const ttt_view* gk_out, const ttt_view* gv_out, void* workspace,
                     int64_t workspace_bytes, void* stream) {
+  return ttt_attn_gg_col_shape(pr, nullptr, q, k, v, dout, lse, p, rowsum, e_in, f_in, gq, gk, gv, gk_out, gv_out,
+                               workspace, workspace_bytes, stream);
+}
+
+int ttt_attn_gg_col_shape(const ttt_problem* problem, const ttt_shape* shape, const ttt_view* q, const ttt_view* k,
+                          const ttt_view* v, const ttt_view* dout, const float* lse, const ttt_view* p,
+                          const float* rowsum, const float* e_in, const float* f_in, const ttt_view* gq,
+                          const ttt_view* gk, const ttt_view* gv, const ttt_view* gk_out, const ttt_view* gv_out,
+                          void* workspace, int64_t workspace_bytes, void* stream) {
   Prob prob;
   const Prob* pr = &prob;
-  TRY(make_prob(problem, nullptr, &prob));
+  TRY(make_prob(problem, shape, &prob));
   return gg_col_impl(pr, q, k, v, dout, lse, p, rowsum, e_in, f_in, gq, gk, gv, gk_out, gv_out, workspace,
                      workspace_bytes, stream, -1);
 }

@@ -94,9 +94,8 @@ void check(int rc, const char* what) {
   TORCH_CHECK(rc == 0, what, " failed (status ", rc, "): ", ttt_last_error());
 }
 
-// The shape of q [B,H,Tq,d] against k [B,H,Tk,d], for the entry points that
-// take one; their problem's head_dim is d rounded up to 64 or 128 (the others
-// refuse rows of any other length).
+// The shape of q [B,H,Tq,d] against k [B,H,Tk,d]; its problem's head_dim is d
+// rounded up to 64 or 128.
 ttt_shape shape_of(const at::Tensor& q, const at::Tensor& k, ttt_problem* pr) {
   const int64_t d = q.size(3);
   pr->head_dim = d <= 64 ? 64 : d <= 128 ? 128 : d;
@@ -118,7 +117,7 @@ at::Tensor alloc_p(const at::Tensor& x, int64_t t) {
   return tp == t ? buf : buf.narrow(3, 0, t);
 }
 
-int64_t workspace_size(const ttt_problem& pr, int32_t entry, bool gdo, const ttt_shape* shape = nullptr) {
+int64_t workspace_size(const ttt_problem& pr, int32_t entry, bool gdo, const ttt_shape* shape) {
   const int64_t n = ttt_attn_workspace_size_shape(&pr, shape, entry, gdo ? 1 : 0);
   TORCH_CHECK(n >= 0, "ttt_attn_workspace_size failed: ", ttt_last_error());
   return n;
@@ -133,9 +132,9 @@ at::Tensor workspace(const ttt_problem& pr, const ttt_shape& shape, int32_t entr
 
 // One workspace for two launches in stream order (the second starts after
 // the first, its combine included, has finished with it).
-at::Tensor workspace2(const ttt_problem& pr0, int32_t e0, const ttt_problem& pr1, int32_t e1, bool gdo,
-                      const at::Tensor& like, int64_t* bytes) {
-  const int64_t n = std::max(workspace_size(pr0, e0, gdo), workspace_size(pr1, e1, gdo));
+at::Tensor workspace2(const ttt_problem& pr0, int32_t e0, const ttt_problem& pr1, int32_t e1,
+                      const ttt_shape& shape, bool gdo, const at::Tensor& like, int64_t* bytes) {
+  const int64_t n = std::max(workspace_size(pr0, e0, gdo, &shape), workspace_size(pr1, e1, gdo, &shape));
   *bytes = n;
   return n > 0 ? at::empty({n}, like.options().dtype(at::kByte)) : at::Tensor();
 }
@@ -172,32 +171,33 @@ std::vector<at::Tensor> bwd(const at::Tensor& q_, const at::Tensor& k_, const at
                             bool causal, double scale, int64_t split_dq, int64_t split_dkdv, int64_t window,
                             int64_t window_kind, const c10::optional<at::Tensor>& bias) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), o = ready(o_), dout = ready(dout_);
-  const ttt_problem pq = problem_of(q, causal, scale, split_dq, window, window_kind, bias);
-  const ttt_problem pk = problem_of(q, causal, scale, split_dkdv, window, window_kind, bias);
+  ttt_problem pq = problem_of(q, causal, scale, split_dq, window, window_kind, bias);
+  const ttt_shape sh = shape_of(q, k, &pq);
+  ttt_problem pk = pq;
+  pk.split_chunk = static_cast<int32_t>(split_dkdv);
   at::Tensor dq = at::empty(q.sizes(), q.options());
   at::Tensor dk = at::empty(k.sizes(), k.options());
   at::Tensor dv = at::empty(v.sizes(), v.options());
   at::Tensor rowsum = stats_of(q);
   int64_t wsb = 0;
-  at::Tensor ws = workspace2(pq, TTT_ENTRY_BWD_DQ, pk, TTT_ENTRY_BWD_DKDV, false, q, &wsb);
+  at::Tensor ws = workspace2(pq, TTT_ENTRY_BWD_DQ, pk, TTT_ENTRY_BWD_DKDV, sh, false, q, &wsb);
   const bool lp = p && p->defined();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
   const ttt_view vdq = view_of(dq), vdk = view_of(dk), vdv = view_of(dv);
   void* st = stream_of(q);
   float* rs = rowsum.data_ptr<float>();
-  check(ttt_attn_bwd_dq(&pq, &vq, &vk, &vv, &vo, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, nullptr, rs, &vdq,
-                        ptr_or_null(ws), wsb, st),
+  check(ttt_attn_bwd_dq_shape(&pq, &sh, &vq, &vk, &vv, &vo, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, nullptr,
+                              rs, &vdq, ptr_or_null(ws), wsb, st),
         "ttt_attn_bwd_dq");
-  check(ttt_attn_bwd_dkdv(&pk, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rs, &vdk, &vdv,
-                          ptr_or_null(ws), wsb, st),
+  check(ttt_attn_bwd_dkdv_shape(&pk, &sh, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rs, &vdk,
+                                &vdv, ptr_or_null(ws), wsb, st),
         "ttt_attn_bwd_dkdv");
   return {dq, dk, dv, rowsum};
 }
 
 // The same through ttt_attn_bwd, both families with one split (0: the
-// library's): the dK/dV launch also finishes dQ's split blocks.  Also for
-// fewer or more keys than queries (ttt_shape).
+// library's): the dK/dV launch also finishes dQ's split blocks.
 std::vector<at::Tensor> bwd_fused(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_,
                                   const at::Tensor& o_, const at::Tensor& dout_, const at::Tensor& lse,
                                   const c10::optional<at::Tensor>& p, bool causal, double scale, int64_t window,
@@ -232,15 +232,17 @@ std::vector<at::Tensor> gg(const at::Tensor& q_, const at::Tensor& k_, const at:
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), dout = ready(dout_);
   const at::Tensor gq = ready(gq_), gk = ready(gk_), gv = ready(gv_);
   const c10::optional<at::Tensor> dq = ready(dq_);
-  const ttt_problem pr = problem_of(q, causal, scale, split_row, window, window_kind, bias);
-  const ttt_problem pc = problem_of(q, causal, scale, split_col, window, window_kind, bias);
+  ttt_problem pr = problem_of(q, causal, scale, split_row, window, window_kind, bias);
+  const ttt_shape sh = shape_of(q, k, &pr);
+  ttt_problem pc = pr;
+  pc.split_chunk = static_cast<int32_t>(split_col);
   at::Tensor gq_out = at::empty(q.sizes(), q.options());
   at::Tensor gk_out = at::empty(k.sizes(), k.options());
   at::Tensor gv_out = at::empty(v.sizes(), v.options());
   at::Tensor gdo = want_gdo ? at::empty(dout.sizes(), dout.options()) : at::Tensor();
   at::Tensor e = stats_of(q), f = stats_of(q);
   int64_t wsb = 0;
-  at::Tensor ws = workspace2(pr, TTT_ENTRY_GG_ROW, pc, TTT_ENTRY_GG_COL, want_gdo, q, &wsb);
+  at::Tensor ws = workspace2(pr, TTT_ENTRY_GG_ROW, pc, TTT_ENTRY_GG_COL, sh, want_gdo, q, &wsb);
   const bool lp = p && p->defined();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
@@ -251,20 +253,19 @@ std::vector<at::Tensor> gg(const at::Tensor& q_, const at::Tensor& k_, const at:
   const ttt_view vdq = ldq ? view_of(*dq) : none_view();
   void* st = stream_of(q);
   const float* rs = rowsum.data_ptr<float>();
-  check(ttt_attn_gg_row(&pr, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rs,
-                        ldq ? &vdq : nullptr, &vgq, &vgk, &vgv, &ogq, want_gdo ? &ogdo : nullptr,
-                        e.data_ptr<float>(), f.data_ptr<float>(), ptr_or_null(ws), wsb, st),
+  check(ttt_attn_gg_row_shape(&pr, &sh, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rs,
+                              ldq ? &vdq : nullptr, &vgq, &vgk, &vgv, &ogq, want_gdo ? &ogdo : nullptr,
+                              e.data_ptr<float>(), f.data_ptr<float>(), ptr_or_null(ws), wsb, st),
         "ttt_attn_gg_row");
-  check(ttt_attn_gg_col(&pc, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rs,
-                        e.data_ptr<float>(), f.data_ptr<float>(), &vgq, &vgk, &vgv, &ogk, &ogv, ptr_or_null(ws), wsb,
-                        st),
+  check(ttt_attn_gg_col_shape(&pc, &sh, &vq, &vk, &vv, &vdo, lse.data_ptr<float>(), lp ? &vp : nullptr, rs,
+                              e.data_ptr<float>(), f.data_ptr<float>(), &vgq, &vgk, &vgv, &ogk, &ogv, ptr_or_null(ws),
+                              wsb, st),
         "ttt_attn_gg_col");
   return {gq_out, gk_out, gv_out, gdo};
 }
 
 // The same through ttt_attn_gg, both passes with one split (0: the library's):
-// the column launch also finishes the row pass's split blocks.  Also for
-// fewer or more keys than queries (ttt_shape).
+// the column launch also finishes the row pass's split blocks.
 std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_,
                                  const at::Tensor& dout_, const at::Tensor& lse, const c10::optional<at::Tensor>& p,
                                  const at::Tensor& rowsum, const c10::optional<at::Tensor>& dq_,
