@@ -178,7 +178,9 @@ def ext():
         spec = importlib.util.spec_from_file_location("testtimeideas_amd._ttt_torch", EXT_PATH)
         mod = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(mod)
+        mod.set_python_gg(_node_gg)
         _ext_mod = mod
+        _choice_changed()
     return _ext_mod
 
 
@@ -208,10 +210,12 @@ def kernel_timing():
     global _timing
     prev = _timing
     _timing = {}
+    _choice_changed()
     try:
         yield _timing
     finally:
         _timing = prev
+        _choice_changed()
 
 
 def _timed_call(name: str, fn, *args):
@@ -353,10 +357,12 @@ def split_chunk(n: int):
     global _split_chunk
     prev = _split_chunk
     _split_chunk = int(n)
+    _choice_changed()
     try:
         yield
     finally:
         _split_chunk = prev
+        _choice_changed()
 
 
 # Query rows per workgroup of the O + LSE forward (ttt_problem.block_rows);
@@ -372,10 +378,12 @@ def block_rows(n: int):
     global _block_rows
     prev = _block_rows
     _block_rows = int(n)
+    _choice_changed()
     try:
         yield
     finally:
         _block_rows = prev
+        _choice_changed()
 
 
 def _problem(x: torch.Tensor, mask, scale: float, split: Optional[int] = None, rows: int = 0) -> _Problem:
@@ -566,6 +574,15 @@ def library_choice() -> bool:
     return not _split_chunk and not _block_rows and _timing is None and not autotune.enabled()
 
 
+def _choice_changed() -> None:
+    """Tells the binding, whose autograd node does not ask (``bwd_graph``)."""
+    if _ext_mod is not None:
+        _ext_mod.set_library_choice(library_choice())
+
+
+autotune.on_change(_choice_changed)
+
+
 def fwd(q, k, v, mask, scale: float, want_p: bool):
     """Forward: O, LSE and (save_p) P.  Reference: TritonAttentionFn.forward,
     ttt_kernels/triton_attention.py:261-337 (P path :51-59, :270-273)."""
@@ -739,6 +756,11 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
                  lse_p, _view(p), rowsum.data_ptr(), e.data_ptr(), f.data_ptr(), _view(gq), _view(gk), _view(gv),
                  _view(gk_out), _view(gv_out), wp, wn, st)
     return gq_out, gk_out, gv_out, gdo
+
+
+def _node_gg(q, k, v, do, lse, p, rowsum, dq, gq, gk, gv, causal, scale, want_gdo, window, window_kind, bias):
+    """``gg`` for the binding's autograd node (``bwd_graph``)."""
+    return gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, Mask(causal, window, window_kind, bias), scale, want_gdo, dq=dq)
 
 
 def gg_noalloc(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bool, dq=None):

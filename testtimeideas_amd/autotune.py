@@ -33,9 +33,19 @@ _MIN_CHUNK = 4  # the library's smallest split (kMinChunk)
 _REPS = 3
 
 
+_listeners: List[Callable[[], None]] = []
+
+
+def on_change(fn: Callable[[], None]) -> None:
+    """Have `fn` called whenever tuning is switched on or off."""
+    _listeners.append(fn)
+
+
 def enable(on: bool = True) -> None:
     global _enabled
     _enabled = bool(on)
+    for fn in _listeners:
+        fn()
 
 
 def enabled() -> bool:

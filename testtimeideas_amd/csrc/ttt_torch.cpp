@@ -20,6 +20,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
+#include <atomic>
 #include <string>
 #include <cstring>
 #include <vector>
@@ -299,6 +300,17 @@ std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, con
   return {gq_out, gk_out, gv_out, gdo};
 }
 
+// What library_choice() of testtimeideas_amd/_lib.py would say (_lib.py sets it
+// whenever a split is forced, kernels are timed or tuning is switched), and its
+// gg (set once, when the module is loaded, and never released: graphs may
+// outlive the interpreter's modules).
+std::atomic<bool> g_library_choice{true};
+PyObject* g_python_gg = nullptr;
+
+void set_library_choice(bool on) { g_library_choice.store(on); }
+
+void set_python_gg(const py::function& gg) { g_python_gg = py::function(gg).release().ptr(); }
+
 // The first backward as a differentiable function of (q, k, v, dO), for
 // create_graph=True on operands that go to the kernels as they are; its
 // backward is the double backward.  The Python Function of the same role
@@ -306,7 +318,10 @@ std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, con
 // other call and says what is saved and why.  In C++ neither pass enters the
 // interpreter: a step at b1 h1 T64, where the host is all there is, takes 79
 // instead of 93 us of host time (73 instead of 89 with P recomputed), the
-// splits kept per thread (ttt_capi.hip) included.
+// splits kept per thread (ttt_capi.hip) included.  Only where a split is forced
+// or kernels are timed or tuned when the double backward runs does it go
+// through _lib.py's gg, whatever held at the first backward (asking _lib.py each
+// time took the step at T512 from 76 to 83 us).
 struct SavedForward {
   at::Tensor o, lse;
   c10::optional<at::Tensor> p, bias;
@@ -332,6 +347,20 @@ struct AttnBwd : public torch::autograd::Function<AttnBwd> {
     return {r[0], r[1], r[2]};
   }
 
+  // The double backward through _lib.py's gg, unless every launch is to take the
+  // library's choice.
+  static bool forced(std::vector<at::Tensor>* r, const torch::autograd::variable_list& s,
+                     const torch::autograd::variable_list& g, const c10::optional<at::Tensor>& p, bool causal,
+                     double scale, bool want_gdo, int64_t window, int64_t window_kind,
+                     const c10::optional<at::Tensor>& bias) {
+    if (g_library_choice.load()) return false;
+    py::gil_scoped_acquire gil;
+    const py::tuple out = py::handle(g_python_gg)(s[0], s[1], s[2], s[3], s[4], p, s[6], s[7], g[0], g[1], g[2],
+                                                  causal, scale, want_gdo, window, window_kind, bias);
+    for (const py::handle t : out) r->push_back(t.is_none() ? at::Tensor() : t.cast<at::Tensor>());
+    return true;
+  }
+
   static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
                                                  torch::autograd::variable_list g) {
     const bool twice = at::GradMode::is_enabled() &&
@@ -344,11 +373,14 @@ struct AttnBwd : public torch::autograd::Function<AttnBwd> {
         if (t.scalar_type() != s[0].scalar_type()) t = t.to(s[0].scalar_type());
       const bool want_gdo = ctx->needs_input_grad(3);
       const c10::optional<at::Tensor> p = s[5].defined() ? c10::make_optional(s[5]) : c10::nullopt;
-      std::vector<at::Tensor> r =
-          gg_fused(s[0], s[1], s[2], s[3], s[4], p, s[6], s[7], g[0], g[1], g[2],
-                   ctx->saved_data["causal"].toBool(), ctx->saved_data["scale"].toDouble(), want_gdo,
-                   ctx->saved_data["window"].toInt(), ctx->saved_data["window_kind"].toInt(),
-                   ctx->saved_data["bias"].toOptional<at::Tensor>(), 0);
+      const bool causal = ctx->saved_data["causal"].toBool();
+      const double scale = ctx->saved_data["scale"].toDouble();
+      const int64_t window = ctx->saved_data["window"].toInt(), window_kind = ctx->saved_data["window_kind"].toInt();
+      const c10::optional<at::Tensor> bias = ctx->saved_data["bias"].toOptional<at::Tensor>();
+      std::vector<at::Tensor> r;
+      if (!forced(&r, s, g, p, causal, scale, want_gdo, window, window_kind, bias))
+        r = gg_fused(s[0], s[1], s[2], s[3], s[4], p, s[6], s[7], g[0], g[1], g[2], causal, scale, want_gdo, window,
+                     window_kind, bias, 0);
       for (int i = 0; i < 4; ++i)
         out.push_back(ctx->needs_input_grad(i) ? r[i] : at::Tensor());
       out.emplace_back();  // the saved forward
@@ -386,6 +418,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bwd", &bwd, "first backward: (dQ, dK, dV, D)");
   m.def("bwd_fused", &bwd_fused, "first backward in one entry call: (dQ, dK, dV, D)");
   m.def("bwd_graph", &bwd_graph, "differentiable first backward: (dQ, dK, dV)");
+  m.def("set_library_choice", &set_library_choice, "whether bwd_graph's double backward takes the library's choice");
+  m.def("set_python_gg", &set_python_gg, "the Python layer's double backward, for every other case");
   m.def("gg", &gg, "double backward: (GQ, GK, GV, GdO or None)");
   m.def("gg_fused", &gg_fused, "double backward in one entry call: (GQ, GK, GV, GdO or None)");
 }

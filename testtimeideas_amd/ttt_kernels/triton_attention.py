@@ -108,9 +108,10 @@ def mode_kind(bwd_mode: str) -> str:
 
 class _AttnBwdFn(torch.autograd.Function):
     """First backward as a function of (q, k, v, dO); its backward is the
-    double backward.  For padded operands, and while a split is forced or
-    kernels are timed or tuned; other calls take the same Function in C++
-    (``bwd_graph`` of the binding).  The kernel-layout dQ is kept for it: the row pass of the
+    double backward.  For padded operands, and where a split is forced or
+    kernels are timed or tuned when the first backward runs; other calls take
+    the same Function in C++ (``bwd_graph`` of the binding).  In both, the
+    double backward takes what holds when it runs itself.  The kernel-layout dQ is kept for it: the row pass of the
     double backward reads dQ = s*(dS*K) instead of forming that product.
 
     `fwd` = (qp, kp, vp, op, lse, p, mask, scale, lay), the saved forward in
