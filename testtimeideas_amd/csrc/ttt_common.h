@@ -272,6 +272,13 @@ enum : int { kMaskNone = 0, kMaskWindow = 1, kMaskBias = 2 };
 template <typename T, int D>
 constexpr bool kBiasAhead = (sizeof(T) == 4) == (D == 64);
 
+// The fp32 D = 128 grad-grad row kernel fills its 512 registers: loaded at the
+// head of its step, a tile's bias makes it spill 74.  There each fragment is
+// loaded and used by itself: 494 registers, no spills (b2 h4 T1500 with key
+// padding: gg-row 561 -> 430 us, the step 1546 -> 1420).
+template <typename T, int D>
+constexpr bool kBiasLate = sizeof(T) == 4 && D == 128;
+
 // The column's chunk: causal_item for plain causal split slices (XM = kMaskNone),
 // else x % nblk, x / nblk (chunk index by chunk index, blocks in launch
 // order; columns past a block's chunks exit on their chunk test).
@@ -1742,6 +1749,22 @@ __device__ __forceinline__ void recompute_p_row(Tile& p, const typename Elem<T>:
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       p.set(kb, j, fast_exp2(XM == kMaskBias ? p.at(kb, j) - lse2 : p.at(kb, j) * sl2 - lse2));
+}
+
+// The same for the bias form with the tile's bias loaded here, one fragment at
+// a time (kBiasLate): brow, this lane's row of it.
+template <typename T>
+__device__ __forceinline__ void recompute_p_row_late(Tile& p, const T* brow, int n0, int T_, float lse2, float sl2) {
+  const int g = (threadIdx.x & 63) >> 4;
+  scale_scores(p, sl2);
+#pragma unroll
+  for (int kb = 0; kb < 2; ++kb) {
+    const int n = n0 + stream_index(kb, g, 0);
+    const typename Elem<T>::frag f = load_frag_g<T>(brow + (n < T_ ? n : 0));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p.set(kb, j, fast_exp2(p.at(kb, j) + Elem<T>::f32(f[j]) * kLog2e - lse2));
+    __builtin_amdgcn_sched_barrier(0);
+  }
 }
 
 // The same for a column-block tile: statistic `slot` of sS holds the streamed

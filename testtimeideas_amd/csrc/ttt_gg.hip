@@ -193,13 +193,13 @@ __device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
   constexpr bool kBias = XM == kMaskBias;
   static_assert(!(LOADP && kBias), "a saved P holds the bias");
   const T* brow = kBias ? at<const T>(a.bias, b, h) + (int64_t)(row_ok ? m : 0) * a.bias.st : nullptr;
-  constexpr bool kAhead = kBias && kBiasAhead<T, D>;
+  constexpr bool kAhead = kBias && kBiasAhead<T, D>, kLate = kBias && kBiasLate<T, D>;
   frag bn[2], bc[2];  // bias of the next tile and of this one
   auto take_bias = [&](int nb) __attribute__((always_inline)) {
     if constexpr (kAhead) {
       bc[0] = bn[0];
       bc[1] = bn[1];
-    } else if constexpr (kBias) {
+    } else if constexpr (kBias && !kLate) {
       load_p_frags<T>(bc, brow, nb * kBlk, Tk_);
       if constexpr (sizeof(T) == 2) __builtin_amdgcn_sched_barrier(0);  // see kBiasAhead
     }
@@ -317,7 +317,10 @@ __device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
     if constexpr (!LOADP) {
       p.zero();
       mm_d<M>(p, cK, qf);
-      recompute_p_row<T, XM>(p, bc, lse2, kSl2);
+      if constexpr (kLate)
+        recompute_p_row_late<T>(p, brow, n0, Tk_, lse2, kSl2);
+      else
+        recompute_p_row<T, XM>(p, bc, lse2, kSl2);
     }
     if (mk.tile(nb)) {
 #pragma unroll
