@@ -60,3 +60,10 @@ def test_splits_follow_the_shape():
                          (_lib.ENTRY_GG_COL, 10)):
         assert _lib.split_info(pr, entry, False, shape=_lib._Shape(128, 80))[0] == tiles
         assert _lib.split_info(pr, entry, False)[0] == 10
+
+
+def test_version_tells_the_entry_points_with_a_shape():
+    lib = _lib.load()
+    for name in _lib._SHAPED:
+        assert hasattr(lib, name + "_shape")
+    assert lib.ttt_version() >= 500

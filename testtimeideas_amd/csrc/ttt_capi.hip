@@ -619,7 +619,7 @@ void timing_mark(hipStream_t st, int tag, bool end) {
 
 extern "C" {
 
-int ttt_version(void) { return 400; }
+int ttt_version(void) { return 500; }
 
 int ttt_kernel_timing(int32_t capacity) {
   TimingPool& t = g_timing;
