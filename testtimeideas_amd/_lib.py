@@ -555,7 +555,7 @@ def prep_p(p: torch.Tensor) -> torch.Tensor:
     if p.stride(-1) == 1 and p.data_ptr() % 16 == 0 and all(
             (s * p.element_size()) % 16 == 0 for s in p.stride()[:-1]) and _rows_readable(p):
         return p
-    out = alloc_p(p)
+    out = alloc_p(p, p.shape[3])
     out.copy_(p)
     return out
 
@@ -639,6 +639,7 @@ def bwd(q, k, v, o, do, lse, p, mask, scale: float):
                                          int(m.window_kind), m.bias, 0))
         return tuple(run(cq, ck))
     q, k, v, o, do = _ready(q), _ready(k), _ready(v), _ready(o), _ready(do)
+    p = None if p is None else prep_p(p)
     dq = _empty_like_out(q)
     dk = _empty_like_out(k)
     dv = _empty_like_out(v)
@@ -737,6 +738,7 @@ def gg(q, k, v, do, lse, p, rowsum, gq, gk, gv, mask, scale: float, want_gdo: bo
                                         bool(want_gdo), int(m.window), int(m.window_kind), m.bias, 0))
         return tuple(run(cr, cc))
     q, k, v, do, dq, gq, gk, gv = (_ready(t) for t in (q, k, v, do, dq, gq, gk, gv))
+    p = None if p is None else prep_p(p)
     gq_out = _empty_like_out(q)
     gk_out = _empty_like_out(k)
     gv_out = _empty_like_out(v)

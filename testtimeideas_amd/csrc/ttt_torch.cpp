@@ -118,6 +118,21 @@ at::Tensor alloc_p(const at::Tensor& x, int64_t t) {
   return tp == t ? buf : buf.narrow(3, 0, t);
 }
 
+// P as the forward wrote it, or, where it came back from a saved-tensor hook
+// without the forward's row storage, a copy that has it.
+c10::optional<at::Tensor> ready_p(const c10::optional<at::Tensor>& p) {
+  if (!p || !p->defined()) return c10::nullopt;
+  const int64_t eb = p->element_size();
+  int64_t end = p->storage_offset() + (p->size(3) + 7) / 8 * 8;  // past the last element read
+  bool ok = p->stride(3) == 1 && reinterpret_cast<uintptr_t>(p->data_ptr()) % 16 == 0;
+  for (int i = 0; i < 3; ++i) {
+    ok = ok && (p->stride(i) * eb) % 16 == 0;
+    end += (p->size(i) - 1) * p->stride(i);
+  }
+  if (ok && end * eb <= static_cast<int64_t>(p->storage().nbytes())) return p;
+  return alloc_p(*p, p->size(3)).copy_(*p);
+}
+
 int64_t workspace_size(const ttt_problem& pr, int32_t entry, bool gdo, const ttt_shape* shape) {
   const int64_t n = ttt_attn_workspace_size_shape(&pr, shape, entry, gdo ? 1 : 0);
   TORCH_CHECK(n >= 0, "ttt_attn_workspace_size failed: ", ttt_last_error());
@@ -168,7 +183,7 @@ std::vector<at::Tensor> fwd(const at::Tensor& q_, const at::Tensor& k_, const at
 
 // First backward: (dQ, dK, dV, D).  split_dq, split_dkdv: each family's split.
 std::vector<at::Tensor> bwd(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_, const at::Tensor& o_,
-                            const at::Tensor& dout_, const at::Tensor& lse, const c10::optional<at::Tensor>& p,
+                            const at::Tensor& dout_, const at::Tensor& lse, const c10::optional<at::Tensor>& p_,
                             bool causal, double scale, int64_t split_dq, int64_t split_dkdv, int64_t window,
                             int64_t window_kind, const c10::optional<at::Tensor>& bias) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), o = ready(o_), dout = ready(dout_);
@@ -182,7 +197,8 @@ std::vector<at::Tensor> bwd(const at::Tensor& q_, const at::Tensor& k_, const at
   at::Tensor rowsum = stats_of(q);
   int64_t wsb = 0;
   at::Tensor ws = workspace2(pq, TTT_ENTRY_BWD_DQ, pk, TTT_ENTRY_BWD_DKDV, sh, false, q, &wsb);
-  const bool lp = p && p->defined();
+  const c10::optional<at::Tensor> p = ready_p(p_);
+  const bool lp = p.has_value();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
   const ttt_view vdq = view_of(dq), vdk = view_of(dk), vdv = view_of(dv);
@@ -201,7 +217,7 @@ std::vector<at::Tensor> bwd(const at::Tensor& q_, const at::Tensor& k_, const at
 // library's): the dK/dV launch also finishes dQ's split blocks.
 std::vector<at::Tensor> bwd_fused(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_,
                                   const at::Tensor& o_, const at::Tensor& dout_, const at::Tensor& lse,
-                                  const c10::optional<at::Tensor>& p, bool causal, double scale, int64_t window,
+                                  const c10::optional<at::Tensor>& p_, bool causal, double scale, int64_t window,
                                   int64_t window_kind, const c10::optional<at::Tensor>& bias, int64_t split) {
   const at::Tensor q = ready(q_), k = ready(k_), v = ready(v_), o = ready(o_), dout = ready(dout_);
   ttt_problem pr = problem_of(q, causal, scale, split, window, window_kind, bias);
@@ -212,7 +228,8 @@ std::vector<at::Tensor> bwd_fused(const at::Tensor& q_, const at::Tensor& k_, co
   at::Tensor rowsum = stats_of(q);
   int64_t wsb = 0;
   at::Tensor ws = workspace(pr, sh, TTT_ENTRY_BWD, false, q, &wsb);
-  const bool lp = p && p->defined();
+  const c10::optional<at::Tensor> p = ready_p(p_);
+  const bool lp = p.has_value();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vo = view_of(o), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
   const ttt_view vdq = view_of(dq), vdk = view_of(dk), vdv = view_of(dv);
@@ -225,7 +242,7 @@ std::vector<at::Tensor> bwd_fused(const at::Tensor& q_, const at::Tensor& k_, co
 // Double backward: (GQ, GK, GV, GdO or None).  dq: the first backward's dQ,
 // or None (ttt_attn_gg_row).
 std::vector<at::Tensor> gg(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_, const at::Tensor& dout_,
-                           const at::Tensor& lse, const c10::optional<at::Tensor>& p, const at::Tensor& rowsum,
+                           const at::Tensor& lse, const c10::optional<at::Tensor>& p_, const at::Tensor& rowsum,
                            const c10::optional<at::Tensor>& dq_, const at::Tensor& gq_, const at::Tensor& gk_,
                            const at::Tensor& gv_, bool causal, double scale, bool want_gdo, int64_t split_row,
                            int64_t split_col, int64_t window, int64_t window_kind,
@@ -244,7 +261,8 @@ std::vector<at::Tensor> gg(const at::Tensor& q_, const at::Tensor& k_, const at:
   at::Tensor e = stats_of(q), f = stats_of(q);
   int64_t wsb = 0;
   at::Tensor ws = workspace2(pr, TTT_ENTRY_GG_ROW, pc, TTT_ENTRY_GG_COL, sh, want_gdo, q, &wsb);
-  const bool lp = p && p->defined();
+  const c10::optional<at::Tensor> p = ready_p(p_);
+  const bool lp = p.has_value();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
   const ttt_view vgq = view_of(gq), vgk = view_of(gk), vgv = view_of(gv);
@@ -268,7 +286,7 @@ std::vector<at::Tensor> gg(const at::Tensor& q_, const at::Tensor& k_, const at:
 // The same through ttt_attn_gg, both passes with one split (0: the library's):
 // the column launch also finishes the row pass's split blocks.
 std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, const at::Tensor& v_,
-                                 const at::Tensor& dout_, const at::Tensor& lse, const c10::optional<at::Tensor>& p,
+                                 const at::Tensor& dout_, const at::Tensor& lse, const c10::optional<at::Tensor>& p_,
                                  const at::Tensor& rowsum, const c10::optional<at::Tensor>& dq_,
                                  const at::Tensor& gq_, const at::Tensor& gk_, const at::Tensor& gv_, bool causal,
                                  double scale, bool want_gdo, int64_t window, int64_t window_kind,
@@ -285,7 +303,8 @@ std::vector<at::Tensor> gg_fused(const at::Tensor& q_, const at::Tensor& k_, con
   at::Tensor e = stats_of(q), f = stats_of(q);
   int64_t wsb = 0;
   at::Tensor ws = workspace(pr, sh, TTT_ENTRY_GG, want_gdo, q, &wsb);
-  const bool lp = p && p->defined();
+  const c10::optional<at::Tensor> p = ready_p(p_);
+  const bool lp = p.has_value();
   const ttt_view vq = view_of(q), vk = view_of(k), vv = view_of(v), vdo = view_of(dout);
   const ttt_view vp = lp ? view_of(*p) : none_view();
   const ttt_view vgq = view_of(gq), vgk = view_of(gk), vgv = view_of(gv);
