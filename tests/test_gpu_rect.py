@@ -30,8 +30,6 @@ def _mask(kind, lq, lk, gen):
                                      (torch.float32, 128)])
 @pytest.mark.parametrize("mask", ["none", "padding", "full", "causal"])
 def test_rectangular_step(lq, lk, dtype, d, mask):
-    if lk == 1 and dtype != torch.float32:
-        pytest.skip("one key: differences of rounded 16-bit terms that cancel exactly, which only fp32 pins")
     gen = torch.Generator().manual_seed(lq * 1000 + lk)
     b, h = 2, 2
     rows = (lq, lk, lk, lq, lq, lk, lk)
@@ -43,6 +41,8 @@ def test_rectangular_step(lq, lk, dtype, d, mask):
     first = closed_form.backward(*n[:4], False, d ** -0.5, bias)
     second = closed_form.double_backward(*n, False, d ** -0.5, bias)
     want = [first[k] for k in ("o", "dq", "dk", "dv")] + [second[k] for k in ("gq", "gk", "gv", "gdo")]
+    # One key in 16 bits: dS, gS and gdP are differences of rounded terms that cancel exactly, which only fp32 pins.
+    cancel = ("dq", "dk", "gq", "gk", "gv") if lk == 1 and dtype != torch.float32 else ()
     dev = [x.cuda() for x in xs]
     for mode, split in (("recompute", 0), ("recompute", 1), ("save_p", 0), ("save_p", 2)):
         q, k, v, do = (x.clone().requires_grad_() for x in dev[:4])
@@ -57,6 +57,8 @@ def test_rectangular_step(lq, lk, dtype, d, mask):
             # cancel (|dP|, |gP| up to ~30, times a cotangent), of random sign, and dK and GK sum lq of them.
             # Elsewhere the key gradients sum up to 700 queries for few keys and reach 10 and more: fp32's bound is
             # then relative to the largest.
+            if name in cancel:
+                continue
             if dtype == torch.float32:
                 check_f32_scaled(f"{name} {mode} split {split}", a, w, MAX_ABS_32 * (lq ** 0.5 if lk == 1 else 1.0))
             else:
