@@ -85,3 +85,31 @@ def test_window_scales(scale, dtype, local, mode):
     for split in (0, 1):
         _check_step(xs, lambda q, k, v: windowed_attention(q, k, v, w, local=local, scale=scale, bwd_mode=mode), want,
                     f"split {split}", split)
+
+
+@pytest.mark.parametrize("t", [15, 17, 80, 97, 113, 129])  # last tiles of 15, 17, 16, 33, 49 and 1 keys
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("form", ["plain", "window", "bias"])
+@pytest.mark.parametrize("mode", ["recompute", "save_p"])
+def test_last_tiles_with_gdo(t, dtype, form, mode):
+    """Head dim 128, whose streamed tiles load in four slices of 16 keys."""
+    xs, gen = _inputs(t, t, 128, dtype)
+    bias = masks.local_bias(t, 16) if form == "window" else None
+    mask = torch.randn((1, 2, t, t), generator=gen).to(dtype) if form == "bias" else None
+    n = [to_np(x) for x in xs]
+    r = closed_form.double_backward(*n, False, 128 ** -0.5, to_np(mask) if mask is not None else bias)
+    q, k, v, do = (x.cuda().requires_grad_() for x in xs[:4])
+    if form == "window":
+        o = windowed_attention(q, k, v, 16, local=True, scale=128 ** -0.5, bwd_mode=mode)
+    else:
+        o = gradgrad_attention(q, k, v, None if mask is None else mask.cuda(), bwd_mode=mode)
+    first = torch.autograd.grad(o, (q, k, v), do, create_graph=True)
+    gx = [x.cuda() for x in xs[4:]]
+    second = torch.autograd.grad(first, (q, k, v, do), gx, retain_graph=True)
+    no_gdo = torch.autograd.grad(first, (q, k, v), gx)
+    for names, got in ((("gq", "gk", "gv", "gdo"), second), (("gq", "gk", "gv"), no_gdo)):
+        for name, a in zip(names, got):
+            if dtype == torch.float32:
+                check_f32_scaled(f"{name} {len(got)}", a, r[name])
+            else:
+                check(f"{name} {len(got)}", a, r[name], dtype)

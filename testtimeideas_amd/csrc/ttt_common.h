@@ -1628,9 +1628,9 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
       issue(lds, g, offset_of(r, c, ld), 0, q);
     }
   }
-  // The compact form (the eight-wave kernels): instruction q of a lane reads
-  // kRowStep rows below instruction 0 at the same column (the row step is a
-  // multiple of 16, so the chunk permutation is the same), so one per-lane
+  // The compact form (the D = 128 grad-grad kernels): instruction q of a lane
+  // reads kRowStep rows below instruction 0 at the same column (the row step is
+  // a multiple of 16, so the chunk permutation is the same), so one per-lane
   // offset per tensor suffices and the step goes into the uniform soffset.
   static constexpr int kRowStep = 1024 * NW / kRowBytes;
   __device__ __forceinline__ int offset0(int64_t ld) const {
@@ -1650,6 +1650,13 @@ struct TileDma {  // for the unpadded (chunk-permuted) layout only: Lds<T, NCOL>
       const int c = col[0] < cols_valid ? col[0] : 0;
       issue(lds, g, offset_of(r, c, ld), 0, q);
     }
+  }
+  // The same with zeros in the rows past rows_valid.
+  __device__ __forceinline__ void load_zero_past0(T* lds, const T* g, int off0, int64_t ld, int rows_valid) const {
+    const int step = (int)(kRowStep * ld * (int64_t)sizeof(T));
+#pragma unroll
+    for (int q = 0; q < kPerWave; ++q)
+      issue(lds, g, row[0] + kRowStep * q < rows_valid ? off0 : kBufPast, q * step, q);
   }
   // One 16-byte-per-lane load into the 1 KB slice (wave + NW q) of lds: uniform
   // base g and step, unsigned 32-bit byte offset per lane.

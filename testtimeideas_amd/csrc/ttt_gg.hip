@@ -321,6 +321,9 @@ __device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
         recompute_p_row_late<T>(p, brow, n0, Tk_, lse2, kSl2);
       else
         recompute_p_row<T, XM>(p, bc, lse2, kSl2);
+      // fp32 D = 128 with GdO: the products below start after P; scheduled into it,
+      // they spill more inside the loop (b2 h8 T1024 663 us, 792 without this).
+      if constexpr (GDO && sizeof(T) == 4 && D == 128 && !kLate) __builtin_amdgcn_sched_barrier(0);
     }
     if (mk.tile(nb)) {
 #pragma unroll
@@ -396,27 +399,55 @@ __device__ __forceinline__ bool gg_row(Params a, GgRowSet<typename M::lds> sr,
   };
 
   if constexpr (kPar) {
-    dd.offsets(oK, a.k.st);
-    dd.offsets(oV, a.v.st);
-    dd.offsets(ogK, a.gk.st);
-    dd.offsets(ogV, a.gv.st);
+    // At D = 128 the compact form: twelve registers fewer than an offset per
+    // fetch, of which the GdO kernels are short (they spill about 1 KB a lane).
+    // A ragged tile's rows past the last read row 0 with GdO and zeros
+    // otherwise: the windowed kernels are 0.6 us of 21 faster with zeros, the
+    // fp16 GdO ones up to 10 % slower.  MI355X, with GdO, P recomputed, offset
+    // per fetch -> compact: b2 h8 T1024 bf16 352 -> 307 us, window 256
+    // 98 -> 87; b1 h4 T2500 bf16 with a bias 859 -> 717, fp16 851 -> 697.
+    constexpr bool kCompact = D == 128;
+    auto offsets = [&](int* o, int64_t ld) __attribute__((always_inline)) {
+      if constexpr (kCompact)
+        o[0] = dd.offset0(ld);
+      else
+        dd.offsets(o, ld);
+    };
+    auto full = [&](lds* to, const T* from, const int* o, int64_t ld) __attribute__((always_inline)) {
+      if constexpr (kCompact)
+        dd.load_full0(to, from, o[0], ld);
+      else
+        dd.load_full(to, from, o);
+    };
+    auto ragged = [&](lds* to, const T* from, const int* o, int64_t ld, int rows) __attribute__((always_inline)) {
+      if constexpr (!kCompact)
+        dd.load_ragged(to, from, ld, rows, D);
+      else if constexpr (GDO)
+        dd.load_ragged0(to, from, ld, rows, D);
+      else
+        dd.load_zero_past0(to, from, o[0], ld, rows);
+    };
+    offsets(oK, a.k.st);
+    offsets(oV, a.v.st);
+    offsets(ogK, a.gk.st);
+    offsets(ogV, a.gv.st);
     auto dma_set = [&](int nb, const GgRowSet<T>& to) __attribute__((always_inline)) {
       const int n0 = nb * kBlk;
       if constexpr (kAhead) load_p_frags<T>(bn, brow, n0, Tk_);
       if (n0 + kBlk <= Tk_) {  // uniform: one test per tile for all four tiles and P
-        dd.load_full(to.k, Kn, oK);
-        dd.load_full(to.v, Vn, oV);
-        dd.load_full(to.gk, gKn, ogK);
-        dd.load_full(to.gv, gVn, ogV);
+        full(to.k, Kn, oK, a.k.st);
+        full(to.v, Vn, oV, a.v.st);
+        full(to.gk, gKn, ogK, a.gk.st);
+        full(to.gv, gVn, ogV, a.gv.st);
         if constexpr (LOADP) {
           pn[0] = load_frag_g<T>(Pn);
           pn[1] = load_frag_g<T>(Pn + 32);
         }
       } else {
-        dd.load_ragged(to.k, Kn, a.k.st, Tk_ - n0, D);
-        dd.load_ragged(to.v, Vn, a.v.st, Tk_ - n0, D);
-        dd.load_ragged(to.gk, gKn, a.gk.st, Tk_ - n0, D);
-        dd.load_ragged(to.gv, gVn, a.gv.st, Tk_ - n0, D);
+        ragged(to.k, Kn, oK, a.k.st, Tk_ - n0);
+        ragged(to.v, Vn, oV, a.v.st, Tk_ - n0);
+        ragged(to.gk, gKn, ogK, a.gk.st, Tk_ - n0);
+        ragged(to.gv, gVn, ogV, a.gv.st, Tk_ - n0);
         if constexpr (LOADP) load_p_frags<T>(pn, Pm, n0, Tk_);
         dma_wait();
       }
